@@ -445,7 +445,7 @@ def main():
     s.time_integration(args.prof_steps, sync=False)
     hip.sync()
     kern = {}
-    for name in ("cell_key", "cell_scatter", "cell_sort", "scan", "fill", "first_half", "pack", "permute", "iota",
+    for name in ("cell_key", "cell_scatter", "cell_rank", "scan", "fill", "first_half", "pack", "permute", "iota",
                  "nlist", "water_x", "water_a", "soil_x", "soil_a", "soil_ab", "water_b", "soil_b", "final_water",
                  "final_soil"):
         n, t = s.profile_get(name)

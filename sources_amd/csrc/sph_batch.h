@@ -110,7 +110,7 @@ SPHG_BATCH_BODY(BodyPermute, permute_multi_body)
 SPHG_BATCH_BODY(BodyScanTile, scan_tile_body)
 SPHG_BATCH_BODY(BodyCellKey, cell_key_body)
 SPHG_BATCH_BODY(BodyCellScatter, cell_scatter_t_body)
-SPHG_BATCH_BODY(BodyCellSort, cell_sort_t_body)
+SPHG_BATCH_BODY(BodyCellRank, cell_rank_body)
 SPHG_BATCH_BODY(BodyPackWater, pack_water_body)
 SPHG_BATCH_BODY(BodyPackSoil, pack_soil_body)
 SPHG_BATCH_BODY(BodyNlist, nlist_body)

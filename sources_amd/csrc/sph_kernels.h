@@ -180,21 +180,29 @@ __global__ void k_scatter(const T* src, T* dst, const int* idx, int n)
 // Exclusive scan of n ints in tiles of SCAN_TILE; out has n+1 entries.
 constexpr int SCAN_BLOCK = 256, SCAN_ITEMS = 8, SCAN_TILE = SCAN_BLOCK * SCAN_ITEMS;
 
+// Exclusive prefix of one int per thread over the workgroup, and the total:
+// wave prefixes by shuffles, then the wave totals through LDS (one barrier
+// before they are read, one before lds is reused).
 __device__ __forceinline__ int block_exclusive_scan(int v, int* lds, int& total)
 {
-    const int tid = threadIdx.x;
-    lds[tid] = v;
-    __syncthreads();
-    for (int off = 1; off < SCAN_BLOCK; off <<= 1) {
-        int t = (tid >= off) ? lds[tid - off] : 0;
-        __syncthreads();
-        lds[tid] += t;
-        __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int incl = v;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int t = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += t;
     }
-    const int incl = lds[tid];
-    total = lds[SCAN_BLOCK - 1];
+    if (lane == 63) lds[wave] = incl;
     __syncthreads();
-    return incl - v;
+    int before = 0;
+    total = 0;
+#pragma unroll
+    for (int w = 0; w < SCAN_BLOCK / 64; ++w) {
+        if (w < wave) before += lds[w];
+        total += lds[w];
+    }
+    __syncthreads();
+    return before + incl - v;
 }
 
 // clear (optional, the same array as in): zeroed after it is read, so that a
@@ -260,27 +268,24 @@ __global__ void k_scan_add(int* out, int n, const int* tile_sums, int ntiles)
 // ------------------------------------------------------------------------
 // Cell list: key + rank (counting sort), scatter, per-cell ordering.
 // ------------------------------------------------------------------------
-__device__ __forceinline__ void cell_key_body(int blk, DPhase P, Grid g, int* err)
+// Cell key of a position (0 with the error flag raised outside the geometry
+// box: grid_geom's range check, m_particles.f90:1131-1136).
+__device__ __forceinline__ int cell_key_of(const Grid& g, double x, double y, int* err)
 {
-    const int i = blk * blockDim.x + threadIdx.x;
-    const bool valid = i < P.n;
-    int key = -1;
-    if (valid) {
-        const double x = P.x[i], y = P.y[i];
-        int cx, cy;
-        grid_cell(g, x, y, cx, cy);
-        // grid_geom's range check (m_particles.f90:1131-1136): the grid spans the
-        // geometry box [x_mingeom, x_maxgeom] x [y_mingeom, y_maxgeom].
-        const bool bad = !(x >= g.x0 && x <= g.x1 && y >= g.y0 && y <= g.y1) || cx < 0 || cy < 0 ||
-                         cx >= g.ncx || cy >= g.ncy;
-        if (bad) atomicOr(err, 1);
-        key = bad ? 0 : cy * g.ncx + cx;
-        P.key[i] = key;
-    }
-    // Rank within the cell.  The state is kept in cell order, so lanes of a
-    // wave mostly hold runs of equal keys: the head lane of each run takes
-    // the run's slots with one atomic and the run's lanes share them out.  The
-    // rank order inside a cell is arbitrary; k_cell_sort fixes it.
+    int cx, cy;
+    grid_cell(g, x, y, cx, cy);
+    const bool bad = !(x >= g.x0 && x <= g.x1 && y >= g.y0 && y <= g.y1) || cx < 0 || cy < 0 ||
+                     cx >= g.ncx || cy >= g.ncy;
+    if (bad) atomicOr(err, 1);
+    return bad ? 0 : cy * g.ncx + cx;
+}
+
+// Arrival rank within the cell of the particle of each group of 1 << lg
+// lanes (all 64 lanes call; key -1: none).  Neighbouring lanes mostly hold
+// runs of equal keys: the head lane of each run takes the run's slots with
+// one atomic and the run's groups share them out.
+__device__ __forceinline__ int cell_slot_of(int* cell_count, int key, int lg)
+{
     const int lane = threadIdx.x & 63;
     const int prev = __shfl_up(key, 1, 64);
     const bool head = lane == 0 || prev != key;
@@ -290,9 +295,21 @@ __device__ __forceinline__ void cell_key_body(int blk, DPhase P, Grid g, int* er
     const uint64_t after = heads & ~upto;
     const int end = after ? __ffsll((long long)after) - 1 : 64;
     int base = 0;
-    if (head && key >= 0) base = atomicAdd(&P.cell_count[key], end - start);
+    if (head && key >= 0) base = atomicAdd(&cell_count[key], (end - start) >> lg);
     base = __shfl(base, start, 64);
-    if (valid) P.slot[i] = base + (lane - start);
+    return base + ((lane - start) >> lg);
+}
+
+__device__ __forceinline__ void cell_key_body(int blk, DPhase P, Grid g, int* err)
+{
+    const int i = blk * blockDim.x + threadIdx.x;
+    const bool valid = i < P.n;
+    const int key = valid ? cell_key_of(g, P.x[i], P.y[i], err) : -1;
+    const int slot = cell_slot_of(P.cell_count, key, 0);
+    if (valid) {
+        P.key[i] = key;
+        P.slot[i] = slot;
+    }
 }
 
 __global__ __launch_bounds__(256) void k_cell_key(DPhase P, Grid g, int* err)
@@ -301,9 +318,25 @@ __global__ __launch_bounds__(256) void k_cell_key(DPhase P, Grid g, int* err)
 }
 
 // Exclusive prefix of the tile sums of k_scan_tile (ntiles <= SCAN_TILE)
-// into LDS tp[0..ntiles], by the whole workgroup (SCAN_BLOCK threads).
+// into LDS tp[0..ntiles], by the whole workgroup (SCAN_BLOCK threads).  Up
+// to 64 tiles (131072 cells) one wave's shuffles do it.
 __device__ __forceinline__ void tile_prefix(const int* tile_sums, int ntiles, int* tp, int* lds)
 {
+    if (ntiles <= 64) {
+        if (threadIdx.x < 64) {
+            const int lane = threadIdx.x, v = lane < ntiles ? tile_sums[lane] : 0;
+            int incl = v;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const int t = __shfl_up(incl, off, 64);
+                if (lane >= off) incl += t;
+            }
+            tp[lane] = incl - v;
+            if (lane == 63) tp[64] = incl;
+        }
+        __syncthreads();
+        return;
+    }
     const int base = threadIdx.x * SCAN_ITEMS;
     int v[SCAN_ITEMS], s = 0;
 #pragma unroll
@@ -324,77 +357,59 @@ __device__ __forceinline__ void tile_prefix(const int* tile_sums, int ntiles, in
 
 // Cell-list scatter on the tile-local prefix of the counts (part, from
 // k_scan_tile) plus the prefix of the tile sums, computed per workgroup:
-// the three-pass scan becomes one pass.
+// the three-pass scan becomes one pass.  arr receives the particles of each
+// cell in arrival order, cell_start the final cell ranges (a grid over the
+// larger of particles and cells).
 __device__ __forceinline__ void cell_scatter_t_body(int blk, DPhase P, const int* part, const int* tile_sums,
-                                                    int ntiles)
+                                                    int ntiles, int ncell, int* arr)
 {
     __shared__ int tp[SCAN_TILE + 1];
     __shared__ int lds[SCAN_BLOCK];
     tile_prefix(tile_sums, ntiles, tp, lds);
     const int i = blk * blockDim.x + threadIdx.x;
+    if (i < ncell) P.cell_start[i] = part[i] + tp[i / SCAN_TILE];
+    if (i == 0) P.cell_start[ncell] = tp[ntiles];
     if (i >= P.n) return;
     const int key = P.key[i];
-    P.order[part[key] + tp[key / SCAN_TILE] + P.slot[i]] = i;
+    arr[part[key] + tp[key / SCAN_TILE] + P.slot[i]] = i;
 }
 
 __global__ __launch_bounds__(SCAN_BLOCK) void k_cell_scatter_t(DPhase P, const int* part, const int* tile_sums,
-                                                               int ntiles)
+                                                               int ntiles, int ncell, int* arr)
 {
-    cell_scatter_t_body(blockIdx.x, P, part, tile_sums, ntiles);
+    cell_scatter_t_body(blockIdx.x, P, part, tile_sums, ntiles, ncell, arr);
 }
 
-// Ascending particle number inside each cell (insertion sort; the ranks of
-// k_cell_key depend on atomic arrival order), which makes the neighbour
-// visiting order and so every floating-point sum deterministic; and the
-// final cell_start from the tile-local prefix and the tile sums.
-__device__ __forceinline__ void cell_sort_t_body(int blk, DPhase P, const int* part, const int* tile_sums, int ntiles,
-                                                 int ncell)
+// Place in the cell order of entry u of the arrival order arr: its particle i
+// goes to the cell's start plus the number of the cell's particles with a
+// smaller number.  The arrival ranks of k_cell_key depend on the order of
+// atomics; this one does not, so the neighbour visiting order, and with it
+// every floating-point sum, is deterministic.  One thread per particle reads
+// its cell's entries (about six, the same lines as its neighbours'); a thread
+// per cell that sorts them, the alternative, serialises on a crowded cell.
+__device__ __forceinline__ int cell_place(const DPhase& P, const int* arr, int u, int& i)
 {
-    __shared__ int tp[SCAN_TILE + 1];
-    __shared__ int lds[SCAN_BLOCK];
-    tile_prefix(tile_sums, ntiles, tp, lds);
-    const int c = blk * blockDim.x + threadIdx.x;
-    if (c >= ncell) return;
-    const int s = part[c] + tp[c / SCAN_TILE];
-    const int e = c + 1 < ncell ? part[c + 1] + tp[(c + 1) / SCAN_TILE] : tp[ntiles];
-    P.cell_start[c] = s;
-    if (c + 1 == ncell) P.cell_start[ncell] = e;
-    constexpr int CS = 16;   // cells up to this size sort in registers
-    if (e - s <= CS) {
-        // the cell's entries in registers (independent loads), an unrolled
-        // odd-even transposition network, one store each
-        int v[CS];
-#pragma unroll
-        for (int q = 0; q < CS; ++q) v[q] = s + q < e ? P.order[s + q] : INT_MAX;
-#pragma unroll
-        for (int r = 0; r < CS; ++r) {
-#pragma unroll
-            for (int q = r & 1; q + 1 < CS; q += 2) {
-                const int a = v[q], b = v[q + 1];
-                v[q] = min(a, b);
-                v[q + 1] = max(a, b);
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < CS; ++q)
-            if (s + q < e) P.order[s + q] = v[q];
-        return;
-    }
-    for (int k = s + 1; k < e; ++k) {
-        const int v = P.order[k];
-        int m = k - 1;
-        while (m >= s && P.order[m] > v) {
-            P.order[m + 1] = P.order[m];
-            --m;
-        }
-        P.order[m + 1] = v;
-    }
+    i = arr[u];
+    const int key = P.key[i];
+    const int s = P.cell_start[key], e = P.cell_start[key + 1];
+    int t = s;
+#pragma unroll 4
+    for (int k = s; k < e; ++k) t += arr[k] < i ? 1 : 0;
+    return t;
 }
 
-__global__ __launch_bounds__(SCAN_BLOCK) void k_cell_sort_t(DPhase P, const int* part, const int* tile_sums,
-                                                            int ntiles, int ncell)
+__device__ __forceinline__ void cell_rank_body(int blk, DPhase P, const int* arr)
 {
-    cell_sort_t_body(blockIdx.x, P, part, tile_sums, ntiles, ncell);
+    const int u = blk * blockDim.x + threadIdx.x;
+    if (u >= P.n) return;
+    int i;
+    const int t = cell_place(P, arr, u, i);
+    P.order[t] = i;
+}
+
+__global__ __launch_bounds__(SCAN_BLOCK) void k_cell_rank(DPhase P, const int* arr)
+{
+    cell_rank_body(blockIdx.x, P, arr);
 }
 
 
@@ -598,46 +613,6 @@ __global__ void k_renorm_water(DPhase P)
     const double v2 = P.vof2[i];
     P.rho[i] = P.rho[i] / P.vof[i] * v2;
     P.vof[i] = v2;
-}
-
-// time_integration_for_water_by_verlet (declarations_sph.f90:889-974), the
-// update after single_step_for_water of step `step`: real particles (the
-// first ntotal of the reference numbering) move by dt v + h2 a with
-// h2 = dt**2./2. and advance their other velocity level by 2 dt a (every
-// 50th step: restart from v + dt a); every particle's other density level
-// advances by 2 dt drho (step 1 and every 50th step: restart); then both
-// levels swap, as the reference's whole-array swaps do (the virtual
-// particles' velocity levels swap unchanged).
-__global__ void k_verlet_water(DPhase P, double* lvx, double* lvy, double* lrho, double dt, double h2, int step)
-{
-#pragma clang fp contract(off)
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= P.n) return;
-    const double vx = P.vx[i], vy = P.vy[i];
-    double nvx = lvx[i], nvy = lvy[i];
-    if (P.id[i] < P.ntotal) {
-        const double ax = P.ax[i], ay = P.ay[i];
-        P.x[i] = P.x[i] + dt * vx + h2 * ax;
-        P.y[i] = P.y[i] + dt * vy + h2 * ay;
-        if (step % 50 != 0) {
-            nvx = nvx + 2.0 * dt * ax;
-            nvy = nvy + 2.0 * dt * ay;
-        } else {
-            nvx = vx + dt * ax;
-            nvy = vy + dt * ay;
-        }
-    }
-    P.vx[i] = nvx;
-    P.vy[i] = nvy;
-    lvx[i] = vx;
-    lvy[i] = vy;
-    const double r = P.rho[i], dr = P.drho[i];
-    double nr;
-    if (step == 1) nr = r + dt * 2.0 * dr;
-    else if (step % 50 != 0) nr = lrho[i] + dt * 2.0 * dr;
-    else nr = r + dt * dr;
-    P.rho[i] = nr;
-    lrho[i] = r;
 }
 
 // volume_fraction_soil (m_particles.f90:3970-3988, applied by single_step
@@ -1257,67 +1232,6 @@ __global__ __launch_bounds__(256) void k_sum_density(DPhase W, Grid g, KParams K
         rs += mb * w;
     });
     W.rho_next[a] = rs / wi;
-}
-
-// After sum_density: drho = -rho*(df2(vx,'x')+df2(vy,'y')) + delta_sph(rho);
-// t via df (:1482-1484); p = b*((rho/rho0)**gamma-1) (:1478); av_vel.
-__global__ __launch_bounds__(256) void k_water1_a(DPhase W, Grid g, KParams K, int mask)
-{
-    const int t = xcd_block() * blockDim.x + threadIdx.x;
-    if (t >= W.n) return;
-    const CellList cw{W.cell_start, W.order};
-    const int a = cw.order[t];
-    const double xa = W.x[a], ya = W.y[a], vxa = W.vx[a], vya = W.vy[a];
-    const double ha = W.hsml[a], rhoa = W.rho[a], ca = W.c[a];
-    const int ita = W.itype[a];
-    const bool link = K.nnps == 2;
-    double d2x = 0.0, d2y = 0.0, drd = 0.0, DXvx = 0.0, DYvy = 0.0, DYvx = 0.0, DXvy = 0.0, avx = 0.0, avy = 0.0;
-    int cnt = 0;
-    for_each_candidate(g, cw, xa, ya, [&](int b) {
-        if (b == a) return;
-        const double xb = W.x[b], yb = W.y[b];
-        const double mh = link ? K.h1_water : sph_mhsml(ha, W.hsml[b]);
-        double dx, dy, r;
-        if (!sph_pair_test(xa, ya, xb, yb, K.scale_k * mh, dx, dy, r)) return;
-        if (link && !ll_reach(g, xa, ya, xb, yb)) return;
-        ++cnt;
-        double w, dwx, dwy;
-        sph_kernel(K.skf, r, dx, dy, mh, w, dwx, dwy);
-        const double mb = W.mass[b], rhob = W.rho[b], vxb = W.vx[b], vyb = W.vy[b];
-        d2x += mb * ((vxb - vxa) * dwx);
-        d2y += mb * ((vyb - vya) * dwy);
-        if (mask & M_DRHO_DELTA) {
-            const double rr = dx * dx + dy * dy;
-            const double muv = 2.0 * (rhoa - rhob) / rr;
-            double h = dx * muv * dwx;
-            h = h + dy * muv * dwy;
-            drd += K.delta * ha * ca * mb * h / rhob;
-        }
-        const double mr = mb / rhob;
-        DXvx += mr * ((vxa + vxb) * dwx);
-        DYvy += mr * ((vya + vyb) * dwy);
-        DYvx += mr * ((vxa + vxb) * dwy);
-        DXvy += mr * ((vya + vyb) * dwx);
-        if (mask & M_XSPH) {
-            const double mrho = (rhoa + rhob) / 2.0;
-            avx -= mb * (vxa - vxb) / mrho * w;
-            avy -= mb * (vya - vyb) / mrho * w;
-        }
-    });
-    {
-#pragma clang fp contract(off)
-        const double a2x = d2x / rhoa, a2y = d2y / rhoa;
-        W.drho[a] = -(rhoa * (a2x + a2y)) + drd;
-        W.txx[a] = SPH_C23_F * (2.0 * DXvx - DYvy);
-        W.txy[a] = DYvx + DXvy;
-        W.tyy[a] = SPH_C23_F * (2.0 * DYvy - DXvx);
-        if (rhoa > 0.0) W.p[a] = K.w_b * (pow(rhoa / K.w_rho0, K.w_gamma) - 1.0);
-        if (mask & M_XSPH) {
-            if (ita > 0) { avx = K.epsilon * avx; avy = K.epsilon * avy; }
-            W.avx[a] = avx; W.avy[a] = avy;
-        }
-        W.countiac[a] = cnt;
-    }
 }
 
 // dvx = -df(p,'x') + df(sxx,'x') + df(sxy,'y') (:1494-1498), /rho,

@@ -16,6 +16,7 @@
 
 #include "../../include/sphg.h"
 #include "sph_fused.h"
+#include "sph_single.h"
 #include "sph_mixed.h"
 #include "sph_gnn.h"
 #include "sph_batch.h"
@@ -95,9 +96,10 @@ struct PhaseBuf {
     bool cells_nl = false;      // the valid cell list is on the neighbour-list grid
     bool counts_zero = false;   // d.cell_count known to be all zero
     int* cell_part = nullptr;   // tile-local exclusive prefix of the cell counts
+    int* arrival = nullptr;     // particles by cell in arrival order, before the ranking
     int* tile_sums = nullptr;   // the scan's tile sums (per phase: the two builds may run concurrently)
     // the other velocity and density levels of the Verlet scheme (water)
-    double *lvx = nullptr, *lvy = nullptr, *lrho = nullptr;
+    double *lvx = nullptr, *lvy = nullptr, *lrho = nullptr, *lshadow[3] = {};
     // materialised pairs
     int *fwd = nullptr, *off = nullptr;
     int *pi = nullptr, *pj = nullptr;
@@ -189,6 +191,9 @@ struct sphg_ctx {
     // the final kernels of the step before also packed this step (first_half
     // applied to the state, records written): the step starts at its stages
     bool packed = false;
+    // single-phase water: the force kernel of the step before applied this
+    // step's first_half and took its cell keys and arrival ranks
+    bool keyed = false;
     int* d_nlflag = nullptr;    // bit 0: rebuild due; bit 1: a particle moved past skin / 2
     int* h_nlflag = nullptr;    // pinned: two slots for the lagged check of sphg_time_integration
     int h_nlstep[2] = {-1, -1}; // nl_seq of the step whose flag each slot holds (-1: none)
@@ -338,17 +343,22 @@ int phase_index(int phase) { return phase == SPHG_WATER ? 0 : (phase == SPHG_SOI
 // Cell list of one phase for the current positions, on the per-step grid
 // (nl = false) or on the neighbour-list grid.  A per-step build replaces the
 // order the neighbour lists index, so it retires them.
-int build_cells(sphg_ctx* c, int k, bool nl = false)
+// keyed: an earlier kernel has taken the keys and arrival ranks of the current
+// positions; ranked false: the rank inside the cells (b.d.order) is left to the
+// kernel that follows.
+int build_cells(sphg_ctx* c, int k, bool nl = false, bool keyed = false, bool ranked = true)
 {
     PhaseBuf& b = c->ph[k];
     if (b.cells_valid && b.cells_nl == nl) return SPHG_OK;
     if (!nl) c->nl_valid = false;
     const Grid& g = nl ? c->gvl[k] : c->gl[k];
     const int ncell = nl ? c->ncell_v : c->ncell;
-    // cell_count is all zero between builds: the scan clears what it reads
-    if (!b.counts_zero) RC(fill_int(c, b.d.cell_count, std::max(c->ncell, c->ncell_v), 0));
-    b.counts_zero = false;
-    RC(launch(c, "cell_key", k_cell_key, nblk(b.n), TPB, b.d, g, c->d_err));
+    if (!keyed) {
+        // cell_count is all zero between builds: the scan clears what it reads
+        if (!b.counts_zero) RC(fill_int(c, b.d.cell_count, std::max(c->ncell, c->ncell_v), 0));
+        b.counts_zero = false;
+        RC(launch(c, "cell_key", k_cell_key, nblk(b.n), TPB, b.d, g, c->d_err));
+    }
     // one scan pass: tile-local prefixes and tile sums; the scatter and the
     // per-cell sort add the prefix of the tile sums themselves
     const int ntiles = std::max((ncell + SCAN_TILE - 1) / SCAN_TILE, 1);
@@ -356,10 +366,9 @@ int build_cells(sphg_ctx* c, int k, bool nl = false)
     RC(launch(c, "scan", k_scan_tile, ntiles, SCAN_BLOCK, (const int*)b.d.cell_count, b.cell_part, ncell, b.tile_sums,
               b.d.cell_count));
     b.counts_zero = true;
-    RC(launch(c, "cell_scatter", k_cell_scatter_t, nblk(b.n, SCAN_BLOCK), SCAN_BLOCK, b.d, (const int*)b.cell_part,
-              (const int*)b.tile_sums, ntiles));
-    RC(launch(c, "cell_sort", k_cell_sort_t, nblk(ncell, SCAN_BLOCK), SCAN_BLOCK, b.d, (const int*)b.cell_part,
-              (const int*)b.tile_sums, ntiles, ncell));
+    RC(launch(c, "cell_scatter", k_cell_scatter_t, nblk(std::max(b.n, ncell), SCAN_BLOCK), SCAN_BLOCK, b.d,
+              (const int*)b.cell_part, (const int*)b.tile_sums, ntiles, ncell, b.arrival));
+    if (ranked) RC(launch(c, "cell_rank", k_cell_rank, nblk(b.n, SCAN_BLOCK), SCAN_BLOCK, b.d, (const int*)b.arrival));
     b.cells_valid = true;
     b.cells_nl = nl;
     return SPHG_OK;
@@ -372,13 +381,15 @@ void state_changed(sphg_ctx* c)
     for (auto& pb : c->ph) pb.cells_valid = false;
     c->nl_valid = false;
     c->packed = false;
+    c->keyed = false;
     c->last_k = 1;   // the rates the state holds count as those of a plain step
 }
 
 // Permute the persistent state of phase k into the current cell order, so
 // that slot t holds the t-th particle of the order (order becomes the
-// identity and the cell list stays valid).
-int reorder(sphg_ctx* c, int k)
+// identity and the cell list stays valid); lv: with the Verlet levels
+// (single-phase, so never in graph mode).
+int reorder(sphg_ctx* c, int k, bool lv = false)
 {
     PhaseBuf& b = c->ph[k];
     DPhase& d = b.d;
@@ -397,7 +408,16 @@ int reorder(sphg_ctx* c, int k)
     A.ni = NI;
     for (int a = 0; a < ND; ++a) { A.sd[a] = *f[a]; A.dd[a] = b.shadow_d[a]; }
     for (int a = 0; a < NI; ++a) { A.si[a] = *fi[a]; A.di[a] = b.shadow_i[a]; }
+    double** lf[] = {&b.lvx, &b.lvy, &b.lrho};
+    static_assert(ND + 3 <= PERM_MAXD, "one pass permutes the Verlet levels too");
+    if (lv)
+        for (int a = 0; a < 3; ++a) {
+            A.sd[A.nd] = *lf[a];
+            A.dd[A.nd++] = b.lshadow[a];
+        }
     RC(launch(c, "permute", k_permute_multi, nblk(b.n), TPB, A, ord, b.n));
+    if (lv)
+        for (int a = 0; a < 3; ++a) std::swap(*lf[a], b.lshadow[a]);
     if (c->stable_ptrs) {
         // captured graphs hold the arrays' addresses: copy back instead
         PermArgs B{};
@@ -847,6 +867,7 @@ int alloc_phase(sphg_ctx* c, int k, const sphg_phase_view* v)
     RC(dalloc(c, b, &d.key, n));
     RC(dalloc(c, b, &d.slot, n));
     RC(dalloc(c, b, &d.order, n));
+    RC(dalloc(c, b, &b.arrival, n));
     double** dbls[] = {&d.x, &d.y, &d.vx, &d.vy, &d.mass, &d.hsml, &d.rho, &d.rho_min, &d.rho_next,
                        &d.vof, &d.vof_min, &d.vof2, &d.dvof, &d.dvof_x, &d.p, &d.c, &d.c_next,
                        &d.drho, &d.ax, &d.ay, &d.avx, &d.avy, &d.vx_min, &d.vy_min,
@@ -1330,21 +1351,67 @@ int rhs_two_phase_fused(sphg_ctx* c, int water_half, int soil_half, int soil_ndp
     return stages_of(c);
 }
 
-// single_step_for_water (declarations_sph.f90:1439-1526).
-int rhs_water(sphg_ctx* c)
+// Lanes per particle (log2) of the single-phase water passes, by the number
+// of particles: the chip's 1024 SIMDs hold one wave each at 65536 particles
+// and one lane per particle, so fewer leave SIMDs idle and each wave alone
+// with the latency of its partner loop, and many more lanes than that repeat
+// the particles' own loads for nothing.  Dam break, us per step (1 / 2 / 4 / 8
+// lanes): 7.5k 57 / 48 / 41 / 39, 14k 58 / 48 / 42 / 42, 44k 60 / 57 / 53 / 60,
+// 85k 75 / 69 / 73 / 86, 168k 93 / 101 / 108 / 137.
+int w1_lanes(int n) { return n <= 16384 ? 3 : n <= 65536 ? 2 : n <= 122880 ? 1 : 0; }
+
+template <int SKF, bool U>
+int w1_passes(sphg_ctx* c, const W1End& end)
 {
     PhaseBuf& W = c->ph[0];
-    RC(build_cells(c, 0));
-    RC(launch(c, "sum_density", k_sum_density, nblk(W.n), TPB, W.d, c->gl[0], c->K, c->K.h1_water));
-    std::swap(W.d.rho, W.d.rho_next);
+    const int lg = w1_lanes(W.n), nb = nblk(W.n << lg);
     int ma = M_DRHO_DELTA | M_XSPH;
     if (!c->P.artificial_density) ma &= ~M_DRHO_DELTA;
     if (!c->P.average_velocity) ma &= ~M_XSPH;
-    RC(launch(c, "water1_a", k_water1_a, nblk(W.n), TPB, W.d, c->gl[0], c->K, ma));
-    int mb = c->P.visc_artificial ? M_ART : 0;
-    RC(launch(c, "water1_b", k_water1_b, nblk(W.n), TPB, W.d, c->gl[0], c->K, mb));
+    RC(launch(c, "water1_d", k_w1_density<SKF, U>, nb, TPB, W.d, W.rec, W.masks, c->gl[0], c->K, c->F, lg));
+    RC(launch(c, "water1_a", k_w1_rates<SKF, U>, nb, TPB, W.d, W.rec, W.masks, c->gl[0], c->K, c->F, ma, lg));
+    return launch(c, "water1_b", k_w1_force<SKF, U>, nb, TPB, W.d, (const double*)W.rec, W.masks, c->gl[0], c->K,
+                  c->F, c->P.visc_artificial ? (int)M_ART : 0, lg, end);
+}
+
+// single_step_for_water (declarations_sph.f90:1439-1526), with first_half
+// before it (half) and the update of end.scheme after it.
+int rhs_water(sphg_ctx* c, bool half, const W1End& end)
+{
+    PhaseBuf& W = c->ph[0];
+    const bool keyed = c->keyed, built = W.cells_valid && !W.cells_nl;
+    c->keyed = false;
+    RC(build_cells(c, 0, false, keyed, false));
+    RC(launch(c, "pack", k_w1_pack, nblk(W.n), TPB, W.d, c->K, W.rec, built ? (const int*)nullptr : W.arrival,
+              half && !keyed ? 1 : 0));
+    const bool u = W.hmin == W.hmax;
+    if (end.ahead) W.counts_zero = false;
+    int rc;
+    switch (c->P.skf) {
+    case 1: rc = u ? w1_passes<1, true>(c, end) : w1_passes<1, false>(c, end); break;
+    case 2: rc = u ? w1_passes<2, true>(c, end) : w1_passes<2, false>(c, end); break;
+    case 3: rc = u ? w1_passes<3, true>(c, end) : w1_passes<3, false>(c, end); break;
+    default: rc = u ? w1_passes<4, true>(c, end) : w1_passes<4, false>(c, end); break;
+    }
+    RC(rc);
+    if (end.scheme) W.cells_valid = false;   // the positions moved
+    c->keyed = end.ahead != 0;
     return SPHG_OK;
 }
+
+// Every reorder_every steps the state is permuted into the cell order of the
+// current positions (b: the water phase; lv: the Verlet levels go along).
+int reorder_water1(sphg_ctx* c, bool lv)
+{
+    if (++c->since_reorder < c->reorder_every) return SPHG_OK;
+    c->since_reorder = 0;
+    RC(build_cells(c, 0));
+    return reorder(c, 0, lv);
+}
+
+// Whether the next step (another of the same call) can be keyed ahead: it
+// does not start with a reorder.
+bool keys_ahead(const sphg_ctx* c, bool ahead_ok) { return ahead_ok && c->since_reorder + 1 < c->reorder_every; }
 
 int check_fused_switches(const sphg_ctx* c)
 {
@@ -1452,11 +1519,9 @@ int one_step(sphg_ctx* c, bool ahead_ok = false)
         return SPHG_OK;
     }
     if (c->P.single_phase) {
-        if (step != 1) RC(launch(c, "first_half", k_first_half_water, nblk(W.n), TPB, W.d, c->K));
-        RC(rhs_water(c));
-        RC(launch(c, "final_water", k_final_water, nblk(W.n), TPB, W.d, c->K, step == 1 ? 1 : 0, 0, 0));
-        W.cells_valid = false;
-        return SPHG_OK;
+        RC(reorder_water1(c, false));
+        return rhs_water(c, step != 1, W1End{1, step, keys_ahead(c, ahead_ok) ? 1 : 0, nullptr, nullptr, nullptr, 0.0,
+                                             c->d_err});
     }
     if (c->legacy) {
         if (step != 1) {
@@ -1513,6 +1578,7 @@ int verlet_steps(sphg_ctx* c, int nsteps)
         RC(dalloc(c, W, &W.lvx, (size_t)W.n));
         RC(dalloc(c, W, &W.lvy, (size_t)W.n));
         RC(dalloc(c, W, &W.lrho, (size_t)W.n));
+        for (double** p : {&W.lshadow[0], &W.lshadow[1], &W.lshadow[2]}) RC(dalloc(c, W, p, (size_t)W.n));
     }
     RC(launch(c, "verlet", k_copy<double>, nblk(W.n), TPB, (const double*)W.d.vx, W.lvx, W.n));
     RC(launch(c, "verlet", k_copy<double>, nblk(W.n), TPB, (const double*)W.d.vy, W.lvy, W.n));
@@ -1520,9 +1586,9 @@ int verlet_steps(sphg_ctx* c, int nsteps)
     const double dt = c->P.dt, h2 = std::pow(dt, 2.0) / 2.0;   // dt**2./2.
     for (int it = 0; it < nsteps; ++it) {
         const int step = ++c->itimestep;
-        RC(rhs_water(c));
-        RC(launch(c, "verlet", k_verlet_water, nblk(W.n), TPB, W.d, W.lvx, W.lvy, W.lrho, dt, h2, step));
-        W.cells_valid = false;
+        RC(reorder_water1(c, true));
+        RC(rhs_water(c, false, W1End{2, step, keys_ahead(c, it + 1 < nsteps) ? 1 : 0, W.lvx, W.lvy, W.lrho, h2,
+                                     c->d_err}));
     }
     return SPHG_OK;
 }
@@ -1862,7 +1928,7 @@ int sphg_single_step(sphg_ctx* c, int sync)
     if (soil_only(c)) {
         RC(rhs_soil_only(c, 0, 1));
     } else if (c->P.single_phase) {
-        RC(rhs_water(c));
+        RC(rhs_water(c, false, W1End{}));
     } else {
         PhaseBuf& S = c->ph[1];
         if (c->legacy) {
@@ -1887,6 +1953,7 @@ int sphg_time_integration(sphg_ctx* c, int nsteps, int sync)
 {
     if (!c || nsteps < 0) return SPHG_ERR_INVALID;
     RC(check_fused_switches(c));
+    c->keyed = false;
     if (c->P.single_phase && c->P.integrate_scheme == 2) RC(verlet_steps(c, nsteps));
     else
         for (int it = 0; it < nsteps; ++it) RC(one_step(c, it + 1 < nsteps));
@@ -2784,7 +2851,7 @@ const std::map<const void*, Batched>& batched_registry()
         reg_batched<BodyScanTile>(r, k_scan_tile);
         reg_batched<BodyCellKey>(r, k_cell_key);
         reg_batched<BodyCellScatter>(r, k_cell_scatter_t);
-        reg_batched<BodyCellSort>(r, k_cell_sort_t);
+        reg_batched<BodyCellRank>(r, k_cell_rank);
         reg_batched<BodyPackWater>(r, k_pack_water);
         reg_batched<BodyPackSoil>(r, k_pack_soil);
         reg_batched<BodyNlist>(r, k_nlist);
@@ -3449,10 +3516,10 @@ int sphg_direct_find_noalloc(const sphg_params* params, int n, const double* x, 
     RC(na_launch(st, k_cell_key, nblk(n), TPB, d, g, flags));
     RC(na_launch(st, k_scan_tile, ntiles, SCAN_BLOCK, (const int*)d.cell_count, cell_part, ncell, tiles,
                  d.cell_count));
-    RC(na_launch(st, k_cell_scatter_t, nblk(n, SCAN_BLOCK), SCAN_BLOCK, d, (const int*)cell_part,
-                 (const int*)tiles, ntiles));
-    RC(na_launch(st, k_cell_sort_t, nblk(ncell, SCAN_BLOCK), SCAN_BLOCK, d, (const int*)cell_part,
-                 (const int*)tiles, ntiles, ncell));
+    // (the arrival order in the counts' array, which is written after it)
+    RC(na_launch(st, k_cell_scatter_t, nblk(std::max(n, ncell), SCAN_BLOCK), SCAN_BLOCK, d, (const int*)cell_part,
+                 (const int*)tiles, ntiles, ncell, fwd));
+    RC(na_launch(st, k_cell_rank, nblk(n, SCAN_BLOCK), SCAN_BLOCK, d, (const int*)fwd));
     // partner counts, their prefix, the total (the kernels of materialise)
     RC(na_launch(st, k_pair_count, nblk(n), TPB, d, d, g, K, 1, 0, 0.0, fwd, countiac));
     RC(na_launch(st, k_scan_tile, ptiles, SCAN_BLOCK, (const int*)fwd, off, n, tiles, (int*)nullptr));
