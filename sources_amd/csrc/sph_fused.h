@@ -4,24 +4,17 @@
 //   pack      thread t of the cell order: half-step update of particle order[t]
 //             and its neighbour record t, cell-sorted and stored as chunk
 //             planes (chunk c of record t is element t of plane c).  Record
-//             chunks (16 bytes): 0 x,y | 1 vx,vy | 2 rho,m | 3 vof,p | 4 s3,c |
-//             5 s1,s2 | 6 h,itype; m carries the sign of itype (negative for
-//             virtual particles).  The lanes of a wave hold nearby particles
-//             whose k-th partners are nearby in the cell order too, so one
-//             chunk load of all lanes touches a few cache lines of a plane (a
-//             128-byte record per particle would touch one line per lane: the
-//             address unit serialises on those).  The loops load only the
-//             chunks they use: 1/rho and m/rho of a partner are recomputed;
-//   stage A   candidate scan of the 3 cell rows with a sqrt-free exact
-//             predicate (dr < T, T precomputed so that dr < T <=> sqrt(dr) < R),
-//             accepted partners kept as one concatenated 128-bit mask; then a
-//             dense loop over the mask bits evaluates the pair terms.  The masks
-//             are stored for stage B, so each pair is tested once per step;
-//   stage B   dense loop over the stored masks (water).  Soil stage B needs
-//             nothing from the stage A of other soil particles, so soil runs
-//             both stages in one kernel over one partner loop.
-// Lanes of a wavefront hold consecutive cell-sorted particles; the dense loops
-// diverge only by the lanes' neighbour-count spread.
+//             chunks (16 bytes): 0 x,y | 1 vx,vy | 2 rho,V | 3 vof,p (soil:
+//             vof/rho,p) | 4 s3,c | 5 s1,s2 | 6 h,itype; V = m/rho carries the
+//             sign of itype (negative for virtual particles), so the pair
+//             terms need no reciprocal of the partner's density.  The loops
+//             load only the chunks they use;
+//   stage A   the same-phase terms that need only the packed values;
+//   stage B   (water) the terms that need the partners' strain rates.  Soil
+//             stage B needs nothing from the stage A of other soil particles,
+//             so soil runs both stages in one kernel over one partner loop.
+// The cross terms have passes of their own.  Lanes of a wavefront hold
+// consecutive cell-sorted particles.
 #pragma once
 #include "sph_kernels.h"
 
@@ -70,110 +63,95 @@ __device__ __forceinline__ double ipow(double q, int n)
     return r;
 }
 
-// 1/d and 1/sqrt(d) from the hardware estimates plus two Newton steps
-// (each step doubles the correct bits), i.e. to about one ulp; far shorter
-// dependency chains than IEEE-exact FP64 division and square root.
+// 1/d and 1/sqrt(d) from the hardware estimates (about 2^-23) plus one
+// third-order step (error below 2^-60 before its rounding), i.e. to about one
+// ulp; far shorter dependency chains than IEEE-exact FP64 division and square
+// root.
 __device__ __forceinline__ double fast_rcp(double d)
 {
-    double x = __builtin_amdgcn_rcp(d);
-    double e = fma(-d, x, 1.0);
-    x = fma(x, e, x);
-    e = fma(-d, x, 1.0);
-    return fma(x, e, x);
+    const double x = __builtin_amdgcn_rcp(d);
+    const double e = fma(-d, x, 1.0);
+    return fma(x, fma(e, e, e), x);
 }
 
 __device__ __forceinline__ double fast_rsq(double d)
 {
-    double y = __builtin_amdgcn_rsq(d);
-    const double h = 0.5 * d;
-    y = y * fma(-h, y * y, 1.5);
-    y = y * fma(-h, y * y, 1.5);
-    return y;
+    const double y = __builtin_amdgcn_rsq(d);
+    const double e = fma(-(d * y), y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
-// r, 1/r and 1/r^2 of a squared distance dr > 0.
-struct Dist {
-    double r, ir, idr;
-};
-
-__device__ __forceinline__ Dist dist_of(double dr)
-{
-    const double ir = fast_rsq(dr);
-    return Dist{dr * ir, ir, ir * ir};
-}
-
-// Kernel constants for one smoothing length (uniform-h fast path).
+// Kernel constants for one smoothing length: the normalisation factor f,
+// and per kernel the coefficients of W and of s = |grad W| / r.
 struct KC {
-    double inv_h, f, fh1, fh2;
+    double inv_h, f, c1, c2, c3;
 };
 
 __device__ __forceinline__ KC make_kc(int skf, double h)
 {
     KC k;
     k.inv_h = 1.0 / h;
-    double f;
-    if (skf == 1) f = 15.0 / (7.0 * SPH_PI_F * h * h);
-    else if (skf == 2) f = 1.0 / ((h * h) * SPH_PI_F);
-    else if (skf == 3) f = 7.0 / (478.0 * SPH_PI_F * h * h);
-    else f = 7.0 / (4.0 * SPH_PI_F * h * h);
-    k.f = f;
-    k.fh1 = f * k.inv_h;
-    k.fh2 = f * k.inv_h * k.inv_h;
+    const double ih2 = k.inv_h * k.inv_h;
+    if (skf == 1) {
+        k.f = 15.0 / (7.0 * SPH_PI_F * h * h);
+        k.c1 = 2.0 * (k.f * ih2);            // s, q <= 1: c1 (0.75 q - 1)
+        k.c2 = -0.5 * (k.f * k.inv_h);       // s, q > 1: c2 (2 - q)^2 / r
+        k.c3 = k.f * (1.0 / 6.0);            // W, q > 1
+    } else if (skf == 2) {
+        k.f = 1.0 / ((h * h) * SPH_PI_F);
+        k.c1 = -2.0 * ih2;
+        k.c2 = k.c3 = 0.0;
+    } else if (skf == 3) {
+        k.f = 7.0 / (478.0 * SPH_PI_F * h * h);
+        k.c1 = k.f * ih2;
+        k.c2 = k.f * k.inv_h;
+        k.c3 = 0.0;
+    } else {
+        k.f = 7.0 / (4.0 * SPH_PI_F * h * h);
+        k.c1 = k.f * ih2;
+        k.c2 = k.c3 = 0.0;
+    }
     return k;
 }
 
-// W and grad W (m_particles.f90:1469-1602) with precomputed constants;
-// inv_r = 1/r is only used where the reference divides by r.
+// W and s (grad W = s (dx, dy); m_particles.f90:1469-1602) of a pair inside
+// the support; inv_r = 1/r.
 template <int SKF, bool NEED_W>
-__device__ __forceinline__ void kern_fast(const KC& k, double r, double inv_r, double dx, double dy,
-                                          double& w, double& gx, double& gy)
+__device__ __forceinline__ void kern_s(const KC& k, double r, double inv_r, double& w, double& s)
 {
     const double q = r * k.inv_h;
-    w = 0.0; gx = 0.0; gy = 0.0;
+    w = 0.0;
     if constexpr (SKF == 1) {
         // both pieces, then a select: no divergent branch in the pair loop
-        const bool in1 = q <= 1.0, in2 = q <= 2.0;
-        const double t = 2.0 - q;
-        const double s1 = k.fh2 * (-2.0 + 1.5 * q);
-        const double s2 = -(0.5 * k.fh1) * (t * t) * inv_r;
-        const double s = in1 ? s1 : (in2 ? s2 : 0.0);
+        const bool in1 = q <= 1.0;
+        const double t = 2.0 - q, t2 = t * t;
+        const double s1 = k.c1 * fma(0.75, q, -1.0), s2 = t2 * (k.c2 * inv_r);
+        s = in1 ? s1 : s2;
         if (NEED_W) {
-            const double w1 = k.f * (SPH_C23_F - q * q + ((q * q) * q) * 0.5);
-            const double w2 = k.f * (1.0 / 6.0) * ((t * t) * t);
-            w = in1 ? w1 : (in2 ? w2 : 0.0);
+            const double w1 = k.f * fma(q * q, fma(0.5, q, -1.0), SPH_C23_F), w2 = t2 * (k.c3 * t);
+            w = in1 ? w1 : w2;
         }
-        gx = s * dx; gy = s * dy;
     } else if constexpr (SKF == 4) {
-        const bool in2 = q <= 2.0;
-        const double t = 1.0 - 0.5 * q;
-        const double t2 = t * t;
-        if (NEED_W) w = in2 ? k.f * ((t2 * t2) * (1.0 + 2.0 * q)) : 0.0;
-        double s = k.fh2 * (-5.0 + 7.5 * q - 3.75 * (q * q) + 0.625 * ((q * q) * q));
-        s = in2 ? s : 0.0;
-        gx = s * dx; gy = s * dy;
+        const double t = fma(-0.5, q, 1.0), t2 = t * t;
+        if (NEED_W) w = k.f * ((t2 * t2) * fma(2.0, q, 1.0));
+        // (the reference's order of the terms: they cancel towards q = 2)
+        s = k.c1 * (-5.0 + 7.5 * q - 3.75 * (q * q) + 0.625 * ((q * q) * q));
     } else if constexpr (SKF == 2) {
-        if (q <= 3.0) {
-            const double e = k.f * exp(-q * q);
-            if (NEED_W) w = e;
-            const double s = -2.0 * e * (k.inv_h * k.inv_h);
-            gx = s * dx; gy = s * dy;
-        }
+        w = k.f * exp(-q * q);
+        s = k.c1 * w;
     } else {
         const double a = 3.0 - q, b = 2.0 - q, c = 1.0 - q;
         const double a2 = a * a, b2 = b * b, c2 = c * c;
         const double a4 = a2 * a2, b4 = b2 * b2, c4 = c2 * c2;
         if (q <= 1.0) {
             if (NEED_W) w = k.f * (a4 * a - 6.0 * (b4 * b) + 15.0 * (c4 * c));
-            const double s = k.fh2 * (-120.0 + 120.0 * q - 50.0 * (q * q));  // reference polynomial
-            gx = s * dx; gy = s * dy;
+            s = k.c1 * (-120.0 + 120.0 * q - 50.0 * (q * q));  // reference polynomial
         } else if (q <= 2.0) {
             if (NEED_W) w = k.f * (a4 * a - 6.0 * (b4 * b));
-            const double s = k.fh1 * (-(5.0 * a4) + 30.0 * b4) * inv_r;
-            gx = s * dx; gy = s * dy;
-        } else if (q <= 3.0) {
+            s = k.c2 * (-(5.0 * a4) + 30.0 * b4) * inv_r;
+        } else {
             if (NEED_W) w = k.f * (a4 * a);
-            const double s = k.fh1 * (-(5.0 * a4)) * inv_r;
-            gx = s * dx; gy = s * dy;
+            s = k.c2 * (-(5.0 * a4)) * inv_r;
         }
     }
 }
@@ -185,7 +163,11 @@ __device__ __forceinline__ void kern_fast(const KC& k, double r, double inv_r, d
 struct RecV {
     const double2* p;
     int n;
-    __device__ __forceinline__ double2 operator()(int k, int c) const { return p[(size_t)c * n + k]; }
+    // (uniform plane address plus a 32-bit lane offset: no 64-bit lane arithmetic)
+    __device__ __forceinline__ double2 operator()(int k, int c) const
+    {
+        return *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(p + (size_t)c * n) + ((uint32_t)k << 4));
+    }
 };
 
 __device__ __forceinline__ RecV recv(const double* rec, int n)
@@ -387,7 +369,8 @@ __device__ __forceinline__ void pack_water_at(const DPhase& P, const KParams& K,
     const size_t pn = (size_t)P.n;
     R[0 * pn] = make_double2(x, y);
     R[1 * pn] = make_double2(vx, vy);
-    R[2 * pn] = make_double2(rho, it < 0 ? -m : m);   // the sign of m marks a virtual particle
+    const double V = m * irho;
+    R[2 * pn] = make_double2(rho, it < 0 ? -V : V);   // the sign of V marks a virtual particle
     R[3 * pn] = make_double2(vof, p);
     R[4 * pn] = make_double2(0.0, cn);
     // (h and itype stay between list rebuilds, in the same slot: a lean pack
@@ -422,7 +405,7 @@ __device__ __forceinline__ void step_water(int blk, DPhase P, KParams K, double*
 {
     const int t = blk * blockDim.x + threadIdx.x;
     if (t >= P.n) return;
-    const int i = P.order[t];
+    const int i = t;   // (lists kept: the state is in record order)
     const WaterEnd e = water_end(P, K, i, first, with_vof, renorm);
     const int it = P.itype[i];
     // the final update's stores that the pack does not overwrite
@@ -520,8 +503,9 @@ __device__ __forceinline__ void pack_soil_at(const DPhase& P, const KParams& K, 
     const size_t pn = (size_t)P.n;
     R[0 * pn] = make_double2(x, y);
     R[1 * pn] = make_double2(vx, vy);
-    R[2 * pn] = make_double2(rho, it < 0 ? -m : m);   // the sign of m marks a virtual particle
-    R[3 * pn] = make_double2(P.vof[i], p);
+    const double V = m * irho;
+    R[2 * pn] = make_double2(rho, it < 0 ? -V : V);   // the sign of V marks a virtual particle
+    R[3 * pn] = make_double2(P.vof[i] * irho, p);
     R[4 * pn] = make_double2(syy, P.c[i]);
     R[5 * pn] = make_double2(sxx, sxy);
     if (!lean) R[6 * pn] = make_double2(P.hsml[i], (double)it);   // (as for water)
@@ -552,7 +536,7 @@ __device__ __forceinline__ void step_soil(int blk, DPhase P, KParams K, double* 
 {
     const int t = blk * blockDim.x + threadIdx.x;
     if (t >= P.n) return;
-    const int i = P.order[t];
+    const int i = t;   // (lists kept: the state is in record order)
     const SoilEnd e = soil_end(P, K, i, first);
     if (K.volume_fraction && K.two_phase) P.vof[i] = e.vof;
     if (P.itype[i] > 0) {
@@ -589,9 +573,33 @@ struct Masks {
 // every pair within R lies in these masks, so each step tests only the
 // listed candidates with the exact predicate instead of scanning the rows.
 // ------------------------------------------------------------------------
+// The same candidates as positions in the window of the workgroup's particles:
+// candidate j of record t is the window's record li[j * n + t], cnt[t] of them
+// (-1: more than cap, the rows are walked).  win: WIN_INTS per workgroup: the
+// first records of the window's three record ranges, their positions in it and
+// its length.  A workgroup holds WIN_LANES >> lg particles.
+struct IdxList {
+    unsigned short* li;
+    int *cnt, *win;
+    int cap, lds;   // lds 0: the windows stay in global memory (predicates that need more than a distance)
+};
+
+constexpr int WIN_INTS = 8;
+constexpr int WIN_CAP = 846;             // records of a window in LDS: two workgroups' six chunks fill a CU's
+constexpr int WIN_STRIDE = WIN_CAP + 1;  // (and the stand-in record)
+// Lanes of a workgroup that take particles.  The window holds three rows' worth
+// of them: 633 records on average and 848 at most for 192 particles of a
+// lattice at h = 1.2 dx (whose cell rows hold two or three lattice rows); with
+// 240 particles one window in four does not fit, and its workgroup takes the
+// slow path at the occupancy the LDS leaves (1M slope, soil_ab 117 us against
+// 102, water_b 72 against 55).
+constexpr int WIN_LANES = 192;
+
 struct NList {
     Masks same, cross;   // candidates within R + skin: same phase, other phase
     const int* cell;     // [n] key of the particle's cell at the rebuild (record order)
+    IdxList is, ix;      // the candidates as indices (FP64 stages): same phase, other phase
+    int lg;
 };
 
 // ------------------------------------------------------------------------
@@ -618,20 +626,6 @@ __device__ __forceinline__ LaneRows lane_rows(const Rows& R)
     return L;
 }
 
-// Scan of one candidate row: accept(k, xy) on the candidates' positions.
-template <class P>
-__device__ __forceinline__ uint64_t scan_row(int k0, int k1, int self, const RecV& rec, P&& accept)
-{
-    uint64_t m = 0;
-    if (k1 - k0 > 64) return 0;
-#pragma unroll 4
-    for (int k = k0; k < k1; ++k) {
-        const bool ok = k != self && accept(k, rec(k, 0));
-        m |= (uint64_t)ok << (k - k0);
-    }
-    return m;
-}
-
 __device__ __forceinline__ int ovf_of(const LaneRows& L)
 {
     int o = 0;
@@ -639,28 +633,6 @@ __device__ __forceinline__ int ovf_of(const LaneRows& L)
     for (int r = 0; r < 3; ++r)
         if (L.k1[r] - L.k0[r] > 64) o |= 1 << r;
     return o;
-}
-
-// Dense visit of the masked partners, then the direct walk of overflowed rows.
-template <class IT, class LD, class B, class P>
-__device__ __forceinline__ void visit(IT it, const LaneRows& L, int ovf, int self, const LD& load, P&& accept, B&& body)
-{
-#pragma unroll 1
-    for (int k = it.next(); k >= 0; k = it.next()) body(load(k));
-    if (ovf) {
-        // one pass over the concatenated rows (row bounds as scalars: an
-        // indexed LaneRows would be kept in scratch memory)
-        const int s1 = L.k1[0] - L.k0[0], s2 = s1 + L.k1[1] - L.k0[1], tot = s2 + L.k1[2] - L.k0[2];
-        const int e0 = L.k0[0], e1 = L.k0[1] - s1, e2 = L.k0[2] - s2;
-#pragma unroll 1
-        for (int c = 0; c < tot; ++c) {
-            const int r = c < s1 ? 0 : (c < s2 ? 1 : 2);
-            if (!(ovf & (1 << r))) continue;
-            const int kk = c + (r == 0 ? e0 : (r == 1 ? e1 : e2));
-            if (kk == self || !accept(kk)) continue;
-            body(load(kk));
-        }
-    }
 }
 
 // The three row masks of a lane concatenated into one 128-bit mask over
@@ -731,76 +703,6 @@ __device__ __forceinline__ CatIter cat_iter(const CatMask& c, const LaneRows& L)
     return it;
 }
 
-// Partner data of the stage kernels: xy = (x, y), v = (vx, vy),
-// rm = (rho, m), hv = (h, vof), pc = (p, c), s12 = (s1, s2), s3 = (s3, itype),
-// iv = (1/rho, m/rho), filled from the record chunks.
-struct Nb {
-    double2 xy, v, rm, hv, pc, s12, s3, iv;
-    double rpre;   // density before the Mohr-Coulomb criterion (record chunk 7)
-    __device__ __forceinline__ void set(int c, double2 q)
-    {
-        switch (c) {
-        case 0: xy = q; break;
-        case 1: v = q; break;
-        case 2: rm = q; break;
-        case 3: hv.y = q.x; pc.x = q.y; break;   // vof, p
-        case 4: s3.x = q.x; pc.y = q.y; break;   // s3, c
-        case 5: s12 = q; break;
-        case 6: hv.x = q.x; s3.y = q.y; break;   // h, itype
-        default: break;
-        }
-    }
-};
-
-constexpr int NEED_IV = 1 << 8;   // recompute 1/rho and m/rho of the partner
-constexpr int CH_H = 1 << 6;      // chunk holding h
-
-// Loads the chunks NEED of partner record k -- plus the h chunk when with_h
-// (non-uniform smoothing length); FROM = 1: all but the positions (chunk 0).
-template <int NEED, int FROM = 0>
-__device__ __forceinline__ Nb load_nb(const RecV& rec, int k, bool with_h)
-{
-    Nb b{};
-#pragma unroll
-    for (int c = FROM; c < 7; ++c) {
-        if (!(NEED & (1 << c)) && !(c == 6 && with_h)) continue;
-        b.set(c, rec(k, c));
-    }
-    if (NEED & 4) {
-        // chunk 2 carries m with the sign of itype (virtual < 0)
-        if (!((NEED & CH_H) || with_h)) b.s3.y = b.rm.y < 0.0 ? -1.0 : 1.0;
-        b.rm.y = fabs(b.rm.y);
-    }
-    if (NEED & NEED_IV) {
-        b.iv.x = fast_rcp(b.rm.x);
-        b.iv.y = b.rm.y * b.iv.x;
-    }
-    return b;
-}
-
-// Partner loader of a dense loop: the chunks NEED of record k (chunk 7, the
-// density before the Mohr-Coulomb criterion, when mc), whole or as positions
-// plus the rest.
-template <int NEED>
-struct Loader {
-    RecV rec;
-    bool with_h, mc;
-    __device__ __forceinline__ double2 xy(int k) const { return rec(k, 0); }
-    __device__ __forceinline__ Nb rest(int k, double2 p) const
-    {
-        Nb b = load_nb<NEED, 1>(rec, k, with_h);
-        b.xy = p;
-        if (mc) b.rpre = rec(k, 7).x;
-        return b;
-    }
-    __device__ __forceinline__ Nb operator()(int k) const
-    {
-        Nb b = load_nb<NEED>(rec, k, with_h);
-        if (mc) b.rpre = rec(k, 7).x;
-        return b;
-    }
-};
-
 // Exact pair predicate on a candidate.
 struct Pred {
     double xa, ya, ha, thr;
@@ -818,7 +720,44 @@ struct Pred {
     }
 };
 
-// Wave-level set-up shared by the stage kernels.
+// The particle and candidate subset of a lane.
+struct SubCtx {
+    int t, tt, sub;
+    bool valid;
+};
+
+// lanes: lanes of the workgroup that take particles (a multiple of 2^lg).
+__device__ __forceinline__ SubCtx sub_ctx(int n, int blk, int lg, int lanes)
+{
+    SubCtx c;
+    const int i = (int)threadIdx.x;
+    c.t = blk * (lanes >> lg) + (i >> lg);
+    c.sub = i & ((1 << lg) - 1);
+    c.valid = i < lanes && c.t < n;
+    c.tt = c.valid ? c.t : n - 1;
+    return c;
+}
+
+// Sum of v over the lanes of a particle (all get it).
+__device__ __forceinline__ void sub_sum(int lg, double& v)
+{
+    for (int o = 1; o < (1 << lg); o <<= 1) v += __shfl_xor(v, o, 64);
+}
+
+template <class... T>
+__device__ __forceinline__ void sub_sum(int lg, double& v, T&... rest)
+{
+    sub_sum(lg, v);
+    sub_sum(lg, rest...);
+}
+
+__device__ __forceinline__ int sub_count(int lg, int v)
+{
+    for (int o = 1; o < (1 << lg); o <<= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+
+// Wave-level set-up of the mixed-precision stage kernels.
 struct WaveCtx {
     int lane, t, tt, last;
     bool valid;
@@ -840,62 +779,6 @@ __device__ __forceinline__ WaveCtx wave_ctx(int n, int blk)
 
 __device__ __forceinline__ WaveCtx wave_ctx(int n) { return wave_ctx(n, xcd_block()); }
 
-// Mask of a particle over its candidate rows in the records rec: scan of the
-// three rows with the predicate P (self: own record index, or -1).
-template <class A>
-__device__ __forceinline__ CatMask scan_mask(const LaneRows& L, int self, const RecV& rec, A&& acc)
-{
-    const uint64_t m0 = scan_row(L.k0[0], L.k1[0], self, rec, acc);
-    const uint64_t m1 = scan_row(L.k0[1], L.k1[1], self, rec, acc);
-    const uint64_t m2 = scan_row(L.k0[2], L.k1[2], self, rec, acc);
-    return cat_masks(L, m0, m1, m2);
-}
-
-// The exact partner mask from a neighbour-list mask: the listed candidates
-// (bits of vm over the rows L) whose current positions pass accept(k, xy).
-// Four candidates' positions are loaded back to back.  A list that
-// overflowed (ovf) stays overflowed: the visit then walks the rows with the
-// exact predicate.
-template <class A>
-__device__ __forceinline__ CatMask filter_mask(const LaneRows& L, const CatMask& vm, const RecV& rec, A&& acc)
-{
-    if (vm.ovf) return vm;
-    const int s1 = L.k1[0] - L.k0[0], s2 = s1 + L.k1[1] - L.k0[1];
-    const int e0 = L.k0[0], e1 = L.k0[1] - s1, e2 = L.k0[2] - s2;
-    uint64_t lo = vm.lo, hi = vm.hi, olo = 0, ohi = 0;
-#pragma unroll 1
-    for (;;) {
-        int c[4], k[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {   // next listed bit: position c, record index k (-1: none)
-            const bool in_lo = lo != 0;
-            const uint64_t m = in_lo ? lo : hi;
-            c[j] = m ? __builtin_ctzll(m) + (in_lo ? 0 : 64) : -1;
-            const uint64_t rest = m & (m - 1);
-            lo = in_lo ? rest : lo;
-            hi = in_lo ? hi : rest;
-            k[j] = c[j] < 0 ? -1 : c[j] + (c[j] < s1 ? e0 : (c[j] < s2 ? e1 : e2));
-        }
-        if (k[0] < 0) break;
-        double2 p[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) p[j] = rec(k[j] >= 0 ? k[j] : k[0], 0);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if (k[j] >= 0 && acc(k[j], p[j])) {
-                if (c[j] < 64) olo |= 1ull << c[j];
-                else ohi |= 1ull << (c[j] - 64);
-            }
-        }
-        if (k[3] < 0) break;
-    }
-    CatMask out;
-    out.lo = olo;
-    out.hi = ohi;
-    out.ovf = 0;
-    return out;
-}
-
 __device__ __forceinline__ CatMask mask_of(const Masks& M, int n, int t)
 {
     CatMask c;
@@ -905,50 +788,52 @@ __device__ __forceinline__ CatMask mask_of(const Masks& M, int n, int t)
     return c;
 }
 
-// Candidate rows of particle tt: the 3 x 3 block of its cell at the list
-// rebuild (row-major key NL.cell[tt]), or (no lists: NL.cell == nullptr) of
-// its current cell.
-__device__ __forceinline__ LaneRows cand_rows(const Grid& g, const int* cell_start, const NList& NL, int tt,
-                                              double xa, double ya)
-{
-    int cx, cy;
-    if (NL.cell) {
-        const int key = NL.cell[tt];
-        cy = key / g.ncx;
-        cx = key - cy * g.ncx;
-    } else {
-        clamped_cell(g, xa, ya, cx, cy);
-    }
-    return lane_rows(block_rows_at(g, cell_start, cx, cy));
-}
-
-// Partner mask of particle tt over the rows L: the list M filtered by the
-// exact predicate, or (no lists: M.m == nullptr) the scan of the rows.
-template <class A>
-__device__ __forceinline__ CatMask cand_mask(const LaneRows& L, const Masks& M, int n, int tt, int self,
-                                             const RecV& rec, A&& acc)
-{
-    if (M.m) return filter_mask(L, mask_of(M, n, tt), rec, acc);
-    return scan_mask(L, self, rec, acc);
-}
-
 // Neighbour lists of phase A against phase B (cell list startB on grid g,
 // candidate k at state slot ordB[k], or k when ordB is null: the state in
 // cell order, as a rebuild leaves it): candidates with dr < thr (thr =
 // (R + skin)^2 of the pair type), the particle itself excluded when same.
 // Also records each particle's cell key.  Positions come from the state, so
 // the FP64 and the FP32 records share the lists.
+// The window of a workgroup of the stage kernels (pb consecutive particles):
+// their cells are a run of row-major keys [ka, kb], so all their candidates
+// lie in the runs [ka - 1, kb + 1] of the row below, the same row and the row
+// above -- three contiguous ranges of records, also where the run wraps from
+// one grid row into the next.
 __device__ __forceinline__ void nlist_body(int blk, const double* xA, const double* yA, const int* ordA, int nA,
                                            const double* xB, const double* yB, const int* ordB, const int* startB,
-                                           Grid g, double thr, int same, Masks VM, int* cell)
+                                           Grid g, double thr, int same, Masks VM, int* cell, IdxList IL, int pb)
 {
     const int t = blk * blockDim.x + threadIdx.x;
     if (t >= nA) return;
+    const int ncell = g.ncx * g.ncy;
+    auto key_of = [&](int u) {
+        const int i = ordA ? ordA[u] : u;
+        int cx, cy;
+        clamped_cell(g, xA[i], yA[i], cx, cy);
+        return cy * g.ncx + cx;
+    };
     const int ia = ordA ? ordA[t] : t;
     const double px = xA[ia], py = yA[ia];
-    int cx, cy;
-    clamped_cell(g, px, py, cx, cy);
-    if (cell) cell[t] = cy * g.ncx + cx;
+    const int key = key_of(t), cy = key / g.ncx, cx = key - cy * g.ncx;
+    if (cell) cell[t] = key;
+    const int wb = t / pb, ka = key_of(wb * pb), kb = key_of(min(nA, (wb + 1) * pb) - 1);
+    int lo[3], off[3], tot = 0;
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        const int a = max(ka + (r - 1) * g.ncx - 1, 0), b = min(kb + (r - 1) * g.ncx + 1, ncell - 1);
+        lo[r] = a <= b ? startB[a] : 0;
+        off[r] = tot;
+        tot += a <= b ? startB[b + 1] - lo[r] : 0;
+    }
+    if (t == wb * pb) {
+        int* w = IL.win + (size_t)wb * WIN_INTS;
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            w[r] = lo[r];
+            w[3 + r] = off[r];
+        }
+        w[6] = tot;
+    }
     const LaneRows L = lane_rows(block_rows_at(g, startB, cx, cy));
     auto acc = [&](int k) {
         const int ib = ordB ? ordB[k] : k;
@@ -957,35 +842,303 @@ __device__ __forceinline__ void nlist_body(int blk, const double* xA, const doub
     };
     const int self = same ? t : -1;
     uint64_t m[3];
+    int cnt = 0;
 #pragma unroll
     for (int r = 0; r < 3; ++r) {
         const int k0 = r == 0 ? L.k0[0] : (r == 1 ? L.k0[1] : L.k0[2]);
         const int k1 = r == 0 ? L.k1[0] : (r == 1 ? L.k1[1] : L.k1[2]);
         uint64_t mm = 0;
-        if (k1 - k0 <= 64) {
 #pragma unroll 4
-            for (int k = k0; k < k1; ++k) mm |= (uint64_t)(k != self && acc(k)) << (k - k0);
+        for (int k = k0; k < k1; ++k) {
+            const bool ok = k != self && acc(k);
+            if (k - k0 < 64) mm |= (uint64_t)ok << (k - k0);
+            if (ok) {
+                if (cnt < IL.cap) IL.li[(size_t)cnt * nA + t] = (unsigned short)(off[r] + (k - lo[r]));
+                ++cnt;
+            }
         }
-        m[r] = mm;
+        m[r] = k1 - k0 <= 64 ? mm : 0;
     }
     const CatMask cm = cat_masks(L, m[0], m[1], m[2]);
     VM.m[t] = cm.lo;
     VM.m[nA + t] = cm.hi;
     VM.ovf[t] = cm.ovf;
+    IL.cnt[t] = cnt <= IL.cap && tot < 65536 ? cnt : -1;
 }
 
 __global__ __launch_bounds__(256) void k_nlist(const double* xA, const double* yA, const int* ordA, int nA,
                                                const double* xB, const double* yB, const int* ordB, const int* startB,
-                                               Grid g, double thr, int same, Masks VM, int* cell)
+                                               Grid g, double thr, int same, Masks VM, int* cell, IdxList IL, int pb)
 {
-    nlist_body(xcd_block(), xA, yA, ordA, nA, xB, yB, ordB, startB, g, thr, same, VM, cell);
+    nlist_body(xcd_block(), xA, yA, ordA, nA, xB, yB, ordB, startB, g, thr, same, VM, cell, IL, pb);
 }
 
-// Chunks read per partner by each loop (h only when it is not uniform).
-constexpr int NEED_SAME_A = 0x07 | NEED_IV;          // x,y v rho,m(itype in its sign); 1/rho, m/rho
-constexpr int NEED_WX_A = 0x0F | NEED_IV;            // soil partners of water: x,y v rho,m vof
-constexpr int NEED_SX_A = 0x0F | NEED_IV;            // water partners of soil: x,y v rho,m vof,p
-constexpr int NEED_B = 0x3F | NEED_IV;               // x,y v rho,m vof,p s3,c s1,s2
+// ------------------------------------------------------------------------
+// Partner visit of the FP64 stage kernels.
+//
+// In list mode with a uniform smoothing length a workgroup first copies its
+// window's record chunks into LDS, then every lane goes through its list,
+// reading the partners there (the next partner's chunks in flight beside the
+// current one's terms); candidates outside the support (about one in six, in
+// the skin) are evaluated with W = s = 0.  What bound the gathers from global
+// memory was the L1's tag lookups: a 64-lane 16-byte gather of such partners
+// takes 34 of them (one per cycle and CU; 16 for contiguous lanes), where the
+// same LDS read takes about 8 cycles.  The copy itself is contiguous.  What
+// bounds the kernels now is the latency of the copy and of the particles' own
+// loads at two to four workgroups per CU (without the partner loop soil_ab still
+// takes 55 us of 102).  1M slope, us per launch, gathers from global memory
+// through 128-bit masks -> this: soil_ab 130 -> 102, soil_x 82 -> 77, water_a
+// 69 -> 48, water_b 73 -> 55, water_x 64 -> 50.
+//
+// Otherwise (no lists, smoothing lengths that vary, link_list's reach, a
+// window that does not fit): the candidates are the particle's list, or its
+// three candidate rows.  Four at a time their positions are tested with the
+// exact predicate; the indices that pass are put into the lane's column of an
+// LDS table, and the dense loop reads them back in order.  The loop control is
+// wave-uniform: the test runs until some lane's column is full or all
+// candidates are done.
+// ------------------------------------------------------------------------
+constexpr int VIS_ROWS = 32;            // column height
+constexpr int VIS_CAP = VIS_ROWS - 1;   // (the loop reads one past the last entry)
+
+// Record index of a position of three concatenated ranges: starts s1 and s2
+// of the second and third, record index - position in each.
+struct Ranges3 {
+    int s1, s2, e0, e1, e2;
+    __device__ __forceinline__ int operator()(int i) const { return i + pick(i < s1, e0, pick(i < s2, e1, e2)); }
+};
+
+// Where a particle's candidates come from: its list, or (none, or one that
+// overflowed: walk) the candidate rows of its cell.
+struct Cand {
+    const Grid& g;
+    const int *cell_start, *cell;   // cell: key at the rebuild (null: the current position's)
+    double xa, ya;
+    __device__ __forceinline__ Ranges3 rows(int tt, int& tot) const
+    {
+        int cx, cy;
+        if (cell) {
+            const int key = cell[tt];
+            cy = key / g.ncx;
+            cx = key - cy * g.ncx;
+        } else {
+            clamped_cell(g, xa, ya, cx, cy);
+        }
+        const Rows R = block_rows_at(g, cell_start, cx, cy);
+        Ranges3 r;
+        r.s1 = R.k1[0] - R.k0[0];
+        r.s2 = r.s1 + R.k1[1] - R.k0[1];
+        tot = r.s2 + R.k1[2] - R.k0[2];
+        r.e0 = R.k0[0];
+        r.e1 = R.k0[1] - r.s1;
+        r.e2 = R.k0[2] - r.s2;
+        return r;
+    }
+};
+
+__device__ __forceinline__ Ranges3 window_ranges(const int* w)
+{
+    return Ranges3{w[4], w[5], w[0], w[1] - w[4], w[2] - w[5]};
+}
+
+// A workgroup's window while its kernel runs.
+struct Window {
+    Ranges3 r;
+    bool listed, lds;   // a list exists; the window is in LDS (or on its way)
+    int cnt, k[4];      // lds: the lane's list length and first entries
+};
+
+// The candidates sub, sub + 2^lg, ... of a particle from global memory:
+// body(v, rec, k) for each that passes accept(k, xy), in order; self: own
+// record index in the candidates' phase (-1: none).  All lanes of the wave call.
+template <int NCH, class A, class B>
+__device__ __forceinline__ void visit_global(int* table, const Cand& C, const IdxList& I, const Window& w, int n,
+                                             const SubCtx& sc, int lg, int self, const RecV& rec, A&& accept,
+                                             B&& body)
+{
+    int* col = table + threadIdx.x;
+    int tot = w.listed ? I.cnt[sc.tt] : -1;
+    const bool walk = tot < 0;
+    Ranges3 rows{0, 0, 0, 0, 0};
+    if (walk) rows = C.rows(sc.tt, tot);
+    if (!sc.valid) tot = 0;
+    int j = 0;
+    do {
+        int c = 0;
+        do {
+            int k[4];
+            double2 p[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int i = j + (q << lg) + sc.sub;
+                k[q] = 0;   // (record 0 stands in past the end)
+                if (i < tot) k[q] = walk ? rows(i) : w.r(I.li[(size_t)i * n + sc.tt]);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) p[q] = rec(k[q], 0);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                col[c * STAGE_BLOCK] = k[q];
+                c += j + (q << lg) + sc.sub < tot && k[q] != self && accept(k[q], p[q]) ? 1 : 0;
+            }
+            j += 4 << lg;
+        } while (__any(j < tot) && !__any(c > VIS_CAP - 4));
+        int next = col[0];
+#pragma unroll 1
+        for (int i = 1; i <= c; ++i) {
+            const int k = next;
+            next = col[i * STAGE_BLOCK];
+            double2 v[NCH];
+#pragma unroll
+            for (int ch = 0; ch < NCH; ++ch) v[ch] = rec(k, ch);
+            body(v, rec, k);
+        }
+    } while (__any(j < tot));
+}
+
+// LDS of a stage kernel that reads NCH chunks per partner.
+template <int NCH>
+constexpr size_t VIS_LDS = sizeof(int) * VIS_ROWS * STAGE_BLOCK > sizeof(double2) * NCH * WIN_STRIDE
+                               ? sizeof(int) * VIS_ROWS * STAGE_BLOCK
+                               : sizeof(double2) * NCH * WIN_STRIDE;
+
+// Sends chunks 0 .. NCH - 1 of the workgroup's window on their way into LDS
+// (straight from global memory, no registers: all of it is in flight at once),
+// and a stand-in record (far away, finite everywhere) at WIN_CAP.  Called after
+// a kernel's own loads: loads return in order, so a use of one issued behind
+// the window would wait for all of it.
+template <bool U, int NCH>
+__device__ __forceinline__ Window open_window(unsigned char* lds, const IdxList& I, int blk, const SubCtx& sc, int lg,
+                                              int n, const RecV& rec)
+{
+    Window w{{0, 0, 0, 0, 0}, I.li != nullptr, false, 0, {0, 0, 0, 0}};
+    if (!I.li) return w;
+    const int* p = I.win + (size_t)blk * WIN_INTS;
+    w.r = window_ranges(p);
+    if constexpr (U) {
+        const int tot = p[6];
+        w.lds = I.lds && tot <= WIN_CAP;
+        if (w.lds) {
+            const uint32_t o = (uint32_t)sc.sub * n + sc.tt;
+            const size_t row = (size_t)n << lg;
+            w.cnt = I.cnt[sc.tt];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) w.k[q] = I.li[q * row + o];
+            double2* wl = reinterpret_cast<double2*>(lds);
+            if (threadIdx.x < NCH) {
+                const double f = threadIdx.x == 0 ? 1.0e18 : 1.0;
+                wl[threadIdx.x * WIN_STRIDE + WIN_CAP] = make_double2(f, f);
+            }
+            const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x & ~63);
+            for (int i0 = wave; i0 < tot; i0 += STAGE_BLOCK) {
+                const int i = i0 + (int)(threadIdx.x & 63);
+                if (i < tot) {
+                    const uint32_t at = (uint32_t)w.r(i) << 4;
+#pragma unroll
+                    for (int c = 0; c < NCH; ++c)
+                        __builtin_amdgcn_global_load_lds(
+                            (const __attribute__((address_space(1))) void*)(reinterpret_cast<const char*>(
+                                                                                rec.p + (size_t)c * rec.n) + at),
+                            (__attribute__((address_space(3))) void*)(wl + c * WIN_STRIDE + i0), 16, 0, 0);
+                }
+            }
+        }
+    }
+    return w;
+}
+
+// body(v, R, k) over the partners of the lane's particle, v the record chunks
+// 0 .. NCH - 1 and R(k, c) any other (all lanes of the workgroup call).
+template <bool U, int NCH, class A, class B>
+__device__ __forceinline__ void visit(unsigned char* lds, const Window& w, const Cand& C, const IdxList& I, int n,
+                                      const SubCtx& sc, int lg, int self, const RecV& rec, A&& accept, B&& body)
+{
+    if constexpr (U) {
+        if (w.lds) {
+            const double2* wl = reinterpret_cast<const double2*>(lds);
+            auto read = [&](double2(&v)[NCH], int k) {
+#pragma unroll
+                for (int c = 0; c < NCH; ++c) v[c] = wl[c * WIN_STRIDE + k];
+            };
+            // The lane's candidates i = 0, 1, ... are sub, sub + 2^lg, ... of
+            // the list; past its end the stand-in.  Indices are loaded two
+            // rounds ahead (the buffer is padded), chunks one.
+            const unsigned short* l = I.li;
+            const uint32_t o = (uint32_t)sc.sub * n + sc.tt;
+            const size_t row = (size_t)n << lg;
+            int k0 = w.k[0], k1 = w.k[1], n0 = w.k[2], n1 = w.k[3];
+            const int cnt = w.cnt;
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+            // candidates of the lane (none of a list that overflowed)
+            const int mine = sc.valid ? (max(cnt, 0) - sc.sub + (1 << lg) - 1) >> lg : 0;
+            double2 a[NCH], b[NCH];
+            read(a, pick(0 < mine, k0, WIN_CAP));
+            k1 = pick(1 < mine, k1, WIN_CAP);
+#pragma unroll 1
+            for (int i = 0; __any(i < mine); i += 2) {
+                l += 2 * row;
+                k0 = pick(i + 2 < mine, n0, WIN_CAP);
+                const int k2 = pick(i + 3 < mine, n1, WIN_CAP);
+                n0 = l[2 * row + o];
+                n1 = l[3 * row + o];
+                read(b, k1);
+                body(a, rec, 0);
+                read(a, k0);
+                k1 = k2;
+                body(b, rec, 0);
+            }
+            // a particle whose list overflowed walks its rows
+            if (cnt < 0 && sc.valid) {
+                int tot;
+                const Ranges3 rows = C.rows(sc.tt, tot);
+#pragma unroll 1
+                for (int i = sc.sub; i < tot; i += 1 << lg) {
+                    const int k = rows(i);
+                    if (k == self || !accept(k, rec(k, 0))) continue;
+#pragma unroll
+                    for (int c = 0; c < NCH; ++c) a[c] = rec(k, c);
+                    body(a, rec, k);
+                }
+            }
+            return;
+        }
+    }
+    visit_global<NCH>(reinterpret_cast<int*>(lds), C, I, w, n, sc, lg, self, rec, accept, body);
+}
+
+// ------------------------------------------------------------------------
+// Pair terms.  With grad W = s d (d the separation) every product of a
+// stage is a combination of s, d, the velocity difference u and vr = u.d:
+// u.grad W = s vr, and delta_sph's 2 (d.grad W) / d^2 = 2 s.  Records hold the
+// partner's volume V = m / rho, so V s d and m = V rho replace its
+// reciprocals.
+// ------------------------------------------------------------------------
+struct Sep {
+    double dx, dy, dr, ir, w, s;
+    bool in;
+};
+
+// thr: W = s = 0 at and beyond dr = thr (the exact predicate of a uniform
+// smoothing length; listed candidates may lie outside the support).
+template <int SKF, bool NEED_W>
+__device__ __forceinline__ Sep sep_of(const KC& kc, double dx, double dy, double thr, bool coincident)
+{
+    Sep p;
+    p.dx = dx;
+    p.dy = dy;
+    {
+#pragma clang fp contract(off)
+        p.dr = dx * dx + dy * dy;
+    }
+    // (co-located particles of two phases: W(0), no gradient direction)
+    p.ir = coincident && !(p.dr > 0.0) ? 0.0 : fast_rsq(p.dr);
+    kern_s<SKF, NEED_W>(kc, p.dr * p.ir, p.ir, p.w, p.s);
+    p.in = p.dr < thr;
+    p.s = p.in ? p.s : 0.0;
+    if (NEED_W) p.w = p.in ? p.w : 0.0;
+    return p;
+}
 
 // ------------------------------------------------------------------------
 // Cross terms, water side (stage A of single_step's interaction block,
@@ -994,59 +1147,63 @@ constexpr int NEED_B = 0x3F | NEED_IV;               // x,y v rho,m vof,p s3,c s
 // soil partners (direct_find_2's pairs, virtual x virtual and r = 0
 // included).  Its own kernel: the loop needs few registers, so it runs at
 // twice the occupancy of the same-phase stage.
+// lean (all stages): another step of the same call follows, so the values
+// that only a download or the last step's diagnostics would read stay out.
 // ------------------------------------------------------------------------
 template <int SKF, bool U>
 __device__ __forceinline__ void water_x4(int blk, DPhase W, DPhase S, const double* recW, const double* recS,
-                                         NList NL, Grid g, KParams K, FusedK F)
+                                         NList NL, Grid g, KParams K, FusedK F, int lean)
 {
     const RecV RW = recv(recW, W.n), RS = recv(recS, S.n);
-    const WaveCtx wc = wave_ctx(W.n, blk);
-    const double2 xy = RW(wc.tt, 0), va = RW(wc.tt, 1), rm = RW(wc.tt, 2);
-    const double xa = xy.x, ya = xy.y, vxa = va.x, vya = va.y, rhoa = rm.x, vofa = RW(wc.tt, 3).x;
+    __shared__ __align__(16) unsigned char lds[VIS_LDS<4>];
+    const SubCtx wc = sub_ctx(W.n, blk, NL.lg, WIN_LANES);
+    const double2 xy = RW(wc.tt, 0), va = RW(wc.tt, 1);
+    const double xa = xy.x, ya = xy.y, vxa = va.x, vya = va.y, vofa = RW(wc.tt, 3).x;
     const double ha = U ? K.h1_water : RW(wc.tt, 6).x;
-    const double irhoa = 1.0 / rhoa;
-    const int a = W.order[wc.tt];
+    const int a = NL.cell ? wc.tt : W.order[wc.tt];
     const bool ux = U || F.uni_x;
-    const LaneRows L = cand_rows(g, S.cell_start, NL, wc.tt, xa, ya);
+    const Window win = open_window<U, 4>(lds, NL.ix, blk, wc, NL.lg, W.n, RS);
+    const Cand C{g, S.cell_start, NL.cell, xa, ya};
     const Pred PX{xa, ya, ha, F.thr_x, ux ? 1 : 0, 0};
-    auto acc = [&](int k, double2 b) { return PX(b, ux ? ha : RS(k, 6).x, g, K); };
-    auto acc_k = [&](int k) { return acc(k, RS(k, 0)); };
-    const CatMask cm = cand_mask(L, NL.cross, W.n, wc.tt, -1, RS, acc);
-    const Loader<NEED_WX_A> load{RS, !ux, false};
-    const double cfa = vofa * rhoa * (-K.numeric_gravity) / K.s_perm;
     const KC kx = make_kc(SKF, sph_mhsml(ha, ux ? RS(0, 6).x : ha));
     double dg_x = 0.0, dg_y = 0.0, dvof_x = 0.0, vof2 = 0.0;
     int cntx = 0;
-    visit(cat_iter(cm, L), L, cm.ovf, -1, load, acc_k, [&](const Nb& b) {
-        const double dx = xa - b.xy.x, dy = ya - b.xy.y;
-        const double dr = dx * dx + dy * dy;
-        const double ir = (dr > 0.0) ? fast_rsq(dr) : 0.0;
-        const double r = dr * ir;
-        double ww, gx, gy;
-        if (ux) kern_fast<SKF, true>(kx, r, ir, dx, dy, ww, gx, gy);
-        else kern_fast<SKF, true>(make_kc(SKF, sph_mhsml(ha, b.hv.x)), r, ir, dx, dy, ww, gx, gy);
-        ++cntx;
-        const double mb = b.rm.y;
-        const double dvx = vxa - b.v.x, dvy = vya - b.v.y;
-        const double sc = mb * (cfa * b.hv.y) * (ww * irhoa * b.iv.x);
-        dg_x += sc * dvx;
-        dg_y += sc * dvy;
-        dvof_x += mb * (dvx * gx + dvy * gy);
-        vof2 += mb * ww;
-    });
-    if (!wc.valid) return;
-    W.drgx[a] = dg_x;
-    W.drgy[a] = dg_y;
+    visit<U, 4>(
+        lds, win, C, NL.ix, W.n, wc, NL.lg, -1, RS, [&](int k, double2 b) { return PX(b, ux ? ha : RS(k, 6).x, g, K); },
+        [&](const auto& v, const auto& R, int k) {
+            const double2 b = v[0], u = v[1], q = v[2];
+            const double vr_b = v[3].x;   // vof / rho
+            KC kc = kx;
+            if (!ux) kc = make_kc(SKF, sph_mhsml(ha, R(k, 6).x));
+            const Sep p = sep_of<SKF, true>(kc, xa - b.x, ya - b.y, U ? F.thr_x : INFINITY, true);
+            cntx += p.in ? 1 : 0;
+            const double m = fabs(q.y) * q.x, mw = m * p.w;
+            const double dvx = vxa - u.x, dvy = vya - u.y;
+            const double sc = mw * vr_b;
+            dg_x += sc * dvx;
+            dg_y += sc * dvy;
+            dvof_x += (m * p.s) * (dvx * p.dx + dvy * p.dy);
+            vof2 += mw;
+        });
+    sub_sum(NL.lg, dg_x, dg_y, dvof_x, vof2);
+    cntx = sub_count(NL.lg, cntx);
+    if (!wc.valid || wc.sub) return;
+    // vof_a vof_b rho_a (-g) / perm * W / (rho_a rho_b): rho_a cancels
+    const double cfa = vofa * (-K.numeric_gravity) / K.s_perm;
+    W.drgx[a] = cfa * dg_x;
+    W.drgy[a] = cfa * dg_y;
     W.dvof_x[a] = dvof_x * (1.0 / K.s_rho0);
-    W.vof2[a] = 1.0 - vof2 / K.s_rho0;
-    W.countiac[a] = cntx;
+    if (!lean) {
+        W.vof2[a] = 1.0 - vof2 / K.s_rho0;
+        W.countiac[a] = cntx;
+    }
 }
 
 template <int SKF, bool U>
 __global__ STAGE_ATTR void k_water_x4(DPhase W, DPhase S, const double* recW, const double* recS, NList NL, Grid g,
-                                      KParams K, FusedK F)
+                                      KParams K, FusedK F, int lean)
 {
-    water_x4<SKF, U>(xcd_block(), W, S, recW, recS, NL, g, K, F);
+    water_x4<SKF, U>(xcd_block(), W, S, recW, recS, NL, g, K, F, lean);
 }
 
 // ------------------------------------------------------------------------
@@ -1056,136 +1213,148 @@ __global__ STAGE_ATTR void k_water_x4(DPhase W, DPhase S, const double* recW, co
 // ------------------------------------------------------------------------
 template <int SKF, bool U>
 __device__ __forceinline__ void soil_x4(int blk, DPhase S, DPhase W, const double* recS, const double* recW, NList NL,
-                                        Grid g, KParams K, FusedK F)
+                                        Grid g, KParams K, FusedK F, int lean)
 {
     const RecV RS = recv(recS, S.n), RW = recv(recW, W.n);
-    const WaveCtx wc = wave_ctx(S.n, blk);
-    const double2 xy = RS(wc.tt, 0), va = RS(wc.tt, 1), rm = RS(wc.tt, 2);
-    const double xa = xy.x, ya = xy.y, vxa = va.x, vya = va.y, rhoa = rm.x, vofa = RS(wc.tt, 3).x;
+    __shared__ __align__(16) unsigned char lds[VIS_LDS<4>];
+    const SubCtx wc = sub_ctx(S.n, blk, NL.lg, WIN_LANES);
+    const double2 xy = RS(wc.tt, 0), va = RS(wc.tt, 1);
+    const double xa = xy.x, ya = xy.y, vxa = va.x, vya = va.y;
+    const double vra = RS(wc.tt, 3).x;   // vof / rho
     const double ha = U ? K.h1_soil : RS(wc.tt, 6).x;
-    const double irhoa = 1.0 / rhoa;
-    const int a = S.order[wc.tt];
+    const int a = NL.cell ? wc.tt : S.order[wc.tt];
     const bool ux = U || F.uni_x;
-    const LaneRows L = cand_rows(g, W.cell_start, NL, wc.tt, xa, ya);
+    const Window win = open_window<U, 4>(lds, NL.ix, blk, wc, NL.lg, S.n, RW);
+    const Cand C{g, W.cell_start, NL.cell, xa, ya};
     const Pred PX{xa, ya, ha, F.thr_x, ux ? 1 : 0, 0};
-    auto acc = [&](int k, double2 b) { return PX(b, ux ? ha : RW(k, 6).x, g, K); };
-    auto acc_k = [&](int k) { return acc(k, RW(k, 0)); };
-    const CatMask cm = cand_mask(L, NL.cross, S.n, wc.tt, -1, RW, acc);
-    const Loader<NEED_SX_A> load{RW, !ux, false};
-    const double cfs = vofa * (-K.numeric_gravity) / K.s_perm;
     const KC kx = make_kc(SKF, sph_mhsml(ux ? RW(0, 6).x : ha, ha));
     double dg_x = 0.0, dg_y = 0.0, po_x = 0.0, po_y = 0.0;
     int cntx = 0;
-    visit(cat_iter(cm, L), L, cm.ovf, -1, load, acc_k, [&](const Nb& b) {
-        const double dx = b.xy.x - xa, dy = b.xy.y - ya;   // water - soil
-        const double dr = dx * dx + dy * dy;
-        const double ir = (dr > 0.0) ? fast_rsq(dr) : 0.0;
-        const double r = dr * ir;
-        double ww, gx, gy;
-        if (ux) kern_fast<SKF, true>(kx, r, ir, dx, dy, ww, gx, gy);
-        else kern_fast<SKF, true>(make_kc(SKF, sph_mhsml(b.hv.x, ha)), r, ir, dx, dy, ww, gx, gy);
-        ++cntx;
-        const double mw = b.rm.y, rhow = b.rm.x;
-        const double sc = mw * (b.hv.y * rhow * cfs) * (ww * b.iv.x * irhoa);
-        dg_x += sc * (b.v.x - vxa);
-        dg_y += sc * (b.v.y - vya);
-        const double mprr = mw * b.pc.x * (b.iv.x * irhoa);
-        po_x += mprr * gx;
-        po_y += mprr * gy;
-    });
-    if (!wc.valid) return;
-    S.drgx[a] = dg_x;
-    S.drgy[a] = dg_y;
-    S.porx[a] = vofa * po_x;
-    S.pory[a] = vofa * po_y;
-    S.countiac[a] = cntx;
+    visit<U, 4>(
+        lds, win, C, NL.ix, S.n, wc, NL.lg, -1, RW, [&](int k, double2 b) { return PX(b, ux ? ha : RW(k, 6).x, g, K); },
+        [&](const auto& v, const auto& R, int k) {
+            const double2 b = v[0], u = v[1], q = v[2], f = v[3];   // f = (vof, p)
+            KC kc = kx;
+            if (!ux) kc = make_kc(SKF, sph_mhsml(R(k, 6).x, ha));
+            // water - soil
+            const Sep p = sep_of<SKF, true>(kc, b.x - xa, b.y - ya, U ? F.thr_x : INFINITY, true);
+            cntx += p.in ? 1 : 0;
+            const double V = fabs(q.y);
+            // m_w vof_w rho_w W / (rho_w rho_s): the soil's factors outside
+            const double sc = (V * q.x) * (f.x * p.w);
+            dg_x += sc * (u.x - vxa);
+            dg_y += sc * (u.y - vya);
+            const double vp = (V * f.y) * p.s;
+            po_x += vp * p.dx;
+            po_y += vp * p.dy;
+        });
+    sub_sum(NL.lg, dg_x, dg_y, po_x, po_y);
+    cntx = sub_count(NL.lg, cntx);
+    if (!wc.valid || wc.sub) return;
+    const double cfs = vra * (-K.numeric_gravity) / K.s_perm;
+    S.drgx[a] = cfs * dg_x;
+    S.drgy[a] = cfs * dg_y;
+    S.porx[a] = vra * po_x;
+    S.pory[a] = vra * po_y;
+    if (!lean) S.countiac[a] = cntx;
 }
 
 template <int SKF, bool U>
 __global__ STAGE_ATTR void k_soil_x4(DPhase S, DPhase W, const double* recS, const double* recW, NList NL, Grid g,
-                                     KParams K, FusedK F)
+                                     KParams K, FusedK F, int lean)
 {
-    soil_x4<SKF, U>(xcd_block(), S, W, recS, recW, NL, g, K, F);
+    soil_x4<SKF, U>(xcd_block(), S, W, recS, recW, NL, g, K, F, lean);
+}
+
+// repulsive_force on a real particle from a virtual partner within r0
+// (m_particles.f90:1605): D ((r0/r)^p1 - (r0/r)^p2) d / r^2; ir = 1/r.
+template <bool U>
+__device__ __forceinline__ double rep_factor(const KParams& K, double r0, double ir)
+{
+    const double q = r0 * ir;
+    return K.dd * (U ? ipow(q, K.ip1) - ipow(q, K.ip2) : pow(q, K.p1) - pow(q, K.p2)) * (ir * ir);
 }
 
 // ------------------------------------------------------------------------
 // Stage A, water: same-phase terms (con_density, delta_sph(rho),
 // shear_strain_rate, av_vel, repulsive_force), then pressure() per particle.
-// Writes a-space outputs, the same-phase masks and the record slots
-// vof*sigma for stage B.  cross: two-phase run (countiac then counts the
-// soil partners, which k_water_x4 writes).
+// Writes a-space outputs and the record slots vof*sigma for stage B.  cross:
+// two-phase run (countiac then counts the soil partners, which k_water_x4
+// writes).
 // ------------------------------------------------------------------------
 template <int SKF, bool U>
-__device__ __forceinline__ void water_a4(int blk, DPhase W, const double* recW, double* recWw, NList NL, Masks MW,
-                                         Grid g, KParams K, FusedK F, int cross)
+__device__ __forceinline__ void water_a4(int blk, DPhase W, const double* recW, double* recWw, NList NL, Grid g,
+                                         KParams K, FusedK F, int cross, int lean)
 {
     const RecV RW = recv(recW, W.n);
-    const WaveCtx wc = wave_ctx(W.n, blk);
+    __shared__ __align__(16) unsigned char lds[VIS_LDS<3>];
+    const SubCtx wc = sub_ctx(W.n, blk, NL.lg, WIN_LANES);
     const int t = wc.t;
     auto RA = [&](int c) { return RW(wc.tt, c); };
-    const double2 xy = RA(0), va = RA(1), rm = RA(2), hi = RA(6);
+    const double2 xy = RA(0), va = RA(1);
     const bool link = K.nnps == 2;
     // U (checked by the host): h uniform in the phase (hsml(1) everywhere, a
     // wave-uniform value), integer repulsion exponents
-    const double xa = xy.x, ya = xy.y, vxa = va.x, vya = va.y, rhoa = rm.x, vofa = RA(3).x;
-    const double ha = U ? K.h1_water : hi.x;
-    const int ita = (int)hi.y;
-    const int a = W.order[wc.tt];
+    const double xa = xy.x, ya = xy.y, vxa = va.x, vya = va.y, rhoa = RA(2).x, vofa = RA(3).x;
+    const double ha = U ? K.h1_water : RA(6).x;
+    const int a = NL.cell ? wc.tt : W.order[wc.tt];
     const double ca = W.c[a];
     const bool uni = U || link || F.uni_w;
-    const KC kc = make_kc(SKF, link ? K.h1_water : ha);
-    const LaneRows L = cand_rows(g, W.cell_start, NL, wc.tt, xa, ya);
+    const KC kc0 = make_kc(SKF, link ? K.h1_water : ha);
+    const int ita = W.itype[a];
+    const Window win = open_window<U, 3>(lds, NL.is, blk, wc, NL.lg, W.n, RW);
+    const Cand C{g, W.cell_start, NL.cell, xa, ya};
     const Pred P{xa, ya, ha, F.thr_w, uni ? 1 : 0, link ? 1 : 0};
-    auto acc = [&](int k, double2 b) { return P(b, uni ? ha : RW(k, 6).x, g, K); };
-    auto acc_k = [&](int k) { return acc(k, RW(k, 0)); };
-    const CatMask cm = cand_mask(L, NL.same, W.n, wc.tt, t, RW, acc);
-    if (wc.valid) {
-        MW.m[t] = cm.lo;
-        MW.m[W.n + t] = cm.hi;
-        MW.ovf[t] = cm.ovf;
-    }
-    const Loader<NEED_SAME_A> load{RW, !uni, false};
-    double con = 0.0, drd = 0.0, txx = 0.0, txy = 0.0, tyy = 0.0, avx = 0.0, avy = 0.0, repx = 0.0, repy = 0.0;
+    const double rep2 = ita > 0 ? W.dspp * W.dspp : -1.0;   // real particles feel the wall
+    double con = 0.0, drd = 0.0, xx = 0.0, yy = 0.0, xy2 = 0.0, avx = 0.0, avy = 0.0, repx = 0.0, repy = 0.0;
     int cnt = 0;
-    visit(cat_iter(cm, L), L, cm.ovf, t, load, acc_k, [&](const Nb& b) {
-        const double dx = xa - b.xy.x, dy = ya - b.xy.y;
-        const double dr = dx * dx + dy * dy;
-        const Dist D = dist_of(dr);
-        const double r = D.r, idr = D.idr;
-        double ww, gx, gy;
-        if (uni) kern_fast<SKF, true>(kc, r, D.ir, dx, dy, ww, gx, gy);
-        else kern_fast<SKF, true>(make_kc(SKF, sph_mhsml(ha, b.hv.x)), r, D.ir, dx, dy, ww, gx, gy);
-        ++cnt;
-        const double mb = b.rm.y, Vb = b.iv.y;
-        const double dvx = vxa - b.v.x, dvy = vya - b.v.y;
-        con += mb * (dvx * gx + dvy * gy);
-        drd += mb * (2.0 * (rhoa - b.rm.x) * idr * (dx * gx + dy * gy)) * b.iv.x;
-        txx += Vb * (-2.0 * dvx * gx + dvy * gy);
-        txy += Vb * (-(dvx * gy) - dvy * gx);
-        tyy += Vb * (-2.0 * dvy * gy + dvx * gx);
-        const double f = mb * ww * (2.0 * fast_rcp(rhoa + b.rm.x));
-        avx -= dvx * f;
-        avy -= dvy * f;
-        if (ita > 0 && !(r > W.dspp) && (int)b.s3.y < 0) {
-            const double q = W.dspp / r;
-            const double fr = (U ? ipow(q, K.ip1) - ipow(q, K.ip2) : pow(q, K.p1) - pow(q, K.p2)) * idr;
-            repx += K.dd * dx * fr;
-            repy += K.dd * dy * fr;
-        }
-    });
-    if (!wc.valid) return;
+    visit<U, 3>(
+        lds, win, C, NL.is, W.n, wc, NL.lg, t, RW, [&](int k, double2 b) { return P(b, uni ? ha : RW(k, 6).x, g, K); },
+        [&](const auto& v, const auto& R, int k) {
+            const double2 b = v[0], u = v[1], q = v[2];
+            KC kc = kc0;
+            if (!uni) kc = make_kc(SKF, sph_mhsml(ha, R(k, 6).x));
+            const Sep p = sep_of<SKF, true>(kc, xa - b.x, ya - b.y, U ? F.thr_w : INFINITY, false);
+            cnt += p.in ? 1 : 0;
+            const double V = fabs(q.y), dvx = vxa - u.x, dvy = vya - u.y, vr = dvx * p.dx + dvy * p.dy;
+            const double Vs = V * p.s, wx = Vs * p.dx, wy = Vs * p.dy;
+            con += (Vs * q.x) * vr;
+            drd += Vs * (rhoa - q.x);
+            xx += wx * dvx;
+            yy += wy * dvy;
+            xy2 += wy * dvx;
+            xy2 += wx * dvy;
+            const double f = (V * q.x) * (p.w * fast_rcp(rhoa + q.x));
+            avx -= f * dvx;
+            avy -= f * dvy;
+            if (q.y < 0.0 && p.dr <= rep2) {
+                const double fr = rep_factor<U>(K, W.dspp, p.ir);
+                repx += p.dx * fr;
+                repy += p.dy * fr;
+            }
+        });
+    sub_sum(NL.lg, con, drd, xx, yy, xy2, avx, avy, repx, repy);
+    cnt = sub_count(NL.lg, cnt);
+    if (!wc.valid || wc.sub) return;
     const double mu = K.w_mu;
-    txx *= SPH_C23_F;
-    tyy *= SPH_C23_F;
+    const double txx = SPH_C23_F * (yy - 2.0 * xx), tyy = SPH_C23_F * (xx - 2.0 * yy), txy = -xy2;
     // delta_sph(rho) and av_vel only under their switches (artificial_density,
     // average_velocity); without av_vel the reference leaves av as it was
-    W.drho[a] = K.artificial_density ? con + (K.delta * ha * ca) * drd : con;
-    W.txx[a] = txx; W.txy[a] = txy; W.tyy[a] = tyy;
-    if (ita > 0) { avx *= K.epsilon; avy *= K.epsilon; }
-    if (K.average_velocity) { W.avx[a] = avx; W.avy[a] = avy; }
-    W.repx[a] = repx; W.repy[a] = repy;
-    if (!cross) W.countiac[a] = cnt;
-    W.nsame[a] = cnt;
+    W.drho[a] = K.artificial_density ? con + (K.delta * ha * ca) * (2.0 * drd) : con;
+    if (K.average_velocity) {
+        const double e = ita > 0 ? 2.0 * K.epsilon : 2.0;
+        W.avx[a] = e * avx;
+        W.avy[a] = e * avy;
+    }
+    W.repx[a] = repx;
+    W.repy[a] = repy;
+    if (!lean) {
+        W.txx[a] = txx;
+        W.txy[a] = txy;
+        W.tyy[a] = tyy;
+        if (!cross) W.countiac[a] = cnt;
+        W.nsame[a] = cnt;
+    }
     // p and the new c (chunks 3 and 4) come from the pack
     double2* WP = reinterpret_cast<double2*>(recWw) + t;
     const size_t nw = (size_t)W.n;
@@ -1194,93 +1363,98 @@ __device__ __forceinline__ void water_a4(int blk, DPhase W, const double* recW, 
 }
 
 template <int SKF, bool U>
-__global__ STAGE_ATTR void k_water_a4(DPhase W, const double* recW, double* recWw, NList NL, Masks MW, Grid g,
-                                      KParams K, FusedK F, int cross)
+__global__ STAGE_ATTR void k_water_a4(DPhase W, const double* recW, double* recWw, NList NL, Grid g, KParams K,
+                                      FusedK F, int cross, int lean)
 {
-    water_a4<SKF, U>(xcd_block(), W, recW, recWw, NL, MW, g, K, F, cross);
+    water_a4<SKF, U>(xcd_block(), W, recW, recWw, NL, g, K, F, cross, lean);
 }
 
 // ------------------------------------------------------------------------
 // Stage B, water: -vof*df(p) + df(vof*sigma) (declarations_sph.f90:1257-1265),
 // art_visc, delta_sph(vof, dvof); /rho, + repulsion, + gravity, - Darcy drag.
-// The partner masks come from stage A.
 // ------------------------------------------------------------------------
 template <int SKF, bool U>
-__device__ __forceinline__ void water_b4(int blk, DPhase W, const double* recW, NList NL, Masks MW, Grid g, KParams K,
-                                         FusedK F, int mask)
+__device__ __forceinline__ void water_b4(int blk, DPhase W, const double* recW, NList NL, Grid g, KParams K, FusedK F,
+                                         int mask)
 {
     const RecV RW = recv(recW, W.n);
-    const WaveCtx wc = wave_ctx(W.n, blk);
+    __shared__ __align__(16) unsigned char lds[VIS_LDS<6>];
+    const SubCtx wc = sub_ctx(W.n, blk, NL.lg, WIN_LANES);
     const int t = wc.t;
     auto RA = [&](int c) { return RW(wc.tt, c); };
-    const double2 axy = RA(0), av = RA(1), arm = RA(2), a3 = RA(3), apc = RA(4), a12 = RA(5);
+    const double2 axy = RA(0), av = RA(1), arv = RA(2), a3 = RA(3), a4 = RA(4), a12 = RA(5);
     // U: h uniform in the phase (checked by the host)
-    const double xa = axy.x, ya = axy.y, vxa = av.x, vya = av.y, rhoa = arm.x, vofa = a3.x;
+    const double xa = axy.x, ya = axy.y, vxa = av.x, vya = av.y, rhoa = arv.x, vofa = a3.x;
     const double ha = U ? K.h1_water : RA(6).x;
-    const double pa = a3.y, ca = apc.y, fxx_a = a12.x, fxy_a = a12.y, fyy_a = apc.x;
-    const double irhoa = 1.0 / rhoa;
-    const int a = W.order[wc.tt];
+    const double pa = a3.y, ca = a4.y;
+    const int a = NL.cell ? wc.tt : W.order[wc.tt];
     const bool link = K.nnps == 2;
     const bool uni = U || link || F.uni_w;
-    const KC kc = make_kc(SKF, link ? K.h1_water : ha);
-    const LaneRows L = cand_rows(g, W.cell_start, NL, wc.tt, xa, ya);
-    const Pred P{xa, ya, ha, F.thr_w, uni ? 1 : 0, link ? 1 : 0};
-    auto acc_k = [&](int k) { return P(RW(k, 0), uni ? ha : RW(k, 6).x, g, K); };
-    const Loader<NEED_B> load{RW, !uni, false};
-    CatMask cm{0, 0, 0};
-    if (wc.valid) {
-        cm.lo = MW.m[t];
-        cm.hi = MW.m[W.n + t];
-        cm.ovf = MW.ovf[t];
+    const KC kc0 = make_kc(SKF, link ? K.h1_water : ha);
+    // (the tail's inputs, loaded before the loop)
+    const double repx = W.repx[a], repy = W.repy[a];
+    double drgx = 0.0, drgy = 0.0, dvx = 0.0;
+    if (mask & M_CROSS) {
+        drgx = W.drgx[a];
+        drgy = W.drgy[a];
+        dvx = W.dvof_x[a];
     }
+    const Window win = open_window<U, 6>(lds, NL.is, blk, wc, NL.lg, W.n, RW);
+    const Cand C{g, W.cell_start, NL.cell, xa, ya};
+    const Pred P{xa, ya, ha, F.thr_w, uni ? 1 : 0, link ? 1 : 0};
     const double et2 = K.etq * K.etq;
-    double Px = 0.0, Py = 0.0, Sxx = 0.0, Sxyy = 0.0, Sxyx = 0.0, Syy = 0.0;
-    double artx = 0.0, arty = 0.0, dvd = 0.0;
-    visit(cat_iter(cm, L), L, cm.ovf, t, load, acc_k, [&](const Nb& b) {
-        const double dx = xa - b.xy.x, dy = ya - b.xy.y;
-        const double dr = dx * dx + dy * dy;
-        const Dist D = dist_of(dr);
-        const double r = D.r, idr = D.idr;
-        double ww, gx, gy;
-        const double amh = uni ? ha : sph_mhsml(ha, b.hv.x);
-        if (uni) kern_fast<SKF, false>(kc, r, D.ir, dx, dy, ww, gx, gy);
-        else kern_fast<SKF, false>(make_kc(SKF, amh), r, D.ir, dx, dy, ww, gx, gy);
-        const double Vb = b.iv.y, mb = b.rm.y;
-        const double ps = pa + b.pc.x;
-        Px += Vb * (ps * gx);
-        Py += Vb * (ps * gy);
-        const double sxy = fxy_a + b.s12.y;
-        Sxx += Vb * ((fxx_a + b.s12.x) * gx);
-        Sxyy += Vb * (sxy * gy);
-        Sxyx += Vb * (sxy * gx);
-        Syy += Vb * ((fyy_a + b.s3.x) * gy);
-        const double vr = (vxa - b.v.x) * dx + (vya - b.v.y) * dy;
-        {   // art_visc, branch-free: approaching pairs only (vr < 0)
-            const double muv = amh * vr * fast_rcp(dr + amh * amh * et2);
-            const double mc = 0.5 * (ca + b.pc.y);
-            double piv = (K.beta * muv - K.alpha * mc) * muv * (2.0 * fast_rcp(rhoa + b.rm.x));
-            piv = vr < 0.0 ? piv : 0.0;
-            artx -= mb * piv * gx;
-            arty -= mb * piv * gy;
-        }
-        dvd += mb * (2.0 * (vofa - b.hv.y) * idr * (dx * gx + dy * gy)) * b.iv.x;
-    });
-    if (!wc.valid) return;
-    double ax = -(vofa * Px) + Sxx + Sxyy;
-    double ay = -(vofa * Py) + Sxyx + Syy;
+    double Wx = 0.0, Wy = 0.0, Fx = 0.0, Fy = 0.0, artx = 0.0, arty = 0.0, dvd = 0.0;
+    visit<U, 6>(
+        lds, win, C, NL.is, W.n, wc, NL.lg, t, RW, [&](int k, double2 b) { return P(b, uni ? ha : RW(k, 6).x, g, K); },
+        [&](const auto& v, const auto& R, int k) {
+            const double2 b = v[0], u = v[1], q = v[2], f = v[3], s3 = v[4], s12 = v[5];
+            KC kc = kc0;
+            double amh = ha;
+            if (!uni) {
+                amh = sph_mhsml(ha, R(k, 6).x);
+                kc = make_kc(SKF, amh);
+            }
+            const Sep p = sep_of<SKF, false>(kc, xa - b.x, ya - b.y, U ? F.thr_w : INFINITY, false);
+            const double Vs = fabs(q.y) * p.s, wx = Vs * p.dx, wy = Vs * p.dy;
+            const double vr = (vxa - u.x) * p.dx + (vya - u.y) * p.dy;
+            // -vof_a (p_a + p_b) + (f_a + f_b) as twice the own value (outside,
+            // times the sum of V grad W) plus the difference, which is small
+            // where the sum is not: fewer digits cancel in the total
+            const double dp = f.y - pa, fxy = a12.y + s12.y;
+            Wx = fma(Vs, p.dx, Wx);
+            Wy = fma(Vs, p.dy, Wy);
+            Fx += ((s12.x - a12.x) - vofa * dp) * wx;
+            Fx += fxy * wy;
+            Fy += ((s3.x - a4.x) - vofa * dp) * wy;
+            Fy += fxy * wx;
+            {   // art_visc, branch-free: approaching pairs only (vr < 0)
+                const double rs = rhoa + q.x, d2 = p.dr + amh * amh * et2;
+                const double it = fast_rcp(rs * d2), hv = amh * vr, muv = hv * (it * rs);
+                const double piv = (K.beta * muv - 0.5 * K.alpha * (ca + s3.y)) * (hv * it);
+                const double mp = vr < 0.0 ? (Vs * q.x) * piv : 0.0;
+                artx -= mp * p.dx;
+                arty -= mp * p.dy;
+            }
+            dvd += Vs * (vofa - f.x);
+        });
+    sub_sum(NL.lg, Wx, Wy, Fx, Fy, artx, arty, dvd);
+    if (!wc.valid || wc.sub) return;
+    double ax = Fx + 2.0 * (a12.x - vofa * pa) * Wx;
+    double ay = Fy + 2.0 * (a4.x - vofa * pa) * Wy;
     if (rhoa > 0.0) {
+        const double irhoa = 1.0 / rhoa;
         ax = ax * irhoa;
         ay = ay * irhoa;
     }
-    if (mask & M_ART) { ax = ax + artx; ay = ay + arty; }
-    ax = ax + W.repx[a];
-    ay = ay + W.repy[a];
+    if (mask & M_ART) { ax = ax + 2.0 * artx; ay = ay + 2.0 * arty; }
+    ax = ax + repx;
+    ay = ay + repy;
     ay = ay + K.gravity;
-    double dvof = (mask & M_DELTA_FIELD) ? (K.delta * ha * ca) * dvd : 0.0;
+    double dvof = (mask & M_DELTA_FIELD) ? (K.delta * ha * ca) * (2.0 * dvd) : 0.0;
     if (mask & M_CROSS) {
-        ax = ax - W.drgx[a];
-        ay = ay - W.drgy[a];
-        dvof = dvof - W.dvof_x[a];
+        ax = ax - drgx;
+        ay = ay - drgy;
+        dvof = dvof - dvx;
     }
     W.ax[a] = ax;
     W.ay[a] = ay;
@@ -1288,10 +1462,9 @@ __device__ __forceinline__ void water_b4(int blk, DPhase W, const double* recW, 
 }
 
 template <int SKF, bool U>
-__global__ STAGE_ATTR void k_water_b4(DPhase W, const double* recW, NList NL, Masks MW, Grid g, KParams K, FusedK F,
-                                      int mask)
+__global__ STAGE_ATTR void k_water_b4(DPhase W, const double* recW, NList NL, Grid g, KParams K, FusedK F, int mask)
 {
-    water_b4<SKF, U>(xcd_block(), W, recW, NL, MW, g, K, F, mask);
+    water_b4<SKF, U>(xcd_block(), W, recW, NL, g, K, F, mask);
 }
 
 // ------------------------------------------------------------------------
@@ -1311,125 +1484,148 @@ __global__ STAGE_ATTR void k_water_b4(DPhase W, const double* recW, NList NL, Ma
 // ------------------------------------------------------------------------
 template <int SKF, bool U, bool SOLO>
 __device__ __forceinline__ void soil_ab4(int blk, DPhase S, const double* recS, NList NL, Grid g, KParams K, FusedK F,
-                                         int cross, int mask)
+                                         int cross, int mask, int lean)
 {
     const RecV RS = recv(recS, S.n);
-    const WaveCtx wc = wave_ctx(S.n, blk);
+    __shared__ __align__(16) unsigned char lds[VIS_LDS<6>];
+    const SubCtx wc = sub_ctx(S.n, blk, NL.lg, WIN_LANES);
     const int t = wc.t;
     auto RA = [&](int c) { return RS(wc.tt, c); };
-    const double2 xy = RA(0), va = RA(1), rm = RA(2), a3 = RA(3), a4 = RA(4), a12 = RA(5), hi = RA(6);
+    const double2 xy = RA(0), va = RA(1), a3 = RA(3), a4 = RA(4), a12 = RA(5);
     // U (checked by the host): h uniform in the phase (hsml(1) everywhere, a
     // wave-uniform value), integer repulsion exponents, Drucker-Prager
-    const double xa = xy.x, ya = xy.y, vxa = va.x, vya = va.y, rhoa = rm.x, vofa = a3.x;
-    const double ha = U ? K.h1_soil : hi.x;
+    const double xa = xy.x, ya = xy.y, vxa = va.x, vya = va.y, rhoa = RA(2).x;
+    const double ha = U ? K.h1_soil : RA(6).x;
     const double pa = a3.y, sxxa = a12.x, sxya = a12.y, syya = a4.x;
-    const double ca = a4.y;          // sound speed before this step (delta_sph of rho)
-    const double cn = K.s_c;         // sound speed after it (stage B)
-    const double irhoa = 1.0 / rhoa, ir2a = irhoa * irhoa;
+    const double cn = K.s_c;         // sound speed after this step (stage B)
     // Mohr-Coulomb (general instantiation only): the criterion may have reset
     // rho; con_density's delta_sph, the strain rate and the divergence come
     // before it in single_step and use the density before it (chunk 7)
     const bool mc = !U && K.yield_criterion == 1;
     const double rhoa_pre = mc ? RA(7).x : rhoa;
-    const double fpa = vofa * pa * ir2a, fxxa = vofa * sxxa * ir2a, fxya = vofa * sxya * ir2a,
-                 fyya = vofa * syya * ir2a;
-    const int ita = (int)hi.y;
-    const int a = S.order[wc.tt];
+    const int a = NL.cell ? wc.tt : S.order[wc.tt];
+    const int ita = S.itype[a];
     const bool link = K.nnps == 2;
     const bool uni = U || link || F.uni_s;
-    const KC kc = make_kc(SKF, link ? K.h1_soil : ha);
-    const LaneRows L = cand_rows(g, S.cell_start, NL, wc.tt, xa, ya);
+    const KC kc0 = make_kc(SKF, link ? K.h1_soil : ha);
+    // (the tail's inputs, loaded before the loop)
+    double drgx = 0.0, drgy = 0.0, porx = 0.0, pory = 0.0;
+    if (mask & M_CROSS) {
+        drgx = S.drgx[a];
+        drgy = S.drgy[a];
+        porx = S.porx[a];
+        pory = S.pory[a];
+    }
+    const Window win = open_window<U, 6>(lds, NL.is, blk, wc, NL.lg, S.n, RS);
+    const Cand C{g, S.cell_start, NL.cell, xa, ya};
     const Pred P{xa, ya, ha, F.thr_s, uni ? 1 : 0, link ? 1 : 0};
-    auto acc = [&](int k, double2 b) { return P(b, uni ? ha : RS(k, 6).x, g, K); };
-    auto acc_k = [&](int k) { return acc(k, RS(k, 0)); };
-    const CatMask cm = cand_mask(L, NL.same, S.n, wc.tt, t, RS, acc);
-    const Loader<NEED_B> load{RS, !uni, mc};
+    const double rep2 = !SOLO && ita > 0 ? S.dspp * S.dspp : -1.0;   // real particles feel the wall
     const double et2 = K.etq * K.etq;
-    double con = 0.0, drd = 0.0, txx = 0.0, txy = 0.0, tyy = 0.0, vcc = 0.0, wxy = 0.0;
-    double avx = 0.0, avy = 0.0, repx = 0.0, repy = 0.0;
+    const bool art = (mask & M_ART) != 0;
+    double con = 0.0, drd = 0.0, sxx = 0.0, syy = 0.0, sxy = 0.0, syx = 0.0, spin = 0.0;
+    double avx = 0.0, avy = 0.0;
+    const double own = SOLO ? 1.0 : a3.x / rhoa;   // vof / rho^2
+    const double oxx = own * (sxxa - pa), oyy = own * (syya - pa), oxy = own * sxya;
     double Fx = 0.0, Fy = 0.0;
     double artx = 0.0, arty = 0.0, dP = 0.0, dXX = 0.0, dXY = 0.0, dYY = 0.0;
     int cnt = 0;
-    visit(cat_iter(cm, L), L, cm.ovf, t, load, acc_k, [&](const Nb& b) {
-        const double dx = xa - b.xy.x, dy = ya - b.xy.y;
-        const double dr = dx * dx + dy * dy;
-        const Dist D = dist_of(dr);
-        const double r = D.r, idr = D.idr;
-        double ww, gx, gy;
-        const double amh = uni ? ha : sph_mhsml(ha, b.hv.x);
-        if (uni) kern_fast<SKF, true>(kc, r, D.ir, dx, dy, ww, gx, gy);
-        else kern_fast<SKF, true>(make_kc(SKF, amh), r, D.ir, dx, dy, ww, gx, gy);
-        ++cnt;
-        const double mb = b.rm.y, Vb = b.iv.y, irb = b.iv.x;
-        // stage A
-        const double dvx = vxa - b.v.x, dvy = vya - b.v.y;
-        const double dvg = dvx * gx + dvy * gy;
-        const double rb_pre = mc ? b.rpre : b.rm.x;
-        const double irb_pre = mc ? fast_rcp(rb_pre) : irb;
-        const double Vb_pre = mc ? mb * irb_pre : Vb;
-        con += mb * dvg;
-        drd += mb * (2.0 * (rhoa_pre - rb_pre) * idr * (dx * gx + dy * gy)) * irb_pre;
-        txx += Vb_pre * (-2.0 * dvx * gx + dvy * gy);
-        txy += Vb_pre * (-(dvx * gy) - dvy * gx);
-        tyy += Vb_pre * (-2.0 * dvy * gy + dvx * gx);
-        vcc -= Vb_pre * dvg;
-        wxy += Vb * (-(dvx * gy) + dvy * gx);
-        const double f = mb * ww * (2.0 * fast_rcp(rhoa + b.rm.x));
-        avx -= dvx * f;
-        avy -= dvy * f;
-        if (!SOLO && ita > 0 && !(r > S.dspp) && (int)b.s3.y < 0) {
-            const double q = S.dspp / r;
-            const double fr = (U ? ipow(q, K.ip1) - ipow(q, K.ip2) : pow(q, K.p1) - pow(q, K.p2)) * idr;
-            repx += K.dd * dx * fr;
-            repy += K.dd * dy * fr;
-        }
-        // stage B
-        const double vofb = b.hv.y, ir2b = irb * irb;
-        const double fp = fpa + vofb * b.pc.x * ir2b;
-        const double fxx = fxxa + vofb * b.s12.x * ir2b;
-        const double fxy = fxya + vofb * b.s12.y * ir2b;
-        const double fyy = fyya + vofb * b.s3.x * ir2b;
-        if constexpr (SOLO) {
-            // -df(p) + df(sigma) (single_step_for_soil :1596-1597):
-            // m_b/rho_b (f_a + f_b) grad W, no vof factors
-            const double ps = pa + b.pc.x, sxy = sxya + b.s12.y;
-            Fx += Vb * ((sxxa + b.s12.x - ps) * gx + sxy * gy);
-            Fy += Vb * ((syya + b.s3.x - ps) * gy + sxy * gx);
-        } else {
-            Fx += mb * ((fxx - fp) * gx + fxy * gy);
-            Fy += mb * ((fyy - fp) * gy + fxy * gx);
-        }
-        const double vr = dvx * dx + dvy * dy;
-        {   // art_visc, branch-free: approaching pairs only (vr < 0)
-            const double muv = amh * vr * fast_rcp(dr + amh * amh * et2);
-            double piv = (K.beta * muv - K.alpha * cn) * muv * (2.0 * fast_rcp(rhoa + b.rm.x));
-            piv = vr < 0.0 ? piv : 0.0;
-            artx -= mb * piv * gx;
-            arty -= mb * piv * gy;
-        }
-        const double hh = 2.0 * idr * (dx * gx + dy * gy) * mb * irb;
-        dP += hh * (pa - b.pc.x);
-        dXX += hh * (sxxa - b.s12.x);
-        dXY += hh * (sxya - b.s12.y);
-        dYY += hh * (syya - b.s3.x);
-    });
+    visit<U, 6>(
+        lds, win, C, NL.is, S.n, wc, NL.lg, t, RS, [&](int k, double2 b) { return P(b, uni ? ha : RS(k, 6).x, g, K); },
+        [&](const auto& v, const auto& R, int k) {
+            const double2 b = v[0], u = v[1], q = v[2], f = v[3], s3 = v[4], s12 = v[5];
+            KC kc = kc0;
+            double amh = ha;
+            if (!uni) {
+                amh = sph_mhsml(ha, R(k, 6).x);
+                kc = make_kc(SKF, amh);
+            }
+            const Sep p = sep_of<SKF, true>(kc, xa - b.x, ya - b.y, U ? F.thr_s : INFINITY, false);
+            cnt += p.in ? 1 : 0;
+            const double V = fabs(q.y), m = V * q.x;
+            const double dvx = vxa - u.x, dvy = vya - u.y, vr = dvx * p.dx + dvy * p.dy;
+            const double Vs = V * p.s, wx = Vs * p.dx, wy = Vs * p.dy;
+            // stage A
+            con += (m * p.s) * vr;
+            if (mc) {
+                const double rp = R(k, 7).x, Vp = (m * fast_rcp(rp)) * p.s;
+                drd += Vp * (rhoa_pre - rp);
+                sxx += Vp * (dvx * p.dx);
+                syy += Vp * (dvy * p.dy);
+                sxy += Vp * (dvx * p.dy);
+                syx += Vp * (dvy * p.dx);
+                spin += wx * dvy - wy * dvx;
+            } else {
+                drd += Vs * (rhoa - q.x);
+                sxx += wx * dvx;
+                syy += wy * dvy;
+                sxy += wy * dvx;
+                syx += wx * dvy;
+            }
+            // one reciprocal for art_visc's denominator and the mean density
+            const double rs = rhoa + q.x, d2 = p.dr + amh * amh * et2;
+            const double it = fast_rcp(rs * d2);
+            const double fv = (m * p.w) * (it * d2);
+            avx -= fv * dvx;
+            avy -= fv * dvy;
+            if (!SOLO && q.y < 0.0 && p.dr <= rep2) {
+                const double fr = rep_factor<U>(K, S.dspp, p.ir);
+                artx += p.dx * (0.5 * fr);
+                arty += p.dy * (0.5 * fr);
+            }
+            // stage B
+            if constexpr (SOLO) {
+                // -df(p) + df(sigma) (single_step_for_soil :1596-1597):
+                // m_b/rho_b (f_a + f_b) grad W, no vof factors
+                const double fxy = oxy + s12.y;
+                Fx += (oxx + (s12.x - f.y)) * wx;
+                Fx += fxy * wy;
+                Fy += (oyy + (s3.x - f.y)) * wy;
+                Fy += fxy * wx;
+            } else {
+                // m (f_a / rho_a^2 + f_b / rho_b^2) grad W with m = V rho_b
+                const double fxy = fma(q.x, oxy, f.x * s12.y);
+                Fx += fma(q.x, oxx, f.x * (s12.x - f.y)) * wx;
+                Fx += fxy * wy;
+                Fy += fma(q.x, oyy, f.x * (s3.x - f.y)) * wy;
+                Fy += fxy * wx;
+            }
+            {   // art_visc, branch-free: approaching pairs only (vr < 0)
+                const double hv = amh * vr, muv = hv * (it * rs);
+                const double piv = (K.beta * muv - K.alpha * cn) * (hv * it);
+                const double mp = art && vr < 0.0 ? (m * p.s) * piv : 0.0;
+                artx -= mp * p.dx;
+                arty -= mp * p.dy;
+            }
+            dP += Vs * (pa - f.y);
+            dXX += Vs * (sxxa - s12.x);
+            dXY += Vs * (sxya - s12.y);
+            dYY += Vs * (syya - s3.x);
+        });
 
-    if (!wc.valid) return;
-    txx *= SPH_C23_F;
-    tyy *= SPH_C23_F;
-    wxy *= 0.5;
+    sub_sum(NL.lg, con, drd, sxx, syy, sxy, syx, avx, avy, Fx, Fy, artx, arty, dP, dXX, dXY, dYY);
+    if (mc) sub_sum(NL.lg, spin);
+    cnt = sub_count(NL.lg, cnt);
+    if (!wc.valid || wc.sub) return;
+    const double irhoa = 1.0 / rhoa;
+    const double ca = a4.y;          // sound speed before this step (delta_sph of rho)
+    const double txx = SPH_C23_F * (syy - 2.0 * sxx), tyy = SPH_C23_F * (sxx - 2.0 * syy);
+    const double txy = -(sxy + syx), vcc = -(sxx + syy), wxy = 0.5 * (mc ? spin : syx - sxy);
     // delta_sph(rho) and av_vel only under their switches (artificial_density,
     // average_velocity); without av_vel the reference leaves av as it was
     // single-phase soil under summation_density: sum_density replaced rho and
     // drho keeps only the delta-SPH term (declarations_sph.f90:1558-1570)
     if (SOLO && K.summation_density) con = 0.0;
-    S.drho[a] = K.artificial_density ? con + (K.delta * ha * ca) * drd : con;
-    S.txx[a] = txx; S.txy[a] = txy; S.tyy[a] = tyy; S.vcc[a] = vcc; S.wxy[a] = wxy;
-    if (ita > 0) { avx *= K.epsilon; avy *= K.epsilon; }
-    if (K.average_velocity) { S.avx[a] = avx; S.avy[a] = avy; }
-    S.repx[a] = repx; S.repy[a] = repy;
-    if (!cross) S.countiac[a] = cnt;
-    S.nsame[a] = cnt;
+    S.drho[a] = K.artificial_density ? con + (K.delta * ha * ca) * (2.0 * drd) : con;
+    if (K.average_velocity) {
+        const double e = ita > 0 ? 2.0 * K.epsilon : 2.0;
+        S.avx[a] = e * avx;
+        S.avy[a] = e * avy;
+    }
+    if (!lean) {
+        S.txx[a] = txx; S.txy[a] = txy; S.tyy[a] = tyy; S.vcc[a] = vcc; S.wxy[a] = wxy;
+        if (!cross) S.countiac[a] = cnt;
+        S.nsame[a] = cnt;
+    }
     S.c_next[a] = cn;
 
     const double alpha = K.s_alpha1, G = K.s_G, Kb = K.s_k;
@@ -1481,19 +1677,20 @@ __device__ __forceinline__ void soil_ab4(int blk, DPhase S, const double* recS, 
     dsyy = dsyy + G * tyy - 2.0 * sxya * wxy;
     dpv = dpv - Kb * vcc;
 
-    double ax = SOLO ? Fx : Fx * rhoa;
-    double ay = SOLO ? Fy : Fy * rhoa;
+    double ax = Fx, ay = Fy;
+    if (!SOLO) { ax = ax * rhoa; ay = ay * rhoa; }
     if (rhoa > 0.0) { ax = ax * irhoa; ay = ay * irhoa; }
-    if (mask & M_ART) { ax = ax + artx; ay = ay + arty; }
-    ax = ax + repx;
-    ay = ay + repy;
+    ax = ax + 2.0 * artx;   // art_visc and repulsion
+    ay = ay + 2.0 * arty;
     ay = ay + K.gravity;
     if (mask & M_CROSS) {
-        ax = ax + S.drgx[a]; ay = ay + S.drgy[a];
-        ax = ax + S.porx[a]; ay = ay + S.pory[a];
+        ax = ax + drgx;
+        ay = ay + drgy;
+        ax = ax + porx;
+        ay = ay + pory;
     }
     if (mask & M_DELTA_FIELD) {
-        const double cf = K.delta * ha * cn;
+        const double cf = K.delta * ha * cn * 2.0;
         dpv = dpv + cf * dP;
         dsxx = dsxx + cf * dXX;
         dsxy = dsxy + cf * dXY;
@@ -1506,7 +1703,7 @@ __device__ __forceinline__ void soil_ab4(int blk, DPhase S, const double* recS, 
 
 template <int SKF, bool U, bool SOLO>
 __global__ STAGE_ATTR_AB void k_soil_ab4(DPhase S, const double* recS, NList NL, Grid g, KParams K, FusedK F,
-                                         int cross, int mask)
+                                         int cross, int mask, int lean)
 {
-    soil_ab4<SKF, U, SOLO>(xcd_block(), S, recS, NL, g, K, F, cross, mask);
+    soil_ab4<SKF, U, SOLO>(xcd_block(), S, recS, NL, g, K, F, cross, mask, lean);
 }

@@ -58,10 +58,10 @@ struct KCf {
 __device__ __forceinline__ KCf make_kcf(int skf, double h)
 {
     const KC k = make_kc(skf, h);
-    return KCf{(float)k.inv_h, (float)k.f, (float)k.fh1, (float)k.fh2};
+    return KCf{(float)k.inv_h, (float)k.f, (float)(k.f * k.inv_h), (float)(k.f * k.inv_h * k.inv_h)};
 }
 
-// W and grad W in FP32 (the forms of kern_fast).
+// W and grad W in FP32 (the forms of kern_s).
 template <int SKF, bool NEED_W>
 __device__ __forceinline__ void kern_f(const KCf& k, float r, float inv_r, float dx, float dy, float& w, float& gx,
                                        float& gy)

@@ -28,42 +28,12 @@
 #pragma once
 #include "sph_fused.h"
 
-// The particle and candidate subset of a lane.
-struct SubCtx {
-    int t, tt, sub;
-    bool valid;
-};
-
-__device__ __forceinline__ SubCtx sub_ctx(int n, int blk, int lg)
-{
-    SubCtx c;
-    const int i = blk * (int)blockDim.x + (int)threadIdx.x;
-    c.t = i >> lg;
-    c.sub = i & ((1 << lg) - 1);
-    c.valid = c.t < n;
-    c.tt = c.valid ? c.t : n - 1;
-    return c;
-}
-
 // Candidate bits of lane sub: every 2^lg-th.
 __device__ __forceinline__ uint64_t sub_bits(int lg, int sub)
 {
     const uint64_t pat = lg == 0 ? ~0ull : lg == 1 ? 0x5555555555555555ull : lg == 2 ? 0x1111111111111111ull
                                                                                      : 0x0101010101010101ull;
     return pat << sub;
-}
-
-// Sum of v over the lanes of a particle (all get it).
-__device__ __forceinline__ void sub_sum(int lg, double& v)
-{
-    for (int o = 1; o < (1 << lg); o <<= 1) v += __shfl_xor(v, o, 64);
-}
-
-template <class... T>
-__device__ __forceinline__ void sub_sum(int lg, double& v, T&... rest)
-{
-    sub_sum(lg, v);
-    sub_sum(lg, rest...);
 }
 
 __device__ __forceinline__ uint64_t sub_or(int lg, uint64_t v)
@@ -214,10 +184,8 @@ __device__ __forceinline__ W1Pair w1_pair(const W1Self& a, const KC& kc, const R
     p.dr = p.dx * p.dx + p.dy * p.dy;
     const double ir = p.dr > 0.0 ? fast_rsq(p.dr) : 0.0, r = p.dr * ir;
     p.h = a.one_h ? a.ha : sph_mhsml(a.ha, R(k, 6).x);
-    double gy;
-    // (the gradient of a unit offset: its factor s)
-    if (a.uni) kern_fast<SKF, NEED_W>(kc, r, ir, 1.0, 0.0, p.w, p.s, gy);
-    else kern_fast<SKF, NEED_W>(make_kc(SKF, p.h), r, ir, 1.0, 0.0, p.w, p.s, gy);
+    if (a.uni) kern_s<SKF, NEED_W>(kc, r, ir, p.w, p.s);
+    else kern_s<SKF, NEED_W>(make_kc(SKF, p.h), r, ir, p.w, p.s);
     return p;
 }
 
@@ -230,7 +198,7 @@ __global__ __launch_bounds__(256) void k_w1_density(DPhase W, double* recw, Mask
                                                     int lg)
 {
     const RecV R = recv(recw, W.n);
-    const SubCtx sc = sub_ctx(W.n, xcd_block(), lg);
+    const SubCtx sc = sub_ctx(W.n, xcd_block(), lg, 256);
     const W1Self a = w1_self<U>(W, R, sc.tt, g, K, F);
     const double2 rm = R(sc.tt, 2);
     const double ma = fabs(rm.y);
@@ -271,7 +239,7 @@ __global__ __launch_bounds__(256) void k_w1_rates(DPhase W, double* recw, Masks 
                                                   int mask, int lg)
 {
     const RecV R = recv(recw, W.n);
-    const SubCtx sc = sub_ctx(W.n, xcd_block(), lg);
+    const SubCtx sc = sub_ctx(W.n, xcd_block(), lg, 256);
     const W1Self a = w1_self<U>(W, R, sc.tt, g, K, F);
     const double2 va = R(sc.tt, 1);
     const double rhoa = R(sc.tt, 3).x;
@@ -345,7 +313,7 @@ __global__ __launch_bounds__(256) void k_w1_force(DPhase W, const double* rec, M
                                                   int mask, int lg, W1End E)
 {
     const RecV R = recv(rec, W.n);
-    const SubCtx sc = sub_ctx(W.n, xcd_block(), lg);
+    const SubCtx sc = sub_ctx(W.n, xcd_block(), lg, 256);
     const W1Self a = w1_self<U>(W, R, sc.tt, g, K, F);
     const double2 va = R(sc.tt, 1), s4 = R(sc.tt, 4), s5 = R(sc.tt, 5);
     const double rhoa = R(sc.tt, 3).x;

@@ -113,6 +113,8 @@ struct PhaseBuf {
     // neighbour lists of the FP64 fused step: candidate masks (same phase,
     // cross), cell key per record and position per particle at the rebuild
     Masks nl_same{}, nl_cross{};
+    IdxList il_same{}, il_cross{};   // the same candidates as indices
+    int lg = 0;                      // log2 of the lanes per particle of the stages that use them
     int* nl_cell = nullptr;
     double *nl_x = nullptr, *nl_y = nullptr;
     // second buffers of the arrays the reorder permutes: the permuted copy is
@@ -841,6 +843,11 @@ int download(sphg_ctx* c, int k, uint64_t m)
     return SPHG_OK;
 }
 
+// Lanes per particle (log2) of the FP64 stages with neighbour lists.  The
+// radius-3h kernels (skf 2, 3) have 50 candidates per particle and windows
+// that only half a workgroup's particles keep within the LDS.
+int nl_lanes(double scale_k) { return scale_k > 2.5 ? 1 : 0; }
+
 int alloc_phase(sphg_ctx* c, int k, const sphg_phase_view* v)
 {
     PhaseBuf& b = c->ph[k];
@@ -893,6 +900,17 @@ int alloc_phase(sphg_ctx* c, int k, const sphg_phase_view* v)
     for (Masks* m : {&b.nl_same, &b.nl_cross}) {
         RC(dalloc(c, b, &m->m, 2 * n));
         RC(dalloc(c, b, &m->ovf, n));
+    }
+    // index lists: a uniform lattice at h = 1.2 dx has 22 candidates within R +
+    // 0.1 R (skf 1, 4) or 50 (skf 2, 3); a particle with more than fit walks
+    // its rows.  (The readers run ahead of the list: padding.)
+    b.lg = nl_lanes(c->K.scale_k);
+    for (IdxList* l : {&b.il_same, &b.il_cross}) {
+        l->cap = c->K.scale_k > 2.5 ? 96 : 48;
+        const size_t slots = (size_t)(l->cap + (8 << b.lg));
+        RC(dalloc(c, b, &l->li, slots * n));
+        RC(dalloc(c, b, &l->cnt, n));
+        RC(dalloc(c, b, &l->win, (size_t)WIN_INTS * (size_t)nblk(b.n, WIN_LANES >> b.lg)));
     }
     RC(dalloc(c, b, &b.nl_cell, n));
     RC(dalloc(c, b, &b.nl_x, n));
@@ -1048,6 +1066,17 @@ struct FinalArgs {
     bool ahead;
 };
 
+// The neighbour lists of a phase for its stage kernels (none without lists;
+// link_list's reach is tested per pair, outside the windows).
+NList nlist_of(const sphg_ctx* c, const PhaseBuf& b, bool nl)
+{
+    if (!nl) return NList{};
+    NList L{b.nl_same, b.nl_cross, b.nl_cell, b.il_same, b.il_cross, b.lg};
+    L.is.lds = c->P.nnps != 2;
+    L.ix.lds = 1;
+    return L;
+}
+
 // The fused step: pack (first_half + soil Drucker-Prager projections +
 // records), cross terms, partner masks, stage A, stage B.  The soil kernels
 // read only the packed records of both phases (the water pressure comes from
@@ -1063,8 +1092,12 @@ int stages_fused(sphg_ctx* c, const FinalArgs* fin)
     const double* rW = W.rec;
     const double* rS = S.rec;
     const bool nl = nl_mode(c);
-    const NList nW = nl ? NList{W.nl_same, W.nl_cross, W.nl_cell} : NList{};
-    const NList nS = nl ? NList{S.nl_same, S.nl_cross, S.nl_cell} : NList{};
+    // (the values of a step that another of the same call follows, and that only
+    // a download would read, stay out)
+    const int lean = fin && fin->ahead ? 1 : 0;
+    const NList nW = nlist_of(c, W, nl);
+    const NList nS = nlist_of(c, S, nl);
+    const int nbW = nblk(W.n, WIN_LANES >> nW.lg), nbS = nblk(S.n, WIN_LANES >> nS.lg);
     const Grid& gW = nl ? c->gvl[0] : c->gl[0];
     const Grid& gS = nl ? c->gvl[1] : c->gl[1];
     // U instantiations: h uniform in the phase(s) the kernel reads (then
@@ -1081,37 +1114,37 @@ int stages_fused(sphg_ctx* c, const FinalArgs* fin)
     {
         SideScope side(c);
         if (cross) {
-            if (ux) RC(launch(c, "soil_x", k_soil_x4<SKF, true>, nblk(S.n, STAGE_BLOCK), STAGE_BLOCK, S.d, W.d, rS, rW,
-                              nS, gS, c->K, c->F));
-            else RC(launch(c, "soil_x", k_soil_x4<SKF, false>, nblk(S.n, STAGE_BLOCK), STAGE_BLOCK, S.d, W.d, rS, rW,
-                           nS, gS, c->K, c->F));
+            if (ux) RC(launch(c, "soil_x", k_soil_x4<SKF, true>, nbS, STAGE_BLOCK, S.d, W.d, rS, rW,
+                              nS, gS, c->K, c->F, lean));
+            else RC(launch(c, "soil_x", k_soil_x4<SKF, false>, nbS, STAGE_BLOCK, S.d, W.d, rS, rW,
+                           nS, gS, c->K, c->F, lean));
         }
         if (split) HIPCHK(c, hipEventRecord(c->ev_sx, c->side));
-        if (us) RC(launch(c, "soil_ab", k_soil_ab4<SKF, true, false>, nblk(S.n, STAGE_BLOCK), STAGE_BLOCK, S.d, rS,
-                          nS, gS, c->K, c->F, cross, mask_b(c, 1)));
-        else RC(launch(c, "soil_ab", k_soil_ab4<SKF, false, false>, nblk(S.n, STAGE_BLOCK), STAGE_BLOCK, S.d, rS,
-                       nS, gS, c->K, c->F, cross, mask_b(c, 1)));
+        if (us) RC(launch(c, "soil_ab", k_soil_ab4<SKF, true, false>, nbS, STAGE_BLOCK, S.d, rS,
+                          nS, gS, c->K, c->F, cross, mask_b(c, 1), lean));
+        else RC(launch(c, "soil_ab", k_soil_ab4<SKF, false, false>, nbS, STAGE_BLOCK, S.d, rS,
+                       nS, gS, c->K, c->F, cross, mask_b(c, 1), lean));
     }
     // water stage A, then the water cross terms (before stage B, whose tail
     // adds them): beside the soil side's cross pass and then its stage,
     // each pair of concurrent kernels reads the same phase's records
-    if (uw) RC(launch(c, "water_a", k_water_a4<SKF, true>, nblk(W.n, STAGE_BLOCK), STAGE_BLOCK, W.d, rW, W.rec,
-                      nW, W.masks, gW, c->K, c->F, cross));
-    else RC(launch(c, "water_a", k_water_a4<SKF, false>, nblk(W.n, STAGE_BLOCK), STAGE_BLOCK, W.d, rW, W.rec,
-                   nW, W.masks, gW, c->K, c->F, cross));
+    if (uw) RC(launch(c, "water_a", k_water_a4<SKF, true>, nbW, STAGE_BLOCK, W.d, rW, W.rec,
+                      nW, gW, c->K, c->F, cross, lean));
+    else RC(launch(c, "water_a", k_water_a4<SKF, false>, nbW, STAGE_BLOCK, W.d, rW, W.rec,
+                   nW, gW, c->K, c->F, cross, lean));
     if (cross) {
-        if (ux) RC(launch(c, "water_x", k_water_x4<SKF, true>, nblk(W.n, STAGE_BLOCK), STAGE_BLOCK, W.d, S.d, rW, rS,
-                          nW, gW, c->K, c->F));
-        else RC(launch(c, "water_x", k_water_x4<SKF, false>, nblk(W.n, STAGE_BLOCK), STAGE_BLOCK, W.d, S.d, rW, rS,
-                       nW, gW, c->K, c->F));
+        if (ux) RC(launch(c, "water_x", k_water_x4<SKF, true>, nbW, STAGE_BLOCK, W.d, S.d, rW, rS,
+                          nW, gW, c->K, c->F, lean));
+        else RC(launch(c, "water_x", k_water_x4<SKF, false>, nbW, STAGE_BLOCK, W.d, S.d, rW, rS,
+                       nW, gW, c->K, c->F, lean));
     }
     if (split) HIPCHK(c, hipEventRecord(c->ev_wx, c->stream));
     swap_c(W);
     swap_c(S);
-    if (uw) RC(launch(c, "water_b", k_water_b4<SKF, true>, nblk(W.n, STAGE_BLOCK), STAGE_BLOCK, W.d, rW, nW,
-                      W.masks, gW, c->K, c->F, mask_b(c, 0)));
-    else RC(launch(c, "water_b", k_water_b4<SKF, false>, nblk(W.n, STAGE_BLOCK), STAGE_BLOCK, W.d, rW, nW,
-                   W.masks, gW, c->K, c->F, mask_b(c, 0)));
+    if (uw) RC(launch(c, "water_b", k_water_b4<SKF, true>, nbW, STAGE_BLOCK, W.d, rW, nW,
+                      gW, c->K, c->F, mask_b(c, 0)));
+    else RC(launch(c, "water_b", k_water_b4<SKF, false>, nbW, STAGE_BLOCK, W.d, rW, nW,
+                   gW, c->K, c->F, mask_b(c, 0)));
     if (fin) {
         auto final_water = [&]() -> int {
             if (fin->ahead)
@@ -1151,11 +1184,11 @@ int stages_soil_only(sphg_ctx* c)
     PhaseBuf& S = c->ph[1];
     const double* rs = S.rec;
     if (S.hmin == S.hmax && c->K.yield_criterion != 1)
-        RC(launch(c, "soil_ab", k_soil_ab4<SKF, true, true>, nblk(S.n, STAGE_BLOCK), STAGE_BLOCK, S.d, rs, NList{},
-                  c->gl[1], c->K, c->F, 0, mask_b(c, 1)));
+        RC(launch(c, "soil_ab", k_soil_ab4<SKF, true, true>, nblk(S.n, WIN_LANES), STAGE_BLOCK, S.d, rs, NList{},
+                  c->gl[1], c->K, c->F, 0, mask_b(c, 1), 0));
     else
-        RC(launch(c, "soil_ab", k_soil_ab4<SKF, false, true>, nblk(S.n, STAGE_BLOCK), STAGE_BLOCK, S.d, rs, NList{},
-                  c->gl[1], c->K, c->F, 0, mask_b(c, 1)));
+        RC(launch(c, "soil_ab", k_soil_ab4<SKF, false, true>, nblk(S.n, WIN_LANES), STAGE_BLOCK, S.d, rs, NList{},
+                  c->gl[1], c->K, c->F, 0, mask_b(c, 1), 0));
     swap_c(S);
     return SPHG_OK;
 }
@@ -1195,8 +1228,8 @@ int stages_mixed(sphg_ctx* c, const FinalArgs* fin)
     // with neighbour lists: the list grid (records hold positions relative
     // to their list cells) and the lists
     const bool nl = nl_mode(c);
-    const NList nW = nl ? NList{W.nl_same, W.nl_cross, W.nl_cell} : NList{};
-    const NList nS = nl ? NList{S.nl_same, S.nl_cross, S.nl_cell} : NList{};
+    const NList nW = nlist_of(c, W, nl);
+    const NList nS = nlist_of(c, S, nl);
     const Grid& gW = nl ? c->gvl[0] : c->gl[0];
     const Grid& gS = nl ? c->gvl[1] : c->gl[1];
     MixK X = c->X;
@@ -1252,16 +1285,16 @@ int build_nlists(sphg_ctx* c)
     RC(launch(c, "nlist", k_keep_bits, 1, TPB, c->d_nlflag, 2));
     RC(launch(c, "nlist", k_nlist, nblk(W.n, 256), 256, (const double*)w.x, (const double*)w.y,
               (const int*)nullptr, W.n, (const double*)w.x, (const double*)w.y, (const int*)nullptr,
-              (const int*)w.cell_start, c->gv, c->nl_thr[0], 1, W.nl_same, W.nl_cell));
+              (const int*)w.cell_start, c->gv, c->nl_thr[0], 1, W.nl_same, W.nl_cell, W.il_same, WIN_LANES >> W.lg));
     RC(launch(c, "nlist", k_nlist, nblk(S.n, 256), 256, (const double*)sd.x, (const double*)sd.y,
               (const int*)nullptr, S.n, (const double*)sd.x, (const double*)sd.y, (const int*)nullptr,
-              (const int*)sd.cell_start, c->gv, c->nl_thr[1], 1, S.nl_same, S.nl_cell));
+              (const int*)sd.cell_start, c->gv, c->nl_thr[1], 1, S.nl_same, S.nl_cell, S.il_same, WIN_LANES >> S.lg));
     RC(launch(c, "nlist", k_nlist, nblk(W.n, 256), 256, (const double*)w.x, (const double*)w.y,
               (const int*)nullptr, W.n, (const double*)sd.x, (const double*)sd.y, (const int*)nullptr,
-              (const int*)sd.cell_start, c->gv, c->nl_thr[2], 0, W.nl_cross, (int*)nullptr));
+              (const int*)sd.cell_start, c->gv, c->nl_thr[2], 0, W.nl_cross, (int*)nullptr, W.il_cross, WIN_LANES >> W.lg));
     RC(launch(c, "nlist", k_nlist, nblk(S.n, 256), 256, (const double*)sd.x, (const double*)sd.y,
               (const int*)nullptr, S.n, (const double*)w.x, (const double*)w.y, (const int*)nullptr,
-              (const int*)w.cell_start, c->gv, c->nl_thr[2], 0, S.nl_cross, (int*)nullptr));
+              (const int*)w.cell_start, c->gv, c->nl_thr[2], 0, S.nl_cross, (int*)nullptr, S.il_cross, WIN_LANES >> S.lg));
     c->nl_valid = true;
     c->nl_due = false;
     c->nl_rebuilt_at = c->nl_seq + 1;   // the step being issued
