@@ -46,8 +46,12 @@ __device__ __forceinline__ void tup_call(int blk, const Tup& a, std::index_seque
 
 // Workgroup b of the batched grid (XCD-aware, so that each XCD works on a
 // contiguous run of cases) runs block tiles[b].y of case tiles[b].x.
+// __restrict__: without it arguments read after a store or a barrier are
+// vector loads, and the two-part bodies took 184 and 304 VGPR instead of the
+// solo kernels' 136 and 208 (16 cases of 0.9M particles: 50.4 ms for 128
+// steps; 43.2 with it).
 template <class F, class... T>
-__global__ __launch_bounds__(256) void k_batched(const ArgTup<T...>* args, const int2* tiles)
+__global__ __launch_bounds__(256) void k_batched(const ArgTup<T...>* __restrict__ args, const int2* __restrict__ tiles)
 {
     const int2 tl = tiles[xcd_block()];
     tup_call<F>(tl.y, args[tl.x], std::index_sequence_for<T...>{});
@@ -57,27 +61,67 @@ __global__ __launch_bounds__(256) void k_batched(const ArgTup<T...>* args, const
 template <int SKF, bool U>
 struct BodyWaterX {
     template <class... A>
-    __device__ __forceinline__ void operator()(int blk, const A&... a) const { water_x4<SKF, U>(blk, a...); }
+    __device__ __forceinline__ void operator()(int blk, const A&... a) const
+    {
+        __shared__ __align__(16) unsigned char lds[VIS_LDS<4>];
+        water_x4<SKF, U>(lds, blk, a...);
+    }
 };
 template <int SKF, bool U>
 struct BodySoilX {
     template <class... A>
-    __device__ __forceinline__ void operator()(int blk, const A&... a) const { soil_x4<SKF, U>(blk, a...); }
+    __device__ __forceinline__ void operator()(int blk, const A&... a) const
+    {
+        __shared__ __align__(16) unsigned char lds[VIS_LDS<4>];
+        soil_x4<SKF, U>(lds, blk, a...);
+    }
 };
 template <int SKF, bool U>
 struct BodyWaterA {
     template <class... A>
-    __device__ __forceinline__ void operator()(int blk, const A&... a) const { water_a4<SKF, U>(blk, a...); }
+    __device__ __forceinline__ void operator()(int blk, const A&... a) const
+    {
+        __shared__ __align__(16) unsigned char lds[VIS_LDS<3>];
+        water_a4<SKF, U>(lds, blk, a...);
+    }
 };
 template <int SKF, bool U>
 struct BodyWaterB {
     template <class... A>
-    __device__ __forceinline__ void operator()(int blk, const A&... a) const { water_b4<SKF, U>(blk, a...); }
+    __device__ __forceinline__ void operator()(int blk, const A&... a) const
+    {
+        __shared__ __align__(16) unsigned char lds[VIS_LDS<6>];
+        water_b4<SKF, U>(lds, blk, a...);
+    }
 };
 template <int SKF, bool U, bool SOLO>
 struct BodySoilAB {
     template <class... A>
-    __device__ __forceinline__ void operator()(int blk, const A&... a) const { soil_ab4<SKF, U, SOLO>(blk, a...); }
+    __device__ __forceinline__ void operator()(int blk, const A&... a) const
+    {
+        __shared__ __align__(16) unsigned char lds[VIS_LDS<6>];
+        soil_ab4<SKF, U, SOLO>(lds, blk, a...);
+    }
+};
+// (a tile is a workgroup of the solo launch, padding included)
+template <int SKF>
+struct BodyStage1 {
+    __device__ __forceinline__ void operator()(int blk, const StageArgs& a) const { stage1<SKF>(blk, a, false); }
+};
+template <int SKF>
+struct BodyStage2 {
+    __device__ __forceinline__ void operator()(int blk, const StageArgs& a) const { stage2<SKF>(blk, a, false); }
+};
+template <int SKF>
+struct BodyStage1Mx {
+    __device__ __forceinline__ void operator()(int blk, const StageArgsMx& a) const { stage1_mx<SKF>(blk, a, false); }
+};
+template <int SKF>
+struct BodyStage2Mx {
+    __device__ __forceinline__ void operator()(int blk, const StageArgsMx& a) const { stage2_mx<SKF>(blk, a, false); }
+};
+struct BodyFinals {
+    __device__ __forceinline__ void operator()(int blk, const FinalsArgs& a) const { finals(blk, a, false); }
 };
 struct BodyStepWater {
     template <class... A>

@@ -1151,11 +1151,10 @@ __device__ __forceinline__ Sep sep_of(const KC& kc, double dx, double dy, double
 // that only a download or the last step's diagnostics would read stay out.
 // ------------------------------------------------------------------------
 template <int SKF, bool U>
-__device__ __forceinline__ void water_x4(int blk, DPhase W, DPhase S, const double* recW, const double* recS,
+__device__ __forceinline__ void water_x4(unsigned char* lds, int blk, DPhase W, DPhase S, const double* recW, const double* recS,
                                          NList NL, Grid g, KParams K, FusedK F, int lean)
 {
     const RecV RW = recv(recW, W.n), RS = recv(recS, S.n);
-    __shared__ __align__(16) unsigned char lds[VIS_LDS<4>];
     const SubCtx wc = sub_ctx(W.n, blk, NL.lg, WIN_LANES);
     const double2 xy = RW(wc.tt, 0), va = RW(wc.tt, 1);
     const double xa = xy.x, ya = xy.y, vxa = va.x, vya = va.y, vofa = RW(wc.tt, 3).x;
@@ -1203,7 +1202,8 @@ template <int SKF, bool U>
 __global__ STAGE_ATTR void k_water_x4(DPhase W, DPhase S, const double* recW, const double* recS, NList NL, Grid g,
                                       KParams K, FusedK F, int lean)
 {
-    water_x4<SKF, U>(xcd_block(), W, S, recW, recS, NL, g, K, F, lean);
+    __shared__ __align__(16) unsigned char lds[VIS_LDS<4>];
+    water_x4<SKF, U>(lds, xcd_block(), W, S, recW, recS, NL, g, K, F, lean);
 }
 
 // ------------------------------------------------------------------------
@@ -1212,11 +1212,10 @@ __global__ STAGE_ATTR void k_water_x4(DPhase W, DPhase S, const double* recW, co
 // (whose pressure is the new one the water pack evaluated).
 // ------------------------------------------------------------------------
 template <int SKF, bool U>
-__device__ __forceinline__ void soil_x4(int blk, DPhase S, DPhase W, const double* recS, const double* recW, NList NL,
+__device__ __forceinline__ void soil_x4(unsigned char* lds, int blk, DPhase S, DPhase W, const double* recS, const double* recW, NList NL,
                                         Grid g, KParams K, FusedK F, int lean)
 {
     const RecV RS = recv(recS, S.n), RW = recv(recW, W.n);
-    __shared__ __align__(16) unsigned char lds[VIS_LDS<4>];
     const SubCtx wc = sub_ctx(S.n, blk, NL.lg, WIN_LANES);
     const double2 xy = RS(wc.tt, 0), va = RS(wc.tt, 1);
     const double xa = xy.x, ya = xy.y, vxa = va.x, vya = va.y;
@@ -1263,7 +1262,8 @@ template <int SKF, bool U>
 __global__ STAGE_ATTR void k_soil_x4(DPhase S, DPhase W, const double* recS, const double* recW, NList NL, Grid g,
                                      KParams K, FusedK F, int lean)
 {
-    soil_x4<SKF, U>(xcd_block(), S, W, recS, recW, NL, g, K, F, lean);
+    __shared__ __align__(16) unsigned char lds[VIS_LDS<4>];
+    soil_x4<SKF, U>(lds, xcd_block(), S, W, recS, recW, NL, g, K, F, lean);
 }
 
 // repulsive_force on a real particle from a virtual partner within r0
@@ -1283,11 +1283,10 @@ __device__ __forceinline__ double rep_factor(const KParams& K, double r0, double
 // writes).
 // ------------------------------------------------------------------------
 template <int SKF, bool U>
-__device__ __forceinline__ void water_a4(int blk, DPhase W, const double* recW, double* recWw, NList NL, Grid g,
+__device__ __forceinline__ void water_a4(unsigned char* lds, int blk, DPhase W, const double* recW, double* recWw, NList NL, Grid g,
                                          KParams K, FusedK F, int cross, int lean)
 {
     const RecV RW = recv(recW, W.n);
-    __shared__ __align__(16) unsigned char lds[VIS_LDS<3>];
     const SubCtx wc = sub_ctx(W.n, blk, NL.lg, WIN_LANES);
     const int t = wc.t;
     auto RA = [&](int c) { return RW(wc.tt, c); };
@@ -1366,7 +1365,8 @@ template <int SKF, bool U>
 __global__ STAGE_ATTR void k_water_a4(DPhase W, const double* recW, double* recWw, NList NL, Grid g, KParams K,
                                       FusedK F, int cross, int lean)
 {
-    water_a4<SKF, U>(xcd_block(), W, recW, recWw, NL, g, K, F, cross, lean);
+    __shared__ __align__(16) unsigned char lds[VIS_LDS<3>];
+    water_a4<SKF, U>(lds, xcd_block(), W, recW, recWw, NL, g, K, F, cross, lean);
 }
 
 // ------------------------------------------------------------------------
@@ -1374,11 +1374,10 @@ __global__ STAGE_ATTR void k_water_a4(DPhase W, const double* recW, double* recW
 // art_visc, delta_sph(vof, dvof); /rho, + repulsion, + gravity, - Darcy drag.
 // ------------------------------------------------------------------------
 template <int SKF, bool U>
-__device__ __forceinline__ void water_b4(int blk, DPhase W, const double* recW, NList NL, Grid g, KParams K, FusedK F,
+__device__ __forceinline__ void water_b4(unsigned char* lds, int blk, DPhase W, const double* recW, NList NL, Grid g, KParams K, FusedK F,
                                          int mask)
 {
     const RecV RW = recv(recW, W.n);
-    __shared__ __align__(16) unsigned char lds[VIS_LDS<6>];
     const SubCtx wc = sub_ctx(W.n, blk, NL.lg, WIN_LANES);
     const int t = wc.t;
     auto RA = [&](int c) { return RW(wc.tt, c); };
@@ -1464,7 +1463,8 @@ __device__ __forceinline__ void water_b4(int blk, DPhase W, const double* recW, 
 template <int SKF, bool U>
 __global__ STAGE_ATTR void k_water_b4(DPhase W, const double* recW, NList NL, Grid g, KParams K, FusedK F, int mask)
 {
-    water_b4<SKF, U>(xcd_block(), W, recW, NL, g, K, F, mask);
+    __shared__ __align__(16) unsigned char lds[VIS_LDS<6>];
+    water_b4<SKF, U>(lds, xcd_block(), W, recW, NL, g, K, F, mask);
 }
 
 // ------------------------------------------------------------------------
@@ -1483,11 +1483,10 @@ __global__ STAGE_ATTR void k_water_b4(DPhase W, const double* recW, NList NL, Gr
 //               (the cross terms k_soil_x4 wrote; cross: two-phase run).
 // ------------------------------------------------------------------------
 template <int SKF, bool U, bool SOLO>
-__device__ __forceinline__ void soil_ab4(int blk, DPhase S, const double* recS, NList NL, Grid g, KParams K, FusedK F,
+__device__ __forceinline__ void soil_ab4(unsigned char* lds, int blk, DPhase S, const double* recS, NList NL, Grid g, KParams K, FusedK F,
                                          int cross, int mask, int lean)
 {
     const RecV RS = recv(recS, S.n);
-    __shared__ __align__(16) unsigned char lds[VIS_LDS<6>];
     const SubCtx wc = sub_ctx(S.n, blk, NL.lg, WIN_LANES);
     const int t = wc.t;
     auto RA = [&](int c) { return RS(wc.tt, c); };
@@ -1705,5 +1704,122 @@ template <int SKF, bool U, bool SOLO>
 __global__ STAGE_ATTR_AB void k_soil_ab4(DPhase S, const double* recS, NList NL, Grid g, KParams K, FusedK F,
                                          int cross, int mask, int lean)
 {
-    soil_ab4<SKF, U, SOLO>(xcd_block(), S, recS, NL, g, K, F, cross, mask, lean);
+    __shared__ __align__(16) unsigned char lds[VIS_LDS<6>];
+    soil_ab4<SKF, U, SOLO>(lds, xcd_block(), S, recS, NL, g, K, F, cross, mask, lean);
+}
+
+// ------------------------------------------------------------------------
+// A whole step in three launches on one stream (the phases uniform in h):
+// stage 1 (water stage A and both cross passes: they read packed records
+// alone), stage 2 (water stage B and the soil pass, which add the cross terms)
+// and the final updates.  The parts of a launch are ranges of its workgroups;
+// each keeps the registers and the LDS of the dearest part, and still the
+// merged step is the faster at every size: the eight launches on two streams
+// with an event at each dependence cost 40 us of a step (us per step, apart
+// and merged: 1.5k particles 83 / 40, 33k 82 / 45, 125k 100 / 77, 258k 127 /
+// 108, 1M 369 / 364).
+// ------------------------------------------------------------------------
+struct StageArgs {
+    DPhase W, S;
+    double *rW, *rS;
+    NList nW, nS;
+    Grid gW, gS;
+    KParams K;
+    FusedK F;
+    int mask_w, mask_s, lean;
+    int nbW, nbS;   // workgroups of a pass over the water, over the soil
+};
+
+// The part of a launch that workgroup l belongs to, in the order of the counts
+// nb (each padded to a multiple of 8, so that a part's workgroups keep the
+// XCDs of their launch index), and its index there (-1: padding).  spread:
+// consecutive workgroups of a part go to the same XCD (a batch gives each XCD
+// a run of its cases instead).
+struct PartIdx {
+    int part, blk;
+};
+
+template <int N>
+__device__ __forceinline__ PartIdx part_of(int l, const int (&nb)[N], bool spread)
+{
+    PartIdx p{0, l};
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int pad = (nb[i] + 7) & ~7;
+        if (p.part == i && i + 1 < N && p.blk >= pad) {
+            p.blk -= pad;
+            p.part = i + 1;
+        }
+    }
+    int n = nb[0];
+#pragma unroll
+    for (int i = 1; i < N; ++i)
+        if (p.part == i) n = nb[i];
+    if (spread) p.blk = (p.blk & 7) * ((n + 7) >> 3) + (p.blk >> 3);
+    if (p.blk >= n) p.blk = -1;
+    return p;
+}
+
+template <int SKF>
+__device__ __forceinline__ void stage1(int l, const StageArgs& A, bool spread)
+{
+    __shared__ __align__(16) unsigned char lds[VIS_LDS<4>];
+    const PartIdx p = part_of<3>(l, {A.nbS, A.nbW, A.nbW}, spread);
+    if (p.blk < 0) return;
+    if (p.part == 0) soil_x4<SKF, true>(lds, p.blk, A.S, A.W, A.rS, A.rW, A.nS, A.gS, A.K, A.F, A.lean);
+    else if (p.part == 1) water_a4<SKF, true>(lds, p.blk, A.W, A.rW, A.rW, A.nW, A.gW, A.K, A.F, 1, A.lean);
+    else water_x4<SKF, true>(lds, p.blk, A.W, A.S, A.rW, A.rS, A.nW, A.gW, A.K, A.F, A.lean);
+}
+
+template <int SKF>
+__device__ __forceinline__ void stage2(int l, const StageArgs& A, bool spread)
+{
+    __shared__ __align__(16) unsigned char lds[VIS_LDS<6>];
+    const PartIdx p = part_of<2>(l, {A.nbS, A.nbW}, spread);
+    if (p.blk < 0) return;
+    if (p.part == 0) soil_ab4<SKF, true, false>(lds, p.blk, A.S, A.rS, A.nS, A.gS, A.K, A.F, 1, A.mask_s, A.lean);
+    else water_b4<SKF, true>(lds, p.blk, A.W, A.rW, A.nW, A.gW, A.K, A.F, A.mask_w);
+}
+
+template <int SKF>
+__global__ STAGE_ATTR void k_stage1(StageArgs A)
+{
+    stage1<SKF>(blockIdx.x, A, true);
+}
+
+template <int SKF>
+__global__ STAGE_ATTR_AB void k_stage2(StageArgs A)
+{
+    stage2<SKF>(blockIdx.x, A, true);
+}
+
+// The final updates of both phases, with the next step's packs when ahead.
+struct FinalsArgs {
+    DPhase W, S;
+    KParams K;
+    double *rW, *rS;
+    int first, vf, renorm, ahead;
+    float *qW, *qS;   // the FP32 records (mixed precision)
+    Grid gW, gS;
+    double cs;
+    NRef nW, nS;
+    int nbW, nbS;
+};
+
+__device__ __forceinline__ void finals(int l, const FinalsArgs& A, bool spread)
+{
+    const PartIdx p = part_of<2>(l, {A.nbS, A.nbW}, spread);
+    if (p.blk < 0) return;
+    if (p.part == 0) {
+        if (A.ahead) step_soil(p.blk, A.S, A.K, A.rS, A.first, A.qS, A.gS, A.cs, A.nS);
+        else final_soil(p.blk, A.S, A.K, A.first);
+    } else {
+        if (A.ahead) step_water(p.blk, A.W, A.K, A.rW, A.first, A.vf, A.renorm, A.qW, A.gW, A.cs, A.nW);
+        else final_water(p.blk, A.W, A.K, A.first, A.vf, A.renorm);
+    }
+}
+
+__global__ __launch_bounds__(256) void k_finals(FinalsArgs A)
+{
+    finals(blockIdx.x, A, true);
 }

@@ -721,3 +721,48 @@ __global__ STAGE_ATTR void k_soil_x_mx(DPhase S, DPhase W, const float* qS, cons
 {
     soil_ab_mx<SKF, 2>(xcd_block(), S, W, qS, qW, NL, g, K, F, X, cross, mask);
 }
+
+// The launches of a whole step (k_stage1, k_stage2), mixed.
+struct StageArgsMx {
+    DPhase W, S;
+    float *qW, *qS;
+    NList nW, nS;
+    Masks MW;
+    Grid gW, gS;
+    KParams K;
+    FusedK F;
+    MixK X;
+    int mask_w, mask_s;
+    int nbW, nbS;
+};
+
+template <int SKF>
+__device__ __forceinline__ void stage1_mx(int l, const StageArgsMx& A, bool spread)
+{
+    const PartIdx p = part_of<3>(l, {A.nbS, A.nbW, A.nbW}, spread);
+    if (p.blk < 0) return;
+    if (p.part == 0) soil_ab_mx<SKF, 2>(p.blk, A.S, A.W, A.qS, A.qW, A.nS, A.gS, A.K, A.F, A.X, 1, A.mask_s);
+    else if (p.part == 1) water_a_mx<SKF, 1>(p.blk, A.W, A.S, A.qW, A.qW, A.qS, A.nW, A.MW, A.gW, A.K, A.F, A.X, 1);
+    else water_a_mx<SKF, 2>(p.blk, A.W, A.S, A.qW, A.qW, A.qS, A.nW, A.MW, A.gW, A.K, A.F, A.X, 1);
+}
+
+template <int SKF>
+__device__ __forceinline__ void stage2_mx(int l, const StageArgsMx& A, bool spread)
+{
+    const PartIdx p = part_of<2>(l, {A.nbS, A.nbW}, spread);
+    if (p.blk < 0) return;
+    if (p.part == 0) soil_ab_mx<SKF, 1>(p.blk, A.S, A.W, A.qS, A.qW, A.nS, A.gS, A.K, A.F, A.X, 1, A.mask_s);
+    else water_b_mx<SKF>(p.blk, A.W, A.qW, A.MW, A.gW, A.K, A.F, A.X, A.mask_w);
+}
+
+template <int SKF>
+__global__ STAGE_ATTR_MX void k_stage1_mx(StageArgsMx A)
+{
+    stage1_mx<SKF>(blockIdx.x, A, true);
+}
+
+template <int SKF>
+__global__ STAGE_ATTR_MX_AB void k_stage2_mx(StageArgsMx A)
+{
+    stage2_mx<SKF>(blockIdx.x, A, true);
+}

@@ -843,10 +843,23 @@ int download(sphg_ctx* c, int k, uint64_t m)
     return SPHG_OK;
 }
 
-// Lanes per particle (log2) of the FP64 stages with neighbour lists.  The
-// radius-3h kernels (skf 2, 3) have 50 candidates per particle and windows
-// that only half a workgroup's particles keep within the LDS.
-int nl_lanes(double scale_k) { return scale_k > 2.5 ? 1 : 0; }
+// Lanes per particle (log2) of the FP64 stages with neighbour lists, by the
+// phase's own size (a batch then sums in the solo order).  One lane per
+// particle leaves a small phase's partner loop a serial chain of 22 pairs on
+// few waves; more lanes cost their reductions and prologues once the chip is
+// full.  us per step at 0 / 1 / 2: 7k particles (water 6k) 44 / 36 / 34, 14k
+// (12k) 51 / 36 / 33, 33k (14k + 19k) 46 / 37 / 42, 64k (27k + 36k) 53 / 51 /
+// 58, 125k 78 / 71 / 89, 258k 108 / 115 / 156; but a batch of 16 cases fills
+// the chip by itself (128 steps, phases to 120k: 43 ms with none, 44.5 with
+// this rule, 48.5 with the solo optimum of 40000 and 8192).
+// The radius-3h kernels (skf 2, 3) have 50 candidates per particle and windows
+// that only half a workgroup's particles keep within the LDS: 14k 91 / 54 /
+// 43, 33k 90 / 57 / 54, 64k 103 / 75 / 75, 258k 195 / 190 / 222.
+int nl_lanes(int n, double scale_k)
+{
+    if (scale_k > 2.5) return n <= 12000 ? 2 : 1;
+    return n <= 4096 ? 2 : n <= 20000 ? 1 : 0;
+}
 
 int alloc_phase(sphg_ctx* c, int k, const sphg_phase_view* v)
 {
@@ -904,7 +917,7 @@ int alloc_phase(sphg_ctx* c, int k, const sphg_phase_view* v)
     // index lists: a uniform lattice at h = 1.2 dx has 22 candidates within R +
     // 0.1 R (skf 1, 4) or 50 (skf 2, 3); a particle with more than fit walks
     // its rows.  (The readers run ahead of the list: padding.)
-    b.lg = nl_lanes(c->K.scale_k);
+    b.lg = nl_lanes(b.n, c->K.scale_k);
     for (IdxList* l : {&b.il_same, &b.il_cross}) {
         l->cap = c->K.scale_k > 2.5 ? 96 : 48;
         const size_t slots = (size_t)(l->cap + (8 << b.lg));
@@ -1077,6 +1090,20 @@ NList nlist_of(const sphg_ctx* c, const PhaseBuf& b, bool nl)
     return L;
 }
 
+int pad8(int nb) { return (nb + 7) & ~7; }
+
+// Both phases' final kernels in one launch (after stages on one stream).
+int launch_finals(sphg_ctx* c, const FinalArgs& f)
+{
+    const PhaseBuf& W = c->ph[0];
+    const PhaseBuf& S = c->ph[1];
+    const bool mx = c->P.precision == SPHG_MIXED;
+    auto q = [&](const PhaseBuf& b) { return mx ? reinterpret_cast<float*>(b.rec) : nullptr; };
+    const FinalsArgs A{W.d, S.d, c->K, W.rec, S.rec, f.first, f.vf, f.renorm, f.ahead ? 1 : 0, q(W), q(S),
+                       c->gvl[0], c->gvl[1], c->csv, nref(c, 0, false), nref(c, 1, false), nblk(W.n), nblk(S.n)};
+    return launch(c, "finals", k_finals, pad8(A.nbS) + pad8(A.nbW), TPB, A);
+}
+
 // The fused step: pack (first_half + soil Drucker-Prager projections +
 // records), cross terms, partner masks, stage A, stage B.  The soil kernels
 // read only the packed records of both phases (the water pressure comes from
@@ -1106,6 +1133,17 @@ int stages_fused(sphg_ctx* c, const FinalArgs* fin)
     const bool us = c->ph[1].hmin == c->ph[1].hmax && rep_int && c->K.yield_criterion != 1;
     const bool uw = c->ph[0].hmin == c->ph[0].hmax && rep_int;
     const bool ux = c->F.uni_x != 0;
+    if (us && uw && ux && cross && !c->prof) {
+        // three launches on one stream (the profile times the passes apart)
+        StageArgs A{W.d, S.d, W.rec, S.rec, nW, nS, gW, gS, c->K, c->F, mask_b(c, 0), mask_b(c, 1), lean, nbW, nbS};
+        RC(launch(c, "stage1", k_stage1<SKF>, pad8(nbS) + 2 * pad8(nbW), STAGE_BLOCK, A));
+        swap_c(W);
+        swap_c(S);
+        A.W = W.d;
+        A.S = S.d;
+        RC(launch(c, "stage2", k_stage2<SKF>, pad8(nbS) + pad8(nbW), STAGE_BLOCK, A));
+        return fin ? launch_finals(c, *fin) : SPHG_OK;
+    }
     SideFork fork(c);
     RC(fork.rc);
     // with the finals on both streams, each phase's final kernel waits only
@@ -1234,6 +1272,17 @@ int stages_mixed(sphg_ctx* c, const FinalArgs* fin)
     const Grid& gS = nl ? c->gvl[1] : c->gl[1];
     MixK X = c->X;
     if (nl) X.cs = (float)c->csv;
+    if (!c->prof) {
+        StageArgsMx A{W.d, S.d, qW, qS, nW, nS, W.masks, gW, gS, c->K, c->F, X, mask_b(c, 0), mask_b(c, 1),
+                      nblk(W.n, STAGE_BLOCK), nblk(S.n, STAGE_BLOCK)};
+        RC(launch(c, "stage1", k_stage1_mx<SKF>, pad8(A.nbS) + 2 * pad8(A.nbW), STAGE_BLOCK, A));
+        swap_c(W);
+        swap_c(S);
+        A.W = W.d;
+        A.S = S.d;
+        RC(launch(c, "stage2", k_stage2_mx<SKF>, pad8(A.nbS) + pad8(A.nbW), STAGE_BLOCK, A));
+        return fin ? launch_finals(c, *fin) : SPHG_OK;
+    }
     SideFork fork(c);   // soil stage beside the water stages
     RC(fork.rc);
     {
@@ -2847,6 +2896,10 @@ void reg_batched(std::map<const void*, Batched>& m, void (*solo)(T...))
 template <int SKF>
 void reg_batched_skf(std::map<const void*, Batched>& m)
 {
+    reg_batched<BodyStage1<SKF>>(m, k_stage1<SKF>);
+    reg_batched<BodyStage2<SKF>>(m, k_stage2<SKF>);
+    reg_batched<BodyStage1Mx<SKF>>(m, k_stage1_mx<SKF>);
+    reg_batched<BodyStage2Mx<SKF>>(m, k_stage2_mx<SKF>);
     reg_batched<BodyWaterX<SKF, true>>(m, k_water_x4<SKF, true>);
     reg_batched<BodyWaterX<SKF, false>>(m, k_water_x4<SKF, false>);
     reg_batched<BodySoilX<SKF, true>>(m, k_soil_x4<SKF, true>);
@@ -2873,6 +2926,7 @@ const std::map<const void*, Batched>& batched_registry()
         reg_batched_skf<2>(r);
         reg_batched_skf<3>(r);
         reg_batched_skf<4>(r);
+        reg_batched<BodyFinals>(r, k_finals);
         reg_batched<BodyStepWater>(r, k_step_water);
         reg_batched<BodyStepSoil>(r, k_step_soil);
         reg_batched<BodyFinalWater>(r, k_final_water);
