@@ -94,13 +94,13 @@ struct BodyWaterB {
         water_b4<SKF, U>(lds, blk, a...);
     }
 };
-template <int SKF, bool U, bool SOLO>
+template <int SKF, bool U>
 struct BodySoilAB {
     template <class... A>
     __device__ __forceinline__ void operator()(int blk, const A&... a) const
     {
         __shared__ __align__(16) unsigned char lds[VIS_LDS<6>];
-        soil_ab4<SKF, U, SOLO>(lds, blk, a...);
+        soil_ab4<SKF, U, false>(lds, blk, a...);
     }
 };
 // (a tile is a workgroup of the solo launch, padding included)

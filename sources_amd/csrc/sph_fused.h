@@ -512,14 +512,19 @@ __device__ __forceinline__ void pack_soil_at(const DPhase& P, const KParams& K, 
     if (K.yield_criterion == 1) R[7 * pn] = make_double2(rho_pre, 0.0);
 }
 
+__device__ __forceinline__ void pack_soil_state(const DPhase& P, const KParams& K, double* rec, int t, int i,
+                                                int do_half, int ndp, float* q, const Grid& g, double cs,
+                                                const NRef& NR)
+{
+    pack_soil_at(P, K, rec, t, i, do_half, false, false, ndp, q, g, cs, NR, P.x[i], P.y[i], P.rho[i], P.vx[i], P.vy[i], P.p[i],
+                 P.sxx[i], P.sxy[i], P.syy[i]);
+}
+
 __device__ __forceinline__ void pack_soil_body(int blk, DPhase P, KParams K, double* rec, int do_half, int ndp,
                                                float* q, Grid g, double cs, NRef NR)
 {
     const int t = blk * blockDim.x + threadIdx.x;
-    if (t >= P.n) return;
-    const int i = P.order[t];
-    pack_soil_at(P, K, rec, t, i, do_half, false, false, ndp, q, g, cs, NR, P.x[i], P.y[i], P.rho[i], P.vx[i], P.vy[i], P.p[i],
-                 P.sxx[i], P.sxy[i], P.syy[i]);
+    if (t < P.n) pack_soil_state(P, K, rec, t, P.order[t], do_half, ndp, q, g, cs, NR);
 }
 
 __global__ void k_pack_soil(DPhase P, KParams K, double* rec, int do_half, int ndp, float* q, Grid g, double cs,
@@ -996,11 +1001,12 @@ __device__ __forceinline__ void visit_global(int* table, const Cand& C, const Id
     } while (__any(j < tot));
 }
 
-// LDS of a stage kernel that reads NCH chunks per partner.
+// LDS of a stage kernel that reads NCH chunks per partner (without a window:
+// the table alone).
+constexpr size_t TABLE_LDS = sizeof(int) * VIS_ROWS * STAGE_BLOCK;
 template <int NCH>
-constexpr size_t VIS_LDS = sizeof(int) * VIS_ROWS * STAGE_BLOCK > sizeof(double2) * NCH * WIN_STRIDE
-                               ? sizeof(int) * VIS_ROWS * STAGE_BLOCK
-                               : sizeof(double2) * NCH * WIN_STRIDE;
+constexpr size_t VIS_LDS = TABLE_LDS > sizeof(double2) * NCH * WIN_STRIDE ? TABLE_LDS
+                                                                         : sizeof(double2) * NCH * WIN_STRIDE;
 
 // Sends chunks 0 .. NCH - 1 of the workgroup's window on their way into LDS
 // (straight from global memory, no registers: all of it is in flight at once),
@@ -1487,7 +1493,7 @@ __device__ __forceinline__ void soil_ab4(unsigned char* lds, int blk, DPhase S, 
                                          int cross, int mask, int lean)
 {
     const RecV RS = recv(recS, S.n);
-    const SubCtx wc = sub_ctx(S.n, blk, NL.lg, WIN_LANES);
+    const SubCtx wc = sub_ctx(S.n, blk, NL.lg, SOLO ? STAGE_BLOCK : WIN_LANES);
     const int t = wc.t;
     auto RA = [&](int c) { return RS(wc.tt, c); };
     const double2 xy = RA(0), va = RA(1), a3 = RA(3), a4 = RA(4), a12 = RA(5);
@@ -1700,12 +1706,12 @@ __device__ __forceinline__ void soil_ab4(unsigned char* lds, int blk, DPhase S, 
     S.ay[a] = ay;
 }
 
-template <int SKF, bool U, bool SOLO>
+template <int SKF, bool U>
 __global__ STAGE_ATTR_AB void k_soil_ab4(DPhase S, const double* recS, NList NL, Grid g, KParams K, FusedK F,
                                          int cross, int mask, int lean)
 {
     __shared__ __align__(16) unsigned char lds[VIS_LDS<6>];
-    soil_ab4<SKF, U, SOLO>(lds, xcd_block(), S, recS, NL, g, K, F, cross, mask, lean);
+    soil_ab4<SKF, U, false>(lds, xcd_block(), S, recS, NL, g, K, F, cross, mask, lean);
 }
 
 // ------------------------------------------------------------------------

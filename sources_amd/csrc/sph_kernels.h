@@ -698,10 +698,9 @@ __device__ __forceinline__ SoilEnd soil_end(const DPhase& P, const KParams& K, i
     return e;
 }
 
-__device__ __forceinline__ void final_soil(int blk, DPhase P, KParams K, int first)
+// The final update of soil particle i.
+__device__ __forceinline__ SoilEnd final_soil_at(const DPhase& P, const KParams& K, int i, int first)
 {
-    const int i = blk * blockDim.x + threadIdx.x;
-    if (i >= P.n) return;
     const SoilEnd e = soil_end(P, K, i, first);
     if (K.volume_fraction && K.two_phase) P.vof[i] = e.vof;
     if (!K.summation_density) P.rho[i] = e.rho;
@@ -713,6 +712,13 @@ __device__ __forceinline__ void final_soil(int blk, DPhase P, KParams K, int fir
     }
     P.fail[i] = e.fail;
     P.sxx[i] = e.sxx; P.sxy[i] = e.sxy; P.syy[i] = e.syy; P.p[i] = e.p;
+    return e;
+}
+
+__device__ __forceinline__ void final_soil(int blk, DPhase P, KParams K, int first)
+{
+    const int i = blk * blockDim.x + threadIdx.x;
+    if (i < P.n) final_soil_at(P, K, i, first);
 }
 
 __global__ void k_final_soil(DPhase P, KParams K, int first)

@@ -429,3 +429,63 @@ __global__ __launch_bounds__(256) void k_w1_force(DPhase W, const double* rec, M
         }
     }
 }
+
+// ------------------------------------------------------------------------
+// Single-phase soil: the pack (with the rank inside the cells, as
+// k_w1_pack), then one pass over the partners (soil_ab4) with the step's final
+// update and the next step's cell keys in its tail (the partners are read from
+// the records alone).  Four launches a step instead of seven, and lanes per
+// particle by size (solo_lanes); bound: launch latency to about 40k particles,
+// then the candidate test and the partner gathers.  Per step: 3k particles 55
+// -> 31 us, 65k 63 -> 47, 128k 84 -> 60.
+// ------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void k_solo_pack(DPhase P, KParams K, double* rec, const int* arr, int do_half,
+                                                   int ndp)
+{
+    const int u = blockIdx.x * blockDim.x + threadIdx.x;
+    if (u >= P.n) return;
+    int t = u, i;
+    if (arr) {
+        t = cell_place(P, arr, u, i);
+        P.order[t] = i;
+    } else {
+        i = P.order[t];
+    }
+    pack_soil_state(P, K, rec, t, i, do_half, ndp, nullptr, Grid{}, 0.0, NRef{});
+}
+
+// What follows the rates: nothing (the right-hand side alone), or the update
+// of the step; ahead: and the cell keys and arrival ranks of the next one
+// (cell_count starts at zero).
+struct SoloEnd {
+    int update, first, ahead;
+    int* err;
+};
+
+template <int SKF, bool U>
+__global__ __launch_bounds__(256) void k_solo_step(DPhase S, const double* recS, Grid g, KParams K, FusedK F, int mask,
+                                                   int lg, SoloEnd E)
+{
+    __shared__ __align__(16) unsigned char lds[TABLE_LDS];
+    NList NL{};
+    NL.lg = lg;
+    soil_ab4<SKF, U, true>(lds, xcd_block(), S, recS, NL, g, K, F, 0, mask, E.ahead);
+    if (!E.update) return;
+    const SubCtx sc = sub_ctx(S.n, xcd_block(), lg, STAGE_BLOCK);
+    const bool own = sc.valid && !sc.sub;
+    const int i = S.order[sc.tt];
+    int key = -1;
+    if (own) {
+        const SoilEnd e = final_soil_at(S, K, i, E.first);
+        if (E.ahead) key = cell_key_of(g, e.x, e.y, E.err);
+    }
+    if (E.ahead) {
+        // (the lanes of a particle share its key)
+        const int gk = lg ? __shfl(key, (int)(threadIdx.x & 63) & ~((1 << lg) - 1), 64) : key;
+        const int slot = cell_slot_of(S.cell_count, gk, lg);
+        if (own) {
+            S.key[i] = key;
+            S.slot[i] = slot;
+        }
+    }
+}

@@ -1158,9 +1158,9 @@ int stages_fused(sphg_ctx* c, const FinalArgs* fin)
                            nS, gS, c->K, c->F, lean));
         }
         if (split) HIPCHK(c, hipEventRecord(c->ev_sx, c->side));
-        if (us) RC(launch(c, "soil_ab", k_soil_ab4<SKF, true, false>, nbS, STAGE_BLOCK, S.d, rS,
+        if (us) RC(launch(c, "soil_ab", k_soil_ab4<SKF, true>, nbS, STAGE_BLOCK, S.d, rS,
                           nS, gS, c->K, c->F, cross, mask_b(c, 1), lean));
-        else RC(launch(c, "soil_ab", k_soil_ab4<SKF, false, false>, nbS, STAGE_BLOCK, S.d, rS,
+        else RC(launch(c, "soil_ab", k_soil_ab4<SKF, false>, nbS, STAGE_BLOCK, S.d, rS,
                        nS, gS, c->K, c->F, cross, mask_b(c, 1), lean));
     }
     // water stage A, then the water cross terms (before stage B, whose tail
@@ -1214,27 +1214,33 @@ int stages_fused(sphg_ctx* c, const FinalArgs* fin)
     return fork.join();
 }
 
+// Lanes per particle (log2) of the single-phase soil pass, by the number of
+// particles, as w1_lanes.  us per step (1 / 2 / 4 / 8 lanes): 3k 42 / 36 / 32 /
+// 31, 14k 44 / 37 / 33 / 33, 25k 45 / 38 / 37 / 46, 34k 46 / 42 / 40 / 48, 65k
+// 50 / 47 / 54 / 65, 128k 60 / 67 / 74 / 104.
+int solo_lanes(int n) { return n <= 10000 ? 3 : n <= 40000 ? 2 : n <= 80000 ? 1 : 0; }
+
 // Single-phase soil (single_step_for_soil, declarations_sph.f90:1530-1655):
 // the one-pass soil kernel in its df form, without water partners.
 template <int SKF>
-int stages_soil_only(sphg_ctx* c)
+int stages_soil_only(sphg_ctx* c, const SoloEnd& end)
 {
     PhaseBuf& S = c->ph[1];
-    const double* rs = S.rec;
-    if (S.hmin == S.hmax && c->K.yield_criterion != 1)
-        RC(launch(c, "soil_ab", k_soil_ab4<SKF, true, true>, nblk(S.n, WIN_LANES), STAGE_BLOCK, S.d, rs, NList{},
-                  c->gl[1], c->K, c->F, 0, mask_b(c, 1), 0));
-    else
-        RC(launch(c, "soil_ab", k_soil_ab4<SKF, false, true>, nblk(S.n, WIN_LANES), STAGE_BLOCK, S.d, rs, NList{},
-                  c->gl[1], c->K, c->F, 0, mask_b(c, 1), 0));
-    swap_c(S);
-    return SPHG_OK;
+    const int lg = solo_lanes(S.n), nb = nblk(S.n, STAGE_BLOCK >> lg);
+    auto kern = S.hmin == S.hmax && c->K.yield_criterion != 1 ? k_solo_step<SKF, true> : k_solo_step<SKF, false>;
+    return launch(c, "soil_ab", kern, nb, STAGE_BLOCK, S.d, (const double*)S.rec, c->gl[1], c->K, c->F, mask_b(c, 1),
+                  lg, end);
 }
 
-int rhs_soil_only(sphg_ctx* c, int soil_half, int soil_ndp)
+// With the projections and first_half (soil_half) of the pack before it and
+// the update of end after it.
+int rhs_soil_only(sphg_ctx* c, int soil_half, int soil_ndp, const SoloEnd& end)
 {
     PhaseBuf& S = c->ph[1];
-    RC(build_cells(c, 1));
+    const bool keyed = c->keyed, built = S.cells_valid && !S.cells_nl;
+    const bool ranked = built || c->P.summation_density;   // (the pack takes the rank otherwise)
+    c->keyed = false;
+    RC(build_cells(c, 1, false, keyed, ranked));
     if (c->P.summation_density) {
         // single_step_for_soil's density approximation (declarations_sph.f90:
         // 1558-1562): rho <- sum_density.  first_half and the Drucker-Prager
@@ -1243,14 +1249,21 @@ int rhs_soil_only(sphg_ctx* c, int soil_half, int soil_ndp)
         RC(launch(c, "sum_density", k_sum_density, nblk(S.n), TPB, S.d, c->gl[1], c->K, c->K.h1_soil));
         std::swap(S.d.rho, S.d.rho_next);
     }
-    RC(launch(c, "pack", k_pack_soil, nblk(S.n), TPB, S.d, c->K, S.rec, soil_half, soil_ndp, (float*)nullptr,
-              c->gl[1], c->cs, NRef{}));
+    RC(launch(c, "pack", k_solo_pack, nblk(S.n), TPB, S.d, c->K, S.rec, ranked ? (const int*)nullptr : S.arrival,
+              soil_half, soil_ndp));
+    if (end.ahead) S.counts_zero = false;
+    int rc;
     switch (c->P.skf) {
-    case 1: return stages_soil_only<1>(c);
-    case 2: return stages_soil_only<2>(c);
-    case 3: return stages_soil_only<3>(c);
-    default: return stages_soil_only<4>(c);
+    case 1: rc = stages_soil_only<1>(c, end); break;
+    case 2: rc = stages_soil_only<2>(c, end); break;
+    case 3: rc = stages_soil_only<3>(c, end); break;
+    default: rc = stages_soil_only<4>(c, end); break;
     }
+    RC(rc);
+    swap_c(S);
+    if (end.update) S.cells_valid = false;   // the positions moved
+    c->keyed = end.ahead != 0;
+    return SPHG_OK;
 }
 
 bool soil_only(const sphg_ctx* c) { return c->P.single_phase && !c->ph[0].bound && c->ph[1].bound; }
@@ -1594,11 +1607,8 @@ int one_step(sphg_ctx* c, bool ahead_ok = false)
             RC(reorder(c, 1));
             c->since_reorder = 0;
         }
-        if (step != 1) RC(rhs_soil_only(c, 1, 2));
-        else RC(rhs_soil_only(c, 0, 1));
-        RC(launch(c, "final_soil", k_final_soil, nblk(S.n), TPB, S.d, c->K, step == 1 ? 1 : 0));
-        S.cells_valid = false;
-        return SPHG_OK;
+        const SoloEnd end{1, step == 1 ? 1 : 0, keys_ahead(c, ahead_ok) ? 1 : 0, c->d_err};
+        return step != 1 ? rhs_soil_only(c, 1, 2, end) : rhs_soil_only(c, 0, 1, end);
     }
     if (c->P.single_phase) {
         RC(reorder_water1(c, false));
@@ -2008,7 +2018,7 @@ int sphg_single_step(sphg_ctx* c, int sync)
     if (!c) return SPHG_ERR_INVALID;
     RC(check_fused_switches(c));
     if (soil_only(c)) {
-        RC(rhs_soil_only(c, 0, 1));
+        RC(rhs_soil_only(c, 0, 1, SoloEnd{0, 0, 0, c->d_err}));
     } else if (c->P.single_phase) {
         RC(rhs_water(c, false, W1End{}));
     } else {
@@ -2908,8 +2918,8 @@ void reg_batched_skf(std::map<const void*, Batched>& m)
     reg_batched<BodyWaterA<SKF, false>>(m, k_water_a4<SKF, false>);
     reg_batched<BodyWaterB<SKF, true>>(m, k_water_b4<SKF, true>);
     reg_batched<BodyWaterB<SKF, false>>(m, k_water_b4<SKF, false>);
-    reg_batched<BodySoilAB<SKF, true, false>>(m, k_soil_ab4<SKF, true, false>);
-    reg_batched<BodySoilAB<SKF, false, false>>(m, k_soil_ab4<SKF, false, false>);
+    reg_batched<BodySoilAB<SKF, true>>(m, k_soil_ab4<SKF, true>);
+    reg_batched<BodySoilAB<SKF, false>>(m, k_soil_ab4<SKF, false>);
     reg_batched<BodyWaterAMx<SKF>>(m, k_water_a_mx<SKF>);
     reg_batched<BodyWaterBMx<SKF>>(m, k_water_b_mx<SKF>);
     reg_batched<BodySoilABMx<SKF>>(m, k_soil_ab_mx<SKF>);
