@@ -156,3 +156,28 @@ __device__ __forceinline__ void for_each_candidate(const Grid& g, const CellList
         for (int k = k0; k < k1; ++k) f(cl.order[k]);
     }
 }
+
+// The candidates sub, sub + lanes, ... of the same block, rows joined (the
+// lanes of one particle share its candidates).
+template <class F>
+__device__ __forceinline__ void for_candidates_of_lane(const Grid& g, const CellList& cl, double x, double y, int sub,
+                                                       int lanes, F&& f)
+{
+    int cx, cy;
+    grid_cell(g, x, y, cx, cy);
+    cx = min(max(cx, 0), g.ncx - 1);   // (as above)
+    cy = min(max(cy, 0), g.ncy - 1);
+    const int c0 = max(cx - 1, 0), c1 = min(cx + 1, g.ncx - 1);
+    int k0[3], k1[3];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        const int row = cy - 1 + r;
+        const bool in = row >= 0 && row < g.ncy;
+        k0[r] = in ? cl.start[row * g.ncx + c0] : 0;
+        k1[r] = in ? cl.start[row * g.ncx + c1 + 1] : 0;
+    }
+    const int s1 = k1[0] - k0[0], s2 = s1 + k1[1] - k0[1], tot = s2 + k1[2] - k0[2];
+#pragma unroll 1
+    for (int c = sub; c < tot; c += lanes)
+        f(cl.order[c < s1 ? k0[0] + c : c < s2 ? k0[1] + c - s1 : k0[2] + c - s2]);
+}

@@ -743,25 +743,6 @@ __device__ __forceinline__ SubCtx sub_ctx(int n, int blk, int lg, int lanes)
     return c;
 }
 
-// Sum of v over the lanes of a particle (all get it).
-__device__ __forceinline__ void sub_sum(int lg, double& v)
-{
-    for (int o = 1; o < (1 << lg); o <<= 1) v += __shfl_xor(v, o, 64);
-}
-
-template <class... T>
-__device__ __forceinline__ void sub_sum(int lg, double& v, T&... rest)
-{
-    sub_sum(lg, v);
-    sub_sum(lg, rest...);
-}
-
-__device__ __forceinline__ int sub_count(int lg, int v)
-{
-    for (int o = 1; o < (1 << lg); o <<= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-
 // Wave-level set-up of the mixed-precision stage kernels.
 struct WaveCtx {
     int lane, t, tt, last;

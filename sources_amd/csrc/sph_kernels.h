@@ -726,6 +726,25 @@ __global__ void k_final_soil(DPhase P, KParams K, int first)
     final_soil(blockIdx.x, P, K, first);
 }
 
+// Sum of v over the lanes of a particle (all get it).
+__device__ __forceinline__ void sub_sum(int lg, double& v)
+{
+    for (int o = 1; o < (1 << lg); o <<= 1) v += __shfl_xor(v, o, 64);
+}
+
+template <class... T>
+__device__ __forceinline__ void sub_sum(int lg, double& v, T&... rest)
+{
+    sub_sum(lg, v);
+    sub_sum(lg, rest...);
+}
+
+__device__ __forceinline__ int sub_count(int lg, int v)
+{
+    for (int o = 1; o < (1 << lg); o <<= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+
 // ------------------------------------------------------------------------
 // Stage A, water: one gather over water neighbours and one over soil
 // neighbours.  Terms (reference routine -> accumulator):
@@ -735,10 +754,13 @@ __global__ void k_final_soil(DPhase P, KParams K, int first)
 //   darcy_law water side (:3832) -> dg      volume_fraction_water2 (:3940) -> dvx_cross
 //   volume_fraction_water (:3912) -> vof2
 // then pressure() (:2133) per particle: p and the new c.
+// (2^lg lanes per particle; this kernel and the three after it serve the
+// granular entries and the unfused step: 33k particles, 66 to 72 us each with
+// one lane, 16 to 29 with four.)
 // ------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_water_a(DPhase W, DPhase S, Grid g, KParams K, int mask)
+__global__ __launch_bounds__(256) void k_water_a(DPhase W, DPhase S, Grid g, KParams K, int mask, int lg)
 {
-    const int t = xcd_block() * blockDim.x + threadIdx.x;
+    const int u = xcd_block() * blockDim.x + threadIdx.x, t = u >> lg, sub = u & ((1 << lg) - 1);
     if (t >= W.n) return;
     const CellList cw{W.cell_start, W.order};
     const int a = cw.order[t];
@@ -749,7 +771,7 @@ __global__ __launch_bounds__(256) void k_water_a(DPhase W, DPhase S, Grid g, KPa
     const double sk = K.scale_k;
     double con = 0.0, drd = 0.0, txx = 0.0, txy = 0.0, tyy = 0.0, avx = 0.0, avy = 0.0, repx = 0.0, repy = 0.0;
     int cnt = 0;
-    for_each_candidate(g, cw, xa, ya, [&](int b) {
+    for_candidates_of_lane(g, cw, xa, ya, sub, 1 << lg, [&](int b) {
         if (b == a) return;
         const double xb = W.x[b], yb = W.y[b];
         const double mh = link ? K.h1_water : sph_mhsml(ha, W.hsml[b]);
@@ -801,7 +823,7 @@ __global__ __launch_bounds__(256) void k_water_a(DPhase W, DPhase S, Grid g, KPa
         const CellList cs{S.cell_start, S.order};
         const double vofa = W.vof[a];
         const double cf0 = -K.numeric_gravity;
-        for_each_candidate(g, cs, xa, ya, [&](int b) {
+        for_candidates_of_lane(g, cs, xa, ya, sub, 1 << lg, [&](int b) {
             const double xb = S.x[b], yb = S.y[b];
             const double mh = sph_mhsml(ha, S.hsml[b]);
             double dx, dy, r;
@@ -820,6 +842,11 @@ __global__ __launch_bounds__(256) void k_water_a(DPhase W, DPhase S, Grid g, KPa
             vof2 += mb * w;
         });
     }
+    sub_sum(lg, con, drd, txx, txy, tyy, avx, avy, repx, repy);
+    if (mask & M_CROSS) sub_sum(lg, dg_x, dg_y, dvof_x, vof2);
+    cnt = sub_count(lg, cnt);
+    cntx = sub_count(lg, cntx);
+    if (sub) return;
     // outputs
     if (mask & (M_CON | M_DRHO_DELTA)) {
         double base = (mask & M_CON) ? con : ((mask & M_DRHO_ACCUM) ? W.drho[a] : 0.0);
@@ -852,9 +879,9 @@ __global__ __launch_bounds__(256) void k_water_a(DPhase W, DPhase S, Grid g, KPa
 // side and pore_water_pressure (:3877, uses the new water p).  Per particle:
 // pressure() sets c, then plastic_or_not + plastic_flow_rule3 and Jaumann_rate.
 // ------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_soil_a(DPhase S, DPhase W, Grid g, KParams K, int mask)
+__global__ __launch_bounds__(256) void k_soil_a(DPhase S, DPhase W, Grid g, KParams K, int mask, int lg)
 {
-    const int t = xcd_block() * blockDim.x + threadIdx.x;
+    const int u = xcd_block() * blockDim.x + threadIdx.x, t = u >> lg, sub = u & ((1 << lg) - 1);
     if (t >= S.n) return;
     const CellList cs{S.cell_start, S.order};
     const int a = cs.order[t];
@@ -866,7 +893,7 @@ __global__ __launch_bounds__(256) void k_soil_a(DPhase S, DPhase W, Grid g, KPar
     double con = 0.0, drd = 0.0, txx = 0.0, txy = 0.0, tyy = 0.0, vcc = 0.0, wxy = 0.0;
     double avx = 0.0, avy = 0.0, repx = 0.0, repy = 0.0;
     int cnt = 0;
-    for_each_candidate(g, cs, xa, ya, [&](int b) {
+    for_candidates_of_lane(g, cs, xa, ya, sub, 1 << lg, [&](int b) {
         if (b == a) return;
         const double xb = S.x[b], yb = S.y[b];
         const double mh = link ? K.h1_soil : sph_mhsml(ha, S.hsml[b]);
@@ -926,7 +953,7 @@ __global__ __launch_bounds__(256) void k_soil_a(DPhase S, DPhase W, Grid g, KPar
         const CellList cw{W.cell_start, W.order};
         const double vofa = S.vof[a];
         const double cf0 = -K.numeric_gravity;
-        for_each_candidate(g, cw, xa, ya, [&](int b) {
+        for_candidates_of_lane(g, cw, xa, ya, sub, 1 << lg, [&](int b) {
             const double xb = W.x[b], yb = W.y[b];
             const double mh = sph_mhsml(W.hsml[b], ha);
             double dx, dy, r;   // oriented water - soil, as direct_find_2
@@ -944,6 +971,11 @@ __global__ __launch_bounds__(256) void k_soil_a(DPhase S, DPhase W, Grid g, KPar
             po_y += mprr * dwy * vofa;
         });
     }
+    sub_sum(lg, con, drd, txx, txy, tyy, vcc, wxy, avx, avy, repx, repy);
+    if (mask & M_CROSS) sub_sum(lg, dg_x, dg_y, po_x, po_y);
+    cnt = sub_count(lg, cnt);
+    cntx = sub_count(lg, cntx);
+    if (sub) return;
     if (mask & (M_CON | M_DRHO_DELTA)) {
         double base = (mask & M_CON) ? con : ((mask & M_DRHO_ACCUM) ? S.drho[a] : 0.0);
         S.drho[a] = base + drd;
@@ -1013,9 +1045,9 @@ __global__ __launch_bounds__(256) void k_soil_a(DPhase S, DPhase W, Grid g, KPar
 // (:1337); then /rho, + repulsion, + gravity, - Darcy drag, and
 // dvof = delta term - cross term.
 // ------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_water_b(DPhase W, Grid g, KParams K, int mask)
+__global__ __launch_bounds__(256) void k_water_b(DPhase W, Grid g, KParams K, int mask, int lg)
 {
-    const int t = xcd_block() * blockDim.x + threadIdx.x;
+    const int u = xcd_block() * blockDim.x + threadIdx.x, t = u >> lg, sub = u & ((1 << lg) - 1);
     if (t >= W.n) return;
     const CellList cw{W.cell_start, W.order};
     const int a = cw.order[t];
@@ -1027,7 +1059,7 @@ __global__ __launch_bounds__(256) void k_water_b(DPhase W, Grid g, KParams K, in
     const double sk = K.scale_k;
     double Px = 0.0, Py = 0.0, Sxx = 0.0, Sxyy = 0.0, Sxyx = 0.0, Syy = 0.0;
     double artx = 0.0, arty = 0.0, dvd = 0.0;
-    for_each_candidate(g, cw, xa, ya, [&](int b) {
+    for_candidates_of_lane(g, cw, xa, ya, sub, 1 << lg, [&](int b) {
         if (b == a) return;
         const double xb = W.x[b], yb = W.y[b], hb = W.hsml[b];
         const double mh = link ? K.h1_water : sph_mhsml(ha, hb);
@@ -1070,6 +1102,8 @@ __global__ __launch_bounds__(256) void k_water_b(DPhase W, Grid g, KParams K, in
             dvd += K.delta * ha * ca * mb * h / rhob;
         }
     });
+    sub_sum(lg, Px, Py, Sxx, Sxyy, Sxyx, Syy, artx, arty, dvd);
+    if (sub) return;
     {
 #pragma clang fp contract(off)
         double ax, ay;
@@ -1099,9 +1133,9 @@ __global__ __launch_bounds__(256) void k_water_b(DPhase W, Grid g, KParams K, in
 // delta_sph on p, sxx, sxy, syy (:1323-1331); then /rho, + repulsion,
 // + gravity, + Darcy drag, + pore-water pressure force.
 // ------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_soil_b(DPhase S, Grid g, KParams K, int mask)
+__global__ __launch_bounds__(256) void k_soil_b(DPhase S, Grid g, KParams K, int mask, int lg)
 {
-    const int t = xcd_block() * blockDim.x + threadIdx.x;
+    const int u = xcd_block() * blockDim.x + threadIdx.x, t = u >> lg, sub = u & ((1 << lg) - 1);
     if (t >= S.n) return;
     const CellList cs{S.cell_start, S.order};
     const int a = cs.order[t];
@@ -1115,7 +1149,7 @@ __global__ __launch_bounds__(256) void k_soil_b(DPhase S, Grid g, KParams K, int
     const double sk = K.scale_k;
     double Ax = 0.0, Ay = 0.0, Bxx = 0.0, Cxyy = 0.0, Cxyx = 0.0, Dyy = 0.0;
     double artx = 0.0, arty = 0.0, dP = 0.0, dXX = 0.0, dXY = 0.0, dYY = 0.0;
-    for_each_candidate(g, cs, xa, ya, [&](int b) {
+    for_candidates_of_lane(g, cs, xa, ya, sub, 1 << lg, [&](int b) {
         if (b == a) return;
         const double xb = S.x[b], yb = S.y[b], hb = S.hsml[b];
         const double mh = link ? K.h1_soil : sph_mhsml(ha, hb);
@@ -1177,6 +1211,8 @@ __global__ __launch_bounds__(256) void k_soil_b(DPhase S, Grid g, KParams K, int
             }
         }
     });
+    sub_sum(lg, Ax, Ay, Bxx, Cxyy, Cxyx, Dyy, artx, arty, dP, dXX, dXY, dYY);
+    if (sub) return;
     {
 #pragma clang fp contract(off)
         double ax, ay;
@@ -1305,7 +1341,17 @@ __global__ __launch_bounds__(256) void k_water1_b(DPhase W, Grid g, KParams K, i
 // Count pass: partners with a larger particle number; write pass: those
 // partners in ascending particle number, i.e. the reference's i-major /
 // j-ascending order, with W and grad W.
+//
+// PAIR_LANES lanes share a particle's candidates (about 50).  The write pass
+// collects the partners that pass into LDS, and an entry's place is the number
+// of entries with a smaller particle number; a particle with more than
+// PAIR_CAP of them counts over its candidates again instead.  A thread per
+// particle that searched its candidates for the next number, once per pair,
+// was a serial chain of 600 candidate tests (33k particles: write 414 us,
+// count 39; now 12 and 8).
 // ------------------------------------------------------------------------
+constexpr int PAIR_LANES = 16, PAIR_CAP = 64;
+
 __device__ __forceinline__ bool pair_pred(const DPhase& A, int a, const DPhase& B, int b, const Grid& g,
                                           const KParams& K, int link, double h1, double& dx, double& dy,
                                           double& r, double& mh)
@@ -1318,54 +1364,82 @@ __device__ __forceinline__ bool pair_pred(const DPhase& A, int a, const DPhase& 
 
 // same == 1: partners b > a of the same phase (and countiac over all partners);
 // same == 0: cross pairs, A = water, B = soil, all partners counted.
-__global__ void k_pair_count(DPhase A, DPhase B, Grid g, KParams K, int same, int link, double h1,
-                             int* fwd, int* countiac)
+__global__ __launch_bounds__(256) void k_pair_count(DPhase A, DPhase B, Grid g, KParams K, int same, int link,
+                                                    double h1, int* fwd, int* countiac)
 {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= A.n) return;
+    const int a = blockIdx.x * (256 / PAIR_LANES) + threadIdx.x / PAIR_LANES, sub = threadIdx.x % PAIR_LANES;
+    if (a >= A.n) return;   // (all lanes of the particle)
     const CellList cl{B.cell_start, B.order};
     const int ida = A.id[a];
     int nf = 0, nall = 0;
-    for_each_candidate(g, cl, A.x[a], A.y[a], [&](int b) {
+    for_candidates_of_lane(g, cl, A.x[a], A.y[a], sub, PAIR_LANES, [&](int b) {
         if (same && b == a) return;
         double dx, dy, r, mh;
         if (!pair_pred(A, a, B, b, g, K, link, h1, dx, dy, r, mh)) return;
         ++nall;
         if (!same || B.id[b] > ida) ++nf;
     });
+    for (int o = 1; o < PAIR_LANES; o <<= 1) {
+        nf += __shfl_xor(nf, o, 64);
+        nall += __shfl_xor(nall, o, 64);
+    }
+    if (sub) return;
     fwd[ida] = nf;
     if (countiac) countiac[a] = nall;
 }
 
-__global__ void k_pair_write(DPhase A, DPhase B, Grid g, KParams K, int same, int link, double h1,
-                             const int* off, int* pi, int* pj, double* w, double* dwdx)
+__global__ __launch_bounds__(256) void k_pair_write(DPhase A, DPhase B, Grid g, KParams K, int same, int link,
+                                                    double h1, const int* off, int* pi, int* pj, double* w,
+                                                    double* dwdx)
 {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= A.n) return;
+    __shared__ int2 list[256 / PAIR_LANES][PAIR_CAP];   // (particle number, slot)
+    __shared__ int count[256 / PAIR_LANES];
+    const int grp = threadIdx.x / PAIR_LANES, sub = threadIdx.x % PAIR_LANES;
+    const int a = blockIdx.x * (256 / PAIR_LANES) + grp;
+    const bool valid = a < A.n;
     const CellList cl{B.cell_start, B.order};
-    const int ida = A.id[a];
-    int o = off[ida];
-    const int cnt = off[ida + 1] - o;
-    int prev = same ? ida : -1;
-    for (int s = 0; s < cnt; ++s) {
-        int best = 0x7fffffff, bestb = 0;
-        for_each_candidate(g, cl, A.x[a], A.y[a], [&](int b) {
+    if (sub == 0) count[grp] = 0;
+    __syncthreads();
+    const int ida = valid ? A.id[a] : 0, prev = same ? ida : -1;
+    if (valid)
+        for_candidates_of_lane(g, cl, A.x[a], A.y[a], sub, PAIR_LANES, [&](int b) {
             const int idb = B.id[b];
-            if (idb <= prev || idb >= best) return;
             double dx, dy, r, mh;
-            if (!pair_pred(A, a, B, b, g, K, link, h1, dx, dy, r, mh)) return;
-            best = idb;
-            bestb = b;
+            if (idb <= prev || !pair_pred(A, a, B, b, g, K, link, h1, dx, dy, r, mh)) return;
+            const int e = atomicAdd(&count[grp], 1);
+            if (e < PAIR_CAP) list[grp][e] = make_int2(idb, b);
         });
+    __syncthreads();
+    if (!valid) return;
+    const int o = off[ida], cnt = count[grp];
+    auto put = [&](int rank, int idb, int b) {
         double dx, dy, r, mh, ww, gx, gy;
-        pair_pred(A, a, B, bestb, g, K, link, h1, dx, dy, r, mh);
+        pair_pred(A, a, B, b, g, K, link, h1, dx, dy, r, mh);
         sph_kernel(K.skf, r, dx, dy, mh, ww, gx, gy);
-        pi[o] = ida + 1;
-        pj[o] = best + 1;
-        w[o] = ww;
-        dwdx[2 * o] = gx;
-        dwdx[2 * o + 1] = gy;
-        ++o;
-        prev = best;
+        pi[o + rank] = ida + 1;
+        pj[o + rank] = idb + 1;
+        w[o + rank] = ww;
+        dwdx[2 * (o + rank)] = gx;
+        dwdx[2 * (o + rank) + 1] = gy;
+    };
+    if (cnt <= PAIR_CAP) {
+        for (int e = sub; e < cnt; e += PAIR_LANES) {
+            const int2 me = list[grp][e];
+            int rank = 0;
+            for (int j = 0; j < cnt; ++j) rank += list[grp][j].x < me.x ? 1 : 0;
+            put(rank, me.x, me.y);
+        }
+        return;
     }
+    for_candidates_of_lane(g, cl, A.x[a], A.y[a], sub, PAIR_LANES, [&](int b) {
+        const int idb = B.id[b];
+        double dx, dy, r, mh;
+        if (idb <= prev || !pair_pred(A, a, B, b, g, K, link, h1, dx, dy, r, mh)) return;
+        int rank = 0;
+        for_each_candidate(g, cl, A.x[a], A.y[a], [&](int b2) {
+            const int id2 = B.id[b2];
+            if (id2 > prev && id2 < idb && pair_pred(A, a, B, b2, g, K, link, h1, dx, dy, r, mh)) ++rank;
+        });
+        put(rank, idb, b);
+    });
 }

@@ -1044,6 +1044,24 @@ bool nl_at(const sphg_ctx* c, int step)
 
 bool nl_mode(const sphg_ctx* c) { return nl_at(c, c->itimestep); }
 
+// Lanes per particle (log2) of the single-phase water passes, by the number
+// of particles: the chip's 1024 SIMDs hold one wave each at 65536 particles
+// and one lane per particle, so fewer leave SIMDs idle and each wave alone
+// with the latency of its partner loop, and many more lanes than that repeat
+// the particles' own loads for nothing.  Dam break, us per step (1 / 2 / 4 / 8
+// lanes): 7.5k 57 / 48 / 41 / 39, 14k 58 / 48 / 42 / 42, 44k 60 / 57 / 53 / 60,
+// 85k 75 / 69 / 73 / 86, 168k 93 / 101 / 108 / 137.
+int w1_lanes(int n) { return n <= 16384 ? 3 : n <= 65536 ? 2 : n <= 122880 ? 1 : 0; }
+
+// A kernel of the granular entries and the unfused step: one thread per
+// particle and lane, the lanes by size as for the single-phase passes.
+template <class... K, class... A>
+int launch_lanes(sphg_ctx* c, const char* name, void (*kern)(K...), int n, const A&... args)
+{
+    const int lg = w1_lanes(n);
+    return launch(c, name, kern, nblk(n << lg), TPB, args..., lg);
+}
+
 // single_step (declarations_sph.f90:1131-1435) after the soil Drucker-Prager
 // projection of :1244 has been applied (legacy unfused kernels).
 int rhs_two_phase_legacy(sphg_ctx* c)
@@ -1052,12 +1070,12 @@ int rhs_two_phase_legacy(sphg_ctx* c)
     PhaseBuf& S = c->ph[1];
     RC(build_cells(c, 0));
     RC(build_cells(c, 1));
-    RC(launch(c, "water_a", k_water_a, nblk(W.n), TPB, W.d, S.d, c->gl[0], c->K, mask_a(c, MASK_A_W)));
-    RC(launch(c, "soil_a", k_soil_a, nblk(S.n), TPB, S.d, W.d, c->gl[1], c->K, mask_a(c, MASK_A_S)));
+    RC(launch_lanes(c, "water_a", k_water_a, W.n, W.d, S.d, c->gl[0], c->K, mask_a(c, MASK_A_W)));
+    RC(launch_lanes(c, "soil_a", k_soil_a, S.n, S.d, W.d, c->gl[1], c->K, mask_a(c, MASK_A_S)));
     swap_c(W);
     swap_c(S);
-    RC(launch(c, "water_b", k_water_b, nblk(W.n), TPB, W.d, c->gl[0], c->K, mask_b(c, 0)));
-    RC(launch(c, "soil_b", k_soil_b, nblk(S.n), TPB, S.d, c->gl[1], c->K, mask_b(c, 1)));
+    RC(launch_lanes(c, "water_b", k_water_b, W.n, W.d, c->gl[0], c->K, mask_b(c, 0)));
+    RC(launch_lanes(c, "soil_b", k_soil_b, S.n, S.d, c->gl[1], c->K, mask_b(c, 1)));
     return SPHG_OK;
 }
 
@@ -1446,15 +1464,6 @@ int rhs_two_phase_fused(sphg_ctx* c, int water_half, int soil_half, int soil_ndp
     return stages_of(c);
 }
 
-// Lanes per particle (log2) of the single-phase water passes, by the number
-// of particles: the chip's 1024 SIMDs hold one wave each at 65536 particles
-// and one lane per particle, so fewer leave SIMDs idle and each wave alone
-// with the latency of its partner loop, and many more lanes than that repeat
-// the particles' own loads for nothing.  Dam break, us per step (1 / 2 / 4 / 8
-// lanes): 7.5k 57 / 48 / 41 / 39, 14k 58 / 48 / 42 / 42, 44k 60 / 57 / 53 / 60,
-// 85k 75 / 69 / 73 / 86, 168k 93 / 101 / 108 / 137.
-int w1_lanes(int n) { return n <= 16384 ? 3 : n <= 65536 ? 2 : n <= 122880 ? 1 : 0; }
-
 template <int SKF, bool U>
 int w1_passes(sphg_ctx* c, const W1End& end)
 {
@@ -1687,6 +1696,8 @@ int verlet_steps(sphg_ctx* c, int nsteps)
 
 // ---- materialised pair lists -------------------------------------------
 
+int pair_blocks(int n) { return nblk(n, 256 / PAIR_LANES); }
+
 int materialise(sphg_ctx* c, int ka, int kb, int same, int link, sphg_phase_view* out_view,
                 int* out_niac)
 {
@@ -1694,7 +1705,7 @@ int materialise(sphg_ctx* c, int ka, int kb, int same, int link, sphg_phase_view
     PhaseBuf& B = c->ph[kb];
     RC(build_cells(c, kb));
     const double h1 = (ka == 0) ? c->K.h1_water : c->K.h1_soil;
-    RC(launch(c, "pair_count", k_pair_count, nblk(A.n), TPB, A.d, B.d, c->gl[ka], c->K, same, link, h1,
+    RC(launch(c, "pair_count", k_pair_count, pair_blocks(A.n), TPB, A.d, B.d, c->gl[ka], c->K, same, link, h1,
               A.fwd, A.d.countiac));
     RC(exclusive_scan(c, A.fwd, A.off, A.n));
     int total = 0;
@@ -1705,7 +1716,7 @@ int materialise(sphg_ctx* c, int ka, int kb, int same, int link, sphg_phase_view
     if (total > out_view->max_interaction) return SPHG_ERR_TOO_MANY_INTERACTIONS;
     if (!out_view->pair_i || !out_view->pair_j || !out_view->w || !out_view->dwdx) return SPHG_ERR_INVALID;
     RC(ensure_pairs(c, A, total > 0 ? total : 1));
-    RC(launch(c, "pair_write", k_pair_write, nblk(A.n), TPB, A.d, B.d, c->gl[ka], c->K, same, link, h1,
+    RC(launch(c, "pair_write", k_pair_write, pair_blocks(A.n), TPB, A.d, B.d, c->gl[ka], c->K, same, link, h1,
               (const int*)A.off, A.pi, A.pj, A.w, A.dwdx));
     if (total > 0) {
         HIPCHK(c, hipMemcpyAsync(out_view->pair_i, A.pi, sizeof(int) * (size_t)total, hipMemcpyDeviceToHost, c->stream));
@@ -1911,7 +1922,7 @@ int sphg_direct_find_2(sphg_ctx* c)
     // countiac of the soil phase: number of water partners
     PhaseBuf& S = c->ph[1];
     RC(build_cells(c, 0));
-    RC(launch(c, "pair_count", k_pair_count, nblk(S.n), TPB, S.d, c->ph[0].d, c->gl[1], c->K, 0, 0, 0.0,
+    RC(launch(c, "pair_count", k_pair_count, pair_blocks(S.n), TPB, S.d, c->ph[0].d, c->gl[1], c->K, 0, 0, 0.0,
               S.fwd, S.d.countiac));
     RC(download(c, 0, SPHG_F_COUNTIAC));
     RC(download(c, 1, SPHG_F_COUNTIAC));
@@ -1927,9 +1938,9 @@ int sphg_con_density(sphg_ctx* c, int phase)
     RC(build_cells(c, k));
     PhaseBuf& b = c->ph[k];
     if (k == 0)
-        RC(launch(c, "water_a", k_water_a, nblk(b.n), TPB, b.d, c->ph[1].d, c->gl[0], c->K, (int)M_CON));
+        RC(launch_lanes(c, "water_a", k_water_a, b.n, b.d, c->ph[1].d, c->gl[0], c->K, (int)M_CON));
     else
-        RC(launch(c, "soil_a", k_soil_a, nblk(b.n), TPB, b.d, c->ph[0].d, c->gl[1], c->K, (int)M_CON));
+        RC(launch_lanes(c, "soil_a", k_soil_a, b.n, b.d, c->ph[0].d, c->gl[1], c->K, (int)M_CON));
     RC(download(c, k, SPHG_F_DRHO));
     return check_flags(c);
 }
@@ -1944,9 +1955,9 @@ int sphg_delta_sph_density(sphg_ctx* c, int phase)
     PhaseBuf& b = c->ph[k];
     const int m = M_DRHO_DELTA | M_DRHO_ACCUM;
     if (k == 0)
-        RC(launch(c, "water_a", k_water_a, nblk(b.n), TPB, b.d, c->ph[1].d, c->gl[0], c->K, m));
+        RC(launch_lanes(c, "water_a", k_water_a, b.n, b.d, c->ph[1].d, c->gl[0], c->K, m));
     else
-        RC(launch(c, "soil_a", k_soil_a, nblk(b.n), TPB, b.d, c->ph[0].d, c->gl[1], c->K, m));
+        RC(launch_lanes(c, "soil_a", k_soil_a, b.n, b.d, c->ph[0].d, c->gl[1], c->K, m));
     RC(download(c, k, SPHG_F_DRHO));
     return check_flags(c);
 }
@@ -1975,9 +1986,9 @@ int sphg_internal_force(sphg_ctx* c, int phase)
     if (k == 0) {
         RC(upload(c, k, SPHG_F_X | SPHG_F_VX | SPHG_F_RHO | SPHG_F_VOF | SPHG_F_C));
         RC(build_cells(c, k));
-        RC(launch(c, "water_a", k_water_a, nblk(b.n), TPB, b.d, c->ph[1].d, c->gl[0], c->K, (int)(M_STRAIN | M_EOS)));
+        RC(launch_lanes(c, "water_a", k_water_a, b.n, b.d, c->ph[1].d, c->gl[0], c->K, (int)(M_STRAIN | M_EOS)));
         swap_c(b);
-        RC(launch(c, "water_b", k_water_b, nblk(b.n), TPB, b.d, c->gl[0], c->K, (int)M_MOMENTUM));
+        RC(launch_lanes(c, "water_b", k_water_b, b.n, b.d, c->gl[0], c->K, (int)M_MOMENTUM));
         RC(download(c, k, SPHG_F_DVX | SPHG_F_P | SPHG_F_C | SPHG_F_STRAIN | SPHG_F_STRESS));
     } else {
         if (c->P.yield_criterion != 2 || (c->P.plasticity != 3 && c->P.plasticity != 0)) return SPHG_ERR_UNSUPPORTED;
@@ -1985,10 +1996,10 @@ int sphg_internal_force(sphg_ctx* c, int phase)
                             SPHG_F_DSTRESS | SPHG_F_EPSP));
         RC(build_cells(c, k));
         RC(launch(c, "first_half", k_first_half_soil, nblk(b.n), TPB, b.d, c->K, 0, 1));
-        RC(launch(c, "soil_a", k_soil_a, nblk(b.n), TPB, b.d, c->ph[0].d, c->gl[1], c->K,
+        RC(launch_lanes(c, "soil_a", k_soil_a, b.n, b.d, c->ph[0].d, c->gl[1], c->K,
                   (int)(M_STRAIN | M_EOS | M_PLASTIC | M_DS_ACCUM)));
         swap_c(b);
-        RC(launch(c, "soil_b", k_soil_b, nblk(b.n), TPB, b.d, c->gl[1], c->K, (int)M_MOMENTUM));
+        RC(launch_lanes(c, "soil_b", k_soil_b, b.n, b.d, c->gl[1], c->K, (int)M_MOMENTUM));
         RC(download(c, k, SPHG_F_DVX | SPHG_F_P | SPHG_F_C | SPHG_F_STRAIN | SPHG_F_STRESS | SPHG_F_DSTRESS |
                               SPHG_F_EPSP | SPHG_F_FAIL));
     }
@@ -2006,9 +2017,9 @@ int sphg_art_visc(sphg_ctx* c, int phase)
     if (c->P.single_phase && k == 0)
         RC(launch(c, "water1_b", k_water1_b, nblk(b.n), TPB, b.d, c->gl[0], c->K, (int)M_ART));
     else if (k == 0)
-        RC(launch(c, "water_b", k_water_b, nblk(b.n), TPB, b.d, c->gl[0], c->K, (int)M_ART));
+        RC(launch_lanes(c, "water_b", k_water_b, b.n, b.d, c->gl[0], c->K, (int)M_ART));
     else
-        RC(launch(c, "soil_b", k_soil_b, nblk(b.n), TPB, b.d, c->gl[1], c->K, (int)M_ART));
+        RC(launch_lanes(c, "soil_b", k_soil_b, b.n, b.d, c->gl[1], c->K, (int)M_ART));
     RC(download(c, k, SPHG_F_DVX));
     return check_flags(c);
 }
@@ -3618,7 +3629,7 @@ int sphg_direct_find_noalloc(const sphg_params* params, int n, const double* x, 
                  (const int*)tiles, ntiles, ncell, fwd));
     RC(na_launch(st, k_cell_rank, nblk(n, SCAN_BLOCK), SCAN_BLOCK, d, (const int*)fwd));
     // partner counts, their prefix, the total (the kernels of materialise)
-    RC(na_launch(st, k_pair_count, nblk(n), TPB, d, d, g, K, 1, 0, 0.0, fwd, countiac));
+    RC(na_launch(st, k_pair_count, pair_blocks(n), TPB, d, d, g, K, 1, 0, 0.0, fwd, countiac));
     RC(na_launch(st, k_scan_tile, ptiles, SCAN_BLOCK, (const int*)fwd, off, n, tiles, (int*)nullptr));
     RC(na_launch(st, k_scan_sums, 1, SCAN_BLOCK, tiles, ptiles));
     RC(na_launch(st, k_scan_add, nblk(n), TPB, off, n, (const int*)tiles, ptiles));
@@ -3630,7 +3641,7 @@ int sphg_direct_find_noalloc(const sphg_params* params, int n, const double* x, 
     *niac = host[0];
     if (host[0] > max_interaction) return SPHG_ERR_TOO_MANY_INTERACTIONS;
     if (host[0] > 0 && (!pair_i || !pair_j || !w || !dwdx)) return SPHG_ERR_INVALID;
-    RC(na_launch(st, k_pair_write, nblk(n), TPB, d, d, g, K, 1, 0, 0.0, (const int*)off, (int*)pair_i,
+    RC(na_launch(st, k_pair_write, pair_blocks(n), TPB, d, d, g, K, 1, 0, 0.0, (const int*)off, (int*)pair_i,
                  (int*)pair_j, w, dwdx));
     NACHK(hipStreamSynchronize(st));
     return SPHG_OK;
