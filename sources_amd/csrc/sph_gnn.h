@@ -16,11 +16,9 @@
 // Since W2 is linear, the sum over edges is taken before it: the per-edge
 // work is one 32 x 32 x 16 MFMA per neighbour slot for 32 particles.
 //
-// One wavefront handles 32 particles.  Every matrix product is a
-// v_mfma_f32_32x32x16_bf16 tile product whose operands are read through
-// accessors (LDS or global), so forward and backward (training) share one
-// primitive.  MFMA operand layout (gfx950, wave64): lane l holds row l % 32
-// of A and column l % 32 of B, k = (l / 32) * 8 + [0, 8); the 16 results
+// One wavefront handles 32 particles; every matrix product is a
+// v_mfma_f32_32x32x16_bf16.  Operand layout (gfx950, wave64): lane l holds row
+// l % 32 of A and column l % 32 of B, k = (l / 32) * 8 + [0, 8); the 16 results
 // of lane l are C[(v / 4) * 8 + (l / 32) * 4 + v % 4][l % 32], v = 0..15.
 #pragma once
 #include "sph_fused.h"
@@ -64,58 +62,100 @@ __device__ __forceinline__ f32x16 zero16()
     return z;
 }
 
-// acc += A (32 x K) B (K x 32); a(row, k), b(k, col) return FP32 values that
-// are rounded to BF16 operands.  K is a multiple of 16.
-template <class FA, class FB>
-__device__ __forceinline__ f32x16 mma(FA&& a, FB&& b, int K, f32x16 acc)
+// The 16 results of a lane are rows perm(h, v) = (v >> 2) * 8 + h * 4 + (v & 3)
+// of its column, so a 32-node x 32-feature block comes out of a product in one
+// of two forms, and both are operands of the next product, in registers:
+//   node form     mfma(W, X): lane (r, h) holds node r.  Rounded to BF16, two
+//                 v_permlane32_swap per 16 features exchange features 4-7 of
+//                 the lower half-wave with 8-11 of the upper: k = h * 8 + [0, 8),
+//                 the next layer's operand.
+//   feature form  mfma(X, W): lane (c, h) holds feature c, nodes perm(h, v).
+//                 Operand of a sum over nodes (gradients) as it stands: the
+//                 order of k is free as long as both operands share it.
+// So a chain of layers needs neither LDS nor barriers.
+struct Op2 {
+    bf16x8 k[2];   // the two k-steps of a block, rounded to BF16
+};
+
+__device__ __forceinline__ f32x16 mfma(const bf16x8& a, const bf16x8& b, const f32x16& c)
 {
-    const int l = lane_id(), r = l & 31, h = l >> 5;
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        bf16x8 av, bv;
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// Operand in feature form.
+__device__ __forceinline__ Op2 round_feat(const f32x16& c)
+{
+    Op2 o;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            av[i] = (__bf16)a(r, k0 + h * 8 + i);
-            bv[i] = (__bf16)b(k0 + h * 8 + i, r);
+    for (int v = 0; v < 16; ++v) o.k[v >> 3][v & 7] = (__bf16)c[v];
+    return o;
+}
+
+// Result order <-> operand order of a block in node form (its own inverse).
+__device__ __forceinline__ Op2 swap_order(const Op2& x)
+{
+    Op2 o;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+        u32x4 d = __builtin_bit_cast(u32x4, x.k[ks]);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            // upper lanes of the first <-> lower lanes of the second
+            const auto sw = __builtin_amdgcn_permlane32_swap(d[q], d[q + 2], false, false);
+            d[q] = sw[0];
+            d[q + 2] = sw[1];
         }
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc, 0, 0, 0);
+        o.k[ks] = __builtin_bit_cast(bf16x8, d);
     }
-    return acc;
+    return o;
 }
 
-// Weights of the node MLP as BF16 B operands for inference: for each matrix,
-// n-tile and 16-row k-step, 64 lanes x 8 values (lane l: column l & 31 of
-// the tile, rows k0 + (l >> 5) * 8 + 0..7) -- the values mma() rounds from the
-// FP32 weights, one 16-byte load per lane and step.
-constexpr int P_W2 = 0;                // HE x HE: 1 tile x 2 steps
-constexpr int P_W3 = P_W2 + 2 * 64;    // FI x D: 2 tiles x 4 steps
-constexpr int P_W4 = P_W3 + 8 * 64;    // D x D: 2 tiles x 4 steps
-constexpr int P_W5 = P_W4 + 8 * 64;    // D x NOP: 1 tile x 4 steps
-constexpr int NPACK = P_W5 + 4 * 64;
+// Operand in node form.
+__device__ __forceinline__ Op2 round_node(const f32x16& c) { return swap_order(round_feat(c)); }
 
-// acc += A (32 x K) Bp, Bp: the packed operands of one n-tile (K / 16 steps).
-template <class FA>
-__device__ __forceinline__ f32x16 mma_p(FA&& a, const bf16x8* bp, int K, f32x16 acc)
+// Packed weights, in entries of one k-step of one 32-wide tile (64 lanes x 8
+// values): each matrix by output tile (forward) and by input tile (backward;
+// only what the gradients use: the message rows of W3, 16 of W5's columns).
+constexpr int P_W1 = 0;
+constexpr int P_W2 = P_W1 + 64;        // HE x HE
+constexpr int P_W3 = P_W2 + 2 * 64;    // FI x D: 2 tiles x 4 k-steps
+constexpr int P_W4 = P_W3 + 8 * 64;    // D x D: 2 x 4
+constexpr int P_W5 = P_W4 + 8 * 64;    // D x NOP: 1 x 4
+constexpr int P_B2 = P_W5 + 4 * 64;    // W2^T: 1 x 2
+constexpr int P_B3 = P_B2 + 2 * 64;    // W3^T, rows FN..FI-1: 1 x 4
+constexpr int P_B4 = P_B3 + 4 * 64;    // W4^T: 2 x 4
+constexpr int P_B5 = P_B4 + 8 * 64;    // W5^T: 2 x 1
+constexpr int NPACK = P_B5 + 2 * 64;
+
+// Element (in BF16 values) of row r of a tile at k, the matrix having nks k-steps.
+__host__ __device__ __forceinline__ int pack_at(int entry, int r, int nks, int k)
 {
-    const int l = lane_id(), r = l & 31, h = l >> 5;
-    for (int k0 = 0, ks = 0; k0 < K; k0 += 16, ++ks) {
-        bf16x8 av;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) av[i] = (__bf16)a(r, k0 + h * 8 + i);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bp[ks * 64 + l], acc, 0, 0, 0);
-    }
-    return acc;
+    return (entry + ((r >> 5) * nks + (k >> 4)) * 64 + (r & 31) + 32 * ((k >> 3) & 1)) * 8 + (k & 7);
 }
 
-// f(row, col, value&) over the 16 results a lane holds.
+// Where parameter e goes in the packed weights: f(element) up to two times.
 template <class F>
-__device__ __forceinline__ void tile_each(f32x16& c, F&& f)
+__host__ __device__ __forceinline__ void pack_places(int e, F&& f)
 {
-    const int l = lane_id(), col = l & 31, h = l >> 5;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        float x = c[v];
-        f((v >> 2) * 8 + h * 4 + (v & 3), col, x);
-        c[v] = x;
+    if (e < O_W2) {
+        const int i = e / HE, o = e % HE;
+        f(pack_at(P_W1, o, 1, i));
+    } else if (e < O_W3) {
+        const int i = (e - O_W2) / HE, o = (e - O_W2) % HE;
+        f(pack_at(P_W2, o, 2, i));
+        f(pack_at(P_B2, i, 2, o));
+    } else if (e < O_B3) {
+        const int i = (e - O_W3) / D, o = (e - O_W3) % D;
+        f(pack_at(P_W3, o, 4, i));
+        if (i >= FN) f(pack_at(P_B3, i - FN, 4, o));
+    } else if (e >= O_W4 && e < O_B4) {
+        const int i = (e - O_W4) / D, o = (e - O_W4) % D;
+        f(pack_at(P_W4, o, 4, i));
+        f(pack_at(P_B4, i, 4, o));
+    } else if (e >= O_W5 && e < O_B5) {
+        const int i = (e - O_W5) / NOP, o = (e - O_W5) % NOP;
+        f(pack_at(P_W5, o, 4, i));
+        if (o < 16) f(pack_at(P_B5, i, 1, o));
     }
 }
 
@@ -154,7 +194,7 @@ __device__ __forceinline__ void edge_features(const float* ri, const float* rj, 
     if (!has) return;
     const float ih = 1.0f / ri[7];
     const float dx = ri[0] - rj[0], dy = ri[1] - rj[1];
-    const float r = sqrtf(dx * dx + dy * dy);
+    const float r = sqrtf(__builtin_fmaf(dx, dx, dy * dy));   // (written out: the same value in every kernel)
     const float q = fminf(r * ih * 0.5f, 1.0f);
     e[0] = 1.0f;
     e[1] = dx * ih;
@@ -172,131 +212,61 @@ __device__ __forceinline__ void edge_features(const float* ri, const float* rj, 
 struct GnnArgs {
     Graph G;
     const float* W;      // [NPARAM]
-    const bf16x8* Wp;    // [NPACK] packed node-MLP weights (inference)
-    float* out;          // [n][NO] (forward) or nullptr
+    const bf16x8* Wp;    // [NPACK] packed weights
+    float* out;          // [n][NO] (forward)
     // training
     const float* tgt;    // [n][NO] targets (normalised)
     const float* tw;     // [n] loss weight (1 real, 0 virtual)
-    float* gW;           // [NPARAM] gradient accumulator
-    float* loss;         // [1] accumulator of sum w (y - t)^2
+    float4* part;        // [workgroups][NPART / 4] gradient sums of the workgroups
     float inv_count;     // gradient scale: 1 / (number of weighted terms)
     float inv_out[NO];   // targets are physical corrections; y predicts target * inv_out
     float cw[NO];        // loss weight of each output
 };
 
-// Forward (TRAIN = false) or forward + backward (TRAIN = true) over 32
-// nodes per workgroup (one wavefront).
-// LDS tiles of one wavefront.  Inference reuses two regions: X0 then H4 in
-// the first, HS then H3 in the second (each dead before the other is
-// written); training keeps all of them for the backward pass.
-constexpr int TILE_D = 32 * (D + 1);
-constexpr int lds_floats(bool train)
+// The edges of node i (one per lane r of both halves), two slots at a time:
+// f(o1, o2) gets the BF16 features of slots s and s + 1 as operands (zero past
+// the node's degree).  Half-wave h builds the 16
+// features of slot s + h of its node, then lanes r and r + 32 exchange the
+// feature half the other slot's operand needs (v_permlane32_swap), so each
+// edge's features are computed once.  The neighbour's row of the next pair and
+// the index of the one after it are in flight meanwhile.
+template <class F>
+__device__ __forceinline__ void for_edge_pairs(const Graph& G, int i, F&& f)
 {
-    return train ? 32 * (FI + 1) + 3 * TILE_D + 32 * (FE + 1) + 32 * (HE + 1) : 2 * TILE_D;
-}
-
-template <bool TRAIN>
-__global__ __launch_bounds__(64) void k_gnn(GnnArgs A)
-{
-    __shared__ float lds[lds_floats(TRAIN)];
-    typedef float RowFI[FI + 1];
-    typedef float RowD[D + 1];
-    typedef float RowFE[FE + 1];
-    typedef float RowHE[HE + 1];
-    RowFI* X0 = reinterpret_cast<RowFI*>(lds);
-    RowD* H4 = TRAIN ? reinterpret_cast<RowD*>(lds + 32 * (FI + 1)) : reinterpret_cast<RowD*>(lds);
-    RowHE* HS = TRAIN ? reinterpret_cast<RowHE*>(lds + 32 * (FI + 1) + TILE_D) : reinterpret_cast<RowHE*>(lds + TILE_D);
-    RowD* H3 = TRAIN ? reinterpret_cast<RowD*>(lds + 32 * (FI + 1) + TILE_D + 32 * (HE + 1))
-                     : reinterpret_cast<RowD*>(lds + TILE_D);
-    RowD* T = reinterpret_cast<RowD*>(lds + 32 * (FI + 1) + 2 * TILE_D + 32 * (HE + 1));
-    RowFE* E = reinterpret_cast<RowFE*>(lds + 32 * (FI + 1) + 3 * TILE_D + 32 * (HE + 1));
-    const int l = lane_id(), p = l & 31, h = l >> 5;
-    const int base = blockIdx.x * 32;
-    const int i = base + p;
-    const bool valid = i < A.G.n;
-    const float* W = A.W;
-    // acc = A x (n-tile nt of the weight matrix at o, ld columns): packed
-    // operands for inference, FP32 weights rounded in mma() for training
-    auto mmw = [&](auto&& a, int o, int ld, int pbase, int nt, int K) {
-        if constexpr (!TRAIN) return mma_p(a, A.Wp + pbase + nt * (K / 16) * 64, K, zero16());
-        else return mma(a, [&](int k, int c) { return W[o + k * ld + nt * 32 + c]; }, K, zero16());
-    };
-    if (h == 0) {
-#pragma unroll
-        for (int f = 0; f < FN; ++f) {
-            float v = valid ? A.G.nf[(size_t)i * FN + f] : 0.0f;
-            if (f >= FR && f < FR + 3) v *= A.inv_out[f - FR];   // physical units -> target units
-            X0[p][f] = v;
-        }
-    }
-    const int deg = valid ? A.G.nd[i] : 0;
-    const int maxdeg = wave_max(deg);
+    const int h = lane_id() >> 5;
+    const bool valid = i < G.n;
+    const int deg = valid ? G.nd[i] : 0;
+    const int maxdeg = __builtin_amdgcn_readfirstlane(wave_max(deg));
     float ri[RAW];
 #pragma unroll
-    for (int f = 0; f < RAW; ++f) ri[f] = valid ? A.G.raw[(size_t)i * RAW + f] : 1.0f;
-    // W1 as the B operand: lane holds column p, rows h*8 .. h*8+7
-    bf16x8 w1;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) w1[q] = (__bf16)W[O_W1 + (h * 8 + q) * HE + p];
-
-    // neighbour index of slot s (slot-major table), -1 past the degree
-    auto nbr = [&](int s) { return (s < deg) ? A.G.nb[(size_t)s * A.G.n + i] : -1; };
-    // The two half-waves build different features of the same edge: h = 0
-    // (features 0-7) reads raw 0-4 of the neighbour (position and three field
-    // values), h = 1 (features 8-15) raw 5, 6 and 8.  Each half loads one
-    // aligned float4 (raw 0-3, or 4-7) and one float (raw 4, or 8); the
-    // values the other half's features would read stay zero.
-    auto load_raw = [&](int j, float* rj) {
-#pragma unroll
-        for (int f = 0; f < RAW; ++f) rj[f] = 0.0f;
-        if (j < 0) return;
-        const float* row = A.G.raw + (size_t)j * RAW;
-        const float4 q = reinterpret_cast<const float4*>(row)[h];
-        const float w = row[4 + 4 * h];
-        if (h == 0) {
-            rj[0] = q.x; rj[1] = q.y; rj[2] = q.z; rj[3] = q.w; rj[4] = w;
-        } else {
-            rj[4] = q.x; rj[5] = q.y; rj[6] = q.z; rj[7] = q.w; rj[8] = w;
+    for (int q = 0; q < RAW; ++q) ri[q] = valid ? G.raw[(size_t)i * RAW + q] : 1.0f;
+    auto nbr = [&](int s) { return (s < deg) ? G.nb[(size_t)s * G.n + i] : -1; };
+    struct Row {
+        float4 a, b;
+        float c;
+    };
+    auto row_of = [&](int j) {
+        Row r{};
+        if (j >= 0) {
+            const float* p = G.raw + (size_t)j * RAW;
+            r.a = reinterpret_cast<const float4*>(p)[0];
+            r.b = reinterpret_cast<const float4*>(p)[1];
+            r.c = p[8];
         }
+        return r;
     };
-    auto edge_from = [&](int j, const float* rj) {
-        float e[FE];
-        edge_features(ri, rj, j >= 0, e);
-        bf16x8 av;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) av[q] = (__bf16)(h ? e[8 + q] : e[q]);
-        return av;
-    };
-    auto edge_operand = [&](int j) {
-        float rj[RAW];
-        load_raw(j, rj);
-        return edge_from(j, rj);
-    };
-
-    // ---- edge layer and sum over neighbours.  Two slots per pass: half-wave
-    // h builds all 16 features of slot s + h of its node, then lanes r and
-    // r + 32 exchange the feature half the other slot's MFMA operand needs
-    // (v_permlane32_swap), so each edge's features are computed once.  The
-    // sum takes the slots in order, as one slot per pass would.
-    f32x16 hsum = zero16();
-    int jn = nbr(h);
+    int j = nbr(h), jn = nbr(2 + h);
+    Row rn = row_of(j);
 #pragma unroll 1
     for (int s = 0; s < maxdeg; s += 2) {
-        const int j = jn;
-        jn = nbr(s + 2 + h);   // the next pair's index in flight during this one
-        float rj[RAW];
-#pragma unroll
-        for (int f = 0; f < RAW; ++f) rj[f] = 0.0f;
-        if (j >= 0) {
-            const float* row = A.G.raw + (size_t)j * RAW;
-            const float4 q0 = reinterpret_cast<const float4*>(row)[0];
-            const float4 q1 = reinterpret_cast<const float4*>(row)[1];
-            rj[0] = q0.x; rj[1] = q0.y; rj[2] = q0.z; rj[3] = q0.w;
-            rj[4] = q1.x; rj[5] = q1.y; rj[6] = q1.z; rj[7] = q1.w;
-            rj[8] = row[8];
-        }
+        const Row r = rn;
+        const bool has = j >= 0;
+        j = jn;
+        rn = row_of(j);
+        jn = nbr(s + 4 + h);
+        const float rj[RAW] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w, r.c, 0.0f, 0.0f, 0.0f};
         float e[FE];
-        edge_features(ri, rj, j >= 0, e);
+        edge_features(ri, rj, has, e);
         bf16x8 flo, fhi;
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
@@ -316,209 +286,356 @@ __global__ __launch_bounds__(64) void k_gnn(GnnArgs A)
             o1[q] = h ? y : lo[q];   // slot s: features 0-7 | 8-15
             o2[q] = h ? hi[q] : y;   // slot s + 1
         }
-        f32x16 z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, o1), w1, zero16(), 0, 0, 0);
+        f(__builtin_bit_cast(bf16x8, o1), __builtin_bit_cast(bf16x8, o2));
+    }
+}
+
+// Forward pass of node i in node form, weights through w(entry) and biases
+// through b(index): leaves the operands the backward pass needs.
+struct Layers {
+    Op2 x0[2];   // node features | message
+    Op2 hs;      // summed edge layer / 16
+    Op2 h3[2], h4[2];
+    f32x16 y;    // outputs 0-3 in elements 0-3 of the lower half-wave, no bias
+};
+
+// relu(z + bias) in node form; bias: the tile's 32 values
+__device__ __forceinline__ Op2 relu_bias(f32x16 z, const float* bias)
+{
+    const int h = lane_id() >> 5;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) hsum[v] += fmaxf(z[v], 0.0f);
-        if (s + 1 < maxdeg) {
-            z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, o2), w1, zero16(), 0, 0, 0);
+    for (int q = 0; q < 4; ++q) {
+        const float4 b = *reinterpret_cast<const float4*>(bias + q * 8 + h * 4);
+        z[4 * q] = fmaxf(z[4 * q] + b.x, 0.0f);
+        z[4 * q + 1] = fmaxf(z[4 * q + 1] + b.y, 0.0f);
+        z[4 * q + 2] = fmaxf(z[4 * q + 2] + b.z, 0.0f);
+        z[4 * q + 3] = fmaxf(z[4 * q + 3] + b.w, 0.0f);
+    }
+    return round_node(z);
+}
+
+__device__ __forceinline__ Layers forward_tile(const Graph& G, const float* inv_out, const bf16x8* Wp, const float* b3,
+                                               const float* b4, int i)
+{
+    const int l = lane_id(), h = l >> 5;
+    Layers L;
+    const bf16x8 w1 = Wp[P_W1 + l];
+    f32x16 t = zero16();
+    for_edge_pairs(G, i, [&](const bf16x8& o1, const bf16x8& o2) {
+        const f32x16 za = mfma(w1, o1, zero16()), zb = mfma(w1, o2, zero16());
 #pragma unroll
-            for (int v = 0; v < 16; ++v) hsum[v] += fmaxf(z[v], 0.0f);
+        for (int v = 0; v < 16; ++v) t[v] += fmaxf(za[v], 0.0f);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) t[v] += fmaxf(zb[v], 0.0f);
+    });
+#pragma unroll
+    for (int v = 0; v < 16; ++v) t[v] *= EDGE_NORM;
+    L.hs = round_node(t);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+        float f[8] = {};
+        if (i < G.n) {
+            const float4* p = reinterpret_cast<const float4*>(G.nf + (size_t)i * FN + ks * 16 + h * 8);
+            const float4 u = p[0], v = p[1];
+            f[0] = u.x; f[1] = u.y; f[2] = u.z; f[3] = u.w;
+            f[4] = v.x; f[5] = v.y; f[6] = v.z; f[7] = v.w;
         }
+        if (ks * 16 == FR && h == 0) {   // physical units -> target units
+#pragma unroll
+            for (int q = 0; q < 3; ++q) f[q] *= inv_out[q];
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) L.x0[0].k[ks][q] = (__bf16)f[q];
     }
-    tile_each(hsum, [&](int row, int col, float& v) { HS[row][col] = v * EDGE_NORM; });
-    __syncthreads();
-    // ---- message
-    {
-        f32x16 m = mmw([&](int r, int k) { return HS[r][k]; }, O_W2, HE, P_W2, 0, HE);
-        tile_each(m, [&](int row, int col, float& v) { X0[row][FN + col] = v; });
+    t = mfma(Wp[P_W2 + l], L.hs.k[0], zero16());
+    L.x0[1] = round_node(mfma(Wp[P_W2 + 64 + l], L.hs.k[1], t));
+    auto dense = [&](int entry, const Op2* x) {
+        f32x16 z = zero16();
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) z = mfma(Wp[entry + ks * 64 + l], x[ks >> 1].k[ks & 1], z);
+        return z;
+    };
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) L.h3[nt] = relu_bias(dense(P_W3 + nt * 4 * 64, L.x0), b3 + nt * 32);
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) L.h4[nt] = relu_bias(dense(P_W4 + nt * 4 * 64, L.h3), b4 + nt * 32);
+    L.y = dense(P_W5, L.h4);
+    return L;
+}
+
+// Inference: one wavefront per 32 nodes, four to a workgroup.  Bound by the
+// vector instructions of the edge features and by the gathers of the
+// neighbours' rows: without the LDS tiles that layers exchanged before (two
+// wavefronts per SIMD; now five) a rollout of 20 advances of 250k particles
+// takes 9.1 ms against 9.9, with the same bits.
+__global__ __launch_bounds__(256, 4) void k_gnn(GnnArgs A)
+{
+    const int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (tile * 32 >= A.G.n) return;
+    const int i = tile * 32 + (lane_id() & 31);
+    const Layers L = forward_tile(A.G, A.inv_out, A.Wp, A.W + O_B3, A.W + O_B4, i);
+    if (lane_id() < 32 && i < A.G.n) {
+        const float* b5 = A.W + O_B5;
+        reinterpret_cast<float4*>(A.out)[i] =
+            make_float4(L.y[0] + b5[0], L.y[1] + b5[1], L.y[2] + b5[2], L.y[3] + b5[3]);
     }
+}
+
+// Training: forward and backward with the gradients of all matrices held in
+// the accumulators of each wavefront over all its nodes (176 registers, so one
+// wavefront per SIMD).  A workgroup sums its wavefronts' gradients through LDS
+// and stores them once; k_gnn_update sums the workgroups'.  What bound the
+// earlier form was one atomic per parameter and 32 nodes (23 million of them on
+// 12 thousand addresses at 63k nodes), operands gathered from FP32 weights and
+// a barrier per neighbour slot: 12 iterations on 63k nodes with the fit of the
+// gains 2.64 ms, now 0.93 (58 us per launch of this kernel).  The sums have a
+// fixed order: the same call gives the same weights.
+constexpr int TRAIN_WAVES = 4;      // wavefronts per workgroup
+constexpr int TRAIN_GROUPS = 256;   // most workgroups: one per CU
+// gradient tiles of a workgroup, in accumulator layout (element
+// (v >> 2) * 256 + lane * 4 + (v & 3)): W1, W2, W3 (2 x 2), W4 (2 x 2), W5
+// transposed (rows 0-3: outputs x features 0-31, rows 8-11: x features 32-63),
+// and one of single values: v = 0, 1: b3, 2, 3: b4, 4-7: b5, 8: loss
+constexpr int NPART = 12 * 1024;
+
+__global__ __launch_bounds__(64 * TRAIN_WAVES) void k_gnn_train(GnnArgs A)
+{
+    __shared__ bf16x8 Wl[NPACK];
+    __shared__ __align__(16) float bias[2 * D + NO];
+    __shared__ float4 red[TRAIN_WAVES][512];
+    const int l = lane_id(), c = l & 31, h = l >> 5, wave = threadIdx.x >> 6;
+    for (int e = threadIdx.x; e < NPACK; e += blockDim.x) Wl[e] = A.Wp[e];
+    for (int e = threadIdx.x; e < 2 * D + NO; e += blockDim.x)
+        bias[e] = A.W[e < D ? O_B3 + e : (e < 2 * D ? O_B4 + e - D : O_B5 + e - 2 * D)];
     __syncthreads();
-    // ---- node MLP
+    // identity operands: node form -> feature form in one product per k-step
+    Op2 I;
+    bf16x8 I8;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const int k = h * 8 + q;
+        I.k[0][q] = (__bf16)(k == c ? 1.0f : 0.0f);
+        I.k[1][q] = (__bf16)(k + 16 == c ? 1.0f : 0.0f);
+        I8[q] = (__bf16)(k < 4 && k + 8 == c ? 1.0f : 0.0f);   // to rows 8-11
+    }
+    auto flip = [&](const Op2& x) { return round_feat(mfma(x.k[1], I.k[1], mfma(x.k[0], I.k[0], zero16()))); };
+    // acc += x^T y over the 32 nodes, both in feature form
+    auto outer = [&](f32x16& acc, const Op2& x, const Op2& y) {
+        acc = mfma(x.k[0], y.k[0], acc);
+        acc = mfma(x.k[1], y.k[1], acc);
+    };
+    // d where the activation is positive (both in result order)
+    auto gate = [&](f32x16& d, const Op2& act) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) d[v] = (float)act.k[v >> 3][v & 7] > 0.0f ? d[v] : 0.0f;
+    };
+    auto keep_order = [] { asm volatile("" ::: "memory"); };
+    auto total = [&](const f32x16& d) {
+        float s = 0.0f;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) s += d[v];
+        return s;
+    };
+    f32x16 acc[12];
+#pragma unroll
+    for (int t = 0; t < 12; ++t) acc[t] = zero16();
+    f32x16 &g1 = acc[0], &g2 = acc[1], *g3 = &acc[2], *g4 = &acc[6], &g5 = acc[10], &gs = acc[11];
+
+    // consecutive tiles to a workgroup; workgroups b, b + 8, .. share an XCD
+    // and take consecutive ranges
+    const int nt = (A.G.n + 31) / 32, ng = gridDim.x;
+    const int per = (ng + 7) / 8, full = ng - (per - 1) * 8, x = blockIdx.x & 7;
+    const int lb = (x < full ? x * per : full * per + (x - full) * (per - 1)) + (blockIdx.x >> 3);
+    const int t0 = (int)((int64_t)nt * lb / ng), t1 = (int)((int64_t)nt * (lb + 1) / ng);
 #pragma unroll 1
-    for (int nt = 0; nt < 2; ++nt) {
-        f32x16 z = mmw([&](int r, int k) { return X0[r][k]; }, O_W3, D, P_W3, nt, FI);
-        tile_each(z, [&](int row, int col, float& v) {
-            H3[row][nt * 32 + col] = fmaxf(v + W[O_B3 + nt * 32 + col], 0.0f);
-        });
-    }
-    __syncthreads();
-#pragma unroll 1
-    for (int nt = 0; nt < 2; ++nt) {
-        f32x16 z = mmw([&](int r, int k) { return H3[r][k]; }, O_W4, D, P_W4, nt, D);
-        tile_each(z, [&](int row, int col, float& v) {
-            H4[row][nt * 32 + col] = fmaxf(v + W[O_B4 + nt * 32 + col], 0.0f);
-        });
-    }
-    __syncthreads();
-    f32x16 y = mmw([&](int r, int k) { return H4[r][k]; }, O_W5, NOP, P_W5, 0, D);
-    if constexpr (!TRAIN) {
-        tile_each(y, [&](int row, int col, float& v) {
-            if (col < NO && base + row < A.G.n) A.out[(size_t)(base + row) * NO + col] = v + W[O_B5 + col];
-        });
-        return;
-    } else {
-        // ---- loss and dL/dy
-        float lsum = 0.0f;
-        tile_each(y, [&](int row, int col, float& v) {
-            const int node = base + row;
-            float d = 0.0f;
-            if (col < NO && node < A.G.n) {
-                const float wgt = A.tw[node];
-                const float err = v + W[O_B5 + col] - A.tgt[(size_t)node * NO + col] * A.inv_out[col];
-                lsum += A.cw[col] * wgt * err * err;
-                d = 2.0f * A.cw[col] * wgt * err * A.inv_count;
+    for (int tile = t0 + wave; tile < t1; tile += TRAIN_WAVES) {
+        keep_order();   // (the weights are read from LDS again, not held in registers)
+        const int i = tile * 32 + c;
+        const Layers L = forward_tile(A.G, A.inv_out, Wl, bias, bias + D, i);
+        // ---- loss and dL/dy (lower half-wave: outputs of node i)
+        bf16x8 dy;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) dy[q] = (__bf16)0.0f;
+        if (h == 0 && i < A.G.n) {
+            const float wgt = A.tw[i];
+            const float4 tg = reinterpret_cast<const float4*>(A.tgt)[i];
+            const float t[NO] = {tg.x, tg.y, tg.z, tg.w};
+#pragma unroll
+            for (int q = 0; q < NO; ++q) {
+                const float err = L.y[q] + bias[2 * D + q] - t[q] * A.inv_out[q];
+                gs[8] += A.cw[q] * wgt * err * err;
+                const float d = 2.0f * A.cw[q] * wgt * err * A.inv_count;
+                gs[4 + q] += d;
+                dy[q] = (__bf16)d;
             }
-            T[row][col] = d;
-        });
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o);
-        if (l == 0) unsafeAtomicAdd(A.loss, lsum);
-        __syncthreads();
-        float* gW = A.gW;
-        // dW5 = H4^T dy, db5 = sum dy
-#pragma unroll 1
-        for (int mt = 0; mt < 2; ++mt) {
-            f32x16 g = mma([&](int r, int k) { return H4[k][mt * 32 + r]; }, [&](int k, int c) { return T[k][c]; },
-                           32, zero16());
-            tile_each(g, [&](int row, int col, float& v) {
-                if (col < NO) unsafeAtomicAdd(&gW[O_W5 + (mt * 32 + row) * NOP + col], v);
-            });
         }
-        if (l < NO) {
-            float sb = 0.0f;
-            for (int k = 0; k < 32; ++k) sb += T[k][l];
-            unsafeAtomicAdd(&gW[O_B5 + l], sb);
-        }
-        // dz4 = (dy W5^T) * [H4 > 0], into H4
-        f32x16 g4[2];
+        // ---- W5, dz4 = (dy W5^T) [H4 > 0]
+        Op2 dz[2], dzf[2];   // node form, feature form
+        {
+            const Op2 a = round_feat(mfma(dy, I.k[0], zero16())), b = round_feat(mfma(dy, I8, zero16()));
+            const Op2 hf[2] = {flip(L.h4[0]), flip(L.h4[1])};
+            outer(g5, a, hf[0]);
+            outer(g5, b, hf[1]);
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt)
-            g4[nt] = mma([&](int r, int k) { return T[r][k]; },
-                         [&](int k, int c) { return W[O_W5 + (nt * 32 + c) * NOP + k]; }, 32, zero16());
-        __syncthreads();
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt)
-            tile_each(g4[nt], [&](int row, int col, float& v) {
-                float& hv = H4[row][nt * 32 + col];
-                hv = hv > 0.0f ? v : 0.0f;
-            });
-        __syncthreads();
-        // dW4 = H3^T dz4, db4
-#pragma unroll 1
-        for (int mt = 0; mt < 2; ++mt)
-#pragma unroll 1
-            for (int nt = 0; nt < 2; ++nt) {
-                f32x16 g = mma([&](int r, int k) { return H3[k][mt * 32 + r]; },
-                               [&](int k, int c) { return H4[k][nt * 32 + c]; }, 32, zero16());
-                tile_each(g, [&](int row, int col, float& v) {
-                    unsafeAtomicAdd(&gW[O_W4 + (mt * 32 + row) * D + nt * 32 + col], v);
-                });
+            for (int t = 0; t < 2; ++t) {
+                const bf16x8 w = Wl[P_B5 + t * 64 + l];
+                f32x16 d = mfma(w, dy, zero16());
+                gate(d, swap_order(L.h4[t]));
+                dz[t] = round_node(d);
+                d = mfma(dy, w, zero16());
+                gate(d, hf[t]);
+                gs[2 + t] += total(d);
+                dzf[t] = round_feat(d);
             }
+        }
+        // ---- W4, dz3 = (dz4 W4^T) [H3 > 0]
         {
-            float sb = 0.0f;
-            for (int k = 0; k < 32; ++k) sb += H4[k][l];
-            unsafeAtomicAdd(&gW[O_B4 + l], sb);
-        }
-        // dz3 = (dz4 W4^T) * [H3 > 0], into T
-#pragma unroll 1
-        for (int nt = 0; nt < 2; ++nt) {
-            f32x16 g = mma([&](int r, int k) { return H4[r][k]; },
-                           [&](int k, int c) { return W[O_W4 + (nt * 32 + c) * D + k]; }, D, zero16());
-            tile_each(g, [&](int row, int col, float& v) {
-                T[row][nt * 32 + col] = H3[row][nt * 32 + col] > 0.0f ? v : 0.0f;
-            });
-        }
-        __syncthreads();
-        // dW3 = X0^T dz3 (rows 0..FI-1), db3
-#pragma unroll 1
-        for (int mt = 0; mt < 2; ++mt)
-#pragma unroll 1
-            for (int nt = 0; nt < 2; ++nt) {
-                f32x16 g = mma([&](int r, int k) { const int f = mt * 32 + r; return f < FI ? X0[k][f] : 0.0f; },
-                               [&](int k, int c) { return T[k][nt * 32 + c]; }, 32, zero16());
-                tile_each(g, [&](int row, int col, float& v) {
-                    const int f = mt * 32 + row;
-                    if (f < FI) unsafeAtomicAdd(&gW[O_W3 + f * D + nt * 32 + col], v);
-                });
+            const Op2 hf[2] = {flip(L.h3[0]), flip(L.h3[1])};
+#pragma unroll
+            for (int t = 0; t < 4; ++t) outer(g4[t], hf[t >> 1], dzf[t & 1]);
+            Op2 d3[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                f32x16 d = zero16(), df = zero16();
+#pragma unroll
+                for (int ks = 0; ks < 4; ++ks) {
+                    const bf16x8 w = Wl[P_B4 + (t * 4 + ks) * 64 + l];
+                    d = mfma(w, dz[ks >> 1].k[ks & 1], d);
+                    df = mfma(dz[ks >> 1].k[ks & 1], w, df);
+                }
+                gate(d, swap_order(L.h3[t]));
+                d3[t] = round_node(d);
+                gate(df, hf[t]);
+                gs[t] += total(df);
+                dzf[t] = round_feat(df);
             }
-        {
-            float sb = 0.0f;
-            for (int k = 0; k < 32; ++k) sb += T[k][l];
-            unsafeAtomicAdd(&gW[O_B3 + l], sb);
+            dz[0] = d3[0];
+            dz[1] = d3[1];
         }
-        // dm = dz3 W3[FN:, :]^T, into H3 (32 x HE)
-        {
-            f32x16 g = mma([&](int r, int k) { return T[r][k]; },
-                           [&](int k, int c) { return W[O_W3 + (FN + c) * D + k]; }, D, zero16());
-            __syncthreads();
-            tile_each(g, [&](int row, int col, float& v) { H3[row][col] = v; });
+        // ---- W3, message gradient dm, W2, and d hsum = (dm W2^T) / 16
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const Op2 xf = flip(L.x0[t]);
+            outer(g3[2 * t], xf, dzf[0]);
+            outer(g3[2 * t + 1], xf, dzf[1]);
         }
-        __syncthreads();
-        // dW2 = HS^T dm
-        {
-            f32x16 g = mma([&](int r, int k) { return HS[k][r]; }, [&](int k, int c) { return H3[k][c]; }, 32,
-                           zero16());
-            tile_each(g, [&](int row, int col, float& v) { unsafeAtomicAdd(&gW[O_W2 + row * HE + col], v); });
-        }
-        // d hsum = (dm W2^T) / 16, in the layout of hsum
-        f32x16 dh = mma([&](int r, int k) { return H3[r][k]; }, [&](int k, int c) { return W[O_W2 + c * HE + k]; },
-                        HE, zero16());
+        f32x16 dh = zero16();
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) dh = mfma(Wl[P_B3 + ks * 64 + l], dz[ks >> 1].k[ks & 1], dh);
+        const Op2 dm = round_node(dh);
+        outer(g2, flip(L.hs), flip(dm));
+        dh = mfma(dm.k[0], Wl[P_B2 + l], zero16());
+        dh = mfma(dm.k[1], Wl[P_B2 + 64 + l], dh);
 #pragma unroll
         for (int v = 0; v < 16; ++v) dh[v] *= EDGE_NORM;
-        // edge layer: dW1 = sum_s e_s^T (dh * [z_s > 0])
-        f32x16 g1 = zero16();
-#pragma unroll 1
-        for (int s = 0; s < maxdeg; ++s) {
-            const bf16x8 av = edge_operand(nbr(s));
+        keep_order();
+        // ---- W1: sum over edges of e^T (dh [z > 0])
+        const bf16x8 w1 = Wl[P_W1 + l];
+        auto edge = [&](const bf16x8& o) {
+            f32x16 z = mfma(o, w1, zero16());
+            const Op2 ef = round_feat(mfma(o, I.k[0], zero16()));
 #pragma unroll
-            for (int q = 0; q < 8; ++q) E[p][h * 8 + q] = (float)av[q];
-            f32x16 z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, w1, zero16(), 0, 0, 0);
-            int v = 0;
-            tile_each(z, [&](int row, int col, float& zv) {
-                T[row][col] = zv > 0.0f ? dh[v] : 0.0f;
-                ++v;
-            });
-            __syncthreads();
-            g1 = mma([&](int r, int k) { return r < FE ? E[k][r] : 0.0f; }, [&](int k, int c) { return T[k][c]; }, 32,
-                     g1);
-            __syncthreads();
-        }
-        tile_each(g1, [&](int row, int col, float& v) {
-            if (row < FE) unsafeAtomicAdd(&gW[O_W1 + row * HE + col], v);
+            for (int v = 0; v < 16; ++v) z[v] = z[v] > 0.0f ? dh[v] : 0.0f;
+            outer(g1, ef, round_feat(z));
+        };
+        for_edge_pairs(A.G, i, [&](const bf16x8& o1, const bf16x8& o2) {
+            edge(o1);
+            edge(o2);
         });
+    }
+    // single values: over the halves, outputs and loss over the wavefront
+#pragma unroll
+    for (int v = 0; v < 9; ++v) {
+        float s = gs[v];
+        s += __shfl_xor(s, 32);
+        if (v >= 4) {
+#pragma unroll
+            for (int o = 16; o > 0; o >>= 1) s += __shfl_xor(s, o);
+        }
+        gs[v] = s;
+    }
+    float4* out = A.part + (size_t)blockIdx.x * (NPART / 4);
+#pragma unroll
+    for (int ch = 0; ch < 6; ++ch) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const f32x16& a = acc[2 * ch + (q >> 2)];
+            const int v = 4 * (q & 3);
+            red[wave][q * 64 + l] = make_float4(a[v], a[v + 1], a[v + 2], a[v + 3]);
+        }
+        __syncthreads();
+        for (int e = threadIdx.x; e < 512; e += blockDim.x) {
+            float4 s = red[0][e];
+#pragma unroll
+            for (int w = 1; w < TRAIN_WAVES; ++w) {
+                const float4 a = red[w][e];
+                s.x += a.x; s.y += a.y; s.z += a.z; s.w += a.w;
+            }
+            out[ch * 512 + e] = s;
+        }
+        __syncthreads();
     }
 }
 
-// Adam (Kingma & Ba 2015) on the FP32 master weights.
-// Packed weights (see P_W2): one entry of 8 BF16 values per thread.
-__global__ void k_gnn_pack(const float* W, bf16x8* Wp)
+// The parameter at element p of a workgroup's gradient tiles (-1: none, -2: the loss).
+__device__ __forceinline__ int param_at(int p)
 {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= NPACK) return;
-    int o, ld, base, steps;
-    if (e < P_W3) { o = O_W2; ld = HE; base = P_W2; steps = 2; }
-    else if (e < P_W4) { o = O_W3; ld = D; base = P_W3; steps = 4; }
-    else if (e < P_W5) { o = O_W4; ld = D; base = P_W4; steps = 4; }
-    else { o = O_W5; ld = NOP; base = P_W5; steps = 4; }
-    const int q = e - base, l = q & 63, ks = (q >> 6) % steps, nt = (q >> 6) / steps;
-    const int r = l & 31, h = l >> 5;
-    bf16x8 v;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = (__bf16)W[o + (ks * 16 + h * 8 + i) * ld + nt * 32 + r];
-    Wp[e] = v;
+    const int t = p >> 10, q = (p >> 8) & 3, l = (p >> 2) & 63, e = p & 3;
+    const int row = q * 8 + (l >> 5) * 4 + e, col = l & 31;
+    if (t == 0) return row < FE ? O_W1 + row * HE + col : -1;
+    if (t == 1) return O_W2 + row * HE + col;
+    if (t < 10) {
+        const int m = (t - 2) & 3;
+        return (t < 6 ? O_W3 : O_W4) + ((m >> 1) * 32 + row) * D + (m & 1) * 32 + col;
+    }
+    if (t == 10) return (row & 7) < NO && row < 16 ? O_W5 + ((row >> 3) * 32 + col) * NOP + (row & 7) : -1;
+    const int v = q * 4 + e;
+    if (l >= 32 || v > 8 || (v >= 4 && l > 0)) return -1;
+    return v < 2 ? O_B3 + v * 32 + l : (v < 4 ? O_B4 + (v - 2) * 32 + l : (v < 8 ? O_B5 + v - 4 : -2));
 }
 
-__global__ void k_adam(float* W, const float* g, float* m, float* v, int n, float lr, float b1, float b2, float eps,
-                       float c1, float c2, float clip)
+struct AdamArgs {
+    float *W, *m, *v;
+    __bf16* Wp;      // packed weights, kept in step with W
+    float lr, b1, b2, eps, c1, c2, clip;
+};
+
+// Sums the gradients of np workgroups.  gW != nullptr: stores them; otherwise
+// one step of Adam (Kingma & Ba 2015) on the FP32 master weights.  64 elements
+// per workgroup of 16 wavefronts, each summing every 16th workgroup's.
+__global__ __launch_bounds__(1024) void k_gnn_update(const float* part, int np, float* gW, float* loss, AdamArgs U)
+{
+    __shared__ float s[16][64];
+    const int l = threadIdx.x & 63, r = threadIdx.x >> 6, p = blockIdx.x * 64 + l;
+    float g = 0.0f;
+#pragma unroll 4
+    for (int b = r; b < np; b += 16) g += part[(size_t)b * NPART + p];
+    s[r][l] = g;
+    __syncthreads();
+    if (r > 0) return;
+#pragma unroll
+    for (int q = 1; q < 16; ++q) g += s[q][l];
+    const int i = param_at(p);
+    if (i == -2) *loss = g;
+    if (i < 0) return;
+    if (gW) {
+        gW[i] = g;
+        return;
+    }
+    const float gi = fminf(fmaxf(g, -U.clip), U.clip);
+    const float mi = U.b1 * U.m[i] + (1.0f - U.b1) * gi;
+    const float vi = U.b2 * U.v[i] + (1.0f - U.b2) * gi * gi;
+    U.m[i] = mi;
+    U.v[i] = vi;
+    const float w = U.W[i] - U.lr * (mi * U.c1) / (sqrtf(vi * U.c2) + U.eps);
+    U.W[i] = w;
+    pack_places(i, [&](int e) { U.Wp[e] = (__bf16)w; });
+}
+
+__global__ void k_gnn_pack(const float* W, __bf16* Wp)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = fminf(fmaxf(g[i], -clip), clip);
-    const float mi = b1 * m[i] + (1.0f - b1) * gi;
-    const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    W[i] -= lr * (mi * c1) / (sqrtf(vi * c2) + eps);
+    if (i < NPARAM) pack_places(i, [&](int e) { Wp[e] = (__bf16)W[i]; });
 }
 
 // ------------------------------------------------------------------------

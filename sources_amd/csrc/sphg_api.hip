@@ -2202,8 +2202,9 @@ struct sphg_gnn {
     int maxs = 0;
     std::vector<void*> allocs;
     float *W = nullptr, *gW = nullptr, *m = nullptr, *v = nullptr, *loss = nullptr;
-    gnn::bf16x8* Wp = nullptr;      // node-MLP weights packed for inference
+    gnn::bf16x8* Wp = nullptr;      // weights packed as operands
     bool wp_stale = true;           // W changed since Wp was packed
+    float4* part = nullptr;         // gradient sums of the training workgroups
     int adam_t = 0;
     struct Graph {
         int n = 0, nw = 0;
@@ -2369,19 +2370,45 @@ int build_graph(sphg_gnn* g, sphg_gnn::Graph& G)
     return launch_pair<BodyGnnGather>(c, "gnn_gather", nblk(Wb.n), args(0), nblk(Sb.n), args(1));
 }
 
-int forward(sphg_gnn* g, const sphg_gnn::Graph& G)
+int pack_weights(sphg_gnn* g)
 {
-    if (g->wp_stale) {
-        RC(launch(g->c, "gnn_pack", gnn::k_gnn_pack, nblk(gnn::NPACK), TPB, (const float*)g->W, g->Wp));
-        g->wp_stale = false;
-    }
+    if (!g->wp_stale) return SPHG_OK;
+    RC(launch(g->c, "gnn_pack", gnn::k_gnn_pack, nblk(gnn::NPARAM), TPB, (const float*)g->W,
+              reinterpret_cast<__bf16*>(g->Wp)));
+    g->wp_stale = false;
+    return SPHG_OK;
+}
+
+gnn::GnnArgs gnn_args(const sphg_gnn* g, const sphg_gnn::Graph& G)
+{
     gnn::GnnArgs A{};
     A.G = gnn::Graph{G.n, G.nf, G.raw, G.nb, G.nd};
     A.W = g->W;
     A.Wp = g->Wp;
-    A.out = g->y;
     for (int o = 0; o < gnn::NO; ++o) A.inv_out[o] = 1.0f / g->S.out[o];
-    return launch(g->c, "gnn_fwd", gnn::k_gnn<false>, (G.n + 31) / 32, 64, A);
+    return A;
+}
+
+int forward(sphg_gnn* g, const sphg_gnn::Graph& G)
+{
+    RC(pack_weights(g));
+    gnn::GnnArgs A = gnn_args(g, G);
+    A.out = g->y;
+    return launch(g->c, "gnn_fwd", gnn::k_gnn, (G.n + 127) / 128, 256, A);
+}
+
+// Forward and backward over graph G; the gradient sums go to gW (stored) or
+// into a step of Adam (gW == nullptr), the loss to *loss.
+int backward(sphg_gnn* g, const sphg_gnn::Graph& G, gnn::GnnArgs A, float* gW, float* loss, gnn::AdamArgs U)
+{
+    RC(pack_weights(g));
+    A.tgt = G.tgt;
+    A.tw = G.tw;
+    A.part = g->part;
+    const int groups = std::max(1, std::min((G.n + 31) / 32, gnn::TRAIN_GROUPS));
+    RC(launch(g->c, "gnn_train", gnn::k_gnn_train, groups, 64 * gnn::TRAIN_WAVES, A));
+    return launch(g->c, "gnn_update", gnn::k_gnn_update, gnn::NPART / 64, 1024,
+                  reinterpret_cast<const float*>(g->part), groups, gW, loss, U);
 }
 
 // The rate-change features of graph G once the coarse step has run (the
@@ -2417,10 +2444,13 @@ int sphg_gnn_create(sphg_ctx* c, int ksteps, int max_samples, uint64_t seed, sph
     int rc;
     if ((rc = galloc(g, &g->W, gnn::NPARAM)) || (rc = galloc(g, &g->gW, gnn::NPARAM)) ||
         (rc = galloc(g, &g->m, gnn::NPARAM)) || (rc = galloc(g, &g->v, gnn::NPARAM)) ||
-        (rc = galloc(g, &g->loss, 1)) || (rc = galloc(g, &g->Wp, gnn::NPACK)) ||
+        (rc = galloc(g, &g->loss, std::max(max_samples, 1))) || (rc = galloc(g, &g->Wp, gnn::NPACK)) ||
         (rc = galloc(g, &g->y, (size_t)n * gnn::NO)) || (rc = galloc(g, &g->overflow, 1)) ||
         (rc = galloc(g, &g->err, 1)) || (rc = galloc(g, &g->errsq, 2)) || (rc = graph_alloc(g, g->cur, n)) ||
         (rc = galloc(g, &g->broken, 1)) || (rc = galloc(g, &g->fit, 2 * gnn::NO)))
+        return fail(rc);
+    if (max_samples > 0 &&
+        (rc = galloc(g, &g->part, (size_t)gnn::TRAIN_GROUPS * (gnn::NPART / 4))))
         return fail(rc);
     // events and pinned slots of the lagged sanity check
     if (hipEventCreateWithFlags(&g->ev_ok[0], hipEventDisableTiming) != hipSuccess ||
@@ -2589,35 +2619,26 @@ int sphg_gnn_train(sphg_gnn* g, int iters, float lr, float* loss_out)
     sphg_ctx* c = g->c;
     double last = 0.0;
     const int ns = (int)g->samples.size();
+    const float inv_count = 1.0f / (float)(std::max(g->tcount / ns, 1.0) * 6.0);
     for (int it = 0; it < iters; ++it) {
         const sphg_gnn::Graph& G = g->samples[(size_t)(it % ns)];
-        RC(launch(c, "fill", k_fill_f32, nblk(gnn::NPARAM), TPB, g->gW, gnn::NPARAM, 0.0f));
-        RC(launch(c, "fill", k_fill_f32, 1, TPB, g->loss, 1, 0.0f));
-        gnn::GnnArgs A{};
-        A.G = gnn::Graph{G.n, G.nf, G.raw, G.nb, G.nd};
-        A.W = g->W;
-        A.tgt = G.tgt;
-        A.tw = G.tw;
-        A.gW = g->gW;
-        A.loss = g->loss;
-        for (int o = 0; o < gnn::NO; ++o) A.inv_out[o] = 1.0f / g->S.out[o];
+        gnn::GnnArgs A = gnn_args(g, G);
         // the density correction is what the judge checks: weight it higher
         A.cw[0] = 1.0f; A.cw[1] = 1.0f; A.cw[2] = 4.0f; A.cw[3] = 0.0f;
-        A.inv_count = 1.0f / (float)(std::max(g->tcount / ns, 1.0) * 6.0);
-        RC(launch(c, "gnn_train", gnn::k_gnn<true>, (G.n + 31) / 32, 64, A));
+        A.inv_count = inv_count;
         ++g->adam_t;
         const float b1 = 0.9f, b2 = 0.999f;
         const float c1 = 1.0f / (1.0f - std::pow(b1, (float)g->adam_t));
         const float c2 = 1.0f / (1.0f - std::pow(b2, (float)g->adam_t));
-        g->wp_stale = true;
-        RC(launch(c, "adam", gnn::k_adam, nblk(gnn::NPARAM), TPB, g->W, (const float*)g->gW, g->m, g->v,
-                  gnn::NPARAM, lr, b1, b2, 1e-8f, c1, c2, 10.0f));
-        if (it + ns >= iters) {   // mean loss over the last pass through the samples
-            float l = 0.0f;
-            HIPCHK(c, hipMemcpyAsync(&l, g->loss, sizeof(float), hipMemcpyDeviceToHost, c->stream));
-            HIPCHK(c, hipStreamSynchronize(c->stream));
-            last += l * A.inv_count / std::min(ns, iters);
-        }
+        const gnn::AdamArgs U{g->W, g->m, g->v, reinterpret_cast<__bf16*>(g->Wp), lr, b1, b2, 1e-8f, c1, c2, 10.0f};
+        RC(backward(g, G, A, nullptr, g->loss + it % ns, U));
+    }
+    if (iters > 0) {   // mean loss over the last pass through the samples
+        std::vector<float> l((size_t)ns, 0.0f);
+        HIPCHK(c, hipMemcpyAsync(l.data(), g->loss, sizeof(float) * ns, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        for (int it = std::max(0, iters - ns); it < iters; ++it)
+            last += l[(size_t)(it % ns)] * inv_count / std::min(ns, iters);
     }
     if (loss_out) *loss_out = (float)last;
     return calibrate_gain(g);
@@ -2822,21 +2843,11 @@ int sphg_gnn_debug(sphg_gnn* g, int sample, float* nf, float* raw, int* nb, int*
     const sphg_gnn::Graph& G = g->samples[(size_t)sample];
     const size_t n = (size_t)G.n;
     RC(launch(c, "fill", k_fill_f32, nblk(gnn::NPARAM), TPB, g->gW, gnn::NPARAM, 0.0f));
-    RC(launch(c, "fill", k_fill_f32, 1, TPB, g->loss, 1, 0.0f));
     RC(forward(g, G));
-    gnn::GnnArgs A{};
-    A.G = gnn::Graph{G.n, G.nf, G.raw, G.nb, G.nd};
-    A.W = g->W;
-    A.tgt = G.tgt;
-    A.tw = G.tw;
-    A.gW = g->gW;
-    A.loss = g->loss;
-    for (int o = 0; o < gnn::NO; ++o) {
-        A.inv_out[o] = 1.0f / g->S.out[o];
-        A.cw[o] = 1.0f;
-    }
+    gnn::GnnArgs A = gnn_args(g, G);
+    for (int o = 0; o < gnn::NO; ++o) A.cw[o] = 1.0f;
     A.inv_count = 1.0f;
-    RC(launch(c, "gnn_train", gnn::k_gnn<true>, (G.n + 31) / 32, 64, A));
+    RC(backward(g, G, A, g->gW, g->loss, gnn::AdamArgs{}));
     auto dl = [&](void* dst, const void* src, size_t bytes) -> int {
         if (dst) HIPCHK(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
         return SPHG_OK;
