@@ -163,27 +163,47 @@ SPHG_BATCH_BODY(BodyNlist, nlist_body)
 template <int SKF>
 struct BodyWaterAMx {
     template <class... A>
-    __device__ __forceinline__ void operator()(int blk, const A&... a) const { water_a_mx<SKF, 1>(blk, a...); }
+    __device__ __forceinline__ void operator()(int blk, const A&... a) const
+    {
+        __shared__ __align__(16) unsigned char lds[MX_LDS<2>];
+        water_a_mx<SKF, 1>(lds, blk, a...);
+    }
 };
 template <int SKF>
 struct BodyWaterXMx {
     template <class... A>
-    __device__ __forceinline__ void operator()(int blk, const A&... a) const { water_a_mx<SKF, 2>(blk, a...); }
+    __device__ __forceinline__ void operator()(int blk, const A&... a) const
+    {
+        __shared__ __align__(16) unsigned char lds[MX_LDS<3>];
+        water_a_mx<SKF, 2>(lds, blk, a...);
+    }
 };
 template <int SKF>
 struct BodyWaterBMx {
     template <class... A>
-    __device__ __forceinline__ void operator()(int blk, const A&... a) const { water_b_mx<SKF>(blk, a...); }
+    __device__ __forceinline__ void operator()(int blk, const A&... a) const
+    {
+        __shared__ __align__(16) unsigned char lds[MX_LDS<4>];
+        water_b_mx<SKF>(lds, blk, a...);
+    }
 };
 template <int SKF>
 struct BodySoilABMx {
     template <class... A>
-    __device__ __forceinline__ void operator()(int blk, const A&... a) const { soil_ab_mx<SKF, 1>(blk, a...); }
+    __device__ __forceinline__ void operator()(int blk, const A&... a) const
+    {
+        __shared__ __align__(16) unsigned char lds[MX_LDS<4>];
+        soil_ab_mx<SKF, 1>(lds, blk, a...);
+    }
 };
 template <int SKF>
 struct BodySoilXMx {
     template <class... A>
-    __device__ __forceinline__ void operator()(int blk, const A&... a) const { soil_ab_mx<SKF, 2>(blk, a...); }
+    __device__ __forceinline__ void operator()(int blk, const A&... a) const
+    {
+        __shared__ __align__(16) unsigned char lds[MX_LDS<3>];
+        soil_ab_mx<SKF, 2>(lds, blk, a...);
+    }
 };
 #undef SPHG_BATCH_BODY
 

@@ -161,8 +161,15 @@ __device__ __forceinline__ void kern_s(const KC& k, double r, double inv_r, doub
 // chunk of nearby partners at a time, so a plane layout touches a few cache
 // lines per load where a 128-byte-per-record layout touches one per lane.
 struct RecV {
+    typedef double2 V;
     const double2* p;
     int n;
+    // a record past the end of a list: far away, finite everywhere
+    __device__ __forceinline__ static double2 stand_in(int c)
+    {
+        const double f = c == 0 ? 1.0e18 : 1.0;
+        return make_double2(f, f);
+    }
     // (uniform plane address plus a 32-bit lane offset: no 64-bit lane arithmetic)
     __device__ __forceinline__ double2 operator()(int k, int c) const
     {
@@ -227,8 +234,13 @@ constexpr int Q_STRIDE = 16;   // floats per record: four float4 chunk planes
 
 // FP32 records of the mixed-precision form, as chunk planes like RecV.
 struct RecQ {
+    typedef float4 V;
     const float4* p;
     int n;
+    __device__ __forceinline__ static float4 stand_in(int c)
+    {
+        return c == 0 ? make_float4(1.0e12f, 1.0e12f, 0.0f, 1.0f) : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+    }
     __device__ __forceinline__ float4 operator()(int k, int c) const { return p[(size_t)c * n + k]; }
 };
 
@@ -994,10 +1006,11 @@ constexpr size_t VIS_LDS = TABLE_LDS > sizeof(double2) * NCH * WIN_STRIDE ? TABL
 // and a stand-in record (far away, finite everywhere) at WIN_CAP.  Called after
 // a kernel's own loads: loads return in order, so a use of one issued behind
 // the window would wait for all of it.
-template <bool U, int NCH>
+template <bool U, int NCH, class R>
 __device__ __forceinline__ Window open_window(unsigned char* lds, const IdxList& I, int blk, const SubCtx& sc, int lg,
-                                              int n, const RecV& rec)
+                                              int n, const R& rec)
 {
+    typedef typename R::V V;
     Window w{{0, 0, 0, 0, 0}, I.li != nullptr, false, 0, {0, 0, 0, 0}};
     if (!I.li) return w;
     const int* p = I.win + (size_t)blk * WIN_INTS;
@@ -1011,11 +1024,8 @@ __device__ __forceinline__ Window open_window(unsigned char* lds, const IdxList&
             w.cnt = I.cnt[sc.tt];
 #pragma unroll
             for (int q = 0; q < 4; ++q) w.k[q] = I.li[q * row + o];
-            double2* wl = reinterpret_cast<double2*>(lds);
-            if (threadIdx.x < NCH) {
-                const double f = threadIdx.x == 0 ? 1.0e18 : 1.0;
-                wl[threadIdx.x * WIN_STRIDE + WIN_CAP] = make_double2(f, f);
-            }
+            V* wl = reinterpret_cast<V*>(lds);
+            if (threadIdx.x < NCH) wl[threadIdx.x * WIN_STRIDE + WIN_CAP] = R::stand_in(threadIdx.x);
             const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x & ~63);
             for (int i0 = wave; i0 < tot; i0 += STAGE_BLOCK) {
                 const int i = i0 + (int)(threadIdx.x & 63);
@@ -1034,6 +1044,46 @@ __device__ __forceinline__ Window open_window(unsigned char* lds, const IdxList&
     return w;
 }
 
+// body(v) over the listed candidates of the lane's particle, v the record
+// chunks 0 .. NCH - 1 from the window in LDS (all lanes of the workgroup call;
+// none of a list that overflowed).
+template <int NCH, class V, class B>
+__device__ __forceinline__ void visit_window(unsigned char* lds, const Window& w, const IdxList& I, int n,
+                                             const SubCtx& sc, int lg, B&& body)
+{
+    const V* wl = reinterpret_cast<const V*>(lds);
+    auto read = [&](V(&v)[NCH], int k) {
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) v[c] = wl[c * WIN_STRIDE + k];
+    };
+    // The lane's candidates i = 0, 1, ... are sub, sub + 2^lg, ... of
+    // the list; past its end the stand-in.  Indices are loaded two
+    // rounds ahead (the buffer is padded), chunks one.
+    const unsigned short* l = I.li;
+    const uint32_t o = (uint32_t)sc.sub * n + sc.tt;
+    const size_t row = (size_t)n << lg;
+    int k0 = w.k[0], k1 = w.k[1], n0 = w.k[2], n1 = w.k[3];
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    const int mine = sc.valid ? (max(w.cnt, 0) - sc.sub + (1 << lg) - 1) >> lg : 0;
+    V a[NCH], b[NCH];
+    read(a, pick(0 < mine, k0, WIN_CAP));
+    k1 = pick(1 < mine, k1, WIN_CAP);
+#pragma unroll 1
+    for (int i = 0; __any(i < mine); i += 2) {
+        l += 2 * row;
+        k0 = pick(i + 2 < mine, n0, WIN_CAP);
+        const int k2 = pick(i + 3 < mine, n1, WIN_CAP);
+        n0 = l[2 * row + o];
+        n1 = l[3 * row + o];
+        read(b, k1);
+        body(a);
+        read(a, k0);
+        k1 = k2;
+        body(b);
+    }
+}
+
 // body(v, R, k) over the partners of the lane's particle, v the record chunks
 // 0 .. NCH - 1 and R(k, c) any other (all lanes of the workgroup call).
 template <bool U, int NCH, class A, class B>
@@ -1042,47 +1092,16 @@ __device__ __forceinline__ void visit(unsigned char* lds, const Window& w, const
 {
     if constexpr (U) {
         if (w.lds) {
-            const double2* wl = reinterpret_cast<const double2*>(lds);
-            auto read = [&](double2(&v)[NCH], int k) {
-#pragma unroll
-                for (int c = 0; c < NCH; ++c) v[c] = wl[c * WIN_STRIDE + k];
-            };
-            // The lane's candidates i = 0, 1, ... are sub, sub + 2^lg, ... of
-            // the list; past its end the stand-in.  Indices are loaded two
-            // rounds ahead (the buffer is padded), chunks one.
-            const unsigned short* l = I.li;
-            const uint32_t o = (uint32_t)sc.sub * n + sc.tt;
-            const size_t row = (size_t)n << lg;
-            int k0 = w.k[0], k1 = w.k[1], n0 = w.k[2], n1 = w.k[3];
-            const int cnt = w.cnt;
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();
-            // candidates of the lane (none of a list that overflowed)
-            const int mine = sc.valid ? (max(cnt, 0) - sc.sub + (1 << lg) - 1) >> lg : 0;
-            double2 a[NCH], b[NCH];
-            read(a, pick(0 < mine, k0, WIN_CAP));
-            k1 = pick(1 < mine, k1, WIN_CAP);
-#pragma unroll 1
-            for (int i = 0; __any(i < mine); i += 2) {
-                l += 2 * row;
-                k0 = pick(i + 2 < mine, n0, WIN_CAP);
-                const int k2 = pick(i + 3 < mine, n1, WIN_CAP);
-                n0 = l[2 * row + o];
-                n1 = l[3 * row + o];
-                read(b, k1);
-                body(a, rec, 0);
-                read(a, k0);
-                k1 = k2;
-                body(b, rec, 0);
-            }
+            visit_window<NCH, double2>(lds, w, I, n, sc, lg, [&](const auto& v) { body(v, rec, 0); });
             // a particle whose list overflowed walks its rows
-            if (cnt < 0 && sc.valid) {
+            if (w.cnt < 0 && sc.valid) {
                 int tot;
                 const Ranges3 rows = C.rows(sc.tt, tot);
 #pragma unroll 1
                 for (int i = sc.sub; i < tot; i += 1 << lg) {
                     const int k = rows(i);
                     if (k == self || !accept(k, rec(k, 0))) continue;
+                    double2 a[NCH];
 #pragma unroll
                     for (int c = 0; c < NCH; ++c) a[c] = rec(k, c);
                     body(a, rec, k);

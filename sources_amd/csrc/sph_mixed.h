@@ -112,6 +112,16 @@ __device__ __forceinline__ void kern_f(const KCf& k, float r, float inv_r, float
     gy = s * dy;
 }
 
+// 1, or 0 and no terms for a listed candidate at or beyond dr = lim.
+__device__ __forceinline__ int inside(float dr, float lim, float& w, float& gx, float& gy)
+{
+    const bool in = dr < lim;
+    w = in ? w : 0.0f;
+    gx = in ? gx : 0.0f;
+    gy = in ? gy : 0.0f;
+    return in ? 1 : 0;
+}
+
 // Mixed-precision constants of a step.
 struct MixK {
     float cs;                  // cell size
@@ -250,17 +260,61 @@ __device__ __forceinline__ CatMask cand_mask_f(const LaneRows& L, const Masks& M
     return cat_masks(L, m0, m1, m2);
 }
 
+// The partners of a lane's particle for the stage kernels.  In list mode with
+// uniform smoothing lengths (the host passes no index lists otherwise) the
+// workgroup's window of FP32 records is in LDS, and every lane goes through
+// its listed candidates there; those outside the support count nothing.  Else
+// (or where the window does not fit) the first lane of each particle goes
+// through its partner mask, reading the records from global memory.
+// Stage 1 was bound by the gathers of the partners' records (1M slope, us per
+// launch: 140 -> 105); stage 2 is bound by its FP32 terms and their sums in
+// FP64, and pays for the candidates in the skin (150 -> 166).  us per step, masks
+// -> windows: slope of 3k 55 -> 46, 33k 57 -> 52, 125k 73 -> 67, 250k 102 -> 100,
+// 1M 419 -> 400; column of 64k 60 -> 50, 400k 131 -> 122.
+// body(v, lim): record chunks v and the squared distance it has yet to be within;
+// mask(R): the partner mask over the rows R = rows().
+template <int NCH, class L, class M, class A, class B>
+__device__ __forceinline__ void visit_mx(unsigned char* lds, const Window& w, const IdxList& I, int n,
+                                         const SubCtx& sc, int lg, int self, const RecQ& rec, float thr, L&& rows,
+                                         M&& mask, A&& accept, B&& body)
+{
+    auto global = [&](int k) {
+        float4 v[NCH];
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) v[c] = rec(k, c);
+        body(v, INFINITY);
+    };
+    if (w.lds) {
+        visit_window<NCH, float4>(lds, w, I, n, sc, lg, [&](const auto& v) { body(v, thr); });
+        if (w.cnt < 0 && sc.valid && sc.sub == 0) {   // a list that overflowed
+            const LaneRows R = rows();
+            visit_f(CatMask{0, 0, 7}, R, self, [&](int k) { return accept(rec(k, 0)); }, global);
+        }
+        return;
+    }
+    if (!sc.valid || sc.sub) return;
+    const LaneRows R = rows();
+    visit_f(mask(R), R, self, [&](int k) { return accept(rec(k, 0)); }, global);
+}
+
+// Lanes of a workgroup that take particles: the windows' with index lists.
+__host__ __device__ __forceinline__ int mx_lanes(const NList& NL) { return NL.is.li ? WIN_LANES : STAGE_BLOCK; }
+
+template <int NCH>
+constexpr size_t MX_LDS = sizeof(float4) * NCH * WIN_STRIDE;
+
 // ------------------------------------------------------------------------
 // Stage A, water (mixed): the terms of k_water_a4 with FP32 pair sums.
 // ------------------------------------------------------------------------
 // XM = 1: the same-phase terms (the cross terms come from the XM = 2 pass,
 // which runs first and stores them); XM = 2: the cross terms alone.
 template <int SKF, int XM>
-__device__ __forceinline__ void water_a_mx(int blk, DPhase W, DPhase S, const float* qW, float* qWw, const float* qS,
-                                           NList NL, Masks MW, Grid g, KParams K, FusedK F, MixK X, int cross)
+__device__ __forceinline__ void water_a_mx(unsigned char* lds, int blk, DPhase W, DPhase S, const float* qW, float* qWw,
+                                           const float* qS, NList NL, Masks MW, Grid g, KParams K, FusedK F, MixK X,
+                                           int cross)
 {
     const RecQ QWv = recqv(qW, W.n), QSv = recqv(qS, S.n);
-    const WaveCtx wc = wave_ctx(W.n, blk);
+    const SubCtx wc = sub_ctx(W.n, blk, NL.lg, mx_lanes(NL));
     const int t = wc.t;
     auto QA = [&](int c) { return QWv(wc.tt, c); };
     const float4 a0 = QA(0), a1 = QA(1), a2 = QA(2);
@@ -274,20 +328,21 @@ __device__ __forceinline__ void water_a_mx(int blk, DPhase W, DPhase S, const fl
         Sum64 dg_x, dg_y, dvof_x, vof2;
         int cntx = 0;
         if (cross) {
-            const LaneRows LX = rows_of_cell(g, S.cell_start, me.cx, me.cy);
             auto accx_q = [&](float4 b0) {
                 float dx, dy;
                 sep(me, b0, X.cs, dx, dy);
                 return pred_f(F.uni_x, X.thr_x, dx * dx + dy * dy, me.h, b0.w, X.scale_k);
             };
-            const CatMask cx3 = cand_mask_f(LX, NL.cross, W.n, wc.tt, -1, QSv, accx_q);
             const double vofa_d = W.vof[a], rhoa_d = W.rho[a];
             const float cfa = (float)(vofa_d * rhoa_d * (-K.numeric_gravity) / K.s_perm);
             const float irhoa = a2.y;
             const KCf kx = make_kcf(SKF, F.uni_x ? 0.5 * ((double)me.h + (double)QSv(0, 0).w) : (double)me.h);
-            visit_f(cx3, LX, -1, [&](int k) { return accx_q(QSv(k, 0)); }, [&](int k) {
-                auto Q = [&](int c) { return QSv(k, c); };
-                const float4 b0 = Q(0), b1 = Q(1), b2 = Q(2);
+            const Window win = open_window<true, 3>(lds, NL.ix, blk, wc, NL.lg, W.n, QSv);
+            visit_mx<3>(lds, win, NL.ix, W.n, wc, NL.lg, -1, QSv, X.thr_x,
+                        [&] { return rows_of_cell(g, S.cell_start, me.cx, me.cy); },
+                        [&](const LaneRows& R) { return cand_mask_f(R, NL.cross, W.n, wc.tt, -1, QSv, accx_q); },
+                        accx_q, [&](const auto& v, float lim) {
+                const float4 b0 = v[0], b1 = v[1], b2 = v[2];
                 float dx, dy;
                 sep(me, b0, X.cs, dx, dy);
                 const float dr = dx * dx + dy * dy;
@@ -296,7 +351,7 @@ __device__ __forceinline__ void water_a_mx(int blk, DPhase W, DPhase S, const fl
                 float ww, gx, gy;
                 if (F.uni_x) kern_f<SKF, true>(kx, r, ir, dx, dy, ww, gx, gy);
                 else kern_f<SKF, true>(make_kcf(SKF, 0.5 * ((double)me.h + (double)b0.w)), r, ir, dx, dy, ww, gx, gy);
-                ++cntx;
+                cntx += inside(dr, lim, ww, gx, gy);
                 const float mb = b1.w;
                 const float dvx = vxa - b1.x, dvy = vya - b1.y;
                 const float sc = mb * (cfa * b2.x) * (ww * irhoa * b2.y);
@@ -305,8 +360,10 @@ __device__ __forceinline__ void water_a_mx(int blk, DPhase W, DPhase S, const fl
                 dvof_x.add(mb * (dvx * gx + dvy * gy));
                 vof2.add(mb * ww);
             });
+            sub_sum(NL.lg, dg_x.s, dg_y.s, dvof_x.s, vof2.s);
+            cntx = sub_count(NL.lg, cntx);
         }
-        if (!wc.valid) return;
+        if (!wc.valid || wc.sub) return;
         if (cross) {
             W.drgx[a] = dg_x.value();
             W.drgy[a] = dg_y.value();
@@ -316,26 +373,28 @@ __device__ __forceinline__ void water_a_mx(int blk, DPhase W, DPhase S, const fl
         }
         return;
     }
-    const LaneRows L = rows_of_cell(g, W.cell_start, me.cx, me.cy);
     auto acc_q = [&](float4 b0) {
         float dx, dy;
         sep(me, b0, X.cs, dx, dy);
         return pred_f(uni, X.thr_w, dx * dx + dy * dy, me.h, b0.w, X.scale_k);
     };
-    const CatMask cm = cand_mask_f(L, NL.same, W.n, wc.tt, t, QWv, acc_q);
-    if (wc.valid) {
-        MW.m[t] = cm.lo;
-        MW.m[W.n + t] = cm.hi;
-        MW.ovf[t] = cm.ovf;
-    }
+    const Window win = open_window<true, 2>(lds, NL.is, blk, wc, NL.lg, W.n, QWv);
     const bool real_a = W.itype[a] > 0;
     const float dspp = (float)W.dspp;
     Sum64 con, drd, txx, txy, tyy, avx, avy;
     float repx = 0.0f, repy = 0.0f;
     int cnt = 0;
-    visit_f(cm, L, t, [&](int k) { return acc_q(QWv(k, 0)); }, [&](int k) {
-        auto Q = [&](int c) { return QWv(k, c); };
-        const float4 b0 = Q(0), b1 = Q(1);   // 1/rho and m/rho recomputed: two loads per partner
+    auto mask_a = [&](const LaneRows& R) {   // (kept for stage B, which has the same window)
+        const CatMask cm = cand_mask_f(R, NL.same, W.n, wc.tt, t, QWv, acc_q);
+        MW.m[t] = cm.lo;
+        MW.m[W.n + t] = cm.hi;
+        MW.ovf[t] = cm.ovf;
+        return cm;
+    };
+    visit_mx<2>(lds, win, NL.is, W.n, wc, NL.lg, t, QWv, X.thr_w,
+                [&] { return rows_of_cell(g, W.cell_start, me.cx, me.cy); }, mask_a, acc_q,
+                [&](const auto& v, float lim) {
+        const float4 b0 = v[0], b1 = v[1];   // 1/rho and m/rho recomputed: two chunks per partner
         float dx, dy;
         sep(me, b0, X.cs, dx, dy);
         const float dr = dx * dx + dy * dy;
@@ -344,7 +403,7 @@ __device__ __forceinline__ void water_a_mx(int blk, DPhase W, DPhase S, const fl
         float ww, gx, gy;
         if (uni) kern_f<SKF, true>(kc, r, ir, dx, dy, ww, gx, gy);
         else kern_f<SKF, true>(make_kcf(SKF, 0.5 * ((double)me.h + (double)b0.w)), r, ir, dx, dy, ww, gx, gy);
-        ++cnt;
+        cnt += inside(dr, lim, ww, gx, gy);
         const float mb = b1.w, irb = __builtin_amdgcn_rcpf(b1.z + X.rho0_w), Vb = mb * irb;
         const float dvx = vxa - b1.x, dvy = vya - b1.y;
         con.add(mb * (dvx * gx + dvy * gy));
@@ -363,7 +422,10 @@ __device__ __forceinline__ void water_a_mx(int blk, DPhase W, DPhase S, const fl
         }
     });
 
-    if (!wc.valid) return;
+    double repx_d = repx, repy_d = repy;
+    sub_sum(NL.lg, con.s, drd.s, txx.s, txy.s, tyy.s, avx.s, avy.s, repx_d, repy_d);
+    cnt = sub_count(NL.lg, cnt);
+    if (!wc.valid || wc.sub) return;
     const double vofa_d = W.vof[a], ha_d = W.hsml[a], ca_d = W.c[a];
     const double mu = K.w_mu;
     const double txx_d = txx.value() * SPH_C23_F, tyy_d = tyy.value() * SPH_C23_F, txy_d = txy.value();
@@ -372,7 +434,7 @@ __device__ __forceinline__ void water_a_mx(int blk, DPhase W, DPhase S, const fl
     double avx_d = avx.value(), avy_d = avy.value();
     if (real_a) { avx_d *= K.epsilon; avy_d *= K.epsilon; }
     if (K.average_velocity) { W.avx[a] = avx_d; W.avy[a] = avy_d; }
-    W.repx[a] = repx; W.repy[a] = repy;
+    W.repx[a] = repx_d; W.repy[a] = repy_d;
     if (!cross) W.countiac[a] = cnt;   // (with cross terms: the XM = 2 pass's count)
     W.nsame[a] = cnt;
     // p (q2.w) and the new c (q3.x) come from the pack
@@ -386,7 +448,8 @@ template <int SKF>
 __global__ STAGE_ATTR_MX void k_water_a_mx(DPhase W, DPhase S, const float* qW, float* qWw, const float* qS, NList NL,
                                            Masks MW, Grid g, KParams K, FusedK F, MixK X, int cross)
 {
-    water_a_mx<SKF, 1>(xcd_block(), W, S, qW, qWw, qS, NL, MW, g, K, F, X, cross);
+    __shared__ __align__(16) unsigned char lds[MX_LDS<2>];
+    water_a_mx<SKF, 1>(lds, xcd_block(), W, S, qW, qWw, qS, NL, MW, g, K, F, X, cross);
 }
 
 // The water side's cross terms (soil partners), before k_water_a_mx.
@@ -394,18 +457,19 @@ template <int SKF>
 __global__ STAGE_ATTR void k_water_x_mx(DPhase W, DPhase S, const float* qW, float* qWw, const float* qS, NList NL,
                                         Masks MW, Grid g, KParams K, FusedK F, MixK X, int cross)
 {
-    water_a_mx<SKF, 2>(xcd_block(), W, S, qW, qWw, qS, NL, MW, g, K, F, X, cross);
+    __shared__ __align__(16) unsigned char lds[MX_LDS<3>];
+    water_a_mx<SKF, 2>(lds, xcd_block(), W, S, qW, qWw, qS, NL, MW, g, K, F, X, cross);
 }
 
 // ------------------------------------------------------------------------
 // Stage B, water (mixed): momentum, art_visc, delta_sph(vof).
 // ------------------------------------------------------------------------
 template <int SKF>
-__device__ __forceinline__ void water_b_mx(int blk, DPhase W, const float* qW, Masks MW, Grid g, KParams K, FusedK F,
-                                           MixK X, int mask)
+__device__ __forceinline__ void water_b_mx(unsigned char* lds, int blk, DPhase W, const float* qW, NList NL, Masks MW,
+                                           Grid g, KParams K, FusedK F, MixK X, int mask)
 {
     const RecQ QWv = recqv(qW, W.n);
-    const WaveCtx wc = wave_ctx(W.n, blk);
+    const SubCtx wc = sub_ctx(W.n, blk, NL.lg, mx_lanes(NL));
     const int t = wc.t;
     auto QA = [&](int c) { return QWv(wc.tt, c); };
     const float4 a0 = QA(0), a1 = QA(1), a2 = QA(2), a3 = QA(3);
@@ -415,24 +479,19 @@ __device__ __forceinline__ void water_b_mx(int blk, DPhase W, const float* qW, M
     const int a = W.order[wc.tt];
     const bool uni = F.uni_w;
     const KCf kc = make_kcf(SKF, me.h);
-    const LaneRows L = rows_of_cell(g, W.cell_start, me.cx, me.cy);
     auto acc_q = [&](float4 b0) {
         float dx, dy;
         sep(me, b0, X.cs, dx, dy);
         return pred_f(uni, X.thr_w, dx * dx + dy * dy, me.h, b0.w, X.scale_k);
     };
-    CatMask cm{0, 0, 0};
-    if (wc.valid) {
-        cm.lo = MW.m[t];
-        cm.hi = MW.m[W.n + t];
-        cm.ovf = MW.ovf[t];
-    }
+    const Window win = open_window<true, 4>(lds, NL.is, blk, wc, NL.lg, W.n, QWv);
     const float et2 = (float)(K.etq * K.etq);
     const float beta = (float)K.beta, alpha = (float)K.alpha;
     Sum64 Px, Py, Sxx, Sxyy, Sxyx, Syy, artx, arty, dvd;
-    visit_f(cm, L, t, [&](int k) { return acc_q(QWv(k, 0)); }, [&](int k) {
-        auto Q = [&](int c) { return QWv(k, c); };
-        const float4 b0 = Q(0), b1 = Q(1), b2 = Q(2), b3 = Q(3);
+    visit_mx<4>(lds, win, NL.is, W.n, wc, NL.lg, t, QWv, X.thr_w,
+                [&] { return rows_of_cell(g, W.cell_start, me.cx, me.cy); },
+                [&](const LaneRows&) { return mask_of(MW, W.n, t); }, acc_q, [&](const auto& v, float lim) {
+        const float4 b0 = v[0], b1 = v[1], b2 = v[2], b3 = v[3];
         float dx, dy;
         sep(me, b0, X.cs, dx, dy);
         const float dr = dx * dx + dy * dy;
@@ -442,6 +501,7 @@ __device__ __forceinline__ void water_b_mx(int blk, DPhase W, const float* qW, M
         const float amh = 0.5f * (me.h + b0.w);
         if (uni) kern_f<SKF, false>(kc, r, ir, dx, dy, ww, gx, gy);
         else kern_f<SKF, false>(make_kcf(SKF, amh), r, ir, dx, dy, ww, gx, gy);
+        inside(dr, lim, ww, gx, gy);
         const float Vb = b2.z, mb = b1.w;
         const float ps = pa + b2.w;
         Px.add(Vb * (ps * gx));
@@ -460,7 +520,8 @@ __device__ __forceinline__ void water_b_mx(int blk, DPhase W, const float* qW, M
         arty.add(-(mb * piv * gy));
         dvd.add(mb * (2.0f * (vofa - b2.x) * idr * (dx * gx + dy * gy)) * b2.y);
     });
-    if (!wc.valid) return;
+    sub_sum(NL.lg, Px.s, Py.s, Sxx.s, Sxyy.s, Sxyx.s, Syy.s, artx.s, arty.s, dvd.s);
+    if (!wc.valid || wc.sub) return;
     const double vofa_d = W.vof[a], rhoa_d = W.rho[a], ha_d = W.hsml[a], ca_d = W.c[a];   // new c
     double ax = -(vofa_d * Px.value()) + Sxx.value() + Sxyy.value();
     double ay = -(vofa_d * Py.value()) + Sxyx.value() + Syy.value();
@@ -484,10 +545,11 @@ __device__ __forceinline__ void water_b_mx(int blk, DPhase W, const float* qW, M
 }
 
 template <int SKF>
-__global__ STAGE_ATTR_MX void k_water_b_mx(DPhase W, const float* qW, Masks MW, Grid g, KParams K, FusedK F, MixK X,
-                                           int mask)
+__global__ STAGE_ATTR_MX void k_water_b_mx(DPhase W, const float* qW, NList NL, Masks MW, Grid g, KParams K, FusedK F,
+                                           MixK X, int mask)
 {
-    water_b_mx<SKF>(xcd_block(), W, qW, MW, g, K, F, X, mask);
+    __shared__ __align__(16) unsigned char lds[MX_LDS<4>];
+    water_b_mx<SKF>(lds, xcd_block(), W, qW, NL, MW, g, K, F, X, mask);
 }
 
 // ------------------------------------------------------------------------
@@ -499,11 +561,12 @@ __global__ STAGE_ATTR_MX void k_water_b_mx(DPhase W, const float* qW, Masks MW, 
 // XM = 1: the same-phase terms and the tail (the cross terms from the XM = 2
 // pass, which runs first and stores them); XM = 2: the cross terms alone.
 template <int SKF, int XM>
-__device__ __forceinline__ void soil_ab_mx(int blk, DPhase S, DPhase W, const float* qS, const float* qW, NList NL,
-                                           Grid g, KParams K, FusedK F, MixK X, int cross, int mask)
+__device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S, DPhase W, const float* qS,
+                                           const float* qW, NList NL, Grid g, KParams K, FusedK F, MixK X, int cross,
+                                           int mask)
 {
     const RecQ QSv = recqv(qS, S.n), QWv = recqv(qW, W.n);
-    const WaveCtx wc = wave_ctx(S.n, blk);
+    const SubCtx wc = sub_ctx(S.n, blk, NL.lg, mx_lanes(NL));
     const int t = wc.t;
     auto QA = [&](int c) { return QSv(wc.tt, c); };
     const float4 a0 = QA(0), a1 = QA(1), a2 = QA(2), a3 = QA(3);
@@ -525,18 +588,19 @@ __device__ __forceinline__ void soil_ab_mx(int blk, DPhase S, DPhase W, const fl
     int cntx = 0;
     const double vofa_d = S.vof[a];
     if (XM == 2 && cross) {
-        const LaneRows LX = rows_of_cell(g, W.cell_start, me.cx, me.cy);
         auto accx_q = [&](float4 b0) {
             float dx, dy;
             sep(me, b0, X.cs, dx, dy);
             return pred_f(F.uni_x, X.thr_x, dx * dx + dy * dy, me.h, b0.w, X.scale_k);
         };
-        const CatMask cx3 = cand_mask_f(LX, NL.cross, S.n, wc.tt, -1, QWv, accx_q);
         const float cfs = (float)(vofa_d * (-K.numeric_gravity) / K.s_perm);
         const KCf kx = make_kcf(SKF, F.uni_x ? 0.5 * ((double)QWv(0, 0).w + (double)me.h) : (double)me.h);
-        visit_f(cx3, LX, -1, [&](int k) { return accx_q(QWv(k, 0)); }, [&](int k) {
-            auto Q = [&](int c) { return QWv(k, c); };
-            const float4 b0 = Q(0), b1 = Q(1), b2 = Q(2);
+        const Window win = open_window<true, 3>(lds, NL.ix, blk, wc, NL.lg, S.n, QWv);
+        visit_mx<3>(lds, win, NL.ix, S.n, wc, NL.lg, -1, QWv, X.thr_x,
+                    [&] { return rows_of_cell(g, W.cell_start, me.cx, me.cy); },
+                    [&](const LaneRows& R) { return cand_mask_f(R, NL.cross, S.n, wc.tt, -1, QWv, accx_q); }, accx_q,
+                    [&](const auto& v, float lim) {
+            const float4 b0 = v[0], b1 = v[1], b2 = v[2];
             float dx, dy;
             sep(me, b0, X.cs, dx, dy);
             dx = -dx;   // water - soil
@@ -547,7 +611,7 @@ __device__ __forceinline__ void soil_ab_mx(int blk, DPhase S, DPhase W, const fl
             float ww, gx, gy;
             if (F.uni_x) kern_f<SKF, true>(kx, r, ir, dx, dy, ww, gx, gy);
             else kern_f<SKF, true>(make_kcf(SKF, 0.5 * ((double)b0.w + (double)me.h)), r, ir, dx, dy, ww, gx, gy);
-            ++cntx;
+            cntx += inside(dr, lim, ww, gx, gy);
             const float mw = b1.w, rhow = b1.z + X.rho0_w;
             const float sc = mw * (b2.x * rhow * cfs) * (ww * b2.y * irhoa);
             dg_x.add(sc * (b1.x - vxa));
@@ -556,10 +620,12 @@ __device__ __forceinline__ void soil_ab_mx(int blk, DPhase S, DPhase W, const fl
             po_x.add(mprr * gx);
             po_y.add(mprr * gy);
         });
+        sub_sum(NL.lg, dg_x.s, dg_y.s, po_x.s, po_y.s);
+        cntx = sub_count(NL.lg, cntx);
     }
 
     if constexpr (XM == 2) {
-        if (!wc.valid) return;
+        if (!wc.valid || wc.sub) return;
         if (cross) {
             S.drgx[a] = dg_x.value();
             S.drgy[a] = dg_y.value();
@@ -570,22 +636,23 @@ __device__ __forceinline__ void soil_ab_mx(int blk, DPhase S, DPhase W, const fl
         return;
     }
 
-    const LaneRows L = rows_of_cell(g, S.cell_start, me.cx, me.cy);
     auto acc_q = [&](float4 b0) {
         float dx, dy;
         sep(me, b0, X.cs, dx, dy);
         return pred_f(uni, X.thr_s, dx * dx + dy * dy, me.h, b0.w, X.scale_k);
     };
-    const CatMask cm = cand_mask_f(L, NL.same, S.n, wc.tt, t, QSv, acc_q);
+    const Window win = open_window<true, 4>(lds, NL.is, blk, wc, NL.lg, S.n, QSv);
     const float et2 = (float)(K.etq * K.etq);
     const float beta = (float)K.beta, alpha = (float)K.alpha;
     Sum64 con, drd, txx, txy, tyy, vcc, wxy, avx, avy;
     Sum64 Fx, Fy, artx, arty, dP, dXX, dXY, dYY;
     float repx = 0.0f, repy = 0.0f;
     int cnt = 0;
-    visit_f(cm, L, t, [&](int k) { return acc_q(QSv(k, 0)); }, [&](int k) {
-        auto Q = [&](int c) { return QSv(k, c); };
-        const float4 b0 = Q(0), b1 = Q(1), b2 = Q(2), b3 = Q(3);
+    visit_mx<4>(lds, win, NL.is, S.n, wc, NL.lg, t, QSv, X.thr_s,
+                [&] { return rows_of_cell(g, S.cell_start, me.cx, me.cy); },
+                [&](const LaneRows& R) { return cand_mask_f(R, NL.same, S.n, wc.tt, t, QSv, acc_q); }, acc_q,
+                [&](const auto& v, float lim) {
+        const float4 b0 = v[0], b1 = v[1], b2 = v[2], b3 = v[3];
         float dx, dy;
         sep(me, b0, X.cs, dx, dy);
         const float dr = dx * dx + dy * dy;
@@ -595,7 +662,7 @@ __device__ __forceinline__ void soil_ab_mx(int blk, DPhase S, DPhase W, const fl
         const float amh = 0.5f * (me.h + b0.w);
         if (uni) kern_f<SKF, true>(kc, r, ir, dx, dy, ww, gx, gy);
         else kern_f<SKF, true>(make_kcf(SKF, 0.5 * ((double)me.h + (double)b0.w)), r, ir, dx, dy, ww, gx, gy);
-        ++cnt;
+        cnt += inside(dr, lim, ww, gx, gy);
         const float mb = b1.w, vofb = b2.x, irb = b2.y, Vb = b2.z;
         // stage A
         const float dvx = vxa - b1.x, dvy = vya - b1.y;
@@ -637,7 +704,11 @@ __device__ __forceinline__ void soil_ab_mx(int blk, DPhase S, DPhase W, const fl
         dXY.add(hh * (sxya - b3.z));
         dYY.add(hh * (syya - b3.w));
     });
-    if (!wc.valid) return;
+    double repx_d = repx, repy_d = repy;
+    sub_sum(NL.lg, con.s, drd.s, txx.s, txy.s, tyy.s, vcc.s, wxy.s, avx.s, avy.s, repx_d, repy_d);
+    sub_sum(NL.lg, Fx.s, Fy.s, artx.s, arty.s, dP.s, dXX.s, dXY.s, dYY.s);
+    cnt = sub_count(NL.lg, cnt);
+    if (!wc.valid || wc.sub) return;
     const double ha_d = S.hsml[a], ca_d = S.c[a], rhoa_d = S.rho[a];
     const double txx_d = txx.value() * SPH_C23_F, tyy_d = tyy.value() * SPH_C23_F, txy_d = txy.value();
     const double vcc_d = vcc.value(), wxy_d = wxy.value() * 0.5;
@@ -646,7 +717,7 @@ __device__ __forceinline__ void soil_ab_mx(int blk, DPhase S, DPhase W, const fl
     double avx_d = avx.value(), avy_d = avy.value();
     if (real_a) { avx_d *= K.epsilon; avy_d *= K.epsilon; }
     if (K.average_velocity) { S.avx[a] = avx_d; S.avy[a] = avy_d; }
-    S.repx[a] = repx; S.repy[a] = repy;
+    S.repx[a] = repx_d; S.repy[a] = repy_d;
     // the cross terms the XM = 2 pass stored
     const double dgx_d = cross ? S.drgx[a] : 0.0, dgy_d = cross ? S.drgy[a] : 0.0;
     const double pox_d = cross ? S.porx[a] : 0.0, poy_d = cross ? S.pory[a] : 0.0;
@@ -688,8 +759,8 @@ __device__ __forceinline__ void soil_ab_mx(int blk, DPhase S, DPhase W, const fl
     double ay = Fy.value() * rhoa_d;
     if (rhoa_d > 0.0) { ax = ax / rhoa_d; ay = ay / rhoa_d; }
     if (mask & M_ART) { ax = ax + artx.value(); ay = ay + arty.value(); }
-    ax = ax + (double)repx;
-    ay = ay + (double)repy;
+    ax = ax + repx_d;
+    ay = ay + repy_d;
     ay = ay + K.gravity;
     if (mask & M_CROSS) {
         ax = ax + dgx_d; ay = ay + dgy_d;
@@ -711,7 +782,8 @@ template <int SKF>
 __global__ STAGE_ATTR_MX_AB void k_soil_ab_mx(DPhase S, DPhase W, const float* qS, const float* qW, NList NL, Grid g,
                                               KParams K, FusedK F, MixK X, int cross, int mask)
 {
-    soil_ab_mx<SKF, 1>(xcd_block(), S, W, qS, qW, NL, g, K, F, X, cross, mask);
+    __shared__ __align__(16) unsigned char lds[MX_LDS<4>];
+    soil_ab_mx<SKF, 1>(lds, xcd_block(), S, W, qS, qW, NL, g, K, F, X, cross, mask);
 }
 
 // The soil side's cross terms (water partners), before k_soil_ab_mx.
@@ -719,7 +791,8 @@ template <int SKF>
 __global__ STAGE_ATTR void k_soil_x_mx(DPhase S, DPhase W, const float* qS, const float* qW, NList NL, Grid g,
                                        KParams K, FusedK F, MixK X, int cross, int mask)
 {
-    soil_ab_mx<SKF, 2>(xcd_block(), S, W, qS, qW, NL, g, K, F, X, cross, mask);
+    __shared__ __align__(16) unsigned char lds[MX_LDS<3>];
+    soil_ab_mx<SKF, 2>(lds, xcd_block(), S, W, qS, qW, NL, g, K, F, X, cross, mask);
 }
 
 // The launches of a whole step (k_stage1, k_stage2), mixed.
@@ -739,20 +812,22 @@ struct StageArgsMx {
 template <int SKF>
 __device__ __forceinline__ void stage1_mx(int l, const StageArgsMx& A, bool spread)
 {
+    __shared__ __align__(16) unsigned char lds[MX_LDS<3>];
     const PartIdx p = part_of<3>(l, {A.nbS, A.nbW, A.nbW}, spread);
     if (p.blk < 0) return;
-    if (p.part == 0) soil_ab_mx<SKF, 2>(p.blk, A.S, A.W, A.qS, A.qW, A.nS, A.gS, A.K, A.F, A.X, 1, A.mask_s);
-    else if (p.part == 1) water_a_mx<SKF, 1>(p.blk, A.W, A.S, A.qW, A.qW, A.qS, A.nW, A.MW, A.gW, A.K, A.F, A.X, 1);
-    else water_a_mx<SKF, 2>(p.blk, A.W, A.S, A.qW, A.qW, A.qS, A.nW, A.MW, A.gW, A.K, A.F, A.X, 1);
+    if (p.part == 0) soil_ab_mx<SKF, 2>(lds, p.blk, A.S, A.W, A.qS, A.qW, A.nS, A.gS, A.K, A.F, A.X, 1, A.mask_s);
+    else if (p.part == 1) water_a_mx<SKF, 1>(lds, p.blk, A.W, A.S, A.qW, A.qW, A.qS, A.nW, A.MW, A.gW, A.K, A.F, A.X, 1);
+    else water_a_mx<SKF, 2>(lds, p.blk, A.W, A.S, A.qW, A.qW, A.qS, A.nW, A.MW, A.gW, A.K, A.F, A.X, 1);
 }
 
 template <int SKF>
 __device__ __forceinline__ void stage2_mx(int l, const StageArgsMx& A, bool spread)
 {
+    __shared__ __align__(16) unsigned char lds[MX_LDS<4>];
     const PartIdx p = part_of<2>(l, {A.nbS, A.nbW}, spread);
     if (p.blk < 0) return;
-    if (p.part == 0) soil_ab_mx<SKF, 1>(p.blk, A.S, A.W, A.qS, A.qW, A.nS, A.gS, A.K, A.F, A.X, 1, A.mask_s);
-    else water_b_mx<SKF>(p.blk, A.W, A.qW, A.MW, A.gW, A.K, A.F, A.X, A.mask_w);
+    if (p.part == 0) soil_ab_mx<SKF, 1>(lds, p.blk, A.S, A.W, A.qS, A.qW, A.nS, A.gS, A.K, A.F, A.X, 1, A.mask_s);
+    else water_b_mx<SKF>(lds, p.blk, A.W, A.qW, A.nW, A.MW, A.gW, A.K, A.F, A.X, A.mask_w);
 }
 
 template <int SKF>

@@ -1297,15 +1297,25 @@ int stages_mixed(sphg_ctx* c, const FinalArgs* fin)
     // with neighbour lists: the list grid (records hold positions relative
     // to their list cells) and the lists
     const bool nl = nl_mode(c);
-    const NList nW = nlist_of(c, W, nl);
-    const NList nS = nlist_of(c, S, nl);
+    NList nW = nlist_of(c, W, nl);
+    NList nS = nlist_of(c, S, nl);
+    if (!(c->F.uni_w && c->F.uni_s && c->F.uni_x) || c->P.nnps == 2) {
+        // the windows' predicate is a distance alone: masks and one lane per
+        // particle over the whole workgroup (the windows' 192 of 256 lanes
+        // would leave a quarter of them idle for nothing)
+        for (NList* L : {&nW, &nS}) {
+            L->is = L->ix = IdxList{};
+            L->lg = 0;
+        }
+    }
+    const int nbW = nblk(W.n, mx_lanes(nW) >> nW.lg), nbS = nblk(S.n, mx_lanes(nS) >> nS.lg);
     const Grid& gW = nl ? c->gvl[0] : c->gl[0];
     const Grid& gS = nl ? c->gvl[1] : c->gl[1];
     MixK X = c->X;
     if (nl) X.cs = (float)c->csv;
     if (!c->prof) {
         StageArgsMx A{W.d, S.d, qW, qS, nW, nS, W.masks, gW, gS, c->K, c->F, X, mask_b(c, 0), mask_b(c, 1),
-                      nblk(W.n, STAGE_BLOCK), nblk(S.n, STAGE_BLOCK)};
+                      nbW, nbS};
         RC(launch(c, "stage1", k_stage1_mx<SKF>, pad8(A.nbS) + 2 * pad8(A.nbW), STAGE_BLOCK, A));
         swap_c(W);
         swap_c(S);
@@ -1319,20 +1329,20 @@ int stages_mixed(sphg_ctx* c, const FinalArgs* fin)
     {
         // the cross terms in a pass of their own before the same-phase pass
         SideScope side(c);
-        RC(launch(c, "soil_x", k_soil_x_mx<SKF>, nblk(S.n, STAGE_BLOCK), STAGE_BLOCK, S.d, W.d, (const float*)qS,
+        RC(launch(c, "soil_x", k_soil_x_mx<SKF>, nbS, STAGE_BLOCK, S.d, W.d, (const float*)qS,
                   (const float*)qW, nS, gS, c->K, c->F, X, 1, mask_b(c, 1)));
-        RC(launch(c, "soil_ab", k_soil_ab_mx<SKF>, nblk(S.n, STAGE_BLOCK), STAGE_BLOCK, S.d, W.d, (const float*)qS,
+        RC(launch(c, "soil_ab", k_soil_ab_mx<SKF>, nbS, STAGE_BLOCK, S.d, W.d, (const float*)qS,
                   (const float*)qW, nS, gS, c->K, c->F, X, 1, mask_b(c, 1)));
     }
     // (stage A before the cross pass: beside the soil side's cross pass and
     // then its stage, each pair of concurrent kernels reads one phase's records)
-    RC(launch(c, "water_a", k_water_a_mx<SKF>, nblk(W.n, STAGE_BLOCK), STAGE_BLOCK, W.d, S.d, (const float*)qW, qW,
+    RC(launch(c, "water_a", k_water_a_mx<SKF>, nbW, STAGE_BLOCK, W.d, S.d, (const float*)qW, qW,
               (const float*)qS, nW, W.masks, gW, c->K, c->F, X, 1));
-    RC(launch(c, "water_x", k_water_x_mx<SKF>, nblk(W.n, STAGE_BLOCK), STAGE_BLOCK, W.d, S.d, (const float*)qW, qW,
+    RC(launch(c, "water_x", k_water_x_mx<SKF>, nbW, STAGE_BLOCK, W.d, S.d, (const float*)qW, qW,
               (const float*)qS, nW, W.masks, gW, c->K, c->F, X, 1));
     swap_c(W);
     swap_c(S);
-    RC(launch(c, "water_b", k_water_b_mx<SKF>, nblk(W.n, STAGE_BLOCK), STAGE_BLOCK, W.d, (const float*)qW, W.masks,
+    RC(launch(c, "water_b", k_water_b_mx<SKF>, nbW, STAGE_BLOCK, W.d, (const float*)qW, nW, W.masks,
               gW, c->K, c->F, X, mask_b(c, 0)));
     RC(fork.join());
     if (fin) {
@@ -2365,7 +2375,8 @@ int build_graph(sphg_gnn* g, sphg_gnn::Graph& G)
         gnn::GatherOut O{G.nf, G.raw, G.nb, G.nd, G.n, G.tw, g->node_of_id[k], g->overflow};
         return args_of(gnn::k_gnn_gather, b.d, lists ? c->gvl[k] : c->gl[k], c->K, k == 0 ? c->F.thr_w : c->F.thr_s,
                        k == 0 ? c->F.uni_w : c->F.uni_s, k == 0 ? 0 : Wb.n, k, g->S, O,
-                       lists ? b.nl_same : Masks{}, lists ? (const int*)b.nl_cell : (const int*)nullptr);
+                       lists ? b.il_same : IdxList{}, WIN_LANES >> b.lg,
+                       lists ? (const int*)b.nl_cell : (const int*)nullptr);
     };
     return launch_pair<BodyGnnGather>(c, "gnn_gather", nblk(Wb.n), args(0), nblk(Sb.n), args(1));
 }
