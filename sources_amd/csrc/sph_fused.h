@@ -1725,6 +1725,26 @@ __global__ STAGE_ATTR_AB void k_soil_ab4(DPhase S, const double* recS, NList NL,
 // and merged: 1.5k particles 83 / 40, 33k 82 / 45, 125k 100 / 77, 258k 127 /
 // 108, 1M 369 / 364).
 // ------------------------------------------------------------------------
+// A device flag word (two bits) that a kernel posts to the host: the word and
+// the number of its step, in pinned memory that the host watches.  A copy
+// engine's copy with an event behind it kept the queue for 10 us of every step
+// (4 us, and 5.5 until the next kernel started).
+struct FlagPost {
+    const int* flag;
+    int* slot;   // null: nothing to post
+    int seq;
+};
+
+// By the first workgroup of a launch; the flag is of kernels before it.
+__device__ __forceinline__ void post_flag(const FlagPost& p, int blk)
+{
+    if (!p.slot || blk != 0 || threadIdx.x != 0) return;
+    const unsigned v = ((unsigned)p.seq << 2) | ((unsigned)*p.flag & 3u);
+    __hip_atomic_store(p.slot, (int)v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ void k_post_flag(FlagPost p) { post_flag(p, blockIdx.x); }
+
 struct StageArgs {
     DPhase W, S;
     double *rW, *rS;
@@ -1734,6 +1754,7 @@ struct StageArgs {
     FusedK F;
     int mask_w, mask_s, lean;
     int nbW, nbS;   // workgroups of a pass over the water, over the soil
+    FlagPost post;  // (stage 1)
 };
 
 // The part of a launch that workgroup l belongs to, in the order of the counts
@@ -1770,6 +1791,7 @@ template <int SKF>
 __device__ __forceinline__ void stage1(int l, const StageArgs& A, bool spread)
 {
     __shared__ __align__(16) unsigned char lds[VIS_LDS<4>];
+    post_flag(A.post, l);
     const PartIdx p = part_of<3>(l, {A.nbS, A.nbW, A.nbW}, spread);
     if (p.blk < 0) return;
     if (p.part == 0) soil_x4<SKF, true>(lds, p.blk, A.S, A.W, A.rS, A.rW, A.nS, A.gS, A.K, A.F, A.lean);

@@ -950,9 +950,10 @@ __global__ __launch_bounds__(256) void k_gnn_fit(const float* y, const float* tg
 
 // The state of a phase copied back from a snapshot (A.s* -> A.d*) when the
 // sanity flag is set: a learned advance that broke the state is undone on
-// the device, before any later kernel reads it.
-__device__ __forceinline__ void restore_if_body(int blk, const int* flag, PermArgs A, int n)
+// the device, before any later kernel reads it.  Posts the flag.
+__device__ __forceinline__ void restore_if_body(int blk, const int* flag, PermArgs A, int n, FlagPost post)
 {
+    post_flag(post, blk);
     if (*flag == 0) return;
     const int i = blk * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -966,9 +967,9 @@ __device__ __forceinline__ void restore_if_body(int blk, const int* flag, PermAr
         if (q < A.ni) A.di[q][i] = A.si[q][i];
 }
 
-__global__ void k_restore_if(const int* flag, PermArgs A, int n)
+__global__ void k_restore_if(const int* flag, PermArgs A, int n, FlagPost post)
 {
-    restore_if_body(blockIdx.x, flag, A, n);
+    restore_if_body(blockIdx.x, flag, A, n, post);
 }
 
 __global__ void k_slot_of_id(DPhase P, int* slot_of_id)

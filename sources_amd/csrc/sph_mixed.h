@@ -807,12 +807,14 @@ struct StageArgsMx {
     MixK X;
     int mask_w, mask_s;
     int nbW, nbS;
+    FlagPost post;
 };
 
 template <int SKF>
 __device__ __forceinline__ void stage1_mx(int l, const StageArgsMx& A, bool spread)
 {
     __shared__ __align__(16) unsigned char lds[MX_LDS<3>];
+    post_flag(A.post, l);
     const PartIdx p = part_of<3>(l, {A.nbS, A.nbW, A.nbW}, spread);
     if (p.blk < 0) return;
     if (p.part == 0) soil_ab_mx<SKF, 2>(lds, p.blk, A.S, A.W, A.qS, A.qW, A.nS, A.gS, A.K, A.F, A.X, 1, A.mask_s);

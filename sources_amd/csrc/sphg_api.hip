@@ -12,6 +12,7 @@
 #include <atomic>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/sphg.h"
@@ -197,9 +198,9 @@ struct sphg_ctx {
     // step's first_half and took its cell keys and arrival ranks
     bool keyed = false;
     int* d_nlflag = nullptr;    // bit 0: rebuild due; bit 1: a particle moved past skin / 2
-    int* h_nlflag = nullptr;    // pinned: two slots for the lagged check of sphg_time_integration
+    int* h_nlflag = nullptr;    // pinned: two slots that the lagged check's flags are posted to
+    FlagPost post{};            // the post that the next stage 1 takes along
     int h_nlstep[2] = {-1, -1}; // nl_seq of the step whose flag each slot holds (-1: none)
-    hipEvent_t ev_nl[2] = {nullptr, nullptr};
 };
 
 namespace {
@@ -457,6 +458,43 @@ int check_flags(sphg_ctx* c)
         return SPHG_ERR_MOVED_TOO_FAR;
     }
     return SPHG_OK;
+}
+
+// Waits for the flag word that a kernel on the context's stream posts to a
+// slot under seq.  A stream that is done without it has failed.
+int await_post(sphg_ctx* c, const int* slot, int seq, int* flag)
+{
+    const unsigned tag = ((unsigned)seq << 2) >> 2;
+    for (unsigned spin = 1;; ++spin) {
+        const bool done = spin % 8192 == 0 && [&] {
+            const hipError_t e = hipStreamQuery(c->stream);
+            if (e != hipSuccess) (void)hipGetLastError();   // (not ready, or reported by the next check)
+            return e != hipErrorNotReady;
+        }();
+        const unsigned v = (unsigned)__atomic_load_n(slot, __ATOMIC_ACQUIRE);
+        if (v >> 2 == tag) {
+            *flag = (int)(v & 3u);
+            return SPHG_OK;
+        }
+        if (done) return SPHG_ERR_HIP;
+        if (spin % 64 == 0) std::this_thread::yield();
+        else __builtin_ia32_pause();
+    }
+}
+
+// The context's pending post (taken: the caller's launch carries it).
+FlagPost take_post(sphg_ctx* c)
+{
+    const FlagPost p = c->post;
+    c->post = FlagPost{};
+    return p;
+}
+
+// ... in a launch of its own, where the step's kernels do not carry it.
+int post_now(sphg_ctx* c)
+{
+    const FlagPost p = take_post(c);
+    return p.slot ? launch(c, "post", k_post_flag, 1, 1, p) : SPHG_OK;
 }
 
 void set_kparams(sphg_ctx* c)
@@ -1153,7 +1191,8 @@ int stages_fused(sphg_ctx* c, const FinalArgs* fin)
     const bool ux = c->F.uni_x != 0;
     if (us && uw && ux && cross && !c->prof) {
         // three launches on one stream (the profile times the passes apart)
-        StageArgs A{W.d, S.d, W.rec, S.rec, nW, nS, gW, gS, c->K, c->F, mask_b(c, 0), mask_b(c, 1), lean, nbW, nbS};
+        StageArgs A{W.d,  S.d,  W.rec,        S.rec,        nW,   nS,  gW,  gS,
+                    c->K, c->F, mask_b(c, 0), mask_b(c, 1), lean, nbW, nbS, take_post(c)};
         RC(launch(c, "stage1", k_stage1<SKF>, pad8(nbS) + 2 * pad8(nbW), STAGE_BLOCK, A));
         swap_c(W);
         swap_c(S);
@@ -1162,6 +1201,7 @@ int stages_fused(sphg_ctx* c, const FinalArgs* fin)
         RC(launch(c, "stage2", k_stage2<SKF>, pad8(nbS) + pad8(nbW), STAGE_BLOCK, A));
         return fin ? launch_finals(c, *fin) : SPHG_OK;
     }
+    RC(post_now(c));
     SideFork fork(c);
     RC(fork.rc);
     // with the finals on both streams, each phase's final kernel waits only
@@ -1315,7 +1355,7 @@ int stages_mixed(sphg_ctx* c, const FinalArgs* fin)
     if (nl) X.cs = (float)c->csv;
     if (!c->prof) {
         StageArgsMx A{W.d, S.d, qW, qS, nW, nS, W.masks, gW, gS, c->K, c->F, X, mask_b(c, 0), mask_b(c, 1),
-                      nbW, nbS};
+                      nbW, nbS, take_post(c)};
         RC(launch(c, "stage1", k_stage1_mx<SKF>, pad8(A.nbS) + 2 * pad8(A.nbW), STAGE_BLOCK, A));
         swap_c(W);
         swap_c(S);
@@ -1324,6 +1364,7 @@ int stages_mixed(sphg_ctx* c, const FinalArgs* fin)
         RC(launch(c, "stage2", k_stage2_mx<SKF>, pad8(A.nbS) + pad8(A.nbW), STAGE_BLOCK, A));
         return fin ? launch_finals(c, *fin) : SPHG_OK;
     }
+    RC(post_now(c));
     SideFork fork(c);   // soil stage beside the water stages
     RC(fork.rc);
     {
@@ -1577,21 +1618,20 @@ bool renorm_active(const sphg_params& P)
 bool renorm_step(const sphg_ctx* c, int step) { return renorm_active(c->P) && step % 40 == 0; }
 
 // Lagged displacement check of the list mode, in each step issued outside
-// a stream capture once its packs are queued: the flag word is copied to
-// pinned memory behind them, and the copy of the step before is read (it
-// has landed by the time the step's packs are queued, so the queue keeps
-// the step's stages and the rest of the step before).  A particle past the
+// a stream capture once its packs are queued: the step's first stage kernel
+// posts the flag word to pinned memory, and the post of the step before is
+// read (it has landed by the time the step's packs are queued, so the queue
+// keeps the step's stages and the rest of the step before).  A particle past the
 // rebuild trigger schedules a rebuild for the step after this one; one past
 // half the skin fails the run (its step may have missed pairs).
 int nl_poll(sphg_ctx* c)
 {
     const int s = ++c->nl_seq, slot = s & 1, o = slot ^ 1;
-    HIPCHK(c, hipMemcpyAsync(&c->h_nlflag[slot], c->d_nlflag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipEventRecord(c->ev_nl[slot], c->stream));
+    c->post = FlagPost{c->d_nlflag, &c->h_nlflag[slot], s};
     c->h_nlstep[slot] = s;
     if (c->h_nlstep[o] != s - 1) return SPHG_OK;
-    HIPCHK(c, hipEventSynchronize(c->ev_nl[o]));
-    const int f = c->h_nlflag[o];
+    int f = 0;
+    RC(await_post(c, &c->h_nlflag[o], s - 1, &f));
     c->h_nlstep[o] = -1;
     if (f & 2) return check_flags(c);
     if ((f & 1) && s - 1 >= c->nl_rebuilt_at) {
@@ -1782,9 +1822,7 @@ int sphg_create(const sphg_params* params, sphg_ctx** out)
         hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->ev_wx, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->ev_sx, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->ev_nl[0], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->ev_nl[1], hipEventDisableTiming) != hipSuccess ||
-        hipHostMalloc((void**)&c->h_nlflag, 2 * sizeof(int), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void**)&c->h_nlflag, 2 * sizeof(int), hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess ||
         hipMalloc(&c->d_err, sizeof(int) * 4) != hipSuccess) {
         delete c;
         return SPHG_ERR_HIP;
@@ -1818,8 +1856,6 @@ void sphg_destroy(sphg_ctx* c)
     if (c->ev_join) hipEventDestroy(c->ev_join);
     if (c->ev_wx) hipEventDestroy(c->ev_wx);
     if (c->ev_sx) hipEventDestroy(c->ev_sx);
-    for (hipEvent_t e : c->ev_nl)
-        if (e) hipEventDestroy(e);
     if (c->h_nlflag) hipHostFree(c->h_nlflag);
     if (c->stream) hipStreamDestroy(c->stream);
     delete c;
@@ -2236,11 +2272,12 @@ struct sphg_gnn {
     // result, 2 the state a judge starts from
     StateCopy snap[3][2];
     int64_t snap_rebuilds[3] = {-1, -1, -1};   // list rebuilds when each slot was taken
-    // lagged sanity check of the learned advances: device flag, its pinned
-    // copies (two slots) and their events; gain fit sums
+    // lagged sanity check of the learned advances: device flag, the pinned
+    // slots it is posted to; gain fit sums
     int* broken = nullptr;
     int* h_broken = nullptr;
-    hipEvent_t ev_ok[2] = {nullptr, nullptr};
+    int sane_seq = 0;               // its posts issued
+    int sane_at[2] = {0, 0};        // the number of the post in each slot
     double* fit = nullptr;
 };
 
@@ -2463,10 +2500,8 @@ int sphg_gnn_create(sphg_ctx* c, int ksteps, int max_samples, uint64_t seed, sph
     if (max_samples > 0 &&
         (rc = galloc(g, &g->part, (size_t)gnn::TRAIN_GROUPS * (gnn::NPART / 4))))
         return fail(rc);
-    // events and pinned slots of the lagged sanity check
-    if (hipEventCreateWithFlags(&g->ev_ok[0], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&g->ev_ok[1], hipEventDisableTiming) != hipSuccess ||
-        hipHostMalloc((void**)&g->h_broken, 2 * sizeof(int), hipHostMallocDefault) != hipSuccess)
+    // pinned slots of the lagged sanity check
+    if (hipHostMalloc((void**)&g->h_broken, 2 * sizeof(int), hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess)
         return fail(SPHG_ERR_HIP);
     g->h_broken[0] = g->h_broken[1] = 0;
     for (int k = 0; k < 2; ++k) {
@@ -2521,8 +2556,6 @@ void sphg_gnn_destroy(sphg_gnn* g)
 {
     if (!g) return;
     if (g->c) hipStreamSynchronize(g->c->stream);
-    for (hipEvent_t e : g->ev_ok)
-        if (e) hipEventDestroy(e);
     if (g->h_broken) hipHostFree(g->h_broken);
     for (void* p : g->allocs) hipFree(p);
     delete g;
@@ -2682,8 +2715,8 @@ int sphg_gnn_step(sphg_gnn* g, int use_net)
 
 // Sanity test of the state after a learned advance, without a host round
 // trip: k_sanity raises the device flag, k_restore_if then copies the last
-// good state (snapshot 0) back on the device, and the flag is copied to the
-// pinned slot `slot` behind them.  The host reads it one advance later.
+// good state (snapshot 0) back on the device and posts the flag to the pinned
+// slot `slot`.  The host reads it one advance later.
 static int sanity_async(sphg_gnn* g, int slot)
 {
     sphg_ctx* c = g->c;
@@ -2691,6 +2724,8 @@ static int sanity_async(sphg_gnn* g, int slot)
     const int nb0 = nblk(c->ph[0].n), nb1 = nblk(c->ph[1].n);
     auto check = [&](int k) { return args_of(gnn::k_sanity, c->ph[k].d, c->g, g->broken); };
     RC(launch_pair<BodySanity>(c, "sanity", nb0, check(0), nb1, check(1)));
+    const FlagPost post{g->broken, &g->h_broken[slot], ++g->sane_seq};
+    g->sane_at[slot] = g->sane_seq;
     auto restore = [&](int k) {
         PhaseBuf& b = c->ph[k];
         StateCopy& sc = g->snap[0][k];
@@ -2702,12 +2737,9 @@ static int sanity_async(sphg_gnn* g, int slot)
         for (int i = 0; i < N_STATE_FIELDS; ++i) { A.sd[i] = sc.f[i]; A.dd[i] = *f[i]; }
         A.si[0] = sc.id; A.si[1] = sc.itype; A.si[2] = sc.fail;
         A.di[0] = b.d.id; A.di[1] = b.d.itype; A.di[2] = b.d.fail;
-        return args_of(gnn::k_restore_if, (const int*)g->broken, A, b.n);
+        return args_of(gnn::k_restore_if, (const int*)g->broken, A, b.n, k == 0 ? post : FlagPost{});
     };
-    RC(launch_pair<BodyRestoreIf>(c, "sanity", nb0, restore(0), nb1, restore(1)));
-    HIPCHK(c, hipMemcpyAsync(&g->h_broken[slot], g->broken, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipEventRecord(g->ev_ok[slot], c->stream));
-    return SPHG_OK;
+    return launch_pair<BodyRestoreIf>(c, "sanity", nb0, restore(0), nb1, restore(1));
 }
 
 int sphg_gnn_rollout(sphg_gnn* g, int nlearned, int judge_every, double tol, int use_net, int* nfallback,
@@ -2742,8 +2774,9 @@ int sphg_gnn_rollout(sphg_gnn* g, int nlearned, int judge_every, double tol, int
     // the sanity flag of the advance before the last (or of the last, at a
     // judge and at the end)
     auto resolve = [&](int slot) -> int {
-        HIPCHK(c, hipEventSynchronize(g->ev_ok[slot]));
-        if (g->h_broken[slot]) return fallback();
+        int f = 0;
+        RC(await_post(c, &g->h_broken[slot], g->sane_at[slot], &f));
+        if (f) return fallback();
         return SPHG_OK;
     };
     // the step's own checks (a particle past half the list skin, or out of
