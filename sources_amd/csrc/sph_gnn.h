@@ -230,8 +230,9 @@ struct GnnArgs {
 // feature half the other slot's operand needs (v_permlane32_swap), so each
 // edge's features are computed once.  The neighbour's row of the next pair and
 // the index of the one after it are in flight meanwhile.
+// s0: the first slot (even); f also gets s.  Returns the largest degree.
 template <class F>
-__device__ __forceinline__ void for_edge_pairs(const Graph& G, int i, F&& f)
+__device__ __forceinline__ int for_edge_pairs(const Graph& G, int i, int s0, F&& f)
 {
     const int h = lane_id() >> 5;
     const bool valid = i < G.n;
@@ -255,10 +256,10 @@ __device__ __forceinline__ void for_edge_pairs(const Graph& G, int i, F&& f)
         }
         return r;
     };
-    int j = nbr(h), jn = nbr(2 + h);
+    int j = nbr(s0 + h), jn = nbr(s0 + 2 + h);
     Row rn = row_of(j);
 #pragma unroll 1
-    for (int s = 0; s < maxdeg; s += 2) {
+    for (int s = s0; s < maxdeg; s += 2) {
         const Row r = rn;
         const bool has = j >= 0;
         j = jn;
@@ -286,8 +287,9 @@ __device__ __forceinline__ void for_edge_pairs(const Graph& G, int i, F&& f)
             o1[q] = h ? y : lo[q];   // slot s: features 0-7 | 8-15
             o2[q] = h ? hi[q] : y;   // slot s + 1
         }
-        f(__builtin_bit_cast(bf16x8, o1), __builtin_bit_cast(bf16x8, o2));
+        f(__builtin_bit_cast(bf16x8, o1), __builtin_bit_cast(bf16x8, o2), s);
     }
+    return maxdeg;
 }
 
 // Forward pass of node i in node form, weights through w(entry) and biases
@@ -297,6 +299,7 @@ struct Layers {
     Op2 hs;      // summed edge layer / 16
     Op2 h3[2], h4[2];
     f32x16 y;    // outputs 0-3 in elements 0-3 of the lower half-wave, no bias
+    int maxdeg;  // largest degree of the tile
 };
 
 // relu(z + bias) in node form; bias: the tile's 32 values
@@ -314,14 +317,18 @@ __device__ __forceinline__ Op2 relu_bias(f32x16 z, const float* bias)
     return round_node(z);
 }
 
+// keep(o, s): sees the edge operand of each slot.
+template <class K>
 __device__ __forceinline__ Layers forward_tile(const Graph& G, const float* inv_out, const bf16x8* Wp, const float* b3,
-                                               const float* b4, int i)
+                                               const float* b4, int i, K&& keep)
 {
     const int l = lane_id(), h = l >> 5;
     Layers L;
     const bf16x8 w1 = Wp[P_W1 + l];
     f32x16 t = zero16();
-    for_edge_pairs(G, i, [&](const bf16x8& o1, const bf16x8& o2) {
+    L.maxdeg = for_edge_pairs(G, i, 0, [&](const bf16x8& o1, const bf16x8& o2, int s) {
+        keep(o1, s);
+        keep(o2, s + 1);
         const f32x16 za = mfma(w1, o1, zero16()), zb = mfma(w1, o2, zero16());
 #pragma unroll
         for (int v = 0; v < 16; ++v) t[v] += fmaxf(za[v], 0.0f);
@@ -373,7 +380,7 @@ __global__ __launch_bounds__(256, 4) void k_gnn(GnnArgs A)
     const int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (tile * 32 >= A.G.n) return;
     const int i = tile * 32 + (lane_id() & 31);
-    const Layers L = forward_tile(A.G, A.inv_out, A.Wp, A.W + O_B3, A.W + O_B4, i);
+    const Layers L = forward_tile(A.G, A.inv_out, A.Wp, A.W + O_B3, A.W + O_B4, i, [](const bf16x8&, int) {});
     if (lane_id() < 32 && i < A.G.n) {
         const float* b5 = A.W + O_B5;
         reinterpret_cast<float4*>(A.out)[i] =
@@ -388,10 +395,16 @@ __global__ __launch_bounds__(256, 4) void k_gnn(GnnArgs A)
 // earlier form was one atomic per parameter and 32 nodes (23 million of them on
 // 12 thousand addresses at 63k nodes), operands gathered from FP32 weights and
 // a barrier per neighbour slot: 12 iterations on 63k nodes with the fit of the
-// gains 2.64 ms, now 0.93 (58 us per launch of this kernel).  The sums have a
-// fixed order: the same call gives the same weights.
+// gains 2.64 ms, now 0.87 (52 us per launch of this kernel; 58 when the backward
+// pass gathered its edges again).  The sums have a fixed order: the same call
+// gives the same weights.
 constexpr int TRAIN_WAVES = 4;      // wavefronts per workgroup
 constexpr int TRAIN_GROUPS = 256;   // most workgroups: one per CU
+// Neighbour slots whose edge operands a wavefront keeps in LDS for its backward
+// pass (a lattice at h = 1.2 dx has 20 neighbours; slots past these are built
+// again): with the weights 152 KB of the CU's 160.
+constexpr int EDGE_SLOTS = 28;
+static_assert(EDGE_SLOTS % 2 == 0 && EDGE_SLOTS * 64 >= 512, "pairs of slots; room for the sums");
 // gradient tiles of a workgroup, in accumulator layout (element
 // (v >> 2) * 256 + lane * 4 + (v & 3)): W1, W2, W3 (2 x 2), W4 (2 x 2), W5
 // transposed (rows 0-3: outputs x features 0-31, rows 8-11: x features 32-63),
@@ -402,7 +415,9 @@ __global__ __launch_bounds__(64 * TRAIN_WAVES) void k_gnn_train(GnnArgs A)
 {
     __shared__ bf16x8 Wl[NPACK];
     __shared__ __align__(16) float bias[2 * D + NO];
-    __shared__ float4 red[TRAIN_WAVES][512];
+    // edge operands of the wavefronts' tiles, then the sums of the wavefronts
+    __shared__ bf16x8 edges[TRAIN_WAVES][EDGE_SLOTS * 64];
+    float4* red = reinterpret_cast<float4*>(edges);   // [TRAIN_WAVES][512]
     const int l = lane_id(), c = l & 31, h = l >> 5, wave = threadIdx.x >> 6;
     for (int e = threadIdx.x; e < NPACK; e += blockDim.x) Wl[e] = A.Wp[e];
     for (int e = threadIdx.x; e < 2 * D + NO; e += blockDim.x)
@@ -451,7 +466,9 @@ __global__ __launch_bounds__(64 * TRAIN_WAVES) void k_gnn_train(GnnArgs A)
     for (int tile = t0 + wave; tile < t1; tile += TRAIN_WAVES) {
         keep_order();   // (the weights are read from LDS again, not held in registers)
         const int i = tile * 32 + c;
-        const Layers L = forward_tile(A.G, A.inv_out, Wl, bias, bias + D, i);
+        const Layers L = forward_tile(A.G, A.inv_out, Wl, bias, bias + D, i, [&](const bf16x8& o, int s) {
+            if (s < EDGE_SLOTS) edges[wave][s * 64 + l] = o;
+        });
         // ---- loss and dL/dy (lower half-wave: outputs of node i)
         bf16x8 dy;
 #pragma unroll
@@ -538,10 +555,18 @@ __global__ __launch_bounds__(64 * TRAIN_WAVES) void k_gnn_train(GnnArgs A)
             for (int v = 0; v < 16; ++v) z[v] = z[v] > 0.0f ? dh[v] : 0.0f;
             outer(g1, ef, round_feat(z));
         };
-        for_edge_pairs(A.G, i, [&](const bf16x8& o1, const bf16x8& o2) {
+        // (the slot past an odd degree holds zeros)
+#pragma unroll 1
+        for (int s = 0; s < min(L.maxdeg, EDGE_SLOTS); s += 2) {
+            const bf16x8 o1 = edges[wave][s * 64 + l], o2 = edges[wave][(s + 1) * 64 + l];
             edge(o1);
             edge(o2);
-        });
+        }
+        if (L.maxdeg > EDGE_SLOTS)
+            for_edge_pairs(A.G, i, EDGE_SLOTS, [&](const bf16x8& o1, const bf16x8& o2, int) {
+                edge(o1);
+                edge(o2);
+            });
     }
     // single values: over the halves, outputs and loss over the wavefront
 #pragma unroll
@@ -555,20 +580,21 @@ __global__ __launch_bounds__(64 * TRAIN_WAVES) void k_gnn_train(GnnArgs A)
         gs[v] = s;
     }
     float4* out = A.part + (size_t)blockIdx.x * (NPART / 4);
+    __syncthreads();   // (red: the edge operands are done)
 #pragma unroll
     for (int ch = 0; ch < 6; ++ch) {
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
             const f32x16& a = acc[2 * ch + (q >> 2)];
             const int v = 4 * (q & 3);
-            red[wave][q * 64 + l] = make_float4(a[v], a[v + 1], a[v + 2], a[v + 3]);
+            red[wave * 512 + q * 64 + l] = make_float4(a[v], a[v + 1], a[v + 2], a[v + 3]);
         }
         __syncthreads();
         for (int e = threadIdx.x; e < 512; e += blockDim.x) {
-            float4 s = red[0][e];
+            float4 s = red[e];
 #pragma unroll
             for (int w = 1; w < TRAIN_WAVES; ++w) {
-                const float4 a = red[w][e];
+                const float4 a = red[w * 512 + e];
                 s.x += a.x; s.y += a.y; s.z += a.z; s.w += a.w;
             }
             out[ch * 512 + e] = s;
