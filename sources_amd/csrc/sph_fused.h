@@ -1740,7 +1740,7 @@ __device__ __forceinline__ void post_flag(const FlagPost& p, int blk)
 {
     if (!p.slot || blk != 0 || threadIdx.x != 0) return;
     const unsigned v = ((unsigned)p.seq << 2) | ((unsigned)*p.flag & 3u);
-    __hip_atomic_store(p.slot, (int)v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(p.slot, (int)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);   // (the word alone)
 }
 
 __global__ void k_post_flag(FlagPost p) { post_flag(p, blockIdx.x); }

@@ -264,18 +264,18 @@ __device__ __forceinline__ CatMask cand_mask_f(const LaneRows& L, const Masks& M
 // uniform smoothing lengths (the host passes no index lists otherwise) the
 // workgroup's window of FP32 records is in LDS, and every lane goes through
 // its listed candidates there; those outside the support count nothing.  Else
-// (or where the window does not fit) the first lane of each particle goes
-// through its partner mask, reading the records from global memory.
+// (or where the window does not fit) it goes through its partner mask, reading
+// the records from global memory.
 // Stage 1 was bound by the gathers of the partners' records (1M slope, us per
 // launch: 140 -> 105); stage 2 is bound by its FP32 terms and their sums in
 // FP64, and pays for the candidates in the skin (150 -> 166).  us per step, masks
-// -> windows: slope of 3k 55 -> 46, 33k 57 -> 52, 125k 73 -> 67, 250k 102 -> 100,
-// 1M 419 -> 400; column of 64k 60 -> 50, 400k 131 -> 122.
+// -> windows: slope of 3k 56 -> 42, 33k 57 -> 46, 64k 61 -> 52, 1M 419 -> 400;
+// column of 33k 56 -> 43, 64k 60 -> 47 (below 1M 5 of these from the posted flag).
 // body(v, lim): record chunks v and the squared distance it has yet to be within;
 // mask(R): the partner mask over the rows R = rows().
 template <int NCH, class L, class M, class A, class B>
 __device__ __forceinline__ void visit_mx(unsigned char* lds, const Window& w, const IdxList& I, int n,
-                                         const SubCtx& sc, int lg, int self, const RecQ& rec, float thr, L&& rows,
+                                         const SubCtx& sc, int self, const RecQ& rec, float thr, L&& rows,
                                          M&& mask, A&& accept, B&& body)
 {
     auto global = [&](int k) {
@@ -285,20 +285,25 @@ __device__ __forceinline__ void visit_mx(unsigned char* lds, const Window& w, co
         body(v, INFINITY);
     };
     if (w.lds) {
-        visit_window<NCH, float4>(lds, w, I, n, sc, lg, [&](const auto& v) { body(v, thr); });
-        if (w.cnt < 0 && sc.valid && sc.sub == 0) {   // a list that overflowed
+        visit_window<NCH, float4>(lds, w, I, n, sc, 0, [&](const auto& v) { body(v, thr); });
+        if (w.cnt < 0 && sc.valid) {   // a list that overflowed
             const LaneRows R = rows();
             visit_f(CatMask{0, 0, 7}, R, self, [&](int k) { return accept(rec(k, 0)); }, global);
         }
         return;
     }
-    if (!sc.valid || sc.sub) return;
+    if (!sc.valid) return;
     const LaneRows R = rows();
     visit_f(mask(R), R, self, [&](int k) { return accept(rec(k, 0)); }, global);
 }
 
-// Lanes of a workgroup that take particles: the windows' with index lists.
-__host__ __device__ __forceinline__ int mx_lanes(const NList& NL) { return NL.is.li ? WIN_LANES : STAGE_BLOCK; }
+// Particles of a workgroup, one lane each: those of its window with index lists.
+// (The FP64 stages give a particle of a small phase two or four lanes; here that
+// would change the order of the sums, and a trajectory in FP32 terms with it.)
+__host__ __device__ __forceinline__ int mx_lanes(const NList& NL)
+{
+    return NL.is.li ? WIN_LANES >> NL.lg : STAGE_BLOCK;
+}
 
 template <int NCH>
 constexpr size_t MX_LDS = sizeof(float4) * NCH * WIN_STRIDE;
@@ -314,7 +319,7 @@ __device__ __forceinline__ void water_a_mx(unsigned char* lds, int blk, DPhase W
                                            int cross)
 {
     const RecQ QWv = recqv(qW, W.n), QSv = recqv(qS, S.n);
-    const SubCtx wc = sub_ctx(W.n, blk, NL.lg, mx_lanes(NL));
+    const SubCtx wc = sub_ctx(W.n, blk, 0, mx_lanes(NL));
     const int t = wc.t;
     auto QA = [&](int c) { return QWv(wc.tt, c); };
     const float4 a0 = QA(0), a1 = QA(1), a2 = QA(2);
@@ -337,8 +342,8 @@ __device__ __forceinline__ void water_a_mx(unsigned char* lds, int blk, DPhase W
             const float cfa = (float)(vofa_d * rhoa_d * (-K.numeric_gravity) / K.s_perm);
             const float irhoa = a2.y;
             const KCf kx = make_kcf(SKF, F.uni_x ? 0.5 * ((double)me.h + (double)QSv(0, 0).w) : (double)me.h);
-            const Window win = open_window<true, 3>(lds, NL.ix, blk, wc, NL.lg, W.n, QSv);
-            visit_mx<3>(lds, win, NL.ix, W.n, wc, NL.lg, -1, QSv, X.thr_x,
+            const Window win = open_window<true, 3>(lds, NL.ix, blk, wc, 0, W.n, QSv);
+            visit_mx<3>(lds, win, NL.ix, W.n, wc, -1, QSv, X.thr_x,
                         [&] { return rows_of_cell(g, S.cell_start, me.cx, me.cy); },
                         [&](const LaneRows& R) { return cand_mask_f(R, NL.cross, W.n, wc.tt, -1, QSv, accx_q); },
                         accx_q, [&](const auto& v, float lim) {
@@ -360,10 +365,8 @@ __device__ __forceinline__ void water_a_mx(unsigned char* lds, int blk, DPhase W
                 dvof_x.add(mb * (dvx * gx + dvy * gy));
                 vof2.add(mb * ww);
             });
-            sub_sum(NL.lg, dg_x.s, dg_y.s, dvof_x.s, vof2.s);
-            cntx = sub_count(NL.lg, cntx);
         }
-        if (!wc.valid || wc.sub) return;
+        if (!wc.valid) return;
         if (cross) {
             W.drgx[a] = dg_x.value();
             W.drgy[a] = dg_y.value();
@@ -378,7 +381,7 @@ __device__ __forceinline__ void water_a_mx(unsigned char* lds, int blk, DPhase W
         sep(me, b0, X.cs, dx, dy);
         return pred_f(uni, X.thr_w, dx * dx + dy * dy, me.h, b0.w, X.scale_k);
     };
-    const Window win = open_window<true, 2>(lds, NL.is, blk, wc, NL.lg, W.n, QWv);
+    const Window win = open_window<true, 2>(lds, NL.is, blk, wc, 0, W.n, QWv);
     const bool real_a = W.itype[a] > 0;
     const float dspp = (float)W.dspp;
     Sum64 con, drd, txx, txy, tyy, avx, avy;
@@ -391,7 +394,7 @@ __device__ __forceinline__ void water_a_mx(unsigned char* lds, int blk, DPhase W
         MW.ovf[t] = cm.ovf;
         return cm;
     };
-    visit_mx<2>(lds, win, NL.is, W.n, wc, NL.lg, t, QWv, X.thr_w,
+    visit_mx<2>(lds, win, NL.is, W.n, wc, t, QWv, X.thr_w,
                 [&] { return rows_of_cell(g, W.cell_start, me.cx, me.cy); }, mask_a, acc_q,
                 [&](const auto& v, float lim) {
         const float4 b0 = v[0], b1 = v[1];   // 1/rho and m/rho recomputed: two chunks per partner
@@ -422,10 +425,7 @@ __device__ __forceinline__ void water_a_mx(unsigned char* lds, int blk, DPhase W
         }
     });
 
-    double repx_d = repx, repy_d = repy;
-    sub_sum(NL.lg, con.s, drd.s, txx.s, txy.s, tyy.s, avx.s, avy.s, repx_d, repy_d);
-    cnt = sub_count(NL.lg, cnt);
-    if (!wc.valid || wc.sub) return;
+    if (!wc.valid) return;
     const double vofa_d = W.vof[a], ha_d = W.hsml[a], ca_d = W.c[a];
     const double mu = K.w_mu;
     const double txx_d = txx.value() * SPH_C23_F, tyy_d = tyy.value() * SPH_C23_F, txy_d = txy.value();
@@ -434,7 +434,7 @@ __device__ __forceinline__ void water_a_mx(unsigned char* lds, int blk, DPhase W
     double avx_d = avx.value(), avy_d = avy.value();
     if (real_a) { avx_d *= K.epsilon; avy_d *= K.epsilon; }
     if (K.average_velocity) { W.avx[a] = avx_d; W.avy[a] = avy_d; }
-    W.repx[a] = repx_d; W.repy[a] = repy_d;
+    W.repx[a] = repx; W.repy[a] = repy;
     if (!cross) W.countiac[a] = cnt;   // (with cross terms: the XM = 2 pass's count)
     W.nsame[a] = cnt;
     // p (q2.w) and the new c (q3.x) come from the pack
@@ -469,7 +469,7 @@ __device__ __forceinline__ void water_b_mx(unsigned char* lds, int blk, DPhase W
                                            Grid g, KParams K, FusedK F, MixK X, int mask)
 {
     const RecQ QWv = recqv(qW, W.n);
-    const SubCtx wc = sub_ctx(W.n, blk, NL.lg, mx_lanes(NL));
+    const SubCtx wc = sub_ctx(W.n, blk, 0, mx_lanes(NL));
     const int t = wc.t;
     auto QA = [&](int c) { return QWv(wc.tt, c); };
     const float4 a0 = QA(0), a1 = QA(1), a2 = QA(2), a3 = QA(3);
@@ -484,11 +484,11 @@ __device__ __forceinline__ void water_b_mx(unsigned char* lds, int blk, DPhase W
         sep(me, b0, X.cs, dx, dy);
         return pred_f(uni, X.thr_w, dx * dx + dy * dy, me.h, b0.w, X.scale_k);
     };
-    const Window win = open_window<true, 4>(lds, NL.is, blk, wc, NL.lg, W.n, QWv);
+    const Window win = open_window<true, 4>(lds, NL.is, blk, wc, 0, W.n, QWv);
     const float et2 = (float)(K.etq * K.etq);
     const float beta = (float)K.beta, alpha = (float)K.alpha;
     Sum64 Px, Py, Sxx, Sxyy, Sxyx, Syy, artx, arty, dvd;
-    visit_mx<4>(lds, win, NL.is, W.n, wc, NL.lg, t, QWv, X.thr_w,
+    visit_mx<4>(lds, win, NL.is, W.n, wc, t, QWv, X.thr_w,
                 [&] { return rows_of_cell(g, W.cell_start, me.cx, me.cy); },
                 [&](const LaneRows&) { return mask_of(MW, W.n, t); }, acc_q, [&](const auto& v, float lim) {
         const float4 b0 = v[0], b1 = v[1], b2 = v[2], b3 = v[3];
@@ -520,8 +520,7 @@ __device__ __forceinline__ void water_b_mx(unsigned char* lds, int blk, DPhase W
         arty.add(-(mb * piv * gy));
         dvd.add(mb * (2.0f * (vofa - b2.x) * idr * (dx * gx + dy * gy)) * b2.y);
     });
-    sub_sum(NL.lg, Px.s, Py.s, Sxx.s, Sxyy.s, Sxyx.s, Syy.s, artx.s, arty.s, dvd.s);
-    if (!wc.valid || wc.sub) return;
+    if (!wc.valid) return;
     const double vofa_d = W.vof[a], rhoa_d = W.rho[a], ha_d = W.hsml[a], ca_d = W.c[a];   // new c
     double ax = -(vofa_d * Px.value()) + Sxx.value() + Sxyy.value();
     double ay = -(vofa_d * Py.value()) + Sxyx.value() + Syy.value();
@@ -566,7 +565,7 @@ __device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S
                                            int mask)
 {
     const RecQ QSv = recqv(qS, S.n), QWv = recqv(qW, W.n);
-    const SubCtx wc = sub_ctx(S.n, blk, NL.lg, mx_lanes(NL));
+    const SubCtx wc = sub_ctx(S.n, blk, 0, mx_lanes(NL));
     const int t = wc.t;
     auto QA = [&](int c) { return QSv(wc.tt, c); };
     const float4 a0 = QA(0), a1 = QA(1), a2 = QA(2), a3 = QA(3);
@@ -595,8 +594,8 @@ __device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S
         };
         const float cfs = (float)(vofa_d * (-K.numeric_gravity) / K.s_perm);
         const KCf kx = make_kcf(SKF, F.uni_x ? 0.5 * ((double)QWv(0, 0).w + (double)me.h) : (double)me.h);
-        const Window win = open_window<true, 3>(lds, NL.ix, blk, wc, NL.lg, S.n, QWv);
-        visit_mx<3>(lds, win, NL.ix, S.n, wc, NL.lg, -1, QWv, X.thr_x,
+        const Window win = open_window<true, 3>(lds, NL.ix, blk, wc, 0, S.n, QWv);
+        visit_mx<3>(lds, win, NL.ix, S.n, wc, -1, QWv, X.thr_x,
                     [&] { return rows_of_cell(g, W.cell_start, me.cx, me.cy); },
                     [&](const LaneRows& R) { return cand_mask_f(R, NL.cross, S.n, wc.tt, -1, QWv, accx_q); }, accx_q,
                     [&](const auto& v, float lim) {
@@ -620,12 +619,10 @@ __device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S
             po_x.add(mprr * gx);
             po_y.add(mprr * gy);
         });
-        sub_sum(NL.lg, dg_x.s, dg_y.s, po_x.s, po_y.s);
-        cntx = sub_count(NL.lg, cntx);
     }
 
     if constexpr (XM == 2) {
-        if (!wc.valid || wc.sub) return;
+        if (!wc.valid) return;
         if (cross) {
             S.drgx[a] = dg_x.value();
             S.drgy[a] = dg_y.value();
@@ -641,14 +638,14 @@ __device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S
         sep(me, b0, X.cs, dx, dy);
         return pred_f(uni, X.thr_s, dx * dx + dy * dy, me.h, b0.w, X.scale_k);
     };
-    const Window win = open_window<true, 4>(lds, NL.is, blk, wc, NL.lg, S.n, QSv);
+    const Window win = open_window<true, 4>(lds, NL.is, blk, wc, 0, S.n, QSv);
     const float et2 = (float)(K.etq * K.etq);
     const float beta = (float)K.beta, alpha = (float)K.alpha;
     Sum64 con, drd, txx, txy, tyy, vcc, wxy, avx, avy;
     Sum64 Fx, Fy, artx, arty, dP, dXX, dXY, dYY;
     float repx = 0.0f, repy = 0.0f;
     int cnt = 0;
-    visit_mx<4>(lds, win, NL.is, S.n, wc, NL.lg, t, QSv, X.thr_s,
+    visit_mx<4>(lds, win, NL.is, S.n, wc, t, QSv, X.thr_s,
                 [&] { return rows_of_cell(g, S.cell_start, me.cx, me.cy); },
                 [&](const LaneRows& R) { return cand_mask_f(R, NL.same, S.n, wc.tt, t, QSv, acc_q); }, acc_q,
                 [&](const auto& v, float lim) {
@@ -704,11 +701,7 @@ __device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S
         dXY.add(hh * (sxya - b3.z));
         dYY.add(hh * (syya - b3.w));
     });
-    double repx_d = repx, repy_d = repy;
-    sub_sum(NL.lg, con.s, drd.s, txx.s, txy.s, tyy.s, vcc.s, wxy.s, avx.s, avy.s, repx_d, repy_d);
-    sub_sum(NL.lg, Fx.s, Fy.s, artx.s, arty.s, dP.s, dXX.s, dXY.s, dYY.s);
-    cnt = sub_count(NL.lg, cnt);
-    if (!wc.valid || wc.sub) return;
+    if (!wc.valid) return;
     const double ha_d = S.hsml[a], ca_d = S.c[a], rhoa_d = S.rho[a];
     const double txx_d = txx.value() * SPH_C23_F, tyy_d = tyy.value() * SPH_C23_F, txy_d = txy.value();
     const double vcc_d = vcc.value(), wxy_d = wxy.value() * 0.5;
@@ -717,7 +710,7 @@ __device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S
     double avx_d = avx.value(), avy_d = avy.value();
     if (real_a) { avx_d *= K.epsilon; avy_d *= K.epsilon; }
     if (K.average_velocity) { S.avx[a] = avx_d; S.avy[a] = avy_d; }
-    S.repx[a] = repx_d; S.repy[a] = repy_d;
+    S.repx[a] = repx; S.repy[a] = repy;
     // the cross terms the XM = 2 pass stored
     const double dgx_d = cross ? S.drgx[a] : 0.0, dgy_d = cross ? S.drgy[a] : 0.0;
     const double pox_d = cross ? S.porx[a] : 0.0, poy_d = cross ? S.pory[a] : 0.0;
@@ -759,8 +752,8 @@ __device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S
     double ay = Fy.value() * rhoa_d;
     if (rhoa_d > 0.0) { ax = ax / rhoa_d; ay = ay / rhoa_d; }
     if (mask & M_ART) { ax = ax + artx.value(); ay = ay + arty.value(); }
-    ax = ax + repx_d;
-    ay = ay + repy_d;
+    ax = ax + (double)repx;
+    ay = ay + (double)repy;
     ay = ay + K.gravity;
     if (mask & M_CROSS) {
         ax = ax + dgx_d; ay = ay + dgy_d;

@@ -1340,15 +1340,11 @@ int stages_mixed(sphg_ctx* c, const FinalArgs* fin)
     NList nW = nlist_of(c, W, nl);
     NList nS = nlist_of(c, S, nl);
     if (!(c->F.uni_w && c->F.uni_s && c->F.uni_x) || c->P.nnps == 2) {
-        // the windows' predicate is a distance alone: masks and one lane per
-        // particle over the whole workgroup (the windows' 192 of 256 lanes
-        // would leave a quarter of them idle for nothing)
-        for (NList* L : {&nW, &nS}) {
-            L->is = L->ix = IdxList{};
-            L->lg = 0;
-        }
+        // the windows' predicate is a distance alone: masks, and particles on
+        // all lanes of a workgroup (not the windows' 192 of 256)
+        for (NList* L : {&nW, &nS}) L->is = L->ix = IdxList{};
     }
-    const int nbW = nblk(W.n, mx_lanes(nW) >> nW.lg), nbS = nblk(S.n, mx_lanes(nS) >> nS.lg);
+    const int nbW = nblk(W.n, mx_lanes(nW)), nbS = nblk(S.n, mx_lanes(nS));
     const Grid& gW = nl ? c->gvl[0] : c->gl[0];
     const Grid& gS = nl ? c->gvl[1] : c->gl[1];
     MixK X = c->X;
