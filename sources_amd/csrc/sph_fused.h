@@ -755,28 +755,6 @@ __device__ __forceinline__ SubCtx sub_ctx(int n, int blk, int lg, int lanes)
     return c;
 }
 
-// Wave-level set-up of the mixed-precision stage kernels.
-struct WaveCtx {
-    int lane, t, tt, last;
-    bool valid;
-};
-
-// blk: the workgroup's block of the phase (the XCD-aware block of a solo
-// launch, the tile's block of a batched one).
-__device__ __forceinline__ WaveCtx wave_ctx(int n, int blk)
-{
-    WaveCtx c;
-    c.lane = threadIdx.x & 63;
-    const int t0 = (blk * SPHG_WPB + (int)(threadIdx.x >> 6)) * 64;
-    c.t = t0 + c.lane;
-    c.valid = c.t < n;
-    c.last = min(63, n - 1 - t0);
-    c.tt = c.valid ? c.t : n - 1;
-    return c;
-}
-
-__device__ __forceinline__ WaveCtx wave_ctx(int n) { return wave_ctx(n, xcd_block()); }
-
 __device__ __forceinline__ CatMask mask_of(const Masks& M, int n, int t)
 {
     CatMask c;
