@@ -7,8 +7,9 @@
 //             chunks (16 bytes): 0 x,y | 1 vx,vy | 2 rho,V | 3 vof,p (soil:
 //             vof/rho,p) | 4 s3,c | 5 s1,s2 | 6 h,itype; V = m/rho carries the
 //             sign of itype (negative for virtual particles), so the pair
-//             terms need no reciprocal of the partner's density.  The loops
-//             load only the chunks they use;
+//             terms need no reciprocal of the partner's density (a step of a
+//             learned run has m and the soil's vof instead, sph_learned.h).
+//             The loops load only the chunks they use;
 //   stage A   the same-phase terms that need only the packed values;
 //   stage B   (water) the terms that need the partners' strain rates.  Soil
 //             stage B needs nothing from the stage A of other soil particles,
@@ -382,7 +383,8 @@ __device__ __forceinline__ void pack_water_at(const DPhase& P, const KParams& K,
     R[0 * pn] = make_double2(x, y);
     R[1 * pn] = make_double2(vx, vy);
     const double V = m * irho;
-    R[2 * pn] = make_double2(rho, it < 0 ? -V : V);   // the sign of V marks a virtual particle
+    const double mv = K.learned ? m : V;
+    R[2 * pn] = make_double2(rho, it < 0 ? -mv : mv);   // the sign marks a virtual particle
     R[3 * pn] = make_double2(vof, p);
     R[4 * pn] = make_double2(0.0, cn);
     // (h and itype stay between list rebuilds, in the same slot: a lean pack
@@ -516,8 +518,9 @@ __device__ __forceinline__ void pack_soil_at(const DPhase& P, const KParams& K, 
     R[0 * pn] = make_double2(x, y);
     R[1 * pn] = make_double2(vx, vy);
     const double V = m * irho;
-    R[2 * pn] = make_double2(rho, it < 0 ? -V : V);   // the sign of V marks a virtual particle
-    R[3 * pn] = make_double2(P.vof[i] * irho, p);
+    const double mv = K.learned ? m : V, vof = P.vof[i];
+    R[2 * pn] = make_double2(rho, it < 0 ? -mv : mv);   // the sign marks a virtual particle
+    R[3 * pn] = make_double2(K.learned ? vof : vof * irho, p);
     R[4 * pn] = make_double2(syy, P.c[i]);
     R[5 * pn] = make_double2(sxx, sxy);
     if (!lean) R[6 * pn] = make_double2(P.hsml[i], (double)it);   // (as for water)
@@ -742,6 +745,13 @@ struct SubCtx {
     int t, tt, sub;
     bool valid;
 };
+
+// Particles of a workgroup whose kernel gives each one lane: those of its window
+// with index lists.
+__host__ __device__ __forceinline__ int lanes_of_one(const NList& NL)
+{
+    return NL.is.li ? WIN_LANES >> NL.lg : STAGE_BLOCK;
+}
 
 // lanes: lanes of the workgroup that take particles (a multiple of 2^lg).
 __device__ __forceinline__ SubCtx sub_ctx(int n, int blk, int lg, int lanes)
@@ -1451,6 +1461,68 @@ __global__ STAGE_ATTR void k_water_b4(DPhase W, const double* recW, NList NL, Gr
     water_b4<SKF, U>(lds, xcd_block(), W, recW, NL, g, K, F, mask);
 }
 
+// Stress and pressure rates of soil particle a from its strain rate t, divergence
+// and spin: plastic_or_not + plastic_flow_rule3 + Jaumann_rate (and the
+// accumulated plastic strain).
+struct StressRates {
+    double xx, xy, yy, p;
+};
+
+__device__ __forceinline__ StressRates stress_rates(const DPhase& S, const KParams& K, int a, double txx, double txy,
+                                                    double tyy, double vcc, double wxy, double pa, double sxxa,
+                                                    double sxya, double syya)
+{
+    const double alpha = K.s_alpha1, G = K.s_G, Kb = K.s_k;
+    double dsxx = 0.0, dsxy = 0.0, dsyy = 0.0, dpv = 0.0;
+    // plasticity 3: plastic_or_not + plastic_flow_rule3 (failed points);
+    // plasticity 1: plastic_flow_rule (m_particles.f90:3571-3633), the same
+    // correction at every point, with the criterion's fail flags left as they are
+    if (K.plasticity == 3 || K.plasticity == 1) {
+        const double I1 = 3.0 * pa;
+        const double j2r = sxxa * sxxa + 2.0 * (sxya * sxya) + syya * syya + (sxxa + syya) * (sxxa + syya);
+        const double J2 = __builtin_sqrt(j2r / 2.0) + 1.0e-6;
+        const int fail = fabs(J2 - alpha * I1) < SPH_YIELD_TOL_F ? 1 : 0;
+        if (fail || K.plasticity == 1) {
+            const double exx = txx * 0.5 + vcc * (1.0 / 3.0);
+            const double exy = txy * 0.5;
+            const double eyy = tyy * 0.5 + vcc * (1.0 / 3.0);
+            const double sde = sxxa * exx + 2.0 * sxya * exy + syya * eyy;
+            const double sj = __builtin_sqrt(j2r / 2.0 + 1.0e-10);
+            const double gs = G / sj;
+            const double dl = (3.0 * alpha * Kb * vcc + gs * sde) / (9.0 * (alpha * alpha) * Kb + G);
+            if (!(dl < 0.0)) {
+                dsxx = -dl * (gs * sxxa);
+                dsxy = -dl * (gs * sxya);
+                dsyy = -dl * (gs * syya);
+                dpv = 3.0 * Kb * alpha * dl;
+                S.eps_p[a] = S.eps_p[a] + dl * sxya / (2.0 * sj) * SPH_EPSP_F;
+            }
+        }
+        if (K.plasticity == 3) S.fail[a] = fail;
+    }
+    if (K.plasticity == 2) {
+        // plastic_flow_rule2 (m_particles.f90:3636-3697): at every point and
+        // without the sign test; its rates act in the return mapping
+        const double j2r = sxxa * sxxa + 2.0 * (sxya * sxya) + syya * syya + (sxxa + syya) * (sxxa + syya);
+        const double exx = txx * 0.5 + vcc * (1.0 / 3.0);
+        const double exy = txy * 0.5;
+        const double eyy = tyy * 0.5 + vcc * (1.0 / 3.0);
+        const double sde = sxxa * exx + 2.0 * sxya * exy + syya * eyy;
+        const double sj = __builtin_sqrt(j2r / 2.0 + 1.0e-10);
+        const double gs = G / sj;
+        const double dl = (3.0 * alpha * Kb * vcc + gs * sde) / (9.0 * (alpha * alpha) * Kb + G);
+        S.dsxx2[a] = -dl * (gs * sxxa);
+        S.dsxy2[a] = -dl * (gs * sxya);
+        S.dsyy2[a] = -dl * (gs * syya);
+        S.dp2[a] = 3.0 * Kb * alpha * dl;
+    }
+    dsxx = dsxx + G * txx + 2.0 * sxya * wxy;
+    dsxy = dsxy + G * txy - (sxxa - syya) * wxy;
+    dsyy = dsyy + G * tyy - 2.0 * sxya * wxy;
+    dpv = dpv - Kb * vcc;
+    return StressRates{dsxx, dsxy, dsyy, dpv};
+}
+
 // ------------------------------------------------------------------------
 // Soil, stages A and B in one kernel (SOLO: single-phase soil,
 // single_step_for_soil, declarations_sph.f90:1530-1655: the df form of the
@@ -1611,54 +1683,7 @@ __device__ __forceinline__ void soil_ab4(unsigned char* lds, int blk, DPhase S, 
     }
     S.c_next[a] = cn;
 
-    const double alpha = K.s_alpha1, G = K.s_G, Kb = K.s_k;
-    double dsxx = 0.0, dsxy = 0.0, dsyy = 0.0, dpv = 0.0;
-    // plasticity 3: plastic_or_not + plastic_flow_rule3 (failed points);
-    // plasticity 1: plastic_flow_rule (m_particles.f90:3571-3633), the same
-    // correction at every point, with the criterion's fail flags left as they are
-    if (K.plasticity == 3 || K.plasticity == 1) {
-        const double I1 = 3.0 * pa;
-        const double j2r = sxxa * sxxa + 2.0 * (sxya * sxya) + syya * syya + (sxxa + syya) * (sxxa + syya);
-        const double J2 = __builtin_sqrt(j2r / 2.0) + 1.0e-6;
-        const int fail = fabs(J2 - alpha * I1) < SPH_YIELD_TOL_F ? 1 : 0;
-        if (fail || K.plasticity == 1) {
-            const double exx = txx * 0.5 + vcc * (1.0 / 3.0);
-            const double exy = txy * 0.5;
-            const double eyy = tyy * 0.5 + vcc * (1.0 / 3.0);
-            const double sde = sxxa * exx + 2.0 * sxya * exy + syya * eyy;
-            const double sj = __builtin_sqrt(j2r / 2.0 + 1.0e-10);
-            const double gs = G / sj;
-            const double dl = (3.0 * alpha * Kb * vcc + gs * sde) / (9.0 * (alpha * alpha) * Kb + G);
-            if (!(dl < 0.0)) {
-                dsxx = -dl * (gs * sxxa);
-                dsxy = -dl * (gs * sxya);
-                dsyy = -dl * (gs * syya);
-                dpv = 3.0 * Kb * alpha * dl;
-                S.eps_p[a] = S.eps_p[a] + dl * sxya / (2.0 * sj) * SPH_EPSP_F;
-            }
-        }
-        if (K.plasticity == 3) S.fail[a] = fail;
-    }
-    if (K.plasticity == 2) {
-        // plastic_flow_rule2 (m_particles.f90:3636-3697): at every point and
-        // without the sign test; its rates act in the return mapping
-        const double j2r = sxxa * sxxa + 2.0 * (sxya * sxya) + syya * syya + (sxxa + syya) * (sxxa + syya);
-        const double exx = txx * 0.5 + vcc * (1.0 / 3.0);
-        const double exy = txy * 0.5;
-        const double eyy = tyy * 0.5 + vcc * (1.0 / 3.0);
-        const double sde = sxxa * exx + 2.0 * sxya * exy + syya * eyy;
-        const double sj = __builtin_sqrt(j2r / 2.0 + 1.0e-10);
-        const double gs = G / sj;
-        const double dl = (3.0 * alpha * Kb * vcc + gs * sde) / (9.0 * (alpha * alpha) * Kb + G);
-        S.dsxx2[a] = -dl * (gs * sxxa);
-        S.dsxy2[a] = -dl * (gs * sxya);
-        S.dsyy2[a] = -dl * (gs * syya);
-        S.dp2[a] = 3.0 * Kb * alpha * dl;
-    }
-    dsxx = dsxx + G * txx + 2.0 * sxya * wxy;
-    dsxy = dsxy + G * txy - (sxxa - syya) * wxy;
-    dsyy = dsyy + G * tyy - 2.0 * sxya * wxy;
-    dpv = dpv - Kb * vcc;
+    StressRates d = stress_rates(S, K, a, txx, txy, tyy, vcc, wxy, pa, sxxa, sxya, syya);
 
     double ax = Fx, ay = Fy;
     if (!SOLO) { ax = ax * rhoa; ay = ay * rhoa; }
@@ -1674,12 +1699,12 @@ __device__ __forceinline__ void soil_ab4(unsigned char* lds, int blk, DPhase S, 
     }
     if (mask & M_DELTA_FIELD) {
         const double cf = K.delta * ha * cn * 2.0;
-        dpv = dpv + cf * dP;
-        dsxx = dsxx + cf * dXX;
-        dsxy = dsxy + cf * dXY;
-        dsyy = dsyy + cf * dYY;
+        d.p = d.p + cf * dP;
+        d.xx = d.xx + cf * dXX;
+        d.xy = d.xy + cf * dXY;
+        d.yy = d.yy + cf * dYY;
     }
-    S.dsxx[a] = dsxx; S.dsxy[a] = dsxy; S.dsyy[a] = dsyy; S.dp[a] = dpv;
+    S.dsxx[a] = d.xx; S.dsxy[a] = d.xy; S.dsyy[a] = d.yy; S.dp[a] = d.p;
     S.ax[a] = ax;
     S.ay[a] = ay;
 }

@@ -51,6 +51,7 @@ struct KParams {
     // Mohr-Coulomb criterion (yield_criterion = 1): cohesion cos(phi), sin(phi)
     // and the tension cut-off pressure -cohesion tan(phi)**(-1.0), host-evaluated
     double mc_ccos, mc_sin, mc_pcut;
+    int learned;                // a step of a learned run (sph_learned.h): FP64 records hold m and vof
 };
 
 // Stage masks (granular entry points run a subset of a fused pass).

@@ -297,14 +297,8 @@ __device__ __forceinline__ void visit_mx(unsigned char* lds, const Window& w, co
     visit_f(mask(R), R, self, [&](int k) { return accept(rec(k, 0)); }, global);
 }
 
-// Particles of a workgroup, one lane each: those of its window with index lists.
-// (The FP64 stages give a particle of a small phase two or four lanes; here that
-// would change the order of the sums, and a trajectory in FP32 terms with it.)
-__host__ __device__ __forceinline__ int mx_lanes(const NList& NL)
-{
-    return NL.is.li ? WIN_LANES >> NL.lg : STAGE_BLOCK;
-}
-
+// (One lane per particle at every size: more, as in the FP64 stages of a small
+// phase, would change the order of the sums, and a trajectory in FP32 terms with it.)
 template <int NCH>
 constexpr size_t MX_LDS = sizeof(float4) * NCH * WIN_STRIDE;
 
@@ -319,7 +313,7 @@ __device__ __forceinline__ void water_a_mx(unsigned char* lds, int blk, DPhase W
                                            int cross)
 {
     const RecQ QWv = recqv(qW, W.n), QSv = recqv(qS, S.n);
-    const SubCtx wc = sub_ctx(W.n, blk, 0, mx_lanes(NL));
+    const SubCtx wc = sub_ctx(W.n, blk, 0, lanes_of_one(NL));
     const int t = wc.t;
     auto QA = [&](int c) { return QWv(wc.tt, c); };
     const float4 a0 = QA(0), a1 = QA(1), a2 = QA(2);
@@ -469,7 +463,7 @@ __device__ __forceinline__ void water_b_mx(unsigned char* lds, int blk, DPhase W
                                            Grid g, KParams K, FusedK F, MixK X, int mask)
 {
     const RecQ QWv = recqv(qW, W.n);
-    const SubCtx wc = sub_ctx(W.n, blk, 0, mx_lanes(NL));
+    const SubCtx wc = sub_ctx(W.n, blk, 0, lanes_of_one(NL));
     const int t = wc.t;
     auto QA = [&](int c) { return QWv(wc.tt, c); };
     const float4 a0 = QA(0), a1 = QA(1), a2 = QA(2), a3 = QA(3);
@@ -565,7 +559,7 @@ __device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S
                                            int mask)
 {
     const RecQ QSv = recqv(qS, S.n), QWv = recqv(qW, W.n);
-    const SubCtx wc = sub_ctx(S.n, blk, 0, mx_lanes(NL));
+    const SubCtx wc = sub_ctx(S.n, blk, 0, lanes_of_one(NL));
     const int t = wc.t;
     auto QA = [&](int c) { return QSv(wc.tt, c); };
     const float4 a0 = QA(0), a1 = QA(1), a2 = QA(2), a3 = QA(3);

@@ -18,6 +18,7 @@
 #include "../../include/sphg.h"
 #include "sph_fused.h"
 #include "sph_single.h"
+#include "sph_learned.h"
 #include "sph_mixed.h"
 #include "sph_gnn.h"
 #include "sph_batch.h"
@@ -1160,6 +1161,38 @@ int launch_finals(sphg_ctx* c, const FinalArgs& f)
     return launch(c, "finals", k_finals, pad8(A.nbS) + pad8(A.nbW), TPB, A);
 }
 
+// The stages of a step of a learned run (us, uw, ux: which parts are uniform).
+template <int SKF>
+int stages_learned(sphg_ctx* c, const FinalArgs* fin, bool us, bool uw, bool ux)
+{
+    PhaseBuf& W = c->ph[0];
+    PhaseBuf& S = c->ph[1];
+    const bool nl = nl_mode(c);
+    const NList nW = nlist_of(c, W, nl), nS = nlist_of(c, S, nl);
+    StageArgs A{W.d,  S.d,  W.rec,        S.rec,        nW, nS, nl ? c->gvl[0] : c->gl[0], nl ? c->gvl[1] : c->gl[1],
+                c->K, c->F, mask_b(c, 0), mask_b(c, 1), 0,  nblk(W.n, lanes_of_one(nW)), nblk(S.n, lanes_of_one(nS)),
+                take_post(c)};
+    const bool all = us && uw && ux;
+    if (all) {
+        RC(launch(c, "stage1", learned::k_stage1<SKF>, pad8(A.nbS) + 2 * pad8(A.nbW), STAGE_BLOCK, A));
+    } else {
+        RC(launch(c, "soil_x", ux ? learned::k_part<SKF, 0, true> : learned::k_part<SKF, 0, false>, A.nbS, STAGE_BLOCK, A));
+        RC(launch(c, "water_a", uw ? learned::k_part<SKF, 1, true> : learned::k_part<SKF, 1, false>, A.nbW, STAGE_BLOCK, A));
+        RC(launch(c, "water_x", ux ? learned::k_part<SKF, 2, true> : learned::k_part<SKF, 2, false>, A.nbW, STAGE_BLOCK, A));
+    }
+    swap_c(W);
+    swap_c(S);
+    A.W = W.d;
+    A.S = S.d;
+    if (all) {
+        RC(launch(c, "stage2", learned::k_stage2<SKF>, pad8(A.nbS) + pad8(A.nbW), STAGE_BLOCK, A));
+    } else {
+        RC(launch(c, "soil_ab", us ? learned::k_part<SKF, 3, true> : learned::k_part<SKF, 3, false>, A.nbS, STAGE_BLOCK, A));
+        RC(launch(c, "water_b", uw ? learned::k_part<SKF, 4, true> : learned::k_part<SKF, 4, false>, A.nbW, STAGE_BLOCK, A));
+    }
+    return fin ? launch_finals(c, *fin) : SPHG_OK;
+}
+
 // The fused step: pack (first_half + soil Drucker-Prager projections +
 // records), cross terms, partner masks, stage A, stage B.  The soil kernels
 // read only the packed records of both phases (the water pressure comes from
@@ -1189,6 +1222,7 @@ int stages_fused(sphg_ctx* c, const FinalArgs* fin)
     const bool us = c->ph[1].hmin == c->ph[1].hmax && rep_int && c->K.yield_criterion != 1;
     const bool uw = c->ph[0].hmin == c->ph[0].hmax && rep_int;
     const bool ux = c->F.uni_x != 0;
+    if (c->K.learned) return stages_learned<SKF>(c, fin, us, uw, ux);
     if (us && uw && ux && cross && !c->prof) {
         // three launches on one stream (the profile times the passes apart)
         StageArgs A{W.d,  S.d,  W.rec,        S.rec,        nW,   nS,  gW,  gS,
@@ -1344,7 +1378,7 @@ int stages_mixed(sphg_ctx* c, const FinalArgs* fin)
         // all lanes of a workgroup (not the windows' 192 of 256)
         for (NList* L : {&nW, &nS}) L->is = L->ix = IdxList{};
     }
-    const int nbW = nblk(W.n, mx_lanes(nW)), nbS = nblk(S.n, mx_lanes(nS));
+    const int nbW = nblk(W.n, lanes_of_one(nW)), nbS = nblk(S.n, lanes_of_one(nS));
     const Grid& gW = nl ? c->gvl[0] : c->gl[0];
     const Grid& gS = nl ? c->gvl[1] : c->gl[1];
     MixK X = c->X;
@@ -2364,12 +2398,21 @@ DPhase snap_view(sphg_gnn* g, int slot, int k)
     return d;
 }
 
+// A step of a learned run, in its arithmetic (sph_learned.h).
+int learned_step(sphg_ctx* c)
+{
+    c->K.learned = 1;
+    const int rc = one_step(c);
+    c->K.learned = 0;
+    return rc;
+}
+
 // One leapfrog step of size K dt (the coarse step of a learned advance).
 int coarse_step(sphg_ctx* c, int K)
 {
     const double dt0 = c->K.dt;
     c->K.dt = dt0 * K;
-    const int rc = one_step(c);
+    const int rc = learned_step(c);
     c->K.dt = dt0;
     RC(rc);
     c->itimestep += K - 1;
@@ -2383,7 +2426,7 @@ int plain_steps(sphg_ctx* c, int n)
     const int prec = c->P.precision;
     c->P.precision = SPHG_FP64;
     int rc = SPHG_OK;
-    for (int s = 0; s < n && rc == SPHG_OK; ++s) rc = one_step(c);
+    for (int s = 0; s < n && rc == SPHG_OK; ++s) rc = learned_step(c);
     c->P.precision = prec;
     return rc;
 }
