@@ -1141,8 +1141,9 @@ __device__ __forceinline__ Sep sep_of(const KC& kc, double dx, double dy, double
 // soil partners (direct_find_2's pairs, virtual x virtual and r = 0
 // included).  Its own kernel: the loop needs few registers, so it runs at
 // twice the occupancy of the same-phase stage.
-// lean (all stages): another step of the same call follows, so the values
-// that only a download or the last step's diagnostics would read stay out.
+// lean (all stages): another step of the same call follows and this one does
+// not renormalise (its final update reads vof2), so the values that only a
+// download or the last step's diagnostics would read stay out.
 // ------------------------------------------------------------------------
 template <int SKF, bool U>
 __device__ __forceinline__ void water_x4(unsigned char* lds, int blk, DPhase W, DPhase S, const double* recW, const double* recS,

@@ -1209,8 +1209,8 @@ int stages_fused(sphg_ctx* c, const FinalArgs* fin)
     const double* rS = S.rec;
     const bool nl = nl_mode(c);
     // (the values of a step that another of the same call follows, and that only
-    // a download would read, stay out)
-    const int lean = fin && fin->ahead ? 1 : 0;
+    // a download would read, stay out; the renormalisation reads vof2)
+    const int lean = fin && fin->ahead && !fin->renorm ? 1 : 0;
     const NList nW = nlist_of(c, W, nl);
     const NList nS = nlist_of(c, S, nl);
     const int nbW = nblk(W.n, WIN_LANES >> nW.lg), nbS = nblk(S.n, WIN_LANES >> nS.lg);
