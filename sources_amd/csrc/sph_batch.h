@@ -58,67 +58,67 @@ __global__ __launch_bounds__(256) void k_batched(const ArgTup<T...>* __restrict_
 }
 
 // The device bodies of the kernels a list-mode FP64 step launches.
-template <int SKF, bool U>
+template <int SKF, int FORM>
 struct BodyWaterX {
     template <class... A>
     __device__ __forceinline__ void operator()(int blk, const A&... a) const
     {
-        __shared__ __align__(16) unsigned char lds[VIS_LDS<4>];
-        water_x4<SKF, U>(lds, blk, a...);
+        __shared__ __align__(16) unsigned char lds[STAGE_LDS<FORM, 4>];
+        water_x4<SKF, FORM>(lds, blk, a...);
     }
 };
-template <int SKF, bool U>
+template <int SKF, int FORM>
 struct BodySoilX {
     template <class... A>
     __device__ __forceinline__ void operator()(int blk, const A&... a) const
     {
-        __shared__ __align__(16) unsigned char lds[VIS_LDS<4>];
-        soil_x4<SKF, U>(lds, blk, a...);
+        __shared__ __align__(16) unsigned char lds[STAGE_LDS<FORM, 4>];
+        soil_x4<SKF, FORM>(lds, blk, a...);
     }
 };
-template <int SKF, bool U>
+template <int SKF, int FORM>
 struct BodyWaterA {
     template <class... A>
     __device__ __forceinline__ void operator()(int blk, const A&... a) const
     {
-        __shared__ __align__(16) unsigned char lds[VIS_LDS<3>];
-        water_a4<SKF, U>(lds, blk, a...);
+        __shared__ __align__(16) unsigned char lds[STAGE_LDS<FORM, 3>];
+        water_a4<SKF, FORM>(lds, blk, a...);
     }
 };
-template <int SKF, bool U>
+template <int SKF, int FORM>
 struct BodyWaterB {
     template <class... A>
     __device__ __forceinline__ void operator()(int blk, const A&... a) const
     {
-        __shared__ __align__(16) unsigned char lds[VIS_LDS<6>];
-        water_b4<SKF, U>(lds, blk, a...);
+        __shared__ __align__(16) unsigned char lds[STAGE_LDS<FORM, 6>];
+        water_b4<SKF, FORM>(lds, blk, a...);
     }
 };
-template <int SKF, bool U>
+template <int SKF, int FORM>
 struct BodySoilAB {
     template <class... A>
     __device__ __forceinline__ void operator()(int blk, const A&... a) const
     {
-        __shared__ __align__(16) unsigned char lds[VIS_LDS<6>];
-        soil_ab4<SKF, U, false>(lds, blk, a...);
+        __shared__ __align__(16) unsigned char lds[STAGE_LDS<FORM, 6>];
+        soil_ab4<SKF, FORM, false>(lds, blk, a...);
     }
 };
 // (a tile is a workgroup of the solo launch, padding included)
-template <int SKF>
+template <int SKF, int FS, int FX>
 struct BodyStage1 {
-    __device__ __forceinline__ void operator()(int blk, const StageArgs& a) const { stage1<SKF>(blk, a, false); }
+    __device__ __forceinline__ void operator()(int blk, const StageArgs& a) const { stage1<SKF, FS, FX>(blk, a, false); }
 };
-template <int SKF>
+template <int SKF, int FS>
 struct BodyStage2 {
-    __device__ __forceinline__ void operator()(int blk, const StageArgs& a) const { stage2<SKF>(blk, a, false); }
+    __device__ __forceinline__ void operator()(int blk, const StageArgs& a) const { stage2<SKF, FS>(blk, a, false); }
 };
-template <int SKF>
+template <int SKF, bool WIN>
 struct BodyStage1Mx {
-    __device__ __forceinline__ void operator()(int blk, const StageArgsMx& a) const { stage1_mx<SKF>(blk, a, false); }
+    __device__ __forceinline__ void operator()(int blk, const StageArgsMx& a) const { stage1_mx<SKF, WIN>(blk, a, false); }
 };
-template <int SKF>
+template <int SKF, bool WIN>
 struct BodyStage2Mx {
-    __device__ __forceinline__ void operator()(int blk, const StageArgsMx& a) const { stage2_mx<SKF>(blk, a, false); }
+    __device__ __forceinline__ void operator()(int blk, const StageArgsMx& a) const { stage2_mx<SKF, WIN>(blk, a, false); }
 };
 struct BodyFinals {
     __device__ __forceinline__ void operator()(int blk, const FinalsArgs& a) const { finals(blk, a, false); }
@@ -158,53 +158,6 @@ SPHG_BATCH_BODY(BodyCellRank, cell_rank_body)
 SPHG_BATCH_BODY(BodyPackWater, pack_water_body)
 SPHG_BATCH_BODY(BodyPackSoil, pack_soil_body)
 SPHG_BATCH_BODY(BodyNlist, nlist_body)
-
-// ... and of the mixed-precision stage kernels.
-template <int SKF>
-struct BodyWaterAMx {
-    template <class... A>
-    __device__ __forceinline__ void operator()(int blk, const A&... a) const
-    {
-        __shared__ __align__(16) unsigned char lds[MX_LDS<2>];
-        water_a_mx<SKF, 1>(lds, blk, a...);
-    }
-};
-template <int SKF>
-struct BodyWaterXMx {
-    template <class... A>
-    __device__ __forceinline__ void operator()(int blk, const A&... a) const
-    {
-        __shared__ __align__(16) unsigned char lds[MX_LDS<3>];
-        water_a_mx<SKF, 2>(lds, blk, a...);
-    }
-};
-template <int SKF>
-struct BodyWaterBMx {
-    template <class... A>
-    __device__ __forceinline__ void operator()(int blk, const A&... a) const
-    {
-        __shared__ __align__(16) unsigned char lds[MX_LDS<4>];
-        water_b_mx<SKF>(lds, blk, a...);
-    }
-};
-template <int SKF>
-struct BodySoilABMx {
-    template <class... A>
-    __device__ __forceinline__ void operator()(int blk, const A&... a) const
-    {
-        __shared__ __align__(16) unsigned char lds[MX_LDS<4>];
-        soil_ab_mx<SKF, 1>(lds, blk, a...);
-    }
-};
-template <int SKF>
-struct BodySoilXMx {
-    template <class... A>
-    __device__ __forceinline__ void operator()(int blk, const A&... a) const
-    {
-        __shared__ __align__(16) unsigned char lds[MX_LDS<3>];
-        soil_ab_mx<SKF, 2>(lds, blk, a...);
-    }
-};
 #undef SPHG_BATCH_BODY
 
 // Two argument sets of one body in one launch (the two phases of a context):

@@ -115,6 +115,23 @@ __device__ __forceinline__ KC make_kc(int skf, double h)
     return k;
 }
 
+// The same for the mean smoothing length of one pair: one short reciprocal
+// instead of two divisions (those were a sixth of a stage's time where h varies).
+template <int SKF>
+__device__ __forceinline__ KC pair_kc(double h)
+{
+    constexpr double norm = SKF == 1 ? 15.0 / (7.0 * SPH_PI_F) : SKF == 2 ? 1.0 / SPH_PI_F
+                          : SKF == 3 ? 7.0 / (478.0 * SPH_PI_F) : 7.0 / (4.0 * SPH_PI_F);
+    KC k;
+    k.inv_h = fast_rcp(h);
+    const double ih2 = k.inv_h * k.inv_h;
+    k.f = norm * ih2;
+    k.c1 = SKF == 1 ? 2.0 * (k.f * ih2) : SKF == 2 ? -2.0 * ih2 : k.f * ih2;
+    k.c2 = SKF == 1 ? -0.5 * (k.f * k.inv_h) : SKF == 3 ? k.f * k.inv_h : 0.0;
+    k.c3 = SKF == 1 ? k.f * (1.0 / 6.0) : 0.0;
+    return k;
+}
+
 // W and s (grad W = s (dx, dy); m_particles.f90:1469-1602) of a pair inside
 // the support; inv_r = 1/r.
 template <int SKF, bool NEED_W>
@@ -597,17 +614,19 @@ struct Masks {
 // candidate j of record t is the window's record li[j * n + t], cnt[t] of them
 // (-1: more than cap, the rows are walked).  win: WIN_INTS per workgroup: the
 // first records of the window's three record ranges, their positions in it and
-// its length.  A workgroup holds WIN_LANES >> lg particles.
+// its length.
 struct IdxList {
     unsigned short* li;
     int *cnt, *win;
     int cap, lds;   // lds 0: the windows stay in global memory (predicates that need more than a distance)
+    int pb;         // particles of a workgroup of the kernels that read it
 };
 
 constexpr int WIN_INTS = 8;
 constexpr int WIN_CAP = 846;             // records of a window in LDS: two workgroups' six chunks fill a CU's
 constexpr int WIN_STRIDE = WIN_CAP + 1;  // (and the stand-in record)
-// Lanes of a workgroup that take particles.  The window holds three rows' worth
+// Lanes of a workgroup that take particles where its window is to fit the LDS (all
+// of them otherwise).  The window holds three rows' worth
 // of them: 633 records on average and 848 at most for 192 particles of a
 // lattice at h = 1.2 dx (whose cell rows hold two or three lattice rows); with
 // 240 particles one window in four does not fit, and its workgroup takes the
@@ -748,10 +767,7 @@ struct SubCtx {
 
 // Particles of a workgroup whose kernel gives each one lane: those of its window
 // with index lists.
-__host__ __device__ __forceinline__ int lanes_of_one(const NList& NL)
-{
-    return NL.is.li ? WIN_LANES >> NL.lg : STAGE_BLOCK;
-}
+__host__ __device__ __forceinline__ int lanes_of_one(const IdxList& I) { return I.li ? I.pb : STAGE_BLOCK; }
 
 // lanes: lanes of the workgroup that take particles (a multiple of 2^lg).
 __device__ __forceinline__ SubCtx sub_ctx(int n, int blk, int lg, int lanes)
@@ -763,6 +779,21 @@ __device__ __forceinline__ SubCtx sub_ctx(int n, int blk, int lg, int lanes)
     c.valid = i < lanes && c.t < n;
     c.tt = c.valid ? c.t : n - 1;
     return c;
+}
+
+// Candidate bits of lane sub: every 2^lg-th.
+__device__ __forceinline__ uint64_t sub_bits(int lg, int sub)
+{
+    const uint64_t pat = lg == 0 ? ~0ull : lg == 1 ? 0x5555555555555555ull : lg == 2 ? 0x1111111111111111ull
+                                                                                     : 0x0101010101010101ull;
+    return pat << sub;
+}
+
+__device__ __forceinline__ uint64_t sub_or(int lg, uint64_t v)
+{
+    for (int o = 1; o < (1 << lg); o <<= 1)
+        v |= (uint64_t)__shfl_xor((unsigned long long)v, o, 64);
+    return v;
 }
 
 __device__ __forceinline__ CatMask mask_of(const Masks& M, int n, int t)
@@ -879,13 +910,16 @@ __global__ __launch_bounds__(256) void k_nlist(const double* xA, const double* y
 // Otherwise (no lists, smoothing lengths that vary, link_list's reach, a
 // window that does not fit): the candidates are the particle's list, or its
 // three candidate rows.  Four at a time their positions are tested with the
-// exact predicate; the indices that pass are put into the lane's column of an
-// LDS table, and the dense loop reads them back in order.  The loop control is
-// wave-uniform: the test runs until some lane's column is full or all
-// candidates are done.
+// exact predicate, into a mask of 128 candidates; the dense loop goes through its
+// bits.
 // ------------------------------------------------------------------------
-constexpr int VIS_ROWS = 32;            // column height
-constexpr int VIS_CAP = VIS_ROWS - 1;   // (the loop reads one past the last entry)
+// The forms of a stage kernel: WINDOWS as described, UNIFORM one smoothing length
+// for all pairs but no windows in LDS (no lists, or link_list's reach), VARYING
+// smoothing lengths that vary, GENERAL other than integer repulsion exponents or
+// Drucker-Prager (pow and the Mohr-Coulomb terms in the pair loop are 47 registers
+// of soil_ab's 204).  All but the first keep all lanes of a workgroup and take no
+// LDS.  1M ...
+enum : int { GENERAL, VARYING, UNIFORM, WINDOWS };
 
 // Record index of a position of three concatenated ranges: starts s1 and s2
 // of the second and third, record index - position in each.
@@ -937,64 +971,118 @@ struct Window {
 // The candidates sub, sub + 2^lg, ... of a particle from global memory:
 // body(v, rec, k) for each that passes accept(k, xy), in order; self: own
 // record index in the candidates' phase (-1: none).  All lanes of the wave call.
-template <int NCH, class A, class B>
-__device__ __forceinline__ void visit_global(int* table, const Cand& C, const IdxList& I, const Window& w, int n,
-                                             const SubCtx& sc, int lg, int self, const RecV& rec, A&& accept,
-                                             B&& body)
+// KEEP: stores the mask of a particle's partners in MW (ovf: more than 128
+// candidates); GIVEN: takes it from there instead of testing again.
+enum : int { TEST, KEEP, GIVEN };
+
+template <int NCH, int MODE, class A, class B>
+__device__ __forceinline__ void visit_global(const Cand& C, const IdxList& I, const Window& w, int n, const SubCtx& sc,
+                                             int lg, int self, const RecV& rec, const Masks& LM, const Masks& MW,
+                                             A&& accept, B&& body)
 {
-    int* col = table + threadIdx.x;
-    int tot = w.listed ? I.cnt[sc.tt] : -1;
-    const bool walk = tot < 0;
-    Ranges3 rows{0, 0, 0, 0, 0};
-    if (walk) rows = C.rows(sc.tt, tot);
+    CatMask kept{0, 0, 1}, listed{0, 0, 1};
+    if (MODE == GIVEN) kept = mask_of(MW, n, sc.tt);
+    if (LM.m && lg == 0) listed = mask_of(LM, n, sc.tt);   // (several lanes: the list deals evenly)
+    int tot = -1;
+    if (w.listed && listed.ovf) tot = I.cnt[sc.tt];
+    const bool by_row = tot < 0;
+    Ranges3 rows = w.r;
+    if (by_row) rows = C.rows(sc.tt, tot);
     if (!sc.valid) tot = 0;
-    int j = 0;
-    do {
-        int c = 0;
-        do {
+    auto at = [&](int i) { return rows(by_row ? i : (int)I.li[(size_t)i * n + sc.tt]); };
+#pragma unroll 1
+    for (int base = 0; base < tot; base += 128) {
+        const int end = min(tot - base, 128);
+        uint64_t lo = 0, hi = 0;
+        auto test = [&](const int(&c)[4]) {
             int k[4];
             double2 p[4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int i = j + (q << lg) + sc.sub;
-                k[q] = 0;   // (record 0 stands in past the end)
-                if (i < tot) k[q] = walk ? rows(i) : w.r(I.li[(size_t)i * n + sc.tt]);
-            }
+            for (int q = 0; q < 4; ++q) k[q] = at(base + c[q]);
 #pragma unroll
             for (int q = 0; q < 4; ++q) p[q] = rec(k[q], 0);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                col[c * STAGE_BLOCK] = k[q];
-                c += j + (q << lg) + sc.sub < tot && k[q] != self && accept(k[q], p[q]) ? 1 : 0;
+                const uint64_t bit = (uint64_t)(k[q] != self && accept(k[q], p[q])) << (c[q] & 63);
+                lo |= pick(c[q] < 64, bit, (uint64_t)0);
+                hi |= pick(c[q] < 64, (uint64_t)0, bit);
             }
-            j += 4 << lg;
-        } while (__any(j < tot) && !__any(c > VIS_CAP - 4));
-        int next = col[0];
+        };
+        if (MODE == GIVEN && !kept.ovf) {
+            lo = kept.lo & sub_bits(lg, sc.sub);
+            hi = kept.hi & sub_bits(lg, sc.sub);
+        } else if (!listed.ovf) {
+            uint64_t clo = listed.lo & sub_bits(lg, sc.sub), chi = listed.hi & sub_bits(lg, sc.sub);
+            while (clo | chi) {
+                int c[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {   // (past the last one: it again)
+                    const bool in_lo = clo != 0;
+                    const uint64_t m = pick(in_lo, clo, chi);
+                    c[q] = m ? __builtin_ctzll(m) + (in_lo ? 0 : 64) : q ? c[q - 1] : 0;
+                    const uint64_t rest = m & (m - 1);
+                    clo = pick(in_lo, rest, clo);
+                    chi = pick(in_lo, chi, rest);
+                }
+                test(c);
+            }
+        } else {
 #pragma unroll 1
-        for (int i = 1; i <= c; ++i) {
-            const int k = next;
-            next = col[i * STAGE_BLOCK];
+            for (int j = sc.sub; j < end; j += 4 << lg) {
+                int c[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) c[q] = j + (q << lg) < end ? j + (q << lg) : j;
+                test(c);
+            }
+        }
+        if (MODE == KEEP) {
+            kept.lo = lo;
+            kept.hi = hi;
+        }
+        auto next = [&]() -> int {
+            const bool in_lo = lo != 0;
+            const uint64_t m = pick(in_lo, lo, hi);
+            if (m == 0) return -1;
+            const int i = __builtin_ctzll(m) + (in_lo ? 0 : 64);
+            const uint64_t rest = m & (m - 1);
+            lo = pick(in_lo, rest, lo);
+            hi = pick(in_lo, hi, rest);
+            return at(base + i);
+        };
+        int ahead = next();
+#pragma unroll 1
+        while (ahead >= 0) {
+            const int k = ahead;
             double2 v[NCH];
 #pragma unroll
             for (int ch = 0; ch < NCH; ++ch) v[ch] = rec(k, ch);
+            ahead = next();
             body(v, rec, k);
         }
-    } while (__any(j < tot));
+    }
+    if (MODE == KEEP) {
+        kept.lo = sub_or(lg, kept.lo);
+        kept.hi = sub_or(lg, kept.hi);
+        if (sc.valid && !sc.sub) {
+            MW.m[sc.t] = kept.lo;
+            MW.m[n + sc.t] = kept.hi;
+            MW.ovf[sc.t] = tot > 128 ? 1 : 0;
+        }
+    }
 }
 
-// LDS of a stage kernel that reads NCH chunks per partner (without a window:
-// the table alone).
-constexpr size_t TABLE_LDS = sizeof(int) * VIS_ROWS * STAGE_BLOCK;
+// LDS of a stage kernel that reads NCH chunks per partner.
 template <int NCH>
-constexpr size_t VIS_LDS = TABLE_LDS > sizeof(double2) * NCH * WIN_STRIDE ? TABLE_LDS
-                                                                         : sizeof(double2) * NCH * WIN_STRIDE;
+constexpr size_t VIS_LDS = sizeof(double2) * NCH * WIN_STRIDE;
+template <int FORM, int NCH>
+constexpr size_t STAGE_LDS = FORM == WINDOWS ? VIS_LDS<NCH> : sizeof(double2);
 
 // Sends chunks 0 .. NCH - 1 of the workgroup's window on their way into LDS
 // (straight from global memory, no registers: all of it is in flight at once),
 // and a stand-in record (far away, finite everywhere) at WIN_CAP.  Called after
 // a kernel's own loads: loads return in order, so a use of one issued behind
 // the window would wait for all of it.
-template <bool U, int NCH, class R>
+template <bool WIN, int NCH, class R>
 __device__ __forceinline__ Window open_window(unsigned char* lds, const IdxList& I, int blk, const SubCtx& sc, int lg,
                                               int n, const R& rec)
 {
@@ -1003,7 +1091,7 @@ __device__ __forceinline__ Window open_window(unsigned char* lds, const IdxList&
     if (!I.li) return w;
     const int* p = I.win + (size_t)blk * WIN_INTS;
     w.r = window_ranges(p);
-    if constexpr (U) {
+    if constexpr (WIN) {
         const int tot = p[6];
         w.lds = I.lds && tot <= WIN_CAP;
         if (w.lds) {
@@ -1074,31 +1162,37 @@ __device__ __forceinline__ void visit_window(unsigned char* lds, const Window& w
 
 // body(v, R, k) over the partners of the lane's particle, v the record chunks
 // 0 .. NCH - 1 and R(k, c) any other (all lanes of the workgroup call).
-template <bool U, int NCH, class A, class B>
+template <bool WIN, int NCH, int MODE = TEST, class A, class B>
 __device__ __forceinline__ void visit(unsigned char* lds, const Window& w, const Cand& C, const IdxList& I, int n,
-                                      const SubCtx& sc, int lg, int self, const RecV& rec, A&& accept, B&& body)
+                                      const SubCtx& sc, int lg, int self, const RecV& rec, const Masks& LM,
+                                      A&& accept, B&& body, const Masks& MW = Masks{})
 {
-    if constexpr (U) {
-        if (w.lds) {
-            visit_window<NCH, double2>(lds, w, I, n, sc, lg, [&](const auto& v) { body(v, rec, 0); });
-            // a particle whose list overflowed walks its rows
-            if (w.cnt < 0 && sc.valid) {
-                int tot;
-                const Ranges3 rows = C.rows(sc.tt, tot);
+    // (a window that does not fit: several lanes go through the list at once, as
+    // through a window, one lane tests it first: savage column of 2k 3.24 ms for 100
+    // steps against 3.39, 250k slope 11.4 against 11.8)
+    if (WIN && (w.lds || lg > 0)) {
+        if (w.lds) visit_window<NCH, double2>(lds, w, I, n, sc, lg, [&](const auto& v) { body(v, rec, 0); });
+        // a particle whose list overflowed walks its rows
+        int tot = w.lds ? min(w.cnt, 0) : I.cnt[sc.tt];
+        const bool walk = tot < 0;
+        Ranges3 rows = w.r;
+        if (walk) rows = C.rows(sc.tt, tot);
+        if (!sc.valid) tot = 0;
+        auto at = [&](int i) { return rows(walk || i >= tot ? i : (int)I.li[(size_t)i * n + sc.tt]); };
+        int next = at(sc.sub);
 #pragma unroll 1
-                for (int i = sc.sub; i < tot; i += 1 << lg) {
-                    const int k = rows(i);
-                    if (k == self || !accept(k, rec(k, 0))) continue;
-                    double2 a[NCH];
+        for (int i = sc.sub; i < tot; i += 1 << lg) {
+            const int k = next;
+            next = at(i + (1 << lg));
+            if (walk && (k == self || !accept(k, rec(k, 0)))) continue;
+            double2 v[NCH];
 #pragma unroll
-                    for (int c = 0; c < NCH; ++c) a[c] = rec(k, c);
-                    body(a, rec, k);
-                }
-            }
-            return;
+            for (int c = 0; c < NCH; ++c) v[c] = rec(k, c);
+            body(v, rec, k);
         }
+        return;
     }
-    visit_global<NCH>(reinterpret_cast<int*>(lds), C, I, w, n, sc, lg, self, rec, accept, body);
+    visit_global<NCH, MODE>(C, I, w, n, sc, lg, self, rec, LM, MW, accept, body);
 }
 
 // ------------------------------------------------------------------------
@@ -1145,30 +1239,31 @@ __device__ __forceinline__ Sep sep_of(const KC& kc, double dx, double dy, double
 // not renormalise (its final update reads vof2), so the values that only a
 // download or the last step's diagnostics would read stay out.
 // ------------------------------------------------------------------------
-template <int SKF, bool U>
+template <int SKF, int FORM>
 __device__ __forceinline__ void water_x4(unsigned char* lds, int blk, DPhase W, DPhase S, const double* recW, const double* recS,
                                          NList NL, Grid g, KParams K, FusedK F, int lean)
 {
+    constexpr bool U = FORM >= UNIFORM, WIN = FORM == WINDOWS;
     const RecV RW = recv(recW, W.n), RS = recv(recS, S.n);
-    const SubCtx wc = sub_ctx(W.n, blk, NL.lg, WIN_LANES);
+    const SubCtx wc = sub_ctx(W.n, blk, NL.lg, NL.ix.pb << NL.lg);
     const double2 xy = RW(wc.tt, 0), va = RW(wc.tt, 1);
     const double xa = xy.x, ya = xy.y, vxa = va.x, vya = va.y, vofa = RW(wc.tt, 3).x;
     const double ha = U ? K.h1_water : RW(wc.tt, 6).x;
     const int a = NL.cell ? wc.tt : W.order[wc.tt];
     const bool ux = U || F.uni_x;
-    const Window win = open_window<U, 4>(lds, NL.ix, blk, wc, NL.lg, W.n, RS);
+    const Window win = open_window<WIN, 4>(lds, NL.ix, blk, wc, NL.lg, W.n, RS);
     const Cand C{g, S.cell_start, NL.cell, xa, ya};
     const Pred PX{xa, ya, ha, F.thr_x, ux ? 1 : 0, 0};
     const KC kx = make_kc(SKF, sph_mhsml(ha, ux ? RS(0, 6).x : ha));
     double dg_x = 0.0, dg_y = 0.0, dvof_x = 0.0, vof2 = 0.0;
     int cntx = 0;
-    visit<U, 4>(
-        lds, win, C, NL.ix, W.n, wc, NL.lg, -1, RS, [&](int k, double2 b) { return PX(b, ux ? ha : RS(k, 6).x, g, K); },
+    visit<WIN, 4>(
+        lds, win, C, NL.ix, W.n, wc, NL.lg, -1, RS, NL.cross, [&](int k, double2 b) { return PX(b, ux ? ha : RS(k, 6).x, g, K); },
         [&](const auto& v, const auto& R, int k) {
             const double2 b = v[0], u = v[1], q = v[2];
             const double vr_b = v[3].x;   // vof / rho
             KC kc = kx;
-            if (!ux) kc = make_kc(SKF, sph_mhsml(ha, R(k, 6).x));
+            if (!ux) kc = pair_kc<SKF>(sph_mhsml(ha, R(k, 6).x));
             const Sep p = sep_of<SKF, true>(kc, xa - b.x, ya - b.y, U ? F.thr_x : INFINITY, true);
             cntx += p.in ? 1 : 0;
             const double m = fabs(q.y) * q.x, mw = m * p.w;
@@ -1193,12 +1288,12 @@ __device__ __forceinline__ void water_x4(unsigned char* lds, int blk, DPhase W, 
     }
 }
 
-template <int SKF, bool U>
+template <int SKF, int FORM>
 __global__ STAGE_ATTR void k_water_x4(DPhase W, DPhase S, const double* recW, const double* recS, NList NL, Grid g,
                                       KParams K, FusedK F, int lean)
 {
-    __shared__ __align__(16) unsigned char lds[VIS_LDS<4>];
-    water_x4<SKF, U>(lds, xcd_block(), W, S, recW, recS, NL, g, K, F, lean);
+    __shared__ __align__(16) unsigned char lds[STAGE_LDS<FORM, 4>];
+    water_x4<SKF, FORM>(lds, xcd_block(), W, S, recW, recS, NL, g, K, F, lean);
 }
 
 // ------------------------------------------------------------------------
@@ -1206,30 +1301,31 @@ __global__ STAGE_ATTR void k_water_x4(DPhase W, DPhase S, const double* recW, co
 // pore_water_pressure (m_particles.f90:3832-3909) from the water partners
 // (whose pressure is the new one the water pack evaluated).
 // ------------------------------------------------------------------------
-template <int SKF, bool U>
+template <int SKF, int FORM>
 __device__ __forceinline__ void soil_x4(unsigned char* lds, int blk, DPhase S, DPhase W, const double* recS, const double* recW, NList NL,
                                         Grid g, KParams K, FusedK F, int lean)
 {
+    constexpr bool U = FORM >= UNIFORM, WIN = FORM == WINDOWS;
     const RecV RS = recv(recS, S.n), RW = recv(recW, W.n);
-    const SubCtx wc = sub_ctx(S.n, blk, NL.lg, WIN_LANES);
+    const SubCtx wc = sub_ctx(S.n, blk, NL.lg, NL.ix.pb << NL.lg);
     const double2 xy = RS(wc.tt, 0), va = RS(wc.tt, 1);
     const double xa = xy.x, ya = xy.y, vxa = va.x, vya = va.y;
     const double vra = RS(wc.tt, 3).x;   // vof / rho
     const double ha = U ? K.h1_soil : RS(wc.tt, 6).x;
     const int a = NL.cell ? wc.tt : S.order[wc.tt];
     const bool ux = U || F.uni_x;
-    const Window win = open_window<U, 4>(lds, NL.ix, blk, wc, NL.lg, S.n, RW);
+    const Window win = open_window<WIN, 4>(lds, NL.ix, blk, wc, NL.lg, S.n, RW);
     const Cand C{g, W.cell_start, NL.cell, xa, ya};
     const Pred PX{xa, ya, ha, F.thr_x, ux ? 1 : 0, 0};
     const KC kx = make_kc(SKF, sph_mhsml(ux ? RW(0, 6).x : ha, ha));
     double dg_x = 0.0, dg_y = 0.0, po_x = 0.0, po_y = 0.0;
     int cntx = 0;
-    visit<U, 4>(
-        lds, win, C, NL.ix, S.n, wc, NL.lg, -1, RW, [&](int k, double2 b) { return PX(b, ux ? ha : RW(k, 6).x, g, K); },
+    visit<WIN, 4>(
+        lds, win, C, NL.ix, S.n, wc, NL.lg, -1, RW, NL.cross, [&](int k, double2 b) { return PX(b, ux ? ha : RW(k, 6).x, g, K); },
         [&](const auto& v, const auto& R, int k) {
             const double2 b = v[0], u = v[1], q = v[2], f = v[3];   // f = (vof, p)
             KC kc = kx;
-            if (!ux) kc = make_kc(SKF, sph_mhsml(R(k, 6).x, ha));
+            if (!ux) kc = pair_kc<SKF>(sph_mhsml(R(k, 6).x, ha));
             // water - soil
             const Sep p = sep_of<SKF, true>(kc, b.x - xa, b.y - ya, U ? F.thr_x : INFINITY, true);
             cntx += p.in ? 1 : 0;
@@ -1253,21 +1349,21 @@ __device__ __forceinline__ void soil_x4(unsigned char* lds, int blk, DPhase S, D
     if (!lean) S.countiac[a] = cntx;
 }
 
-template <int SKF, bool U>
+template <int SKF, int FORM>
 __global__ STAGE_ATTR void k_soil_x4(DPhase S, DPhase W, const double* recS, const double* recW, NList NL, Grid g,
                                      KParams K, FusedK F, int lean)
 {
-    __shared__ __align__(16) unsigned char lds[VIS_LDS<4>];
-    soil_x4<SKF, U>(lds, xcd_block(), S, W, recS, recW, NL, g, K, F, lean);
+    __shared__ __align__(16) unsigned char lds[STAGE_LDS<FORM, 4>];
+    soil_x4<SKF, FORM>(lds, xcd_block(), S, W, recS, recW, NL, g, K, F, lean);
 }
 
 // repulsive_force on a real particle from a virtual partner within r0
 // (m_particles.f90:1605): D ((r0/r)^p1 - (r0/r)^p2) d / r^2; ir = 1/r.
-template <bool U>
+template <bool INT>
 __device__ __forceinline__ double rep_factor(const KParams& K, double r0, double ir)
 {
     const double q = r0 * ir;
-    return K.dd * (U ? ipow(q, K.ip1) - ipow(q, K.ip2) : pow(q, K.p1) - pow(q, K.p2)) * (ir * ir);
+    return K.dd * (INT ? ipow(q, K.ip1) - ipow(q, K.ip2) : pow(q, K.p1) - pow(q, K.p2)) * (ir * ir);
 }
 
 // ------------------------------------------------------------------------
@@ -1277,12 +1373,13 @@ __device__ __forceinline__ double rep_factor(const KParams& K, double r0, double
 // two-phase run (countiac then counts the soil partners, which k_water_x4
 // writes).
 // ------------------------------------------------------------------------
-template <int SKF, bool U>
-__device__ __forceinline__ void water_a4(unsigned char* lds, int blk, DPhase W, const double* recW, double* recWw, NList NL, Grid g,
-                                         KParams K, FusedK F, int cross, int lean)
+template <int SKF, int FORM>
+__device__ __forceinline__ void water_a4(unsigned char* lds, int blk, DPhase W, const double* recW, double* recWw, NList NL, Masks MW,
+                                         Grid g, KParams K, FusedK F, int cross, int lean)
 {
+    constexpr bool U = FORM >= UNIFORM, WIN = FORM == WINDOWS;
     const RecV RW = recv(recW, W.n);
-    const SubCtx wc = sub_ctx(W.n, blk, NL.lg, WIN_LANES);
+    const SubCtx wc = sub_ctx(W.n, blk, NL.lg, NL.is.pb << NL.lg);
     const int t = wc.t;
     auto RA = [&](int c) { return RW(wc.tt, c); };
     const double2 xy = RA(0), va = RA(1);
@@ -1296,18 +1393,18 @@ __device__ __forceinline__ void water_a4(unsigned char* lds, int blk, DPhase W, 
     const bool uni = U || link || F.uni_w;
     const KC kc0 = make_kc(SKF, link ? K.h1_water : ha);
     const int ita = W.itype[a];
-    const Window win = open_window<U, 3>(lds, NL.is, blk, wc, NL.lg, W.n, RW);
+    const Window win = open_window<WIN, 3>(lds, NL.is, blk, wc, NL.lg, W.n, RW);
     const Cand C{g, W.cell_start, NL.cell, xa, ya};
     const Pred P{xa, ya, ha, F.thr_w, uni ? 1 : 0, link ? 1 : 0};
     const double rep2 = ita > 0 ? W.dspp * W.dspp : -1.0;   // real particles feel the wall
     double con = 0.0, drd = 0.0, xx = 0.0, yy = 0.0, xy2 = 0.0, avx = 0.0, avy = 0.0, repx = 0.0, repy = 0.0;
     int cnt = 0;
-    visit<U, 3>(
-        lds, win, C, NL.is, W.n, wc, NL.lg, t, RW, [&](int k, double2 b) { return P(b, uni ? ha : RW(k, 6).x, g, K); },
+    visit<WIN, 3, KEEP>(
+        lds, win, C, NL.is, W.n, wc, NL.lg, t, RW, NL.same, [&](int k, double2 b) { return P(b, uni ? ha : RW(k, 6).x, g, K); },
         [&](const auto& v, const auto& R, int k) {
             const double2 b = v[0], u = v[1], q = v[2];
             KC kc = kc0;
-            if (!uni) kc = make_kc(SKF, sph_mhsml(ha, R(k, 6).x));
+            if (!uni) kc = pair_kc<SKF>(sph_mhsml(ha, R(k, 6).x));
             const Sep p = sep_of<SKF, true>(kc, xa - b.x, ya - b.y, U ? F.thr_w : INFINITY, false);
             cnt += p.in ? 1 : 0;
             const double V = fabs(q.y), dvx = vxa - u.x, dvy = vya - u.y, vr = dvx * p.dx + dvy * p.dy;
@@ -1322,11 +1419,11 @@ __device__ __forceinline__ void water_a4(unsigned char* lds, int blk, DPhase W, 
             avx -= f * dvx;
             avy -= f * dvy;
             if (q.y < 0.0 && p.dr <= rep2) {
-                const double fr = rep_factor<U>(K, W.dspp, p.ir);
+                const double fr = rep_factor<FORM != GENERAL>(K, W.dspp, p.ir);
                 repx += p.dx * fr;
                 repy += p.dy * fr;
             }
-        });
+        }, MW);
     sub_sum(NL.lg, con, drd, xx, yy, xy2, avx, avy, repx, repy);
     cnt = sub_count(NL.lg, cnt);
     if (!wc.valid || wc.sub) return;
@@ -1356,24 +1453,25 @@ __device__ __forceinline__ void water_a4(unsigned char* lds, int blk, DPhase W, 
     WP[5 * nw] = make_double2(vofa * (mu * txx), vofa * (mu * txy));
 }
 
-template <int SKF, bool U>
-__global__ STAGE_ATTR void k_water_a4(DPhase W, const double* recW, double* recWw, NList NL, Grid g, KParams K,
-                                      FusedK F, int cross, int lean)
+template <int SKF, int FORM>
+__global__ STAGE_ATTR void k_water_a4(DPhase W, const double* recW, double* recWw, NList NL, Masks MW, Grid g,
+                                      KParams K, FusedK F, int cross, int lean)
 {
-    __shared__ __align__(16) unsigned char lds[VIS_LDS<3>];
-    water_a4<SKF, U>(lds, xcd_block(), W, recW, recWw, NL, g, K, F, cross, lean);
+    __shared__ __align__(16) unsigned char lds[STAGE_LDS<FORM, 3>];
+    water_a4<SKF, FORM>(lds, xcd_block(), W, recW, recWw, NL, MW, g, K, F, cross, lean);
 }
 
 // ------------------------------------------------------------------------
 // Stage B, water: -vof*df(p) + df(vof*sigma) (declarations_sph.f90:1257-1265),
 // art_visc, delta_sph(vof, dvof); /rho, + repulsion, + gravity, - Darcy drag.
 // ------------------------------------------------------------------------
-template <int SKF, bool U>
-__device__ __forceinline__ void water_b4(unsigned char* lds, int blk, DPhase W, const double* recW, NList NL, Grid g, KParams K, FusedK F,
-                                         int mask)
+template <int SKF, int FORM>
+__device__ __forceinline__ void water_b4(unsigned char* lds, int blk, DPhase W, const double* recW, NList NL, Masks MW, Grid g,
+                                         KParams K, FusedK F, int mask)
 {
+    constexpr bool U = FORM >= UNIFORM, WIN = FORM == WINDOWS;
     const RecV RW = recv(recW, W.n);
-    const SubCtx wc = sub_ctx(W.n, blk, NL.lg, WIN_LANES);
+    const SubCtx wc = sub_ctx(W.n, blk, NL.lg, NL.is.pb << NL.lg);
     const int t = wc.t;
     auto RA = [&](int c) { return RW(wc.tt, c); };
     const double2 axy = RA(0), av = RA(1), arv = RA(2), a3 = RA(3), a4 = RA(4), a12 = RA(5);
@@ -1393,20 +1491,20 @@ __device__ __forceinline__ void water_b4(unsigned char* lds, int blk, DPhase W, 
         drgy = W.drgy[a];
         dvx = W.dvof_x[a];
     }
-    const Window win = open_window<U, 6>(lds, NL.is, blk, wc, NL.lg, W.n, RW);
+    const Window win = open_window<WIN, 6>(lds, NL.is, blk, wc, NL.lg, W.n, RW);
     const Cand C{g, W.cell_start, NL.cell, xa, ya};
     const Pred P{xa, ya, ha, F.thr_w, uni ? 1 : 0, link ? 1 : 0};
     const double et2 = K.etq * K.etq;
     double Wx = 0.0, Wy = 0.0, Fx = 0.0, Fy = 0.0, artx = 0.0, arty = 0.0, dvd = 0.0;
-    visit<U, 6>(
-        lds, win, C, NL.is, W.n, wc, NL.lg, t, RW, [&](int k, double2 b) { return P(b, uni ? ha : RW(k, 6).x, g, K); },
+    visit<WIN, 6, GIVEN>(
+        lds, win, C, NL.is, W.n, wc, NL.lg, t, RW, NL.same, [&](int k, double2 b) { return P(b, uni ? ha : RW(k, 6).x, g, K); },
         [&](const auto& v, const auto& R, int k) {
             const double2 b = v[0], u = v[1], q = v[2], f = v[3], s3 = v[4], s12 = v[5];
             KC kc = kc0;
             double amh = ha;
             if (!uni) {
                 amh = sph_mhsml(ha, R(k, 6).x);
-                kc = make_kc(SKF, amh);
+                kc = pair_kc<SKF>(amh);
             }
             const Sep p = sep_of<SKF, false>(kc, xa - b.x, ya - b.y, U ? F.thr_w : INFINITY, false);
             const double Vs = fabs(q.y) * p.s, wx = Vs * p.dx, wy = Vs * p.dy;
@@ -1430,7 +1528,7 @@ __device__ __forceinline__ void water_b4(unsigned char* lds, int blk, DPhase W, 
                 arty -= mp * p.dy;
             }
             dvd += Vs * (vofa - f.x);
-        });
+        }, MW);
     sub_sum(NL.lg, Wx, Wy, Fx, Fy, artx, arty, dvd);
     if (!wc.valid || wc.sub) return;
     double ax = Fx + 2.0 * (a12.x - vofa * pa) * Wx;
@@ -1455,11 +1553,12 @@ __device__ __forceinline__ void water_b4(unsigned char* lds, int blk, DPhase W, 
     W.dvof[a] = dvof;
 }
 
-template <int SKF, bool U>
-__global__ STAGE_ATTR void k_water_b4(DPhase W, const double* recW, NList NL, Grid g, KParams K, FusedK F, int mask)
+template <int SKF, int FORM>
+__global__ STAGE_ATTR void k_water_b4(DPhase W, const double* recW, NList NL, Masks MW, Grid g, KParams K,
+                                      FusedK F, int mask)
 {
-    __shared__ __align__(16) unsigned char lds[VIS_LDS<6>];
-    water_b4<SKF, U>(lds, xcd_block(), W, recW, NL, g, K, F, mask);
+    __shared__ __align__(16) unsigned char lds[STAGE_LDS<FORM, 6>];
+    water_b4<SKF, FORM>(lds, xcd_block(), W, recW, NL, MW, g, K, F, mask);
 }
 
 // Stress and pressure rates of soil particle a from its strain rate t, divergence
@@ -1539,12 +1638,13 @@ __device__ __forceinline__ StressRates stress_rates(const DPhase& S, const KPara
 //               /rho, + repulsion, + gravity, + Darcy drag, + pore pressure
 //               (the cross terms k_soil_x4 wrote; cross: two-phase run).
 // ------------------------------------------------------------------------
-template <int SKF, bool U, bool SOLO>
+template <int SKF, int FORM, bool SOLO>
 __device__ __forceinline__ void soil_ab4(unsigned char* lds, int blk, DPhase S, const double* recS, NList NL, Grid g, KParams K, FusedK F,
                                          int cross, int mask, int lean)
 {
+    constexpr bool U = FORM >= UNIFORM, WIN = FORM == WINDOWS;
     const RecV RS = recv(recS, S.n);
-    const SubCtx wc = sub_ctx(S.n, blk, NL.lg, SOLO ? STAGE_BLOCK : WIN_LANES);
+    const SubCtx wc = sub_ctx(S.n, blk, NL.lg, SOLO ? STAGE_BLOCK : NL.is.pb << NL.lg);
     const int t = wc.t;
     auto RA = [&](int c) { return RS(wc.tt, c); };
     const double2 xy = RA(0), va = RA(1), a3 = RA(3), a4 = RA(4), a12 = RA(5);
@@ -1557,7 +1657,7 @@ __device__ __forceinline__ void soil_ab4(unsigned char* lds, int blk, DPhase S, 
     // Mohr-Coulomb (general instantiation only): the criterion may have reset
     // rho; con_density's delta_sph, the strain rate and the divergence come
     // before it in single_step and use the density before it (chunk 7)
-    const bool mc = !U && K.yield_criterion == 1;
+    const bool mc = FORM == GENERAL && K.yield_criterion == 1;
     const double rhoa_pre = mc ? RA(7).x : rhoa;
     const int a = NL.cell ? wc.tt : S.order[wc.tt];
     const int ita = S.itype[a];
@@ -1572,7 +1672,7 @@ __device__ __forceinline__ void soil_ab4(unsigned char* lds, int blk, DPhase S, 
         porx = S.porx[a];
         pory = S.pory[a];
     }
-    const Window win = open_window<U, 6>(lds, NL.is, blk, wc, NL.lg, S.n, RS);
+    const Window win = open_window<WIN, 6>(lds, NL.is, blk, wc, NL.lg, S.n, RS);
     const Cand C{g, S.cell_start, NL.cell, xa, ya};
     const Pred P{xa, ya, ha, F.thr_s, uni ? 1 : 0, link ? 1 : 0};
     const double rep2 = !SOLO && ita > 0 ? S.dspp * S.dspp : -1.0;   // real particles feel the wall
@@ -1585,15 +1685,15 @@ __device__ __forceinline__ void soil_ab4(unsigned char* lds, int blk, DPhase S, 
     double Fx = 0.0, Fy = 0.0;
     double artx = 0.0, arty = 0.0, dP = 0.0, dXX = 0.0, dXY = 0.0, dYY = 0.0;
     int cnt = 0;
-    visit<U, 6>(
-        lds, win, C, NL.is, S.n, wc, NL.lg, t, RS, [&](int k, double2 b) { return P(b, uni ? ha : RS(k, 6).x, g, K); },
+    visit<WIN, 6>(
+        lds, win, C, NL.is, S.n, wc, NL.lg, t, RS, NL.same, [&](int k, double2 b) { return P(b, uni ? ha : RS(k, 6).x, g, K); },
         [&](const auto& v, const auto& R, int k) {
             const double2 b = v[0], u = v[1], q = v[2], f = v[3], s3 = v[4], s12 = v[5];
             KC kc = kc0;
             double amh = ha;
             if (!uni) {
                 amh = sph_mhsml(ha, R(k, 6).x);
-                kc = make_kc(SKF, amh);
+                kc = pair_kc<SKF>(amh);
             }
             const Sep p = sep_of<SKF, true>(kc, xa - b.x, ya - b.y, U ? F.thr_s : INFINITY, false);
             cnt += p.in ? 1 : 0;
@@ -1602,13 +1702,13 @@ __device__ __forceinline__ void soil_ab4(unsigned char* lds, int blk, DPhase S, 
             const double Vs = V * p.s, wx = Vs * p.dx, wy = Vs * p.dy;
             // stage A
             con += (m * p.s) * vr;
-            if (mc) {
-                const double rp = R(k, 7).x, Vp = (m * fast_rcp(rp)) * p.s;
-                drd += Vp * (rhoa_pre - rp);
-                sxx += Vp * (dvx * p.dx);
-                syy += Vp * (dvy * p.dy);
-                sxy += Vp * (dvx * p.dy);
-                syx += Vp * (dvy * p.dx);
+            if constexpr (FORM == GENERAL) {   // (a branch for each criterion: 14 more registers and spills)
+                const double rp = mc ? R(k, 7).x : q.x, t = mc ? q.x * fast_rcp(rp) : 1.0, tx = t * wx, ty = t * wy;
+                drd += t * Vs * (rhoa_pre - rp);
+                sxx += tx * dvx;
+                syy += ty * dvy;
+                sxy += ty * dvx;
+                syx += tx * dvy;
                 spin += wx * dvy - wy * dvx;
             } else {
                 drd += Vs * (rhoa - q.x);
@@ -1624,7 +1724,7 @@ __device__ __forceinline__ void soil_ab4(unsigned char* lds, int blk, DPhase S, 
             avx -= fv * dvx;
             avy -= fv * dvy;
             if (!SOLO && q.y < 0.0 && p.dr <= rep2) {
-                const double fr = rep_factor<U>(K, S.dspp, p.ir);
+                const double fr = rep_factor<FORM != GENERAL>(K, S.dspp, p.ir);
                 artx += p.dx * (0.5 * fr);
                 arty += p.dy * (0.5 * fr);
             }
@@ -1710,12 +1810,12 @@ __device__ __forceinline__ void soil_ab4(unsigned char* lds, int blk, DPhase S, 
     S.ay[a] = ay;
 }
 
-template <int SKF, bool U>
+template <int SKF, int FORM>
 __global__ STAGE_ATTR_AB void k_soil_ab4(DPhase S, const double* recS, NList NL, Grid g, KParams K, FusedK F,
                                          int cross, int mask, int lean)
 {
-    __shared__ __align__(16) unsigned char lds[VIS_LDS<6>];
-    soil_ab4<SKF, U, false>(lds, xcd_block(), S, recS, NL, g, K, F, cross, mask, lean);
+    __shared__ __align__(16) unsigned char lds[STAGE_LDS<FORM, 6>];
+    soil_ab4<SKF, FORM, false>(lds, xcd_block(), S, recS, NL, g, K, F, cross, mask, lean);
 }
 
 // ------------------------------------------------------------------------
@@ -1753,12 +1853,13 @@ struct StageArgs {
     DPhase W, S;
     double *rW, *rS;
     NList nW, nS;
+    Masks MW;
     Grid gW, gS;
     KParams K;
     FusedK F;
     int mask_w, mask_s, lean;
-    int nbW, nbS;   // workgroups of a pass over the water, over the soil
-    FlagPost post;  // (stage 1)
+    int nbW, nbS, nbXW, nbXS;   // workgroups of the same-phase and the cross passes
+    FlagPost post;              // (stage 1)
 };
 
 // The part of a launch that workgroup l belongs to, in the order of the counts
@@ -1791,38 +1892,40 @@ __device__ __forceinline__ PartIdx part_of(int l, const int (&nb)[N], bool sprea
     return p;
 }
 
-template <int SKF>
+// FS, FX: the form of the same-phase and of the cross passes.
+template <int SKF, int FS, int FX>
 __device__ __forceinline__ void stage1(int l, const StageArgs& A, bool spread)
 {
-    __shared__ __align__(16) unsigned char lds[VIS_LDS<4>];
+    __shared__ __align__(16) unsigned char lds[STAGE_LDS<FX, 4>];
+    static_assert(STAGE_LDS<FX, 4> >= STAGE_LDS<FS, 3>, "both passes");
     post_flag(A.post, l);
-    const PartIdx p = part_of<3>(l, {A.nbS, A.nbW, A.nbW}, spread);
+    const PartIdx p = part_of<3>(l, {A.nbXS, A.nbW, A.nbXW}, spread);
     if (p.blk < 0) return;
-    if (p.part == 0) soil_x4<SKF, true>(lds, p.blk, A.S, A.W, A.rS, A.rW, A.nS, A.gS, A.K, A.F, A.lean);
-    else if (p.part == 1) water_a4<SKF, true>(lds, p.blk, A.W, A.rW, A.rW, A.nW, A.gW, A.K, A.F, 1, A.lean);
-    else water_x4<SKF, true>(lds, p.blk, A.W, A.S, A.rW, A.rS, A.nW, A.gW, A.K, A.F, A.lean);
+    if (p.part == 0) soil_x4<SKF, FX>(lds, p.blk, A.S, A.W, A.rS, A.rW, A.nS, A.gS, A.K, A.F, A.lean);
+    else if (p.part == 1) water_a4<SKF, FS>(lds, p.blk, A.W, A.rW, A.rW, A.nW, A.MW, A.gW, A.K, A.F, 1, A.lean);
+    else water_x4<SKF, FX>(lds, p.blk, A.W, A.S, A.rW, A.rS, A.nW, A.gW, A.K, A.F, A.lean);
 }
 
-template <int SKF>
+template <int SKF, int FS>
 __device__ __forceinline__ void stage2(int l, const StageArgs& A, bool spread)
 {
-    __shared__ __align__(16) unsigned char lds[VIS_LDS<6>];
+    __shared__ __align__(16) unsigned char lds[STAGE_LDS<FS, 6>];
     const PartIdx p = part_of<2>(l, {A.nbS, A.nbW}, spread);
     if (p.blk < 0) return;
-    if (p.part == 0) soil_ab4<SKF, true, false>(lds, p.blk, A.S, A.rS, A.nS, A.gS, A.K, A.F, 1, A.mask_s, A.lean);
-    else water_b4<SKF, true>(lds, p.blk, A.W, A.rW, A.nW, A.gW, A.K, A.F, A.mask_w);
+    if (p.part == 0) soil_ab4<SKF, FS, false>(lds, p.blk, A.S, A.rS, A.nS, A.gS, A.K, A.F, 1, A.mask_s, A.lean);
+    else water_b4<SKF, FS>(lds, p.blk, A.W, A.rW, A.nW, A.MW, A.gW, A.K, A.F, A.mask_w);
 }
 
-template <int SKF>
+template <int SKF, int FS, int FX>
 __global__ STAGE_ATTR void k_stage1(StageArgs A)
 {
-    stage1<SKF>(blockIdx.x, A, true);
+    stage1<SKF, FS, FX>(blockIdx.x, A, true);
 }
 
-template <int SKF>
+template <int SKF, int FS>
 __global__ STAGE_ATTR_AB void k_stage2(StageArgs A)
 {
-    stage2<SKF>(blockIdx.x, A, true);
+    stage2<SKF, FS>(blockIdx.x, A, true);
 }
 
 // The final updates of both phases, with the next step's packs when ahead.

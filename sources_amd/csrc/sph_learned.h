@@ -152,7 +152,7 @@ __device__ __forceinline__ void water_x(unsigned char* lds, int blk, DPhase W, D
                                         const double* recS, NList NL, Grid g, KParams K, FusedK F)
 {
     const RecV RW = recv(recW, W.n), RS = recv(recS, S.n);
-    const SubCtx wc = sub_ctx(W.n, blk, 0, lanes_of_one(NL));
+    const SubCtx wc = sub_ctx(W.n, blk, 0, lanes_of_one(NL.ix));
     const double2 xy = RW(wc.tt, 0), va = RW(wc.tt, 1), rm = RW(wc.tt, 2);
     const double xa = xy.x, ya = xy.y, vxa = va.x, vya = va.y, rhoa = rm.x, vofa = RW(wc.tt, 3).x;
     const double ha = U ? K.h1_water : RW(wc.tt, 6).x;
@@ -168,7 +168,7 @@ __device__ __forceinline__ void water_x(unsigned char* lds, int blk, DPhase W, D
     double dg_x = 0.0, dg_y = 0.0, dvof_x = 0.0, vof2 = 0.0;
     int cntx = 0;
     visit<U, 4>(
-        lds, win, C, NL.ix, W.n, wc, 0, -1, RS, [&](int k, double2 b) { return PX(b, ux ? ha : RS(k, 6).x, g, K); },
+        lds, win, C, NL.ix, W.n, wc, 0, -1, RS, NL.cross, [&](int k, double2 b) { return PX(b, ux ? ha : RS(k, 6).x, g, K); },
         [&](const auto& v, const auto& R, int k) {
             const double dx = xa - v[0].x, dy = ya - v[0].y;
             if (outside<U>(dx, dy, F.thr_x)) return;
@@ -200,7 +200,7 @@ __device__ __forceinline__ void soil_x(unsigned char* lds, int blk, DPhase S, DP
                                        const double* recW, NList NL, Grid g, KParams K, FusedK F)
 {
     const RecV RS = recv(recS, S.n), RW = recv(recW, W.n);
-    const SubCtx wc = sub_ctx(S.n, blk, 0, lanes_of_one(NL));
+    const SubCtx wc = sub_ctx(S.n, blk, 0, lanes_of_one(NL.ix));
     const double2 xy = RS(wc.tt, 0), va = RS(wc.tt, 1), rm = RS(wc.tt, 2);
     const double xa = xy.x, ya = xy.y, vxa = va.x, vya = va.y, rhoa = rm.x, vofa = RS(wc.tt, 3).x;
     const double ha = U ? K.h1_soil : RS(wc.tt, 6).x;
@@ -215,7 +215,7 @@ __device__ __forceinline__ void soil_x(unsigned char* lds, int blk, DPhase S, DP
     double dg_x = 0.0, dg_y = 0.0, po_x = 0.0, po_y = 0.0;
     int cntx = 0;
     visit<U, 4>(
-        lds, win, C, NL.ix, S.n, wc, 0, -1, RW, [&](int k, double2 b) { return PX(b, ux ? ha : RW(k, 6).x, g, K); },
+        lds, win, C, NL.ix, S.n, wc, 0, -1, RW, NL.cross, [&](int k, double2 b) { return PX(b, ux ? ha : RW(k, 6).x, g, K); },
         [&](const auto& v, const auto& R, int k) {
             const double dx = v[0].x - xa, dy = v[0].y - ya;   // water - soil
             if (outside<U>(dx, dy, F.thr_x)) return;
@@ -247,7 +247,7 @@ __device__ __forceinline__ void water_a(unsigned char* lds, int blk, DPhase W, c
                                         NList NL, Grid g, KParams K, FusedK F)
 {
     const RecV RW = recv(recW, W.n);
-    const SubCtx wc = sub_ctx(W.n, blk, 0, lanes_of_one(NL));
+    const SubCtx wc = sub_ctx(W.n, blk, 0, lanes_of_one(NL.is));
     const int t = wc.t;
     auto RA = [&](int c) { return RW(wc.tt, c); };
     const double2 xy = RA(0), va = RA(1), rm = RA(2), hi = RA(6);
@@ -266,7 +266,7 @@ __device__ __forceinline__ void water_a(unsigned char* lds, int blk, DPhase W, c
     double con = 0.0, drd = 0.0, txx = 0.0, txy = 0.0, tyy = 0.0, avx = 0.0, avy = 0.0, repx = 0.0, repy = 0.0;
     int cnt = 0;
     visit<U, 3>(
-        lds, win, C, NL.is, W.n, wc, 0, t, RW, [&](int k, double2 b) { return P(b, uni ? ha : RW(k, 6).x, g, K); },
+        lds, win, C, NL.is, W.n, wc, 0, t, RW, NL.same, [&](int k, double2 b) { return P(b, uni ? ha : RW(k, 6).x, g, K); },
         [&](const auto& v, const auto& R, int k) {
             const double dx = xa - v[0].x, dy = ya - v[0].y;
             if (outside<U>(dx, dy, F.thr_w)) return;
@@ -313,7 +313,7 @@ __device__ __forceinline__ void water_b(unsigned char* lds, int blk, DPhase W, c
                                         KParams K, FusedK F, int mask)
 {
     const RecV RW = recv(recW, W.n);
-    const SubCtx wc = sub_ctx(W.n, blk, 0, lanes_of_one(NL));
+    const SubCtx wc = sub_ctx(W.n, blk, 0, lanes_of_one(NL.is));
     const int t = wc.t;
     auto RA = [&](int c) { return RW(wc.tt, c); };
     const double2 axy = RA(0), av = RA(1), arm = RA(2), a3 = RA(3), apc = RA(4), a12 = RA(5);
@@ -333,7 +333,7 @@ __device__ __forceinline__ void water_b(unsigned char* lds, int blk, DPhase W, c
     double Px = 0.0, Py = 0.0, Sxx = 0.0, Sxyy = 0.0, Sxyx = 0.0, Syy = 0.0;
     double artx = 0.0, arty = 0.0, dvd = 0.0;
     visit<U, 6>(
-        lds, win, C, NL.is, W.n, wc, 0, t, RW, [&](int k, double2 b) { return P(b, uni ? ha : RW(k, 6).x, g, K); },
+        lds, win, C, NL.is, W.n, wc, 0, t, RW, NL.same, [&](int k, double2 b) { return P(b, uni ? ha : RW(k, 6).x, g, K); },
         [&](const auto& v, const auto& R, int k) {
             const double dx = xa - v[0].x, dy = ya - v[0].y;
             if (outside<U>(dx, dy, F.thr_w)) return;
@@ -390,7 +390,7 @@ __device__ __forceinline__ void soil_ab(unsigned char* lds, int blk, DPhase S, c
                                         KParams K, FusedK F, int mask)
 {
     const RecV RS = recv(recS, S.n);
-    const SubCtx wc = sub_ctx(S.n, blk, 0, lanes_of_one(NL));
+    const SubCtx wc = sub_ctx(S.n, blk, 0, lanes_of_one(NL.is));
     const int t = wc.t;
     auto RA = [&](int c) { return RS(wc.tt, c); };
     const double2 xy = RA(0), va = RA(1), rm = RA(2), a3 = RA(3), a4 = RA(4), a12 = RA(5), hi = RA(6);
@@ -420,7 +420,7 @@ __device__ __forceinline__ void soil_ab(unsigned char* lds, int blk, DPhase S, c
     double artx = 0.0, arty = 0.0, dP = 0.0, dXX = 0.0, dXY = 0.0, dYY = 0.0;
     int cnt = 0;
     visit<U, 6>(
-        lds, win, C, NL.is, S.n, wc, 0, t, RS, [&](int k, double2 b) { return P(b, uni ? ha : RS(k, 6).x, g, K); },
+        lds, win, C, NL.is, S.n, wc, 0, t, RS, NL.same, [&](int k, double2 b) { return P(b, uni ? ha : RS(k, 6).x, g, K); },
         [&](const auto& v, const auto& R, int k) {
             const double dx = xa - v[0].x, dy = ya - v[0].y;
             if (outside<U>(dx, dy, F.thr_s)) return;
@@ -524,7 +524,7 @@ __device__ __forceinline__ void part(unsigned char* lds, int blk, const StageArg
 }
 
 template <int PART, bool U>
-constexpr size_t PART_LDS = !U ? TABLE_LDS : PART >= 3 ? VIS_LDS<6> : PART == 1 ? VIS_LDS<3> : VIS_LDS<4>;
+constexpr size_t PART_LDS = STAGE_LDS<U ? WINDOWS : GENERAL, PART >= 3 ? 6 : PART == 1 ? 3 : 4>;
 
 template <int SKF, int PART, bool U>
 __global__ STAGE_ATTR void k_part(StageArgs A)
@@ -540,7 +540,7 @@ __global__ STAGE_ATTR void k_stage1(StageArgs A)
 {
     __shared__ __align__(16) unsigned char lds[VIS_LDS<4>];
     post_flag(A.post, blockIdx.x);
-    const PartIdx p = part_of<3>(blockIdx.x, {A.nbS, A.nbW, A.nbW}, true);
+    const PartIdx p = part_of<3>(blockIdx.x, {A.nbXS, A.nbW, A.nbXW}, true);
     if (p.blk < 0) return;
     if (p.part == 0) part<SKF, 0, true>(lds, p.blk, A);
     else if (p.part == 1) part<SKF, 1, true>(lds, p.blk, A);

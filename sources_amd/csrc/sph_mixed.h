@@ -273,7 +273,7 @@ __device__ __forceinline__ CatMask cand_mask_f(const LaneRows& L, const Masks& M
 // column of 33k 56 -> 43, 64k 60 -> 47 (below 1M 5 of these from the posted flag).
 // body(v, lim): record chunks v and the squared distance it has yet to be within;
 // mask(R): the partner mask over the rows R = rows().
-template <int NCH, class L, class M, class A, class B>
+template <bool WIN, int NCH, class L, class M, class A, class B>
 __device__ __forceinline__ void visit_mx(unsigned char* lds, const Window& w, const IdxList& I, int n,
                                          const SubCtx& sc, int self, const RecQ& rec, float thr, L&& rows,
                                          M&& mask, A&& accept, B&& body)
@@ -284,7 +284,7 @@ __device__ __forceinline__ void visit_mx(unsigned char* lds, const Window& w, co
         for (int c = 0; c < NCH; ++c) v[c] = rec(k, c);
         body(v, INFINITY);
     };
-    if (w.lds) {
+    if (WIN && w.lds) {
         visit_window<NCH, float4>(lds, w, I, n, sc, 0, [&](const auto& v) { body(v, thr); });
         if (w.cnt < 0 && sc.valid) {   // a list that overflowed
             const LaneRows R = rows();
@@ -307,13 +307,13 @@ constexpr size_t MX_LDS = sizeof(float4) * NCH * WIN_STRIDE;
 // ------------------------------------------------------------------------
 // XM = 1: the same-phase terms (the cross terms come from the XM = 2 pass,
 // which runs first and stores them); XM = 2: the cross terms alone.
-template <int SKF, int XM>
+template <int SKF, int XM, bool WIN>
 __device__ __forceinline__ void water_a_mx(unsigned char* lds, int blk, DPhase W, DPhase S, const float* qW, float* qWw,
                                            const float* qS, NList NL, Masks MW, Grid g, KParams K, FusedK F, MixK X,
                                            int cross)
 {
     const RecQ QWv = recqv(qW, W.n), QSv = recqv(qS, S.n);
-    const SubCtx wc = sub_ctx(W.n, blk, 0, lanes_of_one(NL));
+    const SubCtx wc = sub_ctx(W.n, blk, 0, lanes_of_one(XM == 2 ? NL.ix : NL.is));
     const int t = wc.t;
     auto QA = [&](int c) { return QWv(wc.tt, c); };
     const float4 a0 = QA(0), a1 = QA(1), a2 = QA(2);
@@ -336,8 +336,8 @@ __device__ __forceinline__ void water_a_mx(unsigned char* lds, int blk, DPhase W
             const float cfa = (float)(vofa_d * rhoa_d * (-K.numeric_gravity) / K.s_perm);
             const float irhoa = a2.y;
             const KCf kx = make_kcf(SKF, F.uni_x ? 0.5 * ((double)me.h + (double)QSv(0, 0).w) : (double)me.h);
-            const Window win = open_window<true, 3>(lds, NL.ix, blk, wc, 0, W.n, QSv);
-            visit_mx<3>(lds, win, NL.ix, W.n, wc, -1, QSv, X.thr_x,
+            const Window win = open_window<WIN, 3>(lds, NL.ix, blk, wc, 0, W.n, QSv);
+            visit_mx<WIN, 3>(lds, win, NL.ix, W.n, wc, -1, QSv, X.thr_x,
                         [&] { return rows_of_cell(g, S.cell_start, me.cx, me.cy); },
                         [&](const LaneRows& R) { return cand_mask_f(R, NL.cross, W.n, wc.tt, -1, QSv, accx_q); },
                         accx_q, [&](const auto& v, float lim) {
@@ -375,7 +375,7 @@ __device__ __forceinline__ void water_a_mx(unsigned char* lds, int blk, DPhase W
         sep(me, b0, X.cs, dx, dy);
         return pred_f(uni, X.thr_w, dx * dx + dy * dy, me.h, b0.w, X.scale_k);
     };
-    const Window win = open_window<true, 2>(lds, NL.is, blk, wc, 0, W.n, QWv);
+    const Window win = open_window<WIN, 2>(lds, NL.is, blk, wc, 0, W.n, QWv);
     const bool real_a = W.itype[a] > 0;
     const float dspp = (float)W.dspp;
     Sum64 con, drd, txx, txy, tyy, avx, avy;
@@ -388,7 +388,7 @@ __device__ __forceinline__ void water_a_mx(unsigned char* lds, int blk, DPhase W
         MW.ovf[t] = cm.ovf;
         return cm;
     };
-    visit_mx<2>(lds, win, NL.is, W.n, wc, t, QWv, X.thr_w,
+    visit_mx<WIN, 2>(lds, win, NL.is, W.n, wc, t, QWv, X.thr_w,
                 [&] { return rows_of_cell(g, W.cell_start, me.cx, me.cy); }, mask_a, acc_q,
                 [&](const auto& v, float lim) {
         const float4 b0 = v[0], b1 = v[1];   // 1/rho and m/rho recomputed: two chunks per partner
@@ -443,7 +443,7 @@ __global__ STAGE_ATTR_MX void k_water_a_mx(DPhase W, DPhase S, const float* qW, 
                                            Masks MW, Grid g, KParams K, FusedK F, MixK X, int cross)
 {
     __shared__ __align__(16) unsigned char lds[MX_LDS<2>];
-    water_a_mx<SKF, 1>(lds, xcd_block(), W, S, qW, qWw, qS, NL, MW, g, K, F, X, cross);
+    water_a_mx<SKF, 1, true>(lds, xcd_block(), W, S, qW, qWw, qS, NL, MW, g, K, F, X, cross);
 }
 
 // The water side's cross terms (soil partners), before k_water_a_mx.
@@ -452,18 +452,18 @@ __global__ STAGE_ATTR void k_water_x_mx(DPhase W, DPhase S, const float* qW, flo
                                         Masks MW, Grid g, KParams K, FusedK F, MixK X, int cross)
 {
     __shared__ __align__(16) unsigned char lds[MX_LDS<3>];
-    water_a_mx<SKF, 2>(lds, xcd_block(), W, S, qW, qWw, qS, NL, MW, g, K, F, X, cross);
+    water_a_mx<SKF, 2, true>(lds, xcd_block(), W, S, qW, qWw, qS, NL, MW, g, K, F, X, cross);
 }
 
 // ------------------------------------------------------------------------
 // Stage B, water (mixed): momentum, art_visc, delta_sph(vof).
 // ------------------------------------------------------------------------
-template <int SKF>
+template <int SKF, bool WIN>
 __device__ __forceinline__ void water_b_mx(unsigned char* lds, int blk, DPhase W, const float* qW, NList NL, Masks MW,
                                            Grid g, KParams K, FusedK F, MixK X, int mask)
 {
     const RecQ QWv = recqv(qW, W.n);
-    const SubCtx wc = sub_ctx(W.n, blk, 0, lanes_of_one(NL));
+    const SubCtx wc = sub_ctx(W.n, blk, 0, lanes_of_one(NL.is));
     const int t = wc.t;
     auto QA = [&](int c) { return QWv(wc.tt, c); };
     const float4 a0 = QA(0), a1 = QA(1), a2 = QA(2), a3 = QA(3);
@@ -478,11 +478,11 @@ __device__ __forceinline__ void water_b_mx(unsigned char* lds, int blk, DPhase W
         sep(me, b0, X.cs, dx, dy);
         return pred_f(uni, X.thr_w, dx * dx + dy * dy, me.h, b0.w, X.scale_k);
     };
-    const Window win = open_window<true, 4>(lds, NL.is, blk, wc, 0, W.n, QWv);
+    const Window win = open_window<WIN, 4>(lds, NL.is, blk, wc, 0, W.n, QWv);
     const float et2 = (float)(K.etq * K.etq);
     const float beta = (float)K.beta, alpha = (float)K.alpha;
     Sum64 Px, Py, Sxx, Sxyy, Sxyx, Syy, artx, arty, dvd;
-    visit_mx<4>(lds, win, NL.is, W.n, wc, t, QWv, X.thr_w,
+    visit_mx<WIN, 4>(lds, win, NL.is, W.n, wc, t, QWv, X.thr_w,
                 [&] { return rows_of_cell(g, W.cell_start, me.cx, me.cy); },
                 [&](const LaneRows&) { return mask_of(MW, W.n, t); }, acc_q, [&](const auto& v, float lim) {
         const float4 b0 = v[0], b1 = v[1], b2 = v[2], b3 = v[3];
@@ -542,7 +542,7 @@ __global__ STAGE_ATTR_MX void k_water_b_mx(DPhase W, const float* qW, NList NL, 
                                            MixK X, int mask)
 {
     __shared__ __align__(16) unsigned char lds[MX_LDS<4>];
-    water_b_mx<SKF>(lds, xcd_block(), W, qW, NL, MW, g, K, F, X, mask);
+    water_b_mx<SKF, true>(lds, xcd_block(), W, qW, NL, MW, g, K, F, X, mask);
 }
 
 // ------------------------------------------------------------------------
@@ -553,13 +553,13 @@ __global__ STAGE_ATTR_MX void k_water_b_mx(DPhase W, const float* qW, NList NL, 
 // ------------------------------------------------------------------------
 // XM = 1: the same-phase terms and the tail (the cross terms from the XM = 2
 // pass, which runs first and stores them); XM = 2: the cross terms alone.
-template <int SKF, int XM>
+template <int SKF, int XM, bool WIN>
 __device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S, DPhase W, const float* qS,
                                            const float* qW, NList NL, Grid g, KParams K, FusedK F, MixK X, int cross,
                                            int mask)
 {
     const RecQ QSv = recqv(qS, S.n), QWv = recqv(qW, W.n);
-    const SubCtx wc = sub_ctx(S.n, blk, 0, lanes_of_one(NL));
+    const SubCtx wc = sub_ctx(S.n, blk, 0, lanes_of_one(XM == 2 ? NL.ix : NL.is));
     const int t = wc.t;
     auto QA = [&](int c) { return QSv(wc.tt, c); };
     const float4 a0 = QA(0), a1 = QA(1), a2 = QA(2), a3 = QA(3);
@@ -588,8 +588,8 @@ __device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S
         };
         const float cfs = (float)(vofa_d * (-K.numeric_gravity) / K.s_perm);
         const KCf kx = make_kcf(SKF, F.uni_x ? 0.5 * ((double)QWv(0, 0).w + (double)me.h) : (double)me.h);
-        const Window win = open_window<true, 3>(lds, NL.ix, blk, wc, 0, S.n, QWv);
-        visit_mx<3>(lds, win, NL.ix, S.n, wc, -1, QWv, X.thr_x,
+        const Window win = open_window<WIN, 3>(lds, NL.ix, blk, wc, 0, S.n, QWv);
+        visit_mx<WIN, 3>(lds, win, NL.ix, S.n, wc, -1, QWv, X.thr_x,
                     [&] { return rows_of_cell(g, W.cell_start, me.cx, me.cy); },
                     [&](const LaneRows& R) { return cand_mask_f(R, NL.cross, S.n, wc.tt, -1, QWv, accx_q); }, accx_q,
                     [&](const auto& v, float lim) {
@@ -632,14 +632,14 @@ __device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S
         sep(me, b0, X.cs, dx, dy);
         return pred_f(uni, X.thr_s, dx * dx + dy * dy, me.h, b0.w, X.scale_k);
     };
-    const Window win = open_window<true, 4>(lds, NL.is, blk, wc, 0, S.n, QSv);
+    const Window win = open_window<WIN, 4>(lds, NL.is, blk, wc, 0, S.n, QSv);
     const float et2 = (float)(K.etq * K.etq);
     const float beta = (float)K.beta, alpha = (float)K.alpha;
     Sum64 con, drd, txx, txy, tyy, vcc, wxy, avx, avy;
     Sum64 Fx, Fy, artx, arty, dP, dXX, dXY, dYY;
     float repx = 0.0f, repy = 0.0f;
     int cnt = 0;
-    visit_mx<4>(lds, win, NL.is, S.n, wc, t, QSv, X.thr_s,
+    visit_mx<WIN, 4>(lds, win, NL.is, S.n, wc, t, QSv, X.thr_s,
                 [&] { return rows_of_cell(g, S.cell_start, me.cx, me.cy); },
                 [&](const LaneRows& R) { return cand_mask_f(R, NL.same, S.n, wc.tt, t, QSv, acc_q); }, acc_q,
                 [&](const auto& v, float lim) {
@@ -770,7 +770,7 @@ __global__ STAGE_ATTR_MX_AB void k_soil_ab_mx(DPhase S, DPhase W, const float* q
                                               KParams K, FusedK F, MixK X, int cross, int mask)
 {
     __shared__ __align__(16) unsigned char lds[MX_LDS<4>];
-    soil_ab_mx<SKF, 1>(lds, xcd_block(), S, W, qS, qW, NL, g, K, F, X, cross, mask);
+    soil_ab_mx<SKF, 1, true>(lds, xcd_block(), S, W, qS, qW, NL, g, K, F, X, cross, mask);
 }
 
 // The soil side's cross terms (water partners), before k_soil_ab_mx.
@@ -779,10 +779,11 @@ __global__ STAGE_ATTR void k_soil_x_mx(DPhase S, DPhase W, const float* qS, cons
                                        KParams K, FusedK F, MixK X, int cross, int mask)
 {
     __shared__ __align__(16) unsigned char lds[MX_LDS<3>];
-    soil_ab_mx<SKF, 2>(lds, xcd_block(), S, W, qS, qW, NL, g, K, F, X, cross, mask);
+    soil_ab_mx<SKF, 2, true>(lds, xcd_block(), S, W, qS, qW, NL, g, K, F, X, cross, mask);
 }
 
-// The launches of a whole step (k_stage1, k_stage2), mixed.
+// The launches of a whole step (k_stage1, k_stage2), mixed.  WIN: with index lists
+// (without, no LDS: 250k slope with the lists off, ...).
 struct StageArgsMx {
     DPhase W, S;
     float *qW, *qS;
@@ -793,40 +794,40 @@ struct StageArgsMx {
     FusedK F;
     MixK X;
     int mask_w, mask_s;
-    int nbW, nbS;
+    int nbW, nbS, nbXW, nbXS;
     FlagPost post;
 };
 
-template <int SKF>
+template <int SKF, bool WIN>
 __device__ __forceinline__ void stage1_mx(int l, const StageArgsMx& A, bool spread)
 {
-    __shared__ __align__(16) unsigned char lds[MX_LDS<3>];
+    __shared__ __align__(16) unsigned char lds[WIN ? MX_LDS<3> : sizeof(float4)];
     post_flag(A.post, l);
-    const PartIdx p = part_of<3>(l, {A.nbS, A.nbW, A.nbW}, spread);
+    const PartIdx p = part_of<3>(l, {A.nbXS, A.nbW, A.nbXW}, spread);
     if (p.blk < 0) return;
-    if (p.part == 0) soil_ab_mx<SKF, 2>(lds, p.blk, A.S, A.W, A.qS, A.qW, A.nS, A.gS, A.K, A.F, A.X, 1, A.mask_s);
-    else if (p.part == 1) water_a_mx<SKF, 1>(lds, p.blk, A.W, A.S, A.qW, A.qW, A.qS, A.nW, A.MW, A.gW, A.K, A.F, A.X, 1);
-    else water_a_mx<SKF, 2>(lds, p.blk, A.W, A.S, A.qW, A.qW, A.qS, A.nW, A.MW, A.gW, A.K, A.F, A.X, 1);
+    if (p.part == 0) soil_ab_mx<SKF, 2, WIN>(lds, p.blk, A.S, A.W, A.qS, A.qW, A.nS, A.gS, A.K, A.F, A.X, 1, A.mask_s);
+    else if (p.part == 1) water_a_mx<SKF, 1, WIN>(lds, p.blk, A.W, A.S, A.qW, A.qW, A.qS, A.nW, A.MW, A.gW, A.K, A.F, A.X, 1);
+    else water_a_mx<SKF, 2, WIN>(lds, p.blk, A.W, A.S, A.qW, A.qW, A.qS, A.nW, A.MW, A.gW, A.K, A.F, A.X, 1);
 }
 
-template <int SKF>
+template <int SKF, bool WIN>
 __device__ __forceinline__ void stage2_mx(int l, const StageArgsMx& A, bool spread)
 {
-    __shared__ __align__(16) unsigned char lds[MX_LDS<4>];
+    __shared__ __align__(16) unsigned char lds[WIN ? MX_LDS<4> : sizeof(float4)];
     const PartIdx p = part_of<2>(l, {A.nbS, A.nbW}, spread);
     if (p.blk < 0) return;
-    if (p.part == 0) soil_ab_mx<SKF, 1>(lds, p.blk, A.S, A.W, A.qS, A.qW, A.nS, A.gS, A.K, A.F, A.X, 1, A.mask_s);
-    else water_b_mx<SKF>(lds, p.blk, A.W, A.qW, A.nW, A.MW, A.gW, A.K, A.F, A.X, A.mask_w);
+    if (p.part == 0) soil_ab_mx<SKF, 1, WIN>(lds, p.blk, A.S, A.W, A.qS, A.qW, A.nS, A.gS, A.K, A.F, A.X, 1, A.mask_s);
+    else water_b_mx<SKF, WIN>(lds, p.blk, A.W, A.qW, A.nW, A.MW, A.gW, A.K, A.F, A.X, A.mask_w);
 }
 
-template <int SKF>
+template <int SKF, bool WIN>
 __global__ STAGE_ATTR_MX void k_stage1_mx(StageArgsMx A)
 {
-    stage1_mx<SKF>(blockIdx.x, A, true);
+    stage1_mx<SKF, WIN>(blockIdx.x, A, true);
 }
 
-template <int SKF>
+template <int SKF, bool WIN>
 __global__ STAGE_ATTR_MX_AB void k_stage2_mx(StageArgsMx A)
 {
-    stage2_mx<SKF>(blockIdx.x, A, true);
+    stage2_mx<SKF, WIN>(blockIdx.x, A, true);
 }

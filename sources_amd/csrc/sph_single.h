@@ -28,21 +28,6 @@
 #pragma once
 #include "sph_fused.h"
 
-// Candidate bits of lane sub: every 2^lg-th.
-__device__ __forceinline__ uint64_t sub_bits(int lg, int sub)
-{
-    const uint64_t pat = lg == 0 ? ~0ull : lg == 1 ? 0x5555555555555555ull : lg == 2 ? 0x1111111111111111ull
-                                                                                     : 0x0101010101010101ull;
-    return pat << sub;
-}
-
-__device__ __forceinline__ uint64_t sub_or(int lg, uint64_t v)
-{
-    for (int o = 1; o < (1 << lg); o <<= 1)
-        v |= (uint64_t)__shfl_xor((unsigned long long)v, o, 64);
-    return v;
-}
-
 // Scan of the candidate rows by the lanes of a particle: the concatenated
 // mask of its own candidates (ovf: more than 128 in all).
 template <class A>
@@ -462,14 +447,13 @@ struct SoloEnd {
     int* err;
 };
 
-template <int SKF, bool U>
+template <int SKF, int FORM>
 __global__ __launch_bounds__(256) void k_solo_step(DPhase S, const double* recS, Grid g, KParams K, FusedK F, int mask,
                                                    int lg, SoloEnd E)
 {
-    __shared__ __align__(16) unsigned char lds[TABLE_LDS];
     NList NL{};
     NL.lg = lg;
-    soil_ab4<SKF, U, true>(lds, xcd_block(), S, recS, NL, g, K, F, 0, mask, E.ahead);
+    soil_ab4<SKF, FORM, true>(nullptr, xcd_block(), S, recS, NL, g, K, F, 0, mask, E.ahead);
     if (!E.update) return;
     const SubCtx sc = sub_ctx(S.n, xcd_block(), lg, STAGE_BLOCK);
     const bool own = sc.valid && !sc.sub;

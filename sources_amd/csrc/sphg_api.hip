@@ -1140,7 +1140,12 @@ struct FinalArgs {
 // link_list's reach is tested per pair, outside the windows).
 NList nlist_of(const sphg_ctx* c, const PhaseBuf& b, bool nl)
 {
-    if (!nl) return NList{};
+    if (!nl) {
+        NList none{};
+        none.lg = b.lg;
+        none.is.pb = none.ix.pb = STAGE_BLOCK >> b.lg;
+        return none;
+    }
     NList L{b.nl_same, b.nl_cross, b.nl_cell, b.il_same, b.il_cross, b.lg};
     L.is.lds = c->P.nnps != 2;
     L.ix.lds = 1;
@@ -1148,6 +1153,37 @@ NList nlist_of(const sphg_ctx* c, const PhaseBuf& b, bool nl)
 }
 
 int pad8(int nb) { return (nb + 7) & ~7; }
+
+// Which parts of a step have one smoothing length for all their pairs (then
+// hsml(1) is every h), integer repulsion exponents and Drucker-Prager: the soil's
+// same-phase pass, the water's, and the cross passes (smoothing lengths alone).
+struct UniformParts {
+    bool s, w, x;
+};
+
+bool integer_exponents(const sphg_ctx* c) { return c->K.ip1 >= 0 && c->K.ip2 >= 0; }
+
+UniformParts uniform_parts(const sphg_ctx* c)
+{
+    const bool rep_int = integer_exponents(c);
+    return UniformParts{c->ph[1].hmin == c->ph[1].hmax && rep_int && c->K.yield_criterion != 1,
+                        c->ph[0].hmin == c->ph[0].hmax && rep_int, c->F.uni_x != 0};
+}
+
+// The form of a pass over candidates I (lg: lanes per particle; plain: its terms
+// are not GENERAL's).
+int form_of(bool uniform, bool plain, const IdxList& I, int lg)
+{
+    if (!uniform) return plain ? VARYING : GENERAL;
+    return I.li && I.lds && I.pb << lg == WIN_LANES ? WINDOWS : UNIFORM;
+}
+
+// The kernel of a form (varying: the passes without GENERAL's terms).
+template <class K>
+K kernel_of(int form, K varying, K uniform, K windows)
+{
+    return form == WINDOWS ? windows : form == UNIFORM ? uniform : varying;
+}
 
 // Both phases' final kernels in one launch (after stages on one stream).
 int launch_finals(sphg_ctx* c, const FinalArgs& f)
@@ -1161,24 +1197,29 @@ int launch_finals(sphg_ctx* c, const FinalArgs& f)
     return launch(c, "finals", k_finals, pad8(A.nbS) + pad8(A.nbW), TPB, A);
 }
 
-// The stages of a step of a learned run (us, uw, ux: which parts are uniform).
+// The stages of a step of a learned run.
 template <int SKF>
-int stages_learned(sphg_ctx* c, const FinalArgs* fin, bool us, bool uw, bool ux)
+int stages_learned(sphg_ctx* c, const FinalArgs* fin)
 {
     PhaseBuf& W = c->ph[0];
     PhaseBuf& S = c->ph[1];
     const bool nl = nl_mode(c);
     const NList nW = nlist_of(c, W, nl), nS = nlist_of(c, S, nl);
-    StageArgs A{W.d,  S.d,  W.rec,        S.rec,        nW, nS, nl ? c->gvl[0] : c->gl[0], nl ? c->gvl[1] : c->gl[1],
-                c->K, c->F, mask_b(c, 0), mask_b(c, 1), 0,  nblk(W.n, lanes_of_one(nW)), nblk(S.n, lanes_of_one(nS)),
-                take_post(c)};
-    const bool all = us && uw && ux;
+    StageArgs A{W.d,  S.d,  W.rec,        S.rec,        nW, nS, W.masks, nl ? c->gvl[0] : c->gl[0], nl ? c->gvl[1] : c->gl[1],
+                c->K, c->F, mask_b(c, 0), mask_b(c, 1), 0,
+                nblk(W.n, lanes_of_one(nW.is)), nblk(S.n, lanes_of_one(nS.is)), nblk(W.n, lanes_of_one(nW.ix)),
+                nblk(S.n, lanes_of_one(nS.ix)), take_post(c)};
+    const UniformParts u = uniform_parts(c);
+    const bool all = u.s && u.w && u.x;
+    auto part = [&](const char* name, bool uniform, void (*t)(StageArgs), void (*f)(StageArgs), int nb) {
+        return launch(c, name, uniform ? t : f, nb, STAGE_BLOCK, A);
+    };
     if (all) {
-        RC(launch(c, "stage1", learned::k_stage1<SKF>, pad8(A.nbS) + 2 * pad8(A.nbW), STAGE_BLOCK, A));
+        RC(launch(c, "stage1", learned::k_stage1<SKF>, pad8(A.nbXS) + pad8(A.nbW) + pad8(A.nbXW), STAGE_BLOCK, A));
     } else {
-        RC(launch(c, "soil_x", ux ? learned::k_part<SKF, 0, true> : learned::k_part<SKF, 0, false>, A.nbS, STAGE_BLOCK, A));
-        RC(launch(c, "water_a", uw ? learned::k_part<SKF, 1, true> : learned::k_part<SKF, 1, false>, A.nbW, STAGE_BLOCK, A));
-        RC(launch(c, "water_x", ux ? learned::k_part<SKF, 2, true> : learned::k_part<SKF, 2, false>, A.nbW, STAGE_BLOCK, A));
+        RC(part("soil_x", u.x, learned::k_part<SKF, 0, true>, learned::k_part<SKF, 0, false>, A.nbXS));
+        RC(part("water_a", u.w, learned::k_part<SKF, 1, true>, learned::k_part<SKF, 1, false>, A.nbW));
+        RC(part("water_x", u.x, learned::k_part<SKF, 2, true>, learned::k_part<SKF, 2, false>, A.nbXW));
     }
     swap_c(W);
     swap_c(S);
@@ -1187,8 +1228,8 @@ int stages_learned(sphg_ctx* c, const FinalArgs* fin, bool us, bool uw, bool ux)
     if (all) {
         RC(launch(c, "stage2", learned::k_stage2<SKF>, pad8(A.nbS) + pad8(A.nbW), STAGE_BLOCK, A));
     } else {
-        RC(launch(c, "soil_ab", us ? learned::k_part<SKF, 3, true> : learned::k_part<SKF, 3, false>, A.nbS, STAGE_BLOCK, A));
-        RC(launch(c, "water_b", uw ? learned::k_part<SKF, 4, true> : learned::k_part<SKF, 4, false>, A.nbW, STAGE_BLOCK, A));
+        RC(part("soil_ab", u.s, learned::k_part<SKF, 3, true>, learned::k_part<SKF, 3, false>, A.nbS));
+        RC(part("water_b", u.w, learned::k_part<SKF, 4, true>, learned::k_part<SKF, 4, false>, A.nbW));
     }
     return fin ? launch_finals(c, *fin) : SPHG_OK;
 }
@@ -1204,7 +1245,6 @@ int stages_fused(sphg_ctx* c, const FinalArgs* fin)
     PhaseBuf& W = c->ph[0];
     PhaseBuf& S = c->ph[1];
     const int cross = c->P.single_phase ? 0 : 1;
-    const bool rep_int = c->K.ip1 >= 0 && c->K.ip2 >= 0;
     const double* rW = W.rec;
     const double* rS = S.rec;
     const bool nl = nl_mode(c);
@@ -1213,26 +1253,32 @@ int stages_fused(sphg_ctx* c, const FinalArgs* fin)
     const int lean = fin && fin->ahead && !fin->renorm ? 1 : 0;
     const NList nW = nlist_of(c, W, nl);
     const NList nS = nlist_of(c, S, nl);
-    const int nbW = nblk(W.n, WIN_LANES >> nW.lg), nbS = nblk(S.n, WIN_LANES >> nS.lg);
+    const int nbW = nblk(W.n, nW.is.pb), nbS = nblk(S.n, nS.is.pb);
+    const int nbXW = nblk(W.n, nW.ix.pb), nbXS = nblk(S.n, nS.ix.pb);
     const Grid& gW = nl ? c->gvl[0] : c->gl[0];
     const Grid& gS = nl ? c->gvl[1] : c->gl[1];
-    // U instantiations: h uniform in the phase(s) the kernel reads (then
-    // hsml(1) is every h), integer repulsion exponents, Drucker-Prager; the
-    // general ones read h per particle and partner
-    const bool us = c->ph[1].hmin == c->ph[1].hmax && rep_int && c->K.yield_criterion != 1;
-    const bool uw = c->ph[0].hmin == c->ph[0].hmax && rep_int;
-    const bool ux = c->F.uni_x != 0;
-    if (c->K.learned) return stages_learned<SKF>(c, fin, us, uw, ux);
-    if (us && uw && ux && cross && !c->prof) {
+    const UniformParts u = uniform_parts(c);
+    const bool rep_int = integer_exponents(c);
+    const int fS = form_of(u.s, rep_int && c->K.yield_criterion != 1, nS.is, nS.lg);
+    const int fW = form_of(u.w, rep_int, nW.is, nW.lg);
+    const int fWb = form_of(W.hmin == W.hmax, true, nW.is, nW.lg);   // (water_b has no repulsion)
+    const int fXS = form_of(u.x, true, nS.ix, nS.lg), fXW = form_of(u.x, true, nW.ix, nW.lg);
+    if (c->K.learned) return stages_learned<SKF>(c, fin);
+    if (u.s && u.w && u.x && cross && !c->prof) {
         // three launches on one stream (the profile times the passes apart)
-        StageArgs A{W.d,  S.d,  W.rec,        S.rec,        nW,   nS,  gW,  gS,
-                    c->K, c->F, mask_b(c, 0), mask_b(c, 1), lean, nbW, nbS, take_post(c)};
-        RC(launch(c, "stage1", k_stage1<SKF>, pad8(nbS) + 2 * pad8(nbW), STAGE_BLOCK, A));
+        StageArgs A{W.d,  S.d,  W.rec,        S.rec,        nW,   nS,  W.masks, gW, gS,
+                    c->K, c->F, mask_b(c, 0), mask_b(c, 1), lean, nbW, nbS, nbXW, nbXS, take_post(c)};
+        const bool ws = fS == WINDOWS && fW == WINDOWS, wx = fXS == WINDOWS && fXW == WINDOWS;
+        RC(launch(c, "stage1",
+                  !wx ? k_stage1<SKF, UNIFORM, UNIFORM> : ws ? k_stage1<SKF, WINDOWS, WINDOWS>
+                                                             : k_stage1<SKF, UNIFORM, WINDOWS>,
+                  pad8(nbXS) + pad8(nbW) + pad8(nbXW), STAGE_BLOCK, A));
         swap_c(W);
         swap_c(S);
         A.W = W.d;
         A.S = S.d;
-        RC(launch(c, "stage2", k_stage2<SKF>, pad8(nbS) + pad8(nbW), STAGE_BLOCK, A));
+        RC(launch(c, "stage2", ws ? k_stage2<SKF, WINDOWS> : k_stage2<SKF, UNIFORM>, pad8(nbS) + pad8(nbW),
+                  STAGE_BLOCK, A));
         return fin ? launch_finals(c, *fin) : SPHG_OK;
     }
     RC(post_now(c));
@@ -1243,38 +1289,33 @@ int stages_fused(sphg_ctx* c, const FinalArgs* fin)
     const bool split = fin && fork.open;
     {
         SideScope side(c);
-        if (cross) {
-            if (ux) RC(launch(c, "soil_x", k_soil_x4<SKF, true>, nbS, STAGE_BLOCK, S.d, W.d, rS, rW,
-                              nS, gS, c->K, c->F, lean));
-            else RC(launch(c, "soil_x", k_soil_x4<SKF, false>, nbS, STAGE_BLOCK, S.d, W.d, rS, rW,
-                           nS, gS, c->K, c->F, lean));
-        }
+        if (cross)
+            RC(launch(c, "soil_x",
+                      kernel_of(fXS, k_soil_x4<SKF, VARYING>, k_soil_x4<SKF, UNIFORM>, k_soil_x4<SKF, WINDOWS>), nbXS,
+                      STAGE_BLOCK, S.d, W.d, rS, rW, nS, gS, c->K, c->F, lean));
         if (split) HIPCHK(c, hipEventRecord(c->ev_sx, c->side));
-        if (us) RC(launch(c, "soil_ab", k_soil_ab4<SKF, true>, nbS, STAGE_BLOCK, S.d, rS,
-                          nS, gS, c->K, c->F, cross, mask_b(c, 1), lean));
-        else RC(launch(c, "soil_ab", k_soil_ab4<SKF, false>, nbS, STAGE_BLOCK, S.d, rS,
-                       nS, gS, c->K, c->F, cross, mask_b(c, 1), lean));
+        RC(launch(c, "soil_ab",
+                  fS == GENERAL ? k_soil_ab4<SKF, GENERAL>
+                                : kernel_of(fS, k_soil_ab4<SKF, VARYING>, k_soil_ab4<SKF, UNIFORM>, k_soil_ab4<SKF, WINDOWS>), nbS,
+                  STAGE_BLOCK, S.d, rS, nS, gS, c->K, c->F, cross, mask_b(c, 1), lean));
     }
     // water stage A, then the water cross terms (before stage B, whose tail
     // adds them): beside the soil side's cross pass and then its stage,
     // each pair of concurrent kernels reads the same phase's records
-    if (uw) RC(launch(c, "water_a", k_water_a4<SKF, true>, nbW, STAGE_BLOCK, W.d, rW, W.rec,
-                      nW, gW, c->K, c->F, cross, lean));
-    else RC(launch(c, "water_a", k_water_a4<SKF, false>, nbW, STAGE_BLOCK, W.d, rW, W.rec,
-                   nW, gW, c->K, c->F, cross, lean));
-    if (cross) {
-        if (ux) RC(launch(c, "water_x", k_water_x4<SKF, true>, nbW, STAGE_BLOCK, W.d, S.d, rW, rS,
-                          nW, gW, c->K, c->F, lean));
-        else RC(launch(c, "water_x", k_water_x4<SKF, false>, nbW, STAGE_BLOCK, W.d, S.d, rW, rS,
-                       nW, gW, c->K, c->F, lean));
-    }
+    RC(launch(c, "water_a",
+              fW == GENERAL ? k_water_a4<SKF, GENERAL>
+                            : kernel_of(fW, k_water_a4<SKF, VARYING>, k_water_a4<SKF, UNIFORM>, k_water_a4<SKF, WINDOWS>), nbW,
+              STAGE_BLOCK, W.d, rW, W.rec, nW, W.masks, gW, c->K, c->F, cross, lean));
+    if (cross)
+        RC(launch(c, "water_x",
+                  kernel_of(fXW, k_water_x4<SKF, VARYING>, k_water_x4<SKF, UNIFORM>, k_water_x4<SKF, WINDOWS>), nbXW,
+                  STAGE_BLOCK, W.d, S.d, rW, rS, nW, gW, c->K, c->F, lean));
     if (split) HIPCHK(c, hipEventRecord(c->ev_wx, c->stream));
     swap_c(W);
     swap_c(S);
-    if (uw) RC(launch(c, "water_b", k_water_b4<SKF, true>, nbW, STAGE_BLOCK, W.d, rW, nW,
-                      gW, c->K, c->F, mask_b(c, 0)));
-    else RC(launch(c, "water_b", k_water_b4<SKF, false>, nbW, STAGE_BLOCK, W.d, rW, nW,
-                   gW, c->K, c->F, mask_b(c, 0)));
+    RC(launch(c, "water_b",
+              kernel_of(fWb, k_water_b4<SKF, VARYING>, k_water_b4<SKF, UNIFORM>, k_water_b4<SKF, WINDOWS>), nbW,
+              STAGE_BLOCK, W.d, rW, nW, W.masks, gW, c->K, c->F, mask_b(c, 0)));
     if (fin) {
         auto final_water = [&]() -> int {
             if (fin->ahead)
@@ -1319,7 +1360,9 @@ int stages_soil_only(sphg_ctx* c, const SoloEnd& end)
 {
     PhaseBuf& S = c->ph[1];
     const int lg = solo_lanes(S.n), nb = nblk(S.n, STAGE_BLOCK >> lg);
-    auto kern = S.hmin == S.hmax && c->K.yield_criterion != 1 ? k_solo_step<SKF, true> : k_solo_step<SKF, false>;
+    auto kern = c->K.yield_criterion == 1 ? k_solo_step<SKF, GENERAL>
+                : S.hmin == S.hmax        ? k_solo_step<SKF, UNIFORM>
+                                          : k_solo_step<SKF, VARYING>;
     return launch(c, "soil_ab", kern, nb, STAGE_BLOCK, S.d, (const double*)S.rec, c->gl[1], c->K, c->F, mask_b(c, 1),
                   lg, end);
 }
@@ -1378,20 +1421,23 @@ int stages_mixed(sphg_ctx* c, const FinalArgs* fin)
         // all lanes of a workgroup (not the windows' 192 of 256)
         for (NList* L : {&nW, &nS}) L->is = L->ix = IdxList{};
     }
-    const int nbW = nblk(W.n, lanes_of_one(nW)), nbS = nblk(S.n, lanes_of_one(nS));
+    const int nbW = nblk(W.n, lanes_of_one(nW.is)), nbS = nblk(S.n, lanes_of_one(nS.is));
+    const int nbXW = nblk(W.n, lanes_of_one(nW.ix)), nbXS = nblk(S.n, lanes_of_one(nS.ix));
     const Grid& gW = nl ? c->gvl[0] : c->gl[0];
     const Grid& gS = nl ? c->gvl[1] : c->gl[1];
     MixK X = c->X;
     if (nl) X.cs = (float)c->csv;
     if (!c->prof) {
         StageArgsMx A{W.d, S.d, qW, qS, nW, nS, W.masks, gW, gS, c->K, c->F, X, mask_b(c, 0), mask_b(c, 1),
-                      nbW, nbS, take_post(c)};
-        RC(launch(c, "stage1", k_stage1_mx<SKF>, pad8(A.nbS) + 2 * pad8(A.nbW), STAGE_BLOCK, A));
+                      nbW, nbS, nbXW, nbXS, take_post(c)};
+        const bool win = nW.is.li != nullptr;   // (all four lists, or none)
+        RC(launch(c, "stage1", win ? k_stage1_mx<SKF, true> : k_stage1_mx<SKF, false>, pad8(nbXS) + pad8(nbW) + pad8(nbXW), STAGE_BLOCK, A));
         swap_c(W);
         swap_c(S);
         A.W = W.d;
         A.S = S.d;
-        RC(launch(c, "stage2", k_stage2_mx<SKF>, pad8(A.nbS) + pad8(A.nbW), STAGE_BLOCK, A));
+        RC(launch(c, "stage2", win ? k_stage2_mx<SKF, true> : k_stage2_mx<SKF, false>, pad8(nbS) + pad8(nbW),
+                  STAGE_BLOCK, A));
         return fin ? launch_finals(c, *fin) : SPHG_OK;
     }
     RC(post_now(c));
@@ -1400,7 +1446,7 @@ int stages_mixed(sphg_ctx* c, const FinalArgs* fin)
     {
         // the cross terms in a pass of their own before the same-phase pass
         SideScope side(c);
-        RC(launch(c, "soil_x", k_soil_x_mx<SKF>, nbS, STAGE_BLOCK, S.d, W.d, (const float*)qS,
+        RC(launch(c, "soil_x", k_soil_x_mx<SKF>, nbXS, STAGE_BLOCK, S.d, W.d, (const float*)qS,
                   (const float*)qW, nS, gS, c->K, c->F, X, 1, mask_b(c, 1)));
         RC(launch(c, "soil_ab", k_soil_ab_mx<SKF>, nbS, STAGE_BLOCK, S.d, W.d, (const float*)qS,
                   (const float*)qW, nS, gS, c->K, c->F, X, 1, mask_b(c, 1)));
@@ -1409,7 +1455,7 @@ int stages_mixed(sphg_ctx* c, const FinalArgs* fin)
     // then its stage, each pair of concurrent kernels reads one phase's records)
     RC(launch(c, "water_a", k_water_a_mx<SKF>, nbW, STAGE_BLOCK, W.d, S.d, (const float*)qW, qW,
               (const float*)qS, nW, W.masks, gW, c->K, c->F, X, 1));
-    RC(launch(c, "water_x", k_water_x_mx<SKF>, nbW, STAGE_BLOCK, W.d, S.d, (const float*)qW, qW,
+    RC(launch(c, "water_x", k_water_x_mx<SKF>, nbXW, STAGE_BLOCK, W.d, S.d, (const float*)qW, qW,
               (const float*)qS, nW, W.masks, gW, c->K, c->F, X, 1));
     swap_c(W);
     swap_c(S);
@@ -1441,21 +1487,30 @@ int build_nlists(sphg_ctx* c)
     PhaseBuf& S = c->ph[1];
     const DPhase& w = W.d;
     const DPhase& sd = S.d;
+    // the particles of a workgroup: all its lanes' where the passes of this
+    // context have no windows (1M slope with varying h: 75% of the lanes cost ...)
+    const UniformParts u = uniform_parts(c);
+    const bool mx = c->P.precision == SPHG_MIXED, all = c->F.uni_w && c->F.uni_s && c->F.uni_x;
+    auto groups = [](IdxList& l, bool windows, int lg) { l.pb = (windows ? WIN_LANES : STAGE_BLOCK) >> lg; };
+    groups(W.il_same, c->P.nnps != 2 && (mx ? all : u.w), W.lg);
+    groups(S.il_same, c->P.nnps != 2 && (mx ? all : u.s), S.lg);
+    groups(W.il_cross, u.x, W.lg);
+    groups(S.il_cross, u.x, S.lg);
     // the displacement trigger restarts (a past-the-skin bit stays for the check);
     // the rebuild has just permuted the state into cell order (no order lookups)
     RC(launch(c, "nlist", k_keep_bits, 1, TPB, c->d_nlflag, 2));
     RC(launch(c, "nlist", k_nlist, nblk(W.n, 256), 256, (const double*)w.x, (const double*)w.y,
               (const int*)nullptr, W.n, (const double*)w.x, (const double*)w.y, (const int*)nullptr,
-              (const int*)w.cell_start, c->gv, c->nl_thr[0], 1, W.nl_same, W.nl_cell, W.il_same, WIN_LANES >> W.lg));
+              (const int*)w.cell_start, c->gv, c->nl_thr[0], 1, W.nl_same, W.nl_cell, W.il_same, W.il_same.pb));
     RC(launch(c, "nlist", k_nlist, nblk(S.n, 256), 256, (const double*)sd.x, (const double*)sd.y,
               (const int*)nullptr, S.n, (const double*)sd.x, (const double*)sd.y, (const int*)nullptr,
-              (const int*)sd.cell_start, c->gv, c->nl_thr[1], 1, S.nl_same, S.nl_cell, S.il_same, WIN_LANES >> S.lg));
+              (const int*)sd.cell_start, c->gv, c->nl_thr[1], 1, S.nl_same, S.nl_cell, S.il_same, S.il_same.pb));
     RC(launch(c, "nlist", k_nlist, nblk(W.n, 256), 256, (const double*)w.x, (const double*)w.y,
               (const int*)nullptr, W.n, (const double*)sd.x, (const double*)sd.y, (const int*)nullptr,
-              (const int*)sd.cell_start, c->gv, c->nl_thr[2], 0, W.nl_cross, (int*)nullptr, W.il_cross, WIN_LANES >> W.lg));
+              (const int*)sd.cell_start, c->gv, c->nl_thr[2], 0, W.nl_cross, (int*)nullptr, W.il_cross, W.il_cross.pb));
     RC(launch(c, "nlist", k_nlist, nblk(S.n, 256), 256, (const double*)sd.x, (const double*)sd.y,
               (const int*)nullptr, S.n, (const double*)w.x, (const double*)w.y, (const int*)nullptr,
-              (const int*)w.cell_start, c->gv, c->nl_thr[2], 0, S.nl_cross, (int*)nullptr, S.il_cross, WIN_LANES >> S.lg));
+              (const int*)w.cell_start, c->gv, c->nl_thr[2], 0, S.nl_cross, (int*)nullptr, S.il_cross, S.il_cross.pb));
     c->nl_valid = true;
     c->nl_due = false;
     c->nl_rebuilt_at = c->nl_seq + 1;   // the step being issued
@@ -2451,7 +2506,7 @@ int build_graph(sphg_gnn* g, sphg_gnn::Graph& G)
         gnn::GatherOut O{G.nf, G.raw, G.nb, G.nd, G.n, G.tw, g->node_of_id[k], g->overflow};
         return args_of(gnn::k_gnn_gather, b.d, lists ? c->gvl[k] : c->gl[k], c->K, k == 0 ? c->F.thr_w : c->F.thr_s,
                        k == 0 ? c->F.uni_w : c->F.uni_s, k == 0 ? 0 : Wb.n, k, g->S, O,
-                       lists ? b.il_same : IdxList{}, WIN_LANES >> b.lg,
+                       lists ? b.il_same : IdxList{}, std::max(b.il_same.pb, 1),
                        lists ? (const int*)b.nl_cell : (const int*)nullptr);
     };
     return launch_pair<BodyGnnGather>(c, "gnn_gather", nblk(Wb.n), args(0), nblk(Sb.n), args(1));
@@ -3008,28 +3063,33 @@ void reg_batched(std::map<const void*, Batched>& m, void (*solo)(T...))
     m[reinterpret_cast<const void*>(solo)] = Batched{sizeof(ArgTup<T...>), &go_batched<F, T...>};
 }
 
+template <int SKF, int FORM>
+void reg_batched_form(std::map<const void*, Batched>& m)
+{
+    reg_batched<BodyWaterX<SKF, FORM>>(m, k_water_x4<SKF, FORM>);
+    reg_batched<BodySoilX<SKF, FORM>>(m, k_soil_x4<SKF, FORM>);
+    reg_batched<BodyWaterA<SKF, FORM>>(m, k_water_a4<SKF, FORM>);
+    reg_batched<BodyWaterB<SKF, FORM>>(m, k_water_b4<SKF, FORM>);
+    reg_batched<BodySoilAB<SKF, FORM>>(m, k_soil_ab4<SKF, FORM>);
+}
+
 template <int SKF>
 void reg_batched_skf(std::map<const void*, Batched>& m)
 {
-    reg_batched<BodyStage1<SKF>>(m, k_stage1<SKF>);
-    reg_batched<BodyStage2<SKF>>(m, k_stage2<SKF>);
-    reg_batched<BodyStage1Mx<SKF>>(m, k_stage1_mx<SKF>);
-    reg_batched<BodyStage2Mx<SKF>>(m, k_stage2_mx<SKF>);
-    reg_batched<BodyWaterX<SKF, true>>(m, k_water_x4<SKF, true>);
-    reg_batched<BodyWaterX<SKF, false>>(m, k_water_x4<SKF, false>);
-    reg_batched<BodySoilX<SKF, true>>(m, k_soil_x4<SKF, true>);
-    reg_batched<BodySoilX<SKF, false>>(m, k_soil_x4<SKF, false>);
-    reg_batched<BodyWaterA<SKF, true>>(m, k_water_a4<SKF, true>);
-    reg_batched<BodyWaterA<SKF, false>>(m, k_water_a4<SKF, false>);
-    reg_batched<BodyWaterB<SKF, true>>(m, k_water_b4<SKF, true>);
-    reg_batched<BodyWaterB<SKF, false>>(m, k_water_b4<SKF, false>);
-    reg_batched<BodySoilAB<SKF, true>>(m, k_soil_ab4<SKF, true>);
-    reg_batched<BodySoilAB<SKF, false>>(m, k_soil_ab4<SKF, false>);
-    reg_batched<BodyWaterAMx<SKF>>(m, k_water_a_mx<SKF>);
-    reg_batched<BodyWaterBMx<SKF>>(m, k_water_b_mx<SKF>);
-    reg_batched<BodySoilABMx<SKF>>(m, k_soil_ab_mx<SKF>);
-    reg_batched<BodyWaterXMx<SKF>>(m, k_water_x_mx<SKF>);
-    reg_batched<BodySoilXMx<SKF>>(m, k_soil_x_mx<SKF>);
+    reg_batched<BodyStage1<SKF, UNIFORM, UNIFORM>>(m, k_stage1<SKF, UNIFORM, UNIFORM>);
+    reg_batched<BodyStage1<SKF, UNIFORM, WINDOWS>>(m, k_stage1<SKF, UNIFORM, WINDOWS>);
+    reg_batched<BodyStage1<SKF, WINDOWS, WINDOWS>>(m, k_stage1<SKF, WINDOWS, WINDOWS>);
+    reg_batched<BodyStage2<SKF, UNIFORM>>(m, k_stage2<SKF, UNIFORM>);
+    reg_batched<BodyStage2<SKF, WINDOWS>>(m, k_stage2<SKF, WINDOWS>);
+    reg_batched_form<SKF, VARYING>(m);
+    reg_batched_form<SKF, UNIFORM>(m);
+    reg_batched_form<SKF, WINDOWS>(m);
+    reg_batched<BodyWaterA<SKF, GENERAL>>(m, k_water_a4<SKF, GENERAL>);
+    reg_batched<BodySoilAB<SKF, GENERAL>>(m, k_soil_ab4<SKF, GENERAL>);
+    reg_batched<BodyStage1Mx<SKF, true>>(m, k_stage1_mx<SKF, true>);
+    reg_batched<BodyStage1Mx<SKF, false>>(m, k_stage1_mx<SKF, false>);
+    reg_batched<BodyStage2Mx<SKF, true>>(m, k_stage2_mx<SKF, true>);
+    reg_batched<BodyStage2Mx<SKF, false>>(m, k_stage2_mx<SKF, false>);
 }
 
 // The kernels of a list-mode FP64 step between rebuilds (stages, finals).
