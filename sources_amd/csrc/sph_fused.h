@@ -19,11 +19,8 @@
 #pragma once
 #include "sph_kernels.h"
 
-// record slots (doubles)
-enum : int {
-    R_X = 0, R_Y, R_VX, R_VY, R_RHO, R_M, R_VOF, R_P, R_S3, R_C, R_S1, R_S2, R_H, R_IT, R_PAD0, R_PAD1,
-    R_STRIDE = 16
-};
+// doubles per record
+constexpr int R_STRIDE = 16;
 
 #ifndef SPHG_WPB
 #define SPHG_WPB 4           // waves per workgroup of the stage kernels (consecutive particles share a CU)
@@ -116,7 +113,7 @@ __device__ __forceinline__ KC make_kc(int skf, double h)
 }
 
 // The same for the mean smoothing length of one pair: one short reciprocal
-// instead of two divisions (those were a sixth of a stage's time where h varies).
+// instead of two divisions (2% of a step where h varies).
 template <int SKF>
 __device__ __forceinline__ KC pair_kc(double h)
 {
@@ -589,10 +586,10 @@ __global__ void k_step_soil(DPhase P, KParams K, double* rec, int first, float* 
 }
 
 // ------------------------------------------------------------------------
-// Partner masks of stage A, reused by stage B: per particle t a 128-bit mask
-// over its candidate list (the three cell rows of its 3 x 3 block, in cell
-// order, concatenated): m[t] low and m[n + t] high word, and an overflow
-// flag (rows walked directly).
+// Masks of candidates: per particle t a 128-bit mask over its candidate list
+// (the three cell rows of its 3 x 3 block, in cell order, concatenated, or its
+// index list): m[t] low and m[n + t] high word, and an overflow flag (more
+// candidates, or a row of over 64).
 // ------------------------------------------------------------------------
 struct Masks {
     uint64_t* m;   // [3][n] (the first two words are used)
@@ -603,14 +600,14 @@ struct Masks {
 // Neighbour lists with a skin (FP64 fused step).  At a rebuild the cell
 // list is built on a grid of cell size >= R + skin (R the largest support
 // radius), the records are written in its order, and every particle keeps
-// (a) the key of its cell, (b) a 128-bit mask over its candidate rows of the
-// candidates within R + skin (same phase and cross), and (c) its position.
-// The record order and the cell list then stay fixed until the next rebuild.
-// While no particle has moved more than skin / 2 from its rebuild position,
-// every pair within R lies in these masks, so each step tests only the
-// listed candidates with the exact predicate instead of scanning the rows.
+// (a) the key of its cell, (b) the candidates within R + skin (same phase and
+// cross), as a 128-bit mask over its candidate rows and as a list of indices,
+// and (c) its position.  The record order and the cell list then stay fixed
+// until the next rebuild.  While no particle has moved more than skin / 2 from
+// its rebuild position, every pair within R is listed, so each step tests only
+// these candidates with the exact predicate instead of scanning the rows.
 // ------------------------------------------------------------------------
-// The same candidates as positions in the window of the workgroup's particles:
+// The list: candidates as positions in the window of the workgroup's particles:
 // candidate j of record t is the window's record li[j * n + t], cnt[t] of them
 // (-1: more than cap, the rows are walked).  win: WIN_INTS per workgroup: the
 // first records of the window's three record ranges, their positions in it and
@@ -627,7 +624,7 @@ constexpr int WIN_CAP = 846;             // records of a window in LDS: two work
 constexpr int WIN_STRIDE = WIN_CAP + 1;  // (and the stand-in record)
 // Lanes of a workgroup that take particles where its window is to fit the LDS (all
 // of them otherwise).  The window holds three rows' worth
-// of them: 633 records on average and 848 at most for 192 particles of a
+// of them: 633 records on average (848 at most) for 192 particles of a
 // lattice at h = 1.2 dx (whose cell rows hold two or three lattice rows); with
 // 240 particles one window in four does not fit, and its workgroup takes the
 // slow path at the occupancy the LDS leaves (1M slope, soil_ab 117 us against
@@ -708,8 +705,7 @@ template <class T>
 __device__ __forceinline__ T pick(bool c, T x, T y) { return c ? x : y; }
 
 // Iterator over the set bits of a CatMask; branch-free apart from the loop.
-// next() returns the record index of the next partner (-1 at the end) and
-// i = the index in the staged copy (record index + base of its row).
+// next() returns the record index of the next partner (-1 at the end).
 struct CatIter {
     uint64_t lo, hi;
     int s1, s2;        // start of row 1 and row 2 in the concatenated list
@@ -910,15 +906,21 @@ __global__ __launch_bounds__(256) void k_nlist(const double* xA, const double* y
 // Otherwise (no lists, smoothing lengths that vary, link_list's reach, a
 // window that does not fit): the candidates are the particle's list, or its
 // three candidate rows.  Four at a time their positions are tested with the
-// exact predicate, into a mask of 128 candidates; the dense loop goes through its
-// bits.
+// exact predicate, into a mask of 128 candidates in registers, and the dense loop
+// goes through its bits (water stage B takes the mask of stage A: with a test of its
+// own 72 us against 42 for 250k particles with varying h).  One lane per particle
+// starts from the rebuild's mask of listed candidates, whose rows it can index
+// without a load (900k particles with varying h: 476 us per step, through the index
+// list 557).
 // ------------------------------------------------------------------------
 // The forms of a stage kernel: WINDOWS as described, UNIFORM one smoothing length
 // for all pairs but no windows in LDS (no lists, or link_list's reach), VARYING
 // smoothing lengths that vary, GENERAL other than integer repulsion exponents or
 // Drucker-Prager (pow and the Mohr-Coulomb terms in the pair loop are 47 registers
-// of soil_ab's 204).  All but the first keep all lanes of a workgroup and take no
-// LDS.  1M ...
+// of soil_ab's 204).  All but WINDOWS keep all lanes of a workgroup and take no
+// LDS.  250k slope, us per step, with the windows' LDS and lanes for all -> this:
+// varying h 248 -> 157, link_list 153 -> 114, lists off 231 -> 172 (both 335 -> 237),
+// Mohr-Coulomb 164 -> 138, real exponents 177 -> 141.
 enum : int { GENERAL, VARYING, UNIFORM, WINDOWS };
 
 // Record index of a position of three concatenated ranges: starts s1 and s2

@@ -40,8 +40,6 @@
 #define STAGE_ATTR_MX_AB __launch_bounds__(STAGE_BLOCK)
 #endif
 
-
-
 // FP32 pair terms summed in FP64: a conversion and an add per term (with
 // packed FP32 off, FP32 and FP64 adds issue at the same rate, so this costs
 // half of a compensated FP32 sum and rounds only once per term, in FP64).
@@ -205,8 +203,8 @@ __device__ __forceinline__ void visit_f(const CatMask& cm, const LaneRows& L, in
     }
 }
 
-// The exact FP32 partner mask from a neighbour-list mask (as filter_mask of
-// the FP64 records): the listed candidates whose records pass accept(q0).
+// The exact FP32 partner mask from a neighbour-list mask: the listed
+// candidates whose records pass accept(q0).
 template <class A>
 __device__ __forceinline__ CatMask filter_mask_f(const LaneRows& L, const CatMask& vm, const RecQ& rec, A&& acc)
 {
@@ -782,8 +780,9 @@ __global__ STAGE_ATTR void k_soil_x_mx(DPhase S, DPhase W, const float* qS, cons
     soil_ab_mx<SKF, 2, true>(lds, xcd_block(), S, W, qS, qW, NL, g, K, F, X, cross, mask);
 }
 
-// The launches of a whole step (k_stage1, k_stage2), mixed.  WIN: with index lists
-// (without, no LDS: 250k slope with the lists off, ...).
+// The launches of a whole step (k_stage1, k_stage2), mixed.  WIN: with index lists;
+// without, no LDS and 127 registers instead of 166 in stage 2 (250k slope, us per
+// step: lists off 187 -> 172, varying h 134 -> 124).
 struct StageArgsMx {
     DPhase W, S;
     float *qW, *qS;

@@ -1234,11 +1234,10 @@ int stages_learned(sphg_ctx* c, const FinalArgs* fin)
     return fin ? launch_finals(c, *fin) : SPHG_OK;
 }
 
-// The fused step: pack (first_half + soil Drucker-Prager projections +
-// records), cross terms, partner masks, stage A, stage B.  The soil kernels
+// The stages of the fused step: cross terms, stage A, stage B.  The soil kernels
 // read only the packed records of both phases (the water pressure comes from
-// the pack): they run on the side stream while the water kernels run on the
-// main stream.
+// the pack): in one launch with the water's where both phases are uniform, else on
+// the side stream beside them.
 template <int SKF>
 int stages_fused(sphg_ctx* c, const FinalArgs* fin)
 {
@@ -1487,8 +1486,8 @@ int build_nlists(sphg_ctx* c)
     PhaseBuf& S = c->ph[1];
     const DPhase& w = W.d;
     const DPhase& sd = S.d;
-    // the particles of a workgroup: all its lanes' where the passes of this
-    // context have no windows (1M slope with varying h: 75% of the lanes cost ...)
+    // the particles of a workgroup: those of all its lanes where the passes of this
+    // context have no windows
     const UniformParts u = uniform_parts(c);
     const bool mx = c->P.precision == SPHG_MIXED, all = c->F.uni_w && c->F.uni_s && c->F.uni_x;
     auto groups = [](IdxList& l, bool windows, int lg) { l.pb = (windows ? WIN_LANES : STAGE_BLOCK) >> lg; };
