@@ -1420,7 +1420,7 @@ __device__ __forceinline__ void water_a4(unsigned char* lds, int blk, DPhase W, 
             const double f = (V * q.x) * (p.w * fast_rcp(rhoa + q.x));
             avx -= f * dvx;
             avy -= f * dvy;
-            if (q.y < 0.0 && p.dr <= rep2) {
+            if (q.y < 0.0 && p.dr <= rep2 && p.in) {
                 const double fr = rep_factor<FORM != GENERAL>(K, W.dspp, p.ir);
                 repx += p.dx * fr;
                 repy += p.dy * fr;
@@ -1725,7 +1725,7 @@ __device__ __forceinline__ void soil_ab4(unsigned char* lds, int blk, DPhase S, 
             const double fv = (m * p.w) * (it * d2);
             avx -= fv * dvx;
             avy -= fv * dvy;
-            if (!SOLO && q.y < 0.0 && p.dr <= rep2) {
+            if (!SOLO && q.y < 0.0 && p.dr <= rep2 && p.in) {
                 const double fr = rep_factor<FORM != GENERAL>(K, S.dspp, p.ir);
                 artx += p.dx * (0.5 * fr);
                 arty += p.dy * (0.5 * fr);

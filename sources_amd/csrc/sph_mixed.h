@@ -409,7 +409,7 @@ __device__ __forceinline__ void water_a_mx(unsigned char* lds, int blk, DPhase W
         const float f = mb * ww * (2.0f * __builtin_amdgcn_rcpf(rhoa + b1.z + X.rho0_w));
         avx.add(-(dvx * f));
         avy.add(-(dvy * f));
-        if (real_a && !(r > dspp) && __float_as_int(b0.z) < 0) {
+        if (real_a && !(r > dspp) && dr < lim && __float_as_int(b0.z) < 0) {
             const float q = dspp / r;
             const float fr = (__powf(q, (float)K.p1) - __powf(q, (float)K.p2)) * idr;
             repx += (float)K.dd * dx * fr;
@@ -667,7 +667,7 @@ __device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S
         const float f = mb * ww * rs;
         avx.add(-(dvx * f));
         avy.add(-(dvy * f));
-        if (real_a && !(r > dspp) && __float_as_int(b0.z) < 0) {
+        if (real_a && !(r > dspp) && dr < lim && __float_as_int(b0.z) < 0) {
             const float q = dspp / r;
             const float fr = (__powf(q, (float)K.p1) - __powf(q, (float)K.p2)) * idr;
             repx += (float)K.dd * dx * fr;
