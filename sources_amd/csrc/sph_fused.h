@@ -312,7 +312,15 @@ struct NRef {
     double trig, near, hard2, look;
     int rebuild;
     const int* cell;   // cell key per record slot since the rebuild (FP32 records)
+    int* bad;          // raised by a record with an infinity or a NaN
 };
+
+// Raises bad when one of the values is not finite.
+template <class... T>
+__device__ __forceinline__ void check_finite(int* bad, T... v)
+{
+    if (bad && !((... + ((T)0 * v)) == 0)) atomicOr(bad, 1);
+}
 
 __device__ __forceinline__ int record_cell(const NRef& R, int t) { return R.cell && !R.rebuild ? R.cell[t] : -1; }
 
@@ -390,6 +398,8 @@ __device__ __forceinline__ void pack_water_at(const DPhase& P, const KParams& K,
         write_q01(Q, pn, g, cs, x, y, P.hsml[i], it < 0, vx, vy, rho - K.w_rho0, m, record_cell(NR, t));
         Q[2 * pn] = make_float4((float)vof, (float)irho, (float)(m * irho), (float)p);
         Q[3 * pn] = make_float4((float)cn, 0.0f, 0.0f, 0.0f);
+        check_finite(NR.bad, (float)x, (float)y, (float)vx, (float)vy, (float)rho, (float)m, (float)vof, (float)irho, (float)(m * irho),
+                     (float)p, (float)cn);
         return;
     }
     double2* R = reinterpret_cast<double2*>(rec) + t;
@@ -398,6 +408,7 @@ __device__ __forceinline__ void pack_water_at(const DPhase& P, const KParams& K,
     R[1 * pn] = make_double2(vx, vy);
     const double V = m * irho;
     const double mv = K.learned ? m : V;
+    check_finite(NR.bad, x, y, vx, vy, rho, V, vof, p, cn);
     R[2 * pn] = make_double2(rho, it < 0 ? -mv : mv);   // the sign marks a virtual particle
     R[3 * pn] = make_double2(vof, p);
     R[4 * pn] = make_double2(0.0, cn);
@@ -525,6 +536,8 @@ __device__ __forceinline__ void pack_soil_at(const DPhase& P, const KParams& K, 
         write_q01(Q, pn, g, cs, x, y, P.hsml[i], it < 0, vx, vy, rho - K.s_rho0, m, record_cell(NR, t));
         Q[2 * pn] = make_float4((float)P.vof[i], (float)irho, (float)(m * irho), (float)p);
         Q[3 * pn] = make_float4((float)P.c[i], (float)sxx, (float)sxy, (float)syy);
+        check_finite(NR.bad, (float)x, (float)y, (float)vx, (float)vy, (float)rho, (float)m, (float)P.vof[i], (float)irho,
+                     (float)(m * irho), (float)p, (float)P.c[i], (float)sxx, (float)sxy, (float)syy);
         return;
     }
     double2* R = reinterpret_cast<double2*>(rec) + t;
@@ -533,6 +546,7 @@ __device__ __forceinline__ void pack_soil_at(const DPhase& P, const KParams& K, 
     R[1 * pn] = make_double2(vx, vy);
     const double V = m * irho;
     const double mv = K.learned ? m : V, vof = P.vof[i];
+    check_finite(NR.bad, x, y, vx, vy, rho, V, vof * irho, p, P.c[i], sxx, sxy, syy);
     R[2 * pn] = make_double2(rho, it < 0 ? -mv : mv);   // the sign marks a virtual particle
     R[3 * pn] = make_double2(K.learned ? vof : vof * irho, p);
     R[4 * pn] = make_double2(syy, P.c[i]);
@@ -617,6 +631,7 @@ struct IdxList {
     int *cnt, *win;
     int cap, lds;   // lds 0: the windows stay in global memory (predicates that need more than a distance)
     int pb;         // particles of a workgroup of the kernels that read it
+    int* bad;       // set: a record is not finite, candidates are tested before their terms
 };
 
 constexpr int WIN_INTS = 8;
@@ -893,7 +908,8 @@ __global__ __launch_bounds__(256) void k_nlist(const double* xA, const double* y
 // window's record chunks into LDS, then every lane goes through its list,
 // reading the partners there (the next partner's chunks in flight beside the
 // current one's terms); candidates outside the support (about one in six, in
-// the skin) are evaluated with W = s = 0.  What bound the gathers from global
+// the skin) are evaluated with W = s = 0 (once a record holds an infinity or a
+// NaN, which would count so, the candidates are tested first).  What bound the gathers from global
 // memory was the L1's tag lookups: a 64-lane 16-byte gather of such partners
 // takes 34 of them (one per cycle and CU; 16 for contiguous lanes), where the
 // same LDS read takes about 8 cycles.  The copy itself is contiguous.  What
@@ -967,6 +983,7 @@ __device__ __forceinline__ Ranges3 window_ranges(const int* w)
 struct Window {
     Ranges3 r;
     bool listed, lds;   // a list exists; the window is in LDS (or on its way)
+    bool bad;           // a record is not finite
     int cnt, k[4];      // lds: the lane's list length and first entries
 };
 
@@ -983,7 +1000,7 @@ __device__ __forceinline__ void visit_global(const Cand& C, const IdxList& I, co
                                              A&& accept, B&& body)
 {
     CatMask kept{0, 0, 1}, listed{0, 0, 1};
-    if (MODE == GIVEN) kept = mask_of(MW, n, sc.tt);
+    if (MODE == GIVEN && !w.bad) kept = mask_of(MW, n, sc.tt);   // (bad: stage A may have had its window)
     if (LM.m && lg == 0) listed = mask_of(LM, n, sc.tt);   // (several lanes: the list deals evenly)
     int tot = -1;
     if (w.listed && listed.ovf) tot = I.cnt[sc.tt];
@@ -1089,13 +1106,14 @@ __device__ __forceinline__ Window open_window(unsigned char* lds, const IdxList&
                                               int n, const R& rec)
 {
     typedef typename R::V V;
-    Window w{{0, 0, 0, 0, 0}, I.li != nullptr, false, 0, {0, 0, 0, 0}};
+    Window w{{0, 0, 0, 0, 0}, I.li != nullptr, false, false, 0, {0, 0, 0, 0}};
     if (!I.li) return w;
     const int* p = I.win + (size_t)blk * WIN_INTS;
     w.r = window_ranges(p);
     if constexpr (WIN) {
         const int tot = p[6];
-        w.lds = I.lds && tot <= WIN_CAP;
+        w.bad = *I.bad != 0;
+        w.lds = I.lds && tot <= WIN_CAP && !w.bad;
         if (w.lds) {
             const uint32_t o = (uint32_t)sc.sub * n + sc.tt;
             const size_t row = (size_t)n << lg;
@@ -1172,7 +1190,7 @@ __device__ __forceinline__ void visit(unsigned char* lds, const Window& w, const
     // (a window that does not fit: several lanes go through the list at once, as
     // through a window, one lane tests it first: savage column of 2k 3.24 ms for 100
     // steps against 3.39, 250k slope 11.4 against 11.8)
-    if (WIN && (w.lds || lg > 0)) {
+    if (WIN && (w.lds || (lg > 0 && !w.bad))) {
         if (w.lds) visit_window<NCH, double2>(lds, w, I, n, sc, lg, [&](const auto& v) { body(v, rec, 0); });
         // a particle whose list overflowed walks its rows
         int tot = w.lds ? min(w.cnt, 0) : I.cnt[sc.tt];
@@ -1453,6 +1471,7 @@ __device__ __forceinline__ void water_a4(unsigned char* lds, int blk, DPhase W, 
     const size_t nw = (size_t)W.n;
     reinterpret_cast<double*>(WP + 4 * nw)[0] = vofa * (mu * tyy);
     WP[5 * nw] = make_double2(vofa * (mu * txx), vofa * (mu * txy));
+    if (WIN) check_finite(NL.is.bad, txx, txy, tyy);   // (stage B reads them)
 }
 
 template <int SKF, int FORM>

@@ -147,7 +147,7 @@ struct sphg_ctx {
     bool use_side = true;
     hipStream_t lstream = nullptr;   // stream of the next launches when set
     PhaseBuf ph[2];
-    int* d_err = nullptr;       // [0] out of range
+    int* d_err = nullptr;       // [0] out of range, [2] a record of the list mode is not finite
     int* d_scan = nullptr;      // tile sums
     int scan_cap = 0;
     int last_hip = 0;
@@ -1126,7 +1126,7 @@ NRef nref(const sphg_ctx* c, int k, bool rebuild)
 {
     const double hard = 0.5 * c->skin;
     return NRef{c->ph[k].nl_x, c->ph[k].nl_y, c->d_nlflag, 0.25 * c->skin, 0.45 * c->skin, hard * hard,
-                NL_LOOK * c->K.dt, rebuild ? 1 : 0, c->ph[k].nl_cell};
+                NL_LOOK * c->K.dt, rebuild ? 1 : 0, c->ph[k].nl_cell, c->d_err + 2};
 }
 
 // The final kernels a step's stages launch (FP64 list mode): second_half of
@@ -1147,6 +1147,7 @@ NList nlist_of(const sphg_ctx* c, const PhaseBuf& b, bool nl)
         return none;
     }
     NList L{b.nl_same, b.nl_cross, b.nl_cell, b.il_same, b.il_cross, b.lg};
+    L.is.bad = L.ix.bad = c->d_err + 2;
     L.is.lds = c->P.nnps != 2;
     L.ix.lds = 1;
     return L;
@@ -1565,6 +1566,7 @@ int pack_two_phase(sphg_ctx* c, int water_half, int soil_half, int soil_ndp)
         W.cells_valid = false;
         S.cells_valid = false;
         c->since_reorder = 0;
+        RC(fill_int(c, c->d_err + 2, 1, 0));   // (the packs raise it again)
     }
     auto soil_chain = [&]() -> int {
         RC(build_cells(c, 1, nl));
