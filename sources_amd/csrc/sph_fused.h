@@ -631,7 +631,7 @@ struct IdxList {
     int *cnt, *win;
     int cap, lds;   // lds 0: the windows stay in global memory (predicates that need more than a distance)
     int pb;         // particles of a workgroup of the kernels that read it
-    int* bad;       // set: a record is not finite, candidates are tested before their terms
+    int* bad;       // set: a record is not finite, the rows are walked (their terms follow a test)
 };
 
 constexpr int WIN_INTS = 8;
@@ -909,7 +909,7 @@ __global__ __launch_bounds__(256) void k_nlist(const double* xA, const double* y
 // reading the partners there (the next partner's chunks in flight beside the
 // current one's terms); candidates outside the support (about one in six, in
 // the skin) are evaluated with W = s = 0 (once a record holds an infinity or a
-// NaN, which would count so, the candidates are tested first).  What bound the gathers from global
+// NaN, which would count so, the rows are walked instead).  What bound the gathers from global
 // memory was the L1's tag lookups: a 64-lane 16-byte gather of such partners
 // takes 34 of them (one per cycle and CU; 16 for contiguous lanes), where the
 // same LDS read takes about 8 cycles.  The copy itself is contiguous.  What
@@ -983,8 +983,7 @@ __device__ __forceinline__ Ranges3 window_ranges(const int* w)
 struct Window {
     Ranges3 r;
     bool listed, lds;   // a list exists; the window is in LDS (or on its way)
-    bool bad;           // a record is not finite
-    int cnt, k[4];      // lds: the lane's list length and first entries
+    int cnt, k[4];      // the lane's list length (-1: rows) and, lds, its first entries
 };
 
 // The candidates sub, sub + 2^lg, ... of a particle from global memory:
@@ -1000,7 +999,7 @@ __device__ __forceinline__ void visit_global(const Cand& C, const IdxList& I, co
                                              A&& accept, B&& body)
 {
     CatMask kept{0, 0, 1}, listed{0, 0, 1};
-    if (MODE == GIVEN && !w.bad) kept = mask_of(MW, n, sc.tt);   // (bad: stage A may have had its window)
+    if (MODE == GIVEN) kept = mask_of(MW, n, sc.tt);
     if (LM.m && lg == 0) listed = mask_of(LM, n, sc.tt);   // (several lanes: the list deals evenly)
     int tot = -1;
     if (w.listed && listed.ovf) tot = I.cnt[sc.tt];
@@ -1106,18 +1105,19 @@ __device__ __forceinline__ Window open_window(unsigned char* lds, const IdxList&
                                               int n, const R& rec)
 {
     typedef typename R::V V;
-    Window w{{0, 0, 0, 0, 0}, I.li != nullptr, false, false, 0, {0, 0, 0, 0}};
+    Window w{{0, 0, 0, 0, 0}, I.li != nullptr, false, 0, {0, 0, 0, 0}};
     if (!I.li) return w;
     const int* p = I.win + (size_t)blk * WIN_INTS;
     w.r = window_ranges(p);
     if constexpr (WIN) {
         const int tot = p[6];
-        w.bad = *I.bad != 0;
-        w.lds = I.lds && tot <= WIN_CAP && !w.bad;
+        w.lds = I.lds && tot <= WIN_CAP;
+        // (kernels beside this one may raise bad: read once, by lane; w.lds, on which
+        // a barrier depends, is the workgroup's)
+        w.cnt = __hip_atomic_load(I.bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ? -1 : I.cnt[sc.tt];
         if (w.lds) {
             const uint32_t o = (uint32_t)sc.sub * n + sc.tt;
             const size_t row = (size_t)n << lg;
-            w.cnt = I.cnt[sc.tt];
 #pragma unroll
             for (int q = 0; q < 4; ++q) w.k[q] = I.li[q * row + o];
             V* wl = reinterpret_cast<V*>(lds);
@@ -1190,10 +1190,10 @@ __device__ __forceinline__ void visit(unsigned char* lds, const Window& w, const
     // (a window that does not fit: several lanes go through the list at once, as
     // through a window, one lane tests it first: savage column of 2k 3.24 ms for 100
     // steps against 3.39, 250k slope 11.4 against 11.8)
-    if (WIN && (w.lds || (lg > 0 && !w.bad))) {
+    if (WIN && (w.lds || lg > 0)) {
         if (w.lds) visit_window<NCH, double2>(lds, w, I, n, sc, lg, [&](const auto& v) { body(v, rec, 0); });
         // a particle whose list overflowed walks its rows
-        int tot = w.lds ? min(w.cnt, 0) : I.cnt[sc.tt];
+        int tot = w.lds ? min(w.cnt, 0) : w.cnt;
         const bool walk = tot < 0;
         Ranges3 rows = w.r;
         if (walk) rows = C.rows(sc.tt, tot);

@@ -483,10 +483,7 @@ __device__ __forceinline__ void water_b_mx(unsigned char* lds, int blk, DPhase W
     Sum64 Px, Py, Sxx, Sxyy, Sxyx, Syy, artx, arty, dvd;
     visit_mx<WIN, 4>(lds, win, NL.is, W.n, wc, t, QWv, X.thr_w,
                 [&] { return rows_of_cell(g, W.cell_start, me.cx, me.cy); },
-                [&](const LaneRows& R) {
-                    // (bad: stage A may have had its window)
-                    return win.bad ? cand_mask_f(R, NL.same, W.n, wc.tt, t, QWv, acc_q) : mask_of(MW, W.n, t);
-                }, acc_q, [&](const auto& v, float lim) {
+                [&](const LaneRows&) { return mask_of(MW, W.n, t); }, acc_q, [&](const auto& v, float lim) {
         const float4 b0 = v[0], b1 = v[1], b2 = v[2], b3 = v[3];
         float dx, dy;
         sep(me, b0, X.cs, dx, dy);
