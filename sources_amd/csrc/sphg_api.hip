@@ -469,7 +469,8 @@ int await_post(sphg_ctx* c, const int* slot, int seq, int* flag)
     for (unsigned spin = 1;; ++spin) {
         const bool done = spin % 8192 == 0 && [&] {
             const hipError_t e = hipStreamQuery(c->stream);
-            if (e != hipSuccess) (void)hipGetLastError();   // (not ready, or reported by the next check)
+            if (e != hipSuccess) (void)hipGetLastError();   // (not ready, or kept here)
+            if (e != hipSuccess && e != hipErrorNotReady) c->last_hip = (int)e;
             return e != hipErrorNotReady;
         }();
         const unsigned v = (unsigned)__atomic_load_n(slot, __ATOMIC_ACQUIRE);
@@ -1811,12 +1812,8 @@ int one_step(sphg_ctx* c, bool ahead_ok = false)
 int verlet_steps(sphg_ctx* c, int nsteps)
 {
     PhaseBuf& W = c->ph[0];
-    if (!W.lvx) {
-        RC(dalloc(c, W, &W.lvx, (size_t)W.n));
-        RC(dalloc(c, W, &W.lvy, (size_t)W.n));
-        RC(dalloc(c, W, &W.lrho, (size_t)W.n));
-        for (double** p : {&W.lshadow[0], &W.lshadow[1], &W.lshadow[2]}) RC(dalloc(c, W, p, (size_t)W.n));
-    }
+    for (double** p : {&W.lvx, &W.lvy, &W.lrho, &W.lshadow[0], &W.lshadow[1], &W.lshadow[2]})
+        if (!*p) RC(dalloc(c, W, p, (size_t)W.n));   // (each by itself: a call before may have run out of memory)
     RC(launch(c, "verlet", k_copy<double>, nblk(W.n), TPB, (const double*)W.d.vx, W.lvx, W.n));
     RC(launch(c, "verlet", k_copy<double>, nblk(W.n), TPB, (const double*)W.d.vy, W.lvy, W.n));
     RC(launch(c, "verlet", k_copy<double>, nblk(W.n), TPB, (const double*)W.d.rho, W.lrho, W.n));
