@@ -631,6 +631,7 @@ struct IdxList {
     int *cnt, *win;
     int cap, lds;   // lds 0: the windows stay in global memory (predicates that need more than a distance)
     int pb;         // particles of a workgroup of the kernels that read it
+    int crowd;      // the list of a crowded particle (mask overflow) counts as overflowed
     int* bad;       // set: a record is not finite, the rows are walked (their terms follow a test)
 };
 
@@ -891,7 +892,7 @@ __device__ __forceinline__ void nlist_body(int blk, const double* xA, const doub
     VM.m[t] = cm.lo;
     VM.m[nA + t] = cm.hi;
     VM.ovf[t] = cm.ovf;
-    IL.cnt[t] = cnt <= IL.cap && tot < 65536 ? cnt : -1;
+    IL.cnt[t] = cnt <= IL.cap && tot < 65536 && !(IL.crowd && cm.ovf) ? cnt : -1;
 }
 
 __global__ __launch_bounds__(256) void k_nlist(const double* xA, const double* yA, const int* ordA, int nA,

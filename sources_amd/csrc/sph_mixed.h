@@ -120,6 +120,14 @@ __device__ __forceinline__ int inside(float dr, float lim, float& w, float& gx, 
     return in ? 1 : 0;
 }
 
+// u . d of art_visc (negative for an approaching pair).  The contraction is written
+// out, so that it is the same in every kernel: a crowded particle takes the other one.
+__device__ __forceinline__ float approach(float ux, float uy, float dx, float dy, bool crowded)
+{
+    const float x = ux * dx, y = uy * dy;
+    return crowded ? fmaf(ux, dx, y) : fmaf(uy, dy, x);
+}
+
 // Mixed-precision constants of a step.
 struct MixK {
     float cs;                  // cell size
@@ -162,6 +170,19 @@ __device__ __forceinline__ void sep(const SelfF& a, float4 b0, float cs, float& 
     dx = (a.x - b0.x) + (float)(a.cx - tag_cx(tb)) * cs;
     dy = (a.y - b0.y) + (float)(a.cy - tag_cy(tb)) * cs;
 }
+
+// Crowded: more than 64 candidates in a row of cells or more than 128 in all
+// (the rebuild's mask says so, without lists the particle's rows).
+template <class L>
+__device__ __forceinline__ bool crowded(const Masks& M, int tt, L&& rows)
+{
+    if (M.m) return M.ovf[tt] != 0;
+    const LaneRows R = rows();
+    return ovf_of(R) || R.k1[0] - R.k0[0] + R.k1[1] - R.k0[1] + R.k1[2] - R.k0[2] > 128;
+}
+
+// Whether crowded particles keep their lists: with the radius-3h kernels most are.
+__host__ __device__ constexpr bool mx_lists_crowded(int skf) { return skf == 2 || skf == 3; }
 
 // Scan of one candidate row (FP32 predicate).
 template <class P>
@@ -269,29 +290,38 @@ __device__ __forceinline__ CatMask cand_mask_f(const LaneRows& L, const Masks& M
 // FP64, and pays for the candidates in the skin (150 -> 166).  us per step, masks
 // -> windows: slope of 3k 56 -> 42, 33k 57 -> 46, 64k 61 -> 52, 1M 419 -> 400;
 // column of 33k 56 -> 43, 64k 60 -> 47 (below 1M 5 of these from the posted flag).
-// body(v, lim): record chunks v and the squared distance it has yet to be within;
-// mask(R): the partner mask over the rows R = rows().
-template <bool WIN, int NCH, class L, class M, class A, class B>
+// body(v, lim, other): record chunks v, the squared distance it has yet to be within
+// and the particle's contraction (approach); mask(R): the partner mask over the rows
+// R = rows(); many(): it is crowded.  SEL: crowded particles have lists too (else the
+// rebuild gives theirs as overflowed, which spares the windows' pairs a select).
+struct NotCrowded {
+    __device__ __forceinline__ bool operator()() const { return false; }
+};
+
+template <bool WIN, int NCH, bool SEL = false, class L, class M, class A, class B, class Q = NotCrowded>
 __device__ __forceinline__ void visit_mx(unsigned char* lds, const Window& w, const IdxList& I, int n,
                                          const SubCtx& sc, int self, const RecQ& rec, float thr, L&& rows,
-                                         M&& mask, A&& accept, B&& body)
+                                         M&& mask, A&& accept, B&& body, const Q& many = Q{})
 {
+    bool other = SEL ? many() : false;
     auto global = [&](int k) {
         float4 v[NCH];
 #pragma unroll
         for (int c = 0; c < NCH; ++c) v[c] = rec(k, c);
-        body(v, INFINITY);
+        body(v, INFINITY, other);
     };
     if (WIN && w.lds) {
-        visit_window<NCH, float4>(lds, w, I, n, sc, 0, [&](const auto& v) { body(v, thr); });
+        visit_window<NCH, float4>(lds, w, I, n, sc, 0, [&](const auto& v) { body(v, thr, SEL && other); });
         if (w.cnt < 0 && sc.valid) {   // a list that overflowed
             const LaneRows R = rows();
+            if (!SEL) other = many();
             visit_f(CatMask{0, 0, 7}, R, self, [&](int k) { return accept(rec(k, 0)); }, global);
         }
         return;
     }
     if (!sc.valid) return;
     const LaneRows R = rows();
+    if (!SEL) other = many();
     visit_f(mask(R), R, self, [&](int k) { return accept(rec(k, 0)); }, global);
 }
 
@@ -338,7 +368,7 @@ __device__ __forceinline__ void water_a_mx(unsigned char* lds, int blk, DPhase W
             visit_mx<WIN, 3>(lds, win, NL.ix, W.n, wc, -1, QSv, X.thr_x,
                         [&] { return rows_of_cell(g, S.cell_start, me.cx, me.cy); },
                         [&](const LaneRows& R) { return cand_mask_f(R, NL.cross, W.n, wc.tt, -1, QSv, accx_q); },
-                        accx_q, [&](const auto& v, float lim) {
+                        accx_q, [&](const auto& v, float lim, bool other) {
                 const float4 b0 = v[0], b1 = v[1], b2 = v[2];
                 float dx, dy;
                 sep(me, b0, X.cs, dx, dy);
@@ -388,7 +418,7 @@ __device__ __forceinline__ void water_a_mx(unsigned char* lds, int blk, DPhase W
     };
     visit_mx<WIN, 2>(lds, win, NL.is, W.n, wc, t, QWv, X.thr_w,
                 [&] { return rows_of_cell(g, W.cell_start, me.cx, me.cy); }, mask_a, acc_q,
-                [&](const auto& v, float lim) {
+                [&](const auto& v, float lim, bool other) {
         const float4 b0 = v[0], b1 = v[1];   // 1/rho and m/rho recomputed: two chunks per partner
         float dx, dy;
         sep(me, b0, X.cs, dx, dy);
@@ -477,13 +507,15 @@ __device__ __forceinline__ void water_b_mx(unsigned char* lds, int blk, DPhase W
         sep(me, b0, X.cs, dx, dy);
         return pred_f(uni, X.thr_w, dx * dx + dy * dy, me.h, b0.w, X.scale_k);
     };
+    constexpr bool SEL = mx_lists_crowded(SKF);
+    auto many = [&] { return crowded(NL.same, wc.tt, [&] { return rows_of_cell(g, W.cell_start, me.cx, me.cy); }); };
     const Window win = open_window<WIN, 4>(lds, NL.is, blk, wc, 0, W.n, QWv);
     const float et2 = (float)(K.etq * K.etq);
     const float beta = (float)K.beta, alpha = (float)K.alpha;
     Sum64 Px, Py, Sxx, Sxyy, Sxyx, Syy, artx, arty, dvd;
-    visit_mx<WIN, 4>(lds, win, NL.is, W.n, wc, t, QWv, X.thr_w,
+    visit_mx<WIN, 4, SEL>(lds, win, NL.is, W.n, wc, t, QWv, X.thr_w,
                 [&] { return rows_of_cell(g, W.cell_start, me.cx, me.cy); },
-                [&](const LaneRows&) { return mask_of(MW, W.n, t); }, acc_q, [&](const auto& v, float lim) {
+                [&](const LaneRows&) { return mask_of(MW, W.n, t); }, acc_q, [&](const auto& v, float lim, bool other) {
         const float4 b0 = v[0], b1 = v[1], b2 = v[2], b3 = v[3];
         float dx, dy;
         sep(me, b0, X.cs, dx, dy);
@@ -504,7 +536,7 @@ __device__ __forceinline__ void water_b_mx(unsigned char* lds, int blk, DPhase W
         Sxyy.add(Vb * (sxy * gy));
         Sxyx.add(Vb * (sxy * gx));
         Syy.add(Vb * ((fyy_a + b3.w) * gy));
-        const float vr = (vxa - b1.x) * dx + (vya - b1.y) * dy;
+        const float vr = approach(vxa - b1.x, vya - b1.y, dx, dy, other);
         const float muv = amh * vr * __builtin_amdgcn_rcpf(dr + amh * amh * et2);
         const float mc = 0.5f * (ca + b3.x);
         float piv = (beta * muv - alpha * mc) * muv * (2.0f * __builtin_amdgcn_rcpf(rhoa + b1.z + X.rho0_w));
@@ -512,7 +544,7 @@ __device__ __forceinline__ void water_b_mx(unsigned char* lds, int blk, DPhase W
         artx.add(-(mb * piv * gx));
         arty.add(-(mb * piv * gy));
         dvd.add(mb * (2.0f * (vofa - b2.x) * idr * (dx * gx + dy * gy)) * b2.y);
-    });
+    }, many);
     if (!wc.valid) return;
     const double vofa_d = W.vof[a], rhoa_d = W.rho[a], ha_d = W.hsml[a], ca_d = W.c[a];   // new c
     double ax = -(vofa_d * Px.value()) + Sxx.value() + Sxyy.value();
@@ -591,7 +623,7 @@ __device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S
         visit_mx<WIN, 3>(lds, win, NL.ix, S.n, wc, -1, QWv, X.thr_x,
                     [&] { return rows_of_cell(g, W.cell_start, me.cx, me.cy); },
                     [&](const LaneRows& R) { return cand_mask_f(R, NL.cross, S.n, wc.tt, -1, QWv, accx_q); }, accx_q,
-                    [&](const auto& v, float lim) {
+                    [&](const auto& v, float lim, bool other) {
             const float4 b0 = v[0], b1 = v[1], b2 = v[2];
             float dx, dy;
             sep(me, b0, X.cs, dx, dy);
@@ -631,6 +663,8 @@ __device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S
         sep(me, b0, X.cs, dx, dy);
         return pred_f(uni, X.thr_s, dx * dx + dy * dy, me.h, b0.w, X.scale_k);
     };
+    constexpr bool SEL = mx_lists_crowded(SKF);
+    auto many = [&] { return crowded(NL.same, wc.tt, [&] { return rows_of_cell(g, S.cell_start, me.cx, me.cy); }); };
     const Window win = open_window<WIN, 4>(lds, NL.is, blk, wc, 0, S.n, QSv);
     const float et2 = (float)(K.etq * K.etq);
     const float beta = (float)K.beta, alpha = (float)K.alpha;
@@ -638,10 +672,10 @@ __device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S
     Sum64 Fx, Fy, artx, arty, dP, dXX, dXY, dYY;
     float repx = 0.0f, repy = 0.0f;
     int cnt = 0;
-    visit_mx<WIN, 4>(lds, win, NL.is, S.n, wc, t, QSv, X.thr_s,
+    visit_mx<WIN, 4, SEL>(lds, win, NL.is, S.n, wc, t, QSv, X.thr_s,
                 [&] { return rows_of_cell(g, S.cell_start, me.cx, me.cy); },
                 [&](const LaneRows& R) { return cand_mask_f(R, NL.same, S.n, wc.tt, t, QSv, acc_q); }, acc_q,
-                [&](const auto& v, float lim) {
+                [&](const auto& v, float lim, bool other) {
         const float4 b0 = v[0], b1 = v[1], b2 = v[2], b3 = v[3];
         float dx, dy;
         sep(me, b0, X.cs, dx, dy);
@@ -682,7 +716,7 @@ __device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S
         const float fyy = fyya + vofb * b3.w * ir2b;
         Fx.add(mb * ((fxx - fp) * gx + fxy * gy));
         Fy.add(mb * ((fyy - fp) * gy + fxy * gx));
-        const float vr = dvx * dx + dvy * dy;
+        const float vr = approach(dvx, dvy, dx, dy, other);
         const float muv = amh * vr * __builtin_amdgcn_rcpf(dr + amh * amh * et2);
         float piv = (beta * muv - alpha * cn) * muv * rs;
         piv = vr < 0.0f ? piv : 0.0f;
@@ -693,7 +727,7 @@ __device__ __forceinline__ void soil_ab_mx(unsigned char* lds, int blk, DPhase S
         dXX.add(hh * (sxxa - b3.y));
         dXY.add(hh * (sxya - b3.z));
         dYY.add(hh * (syya - b3.w));
-    });
+    }, many);
     if (!wc.valid) return;
     const double ha_d = S.hsml[a], ca_d = S.c[a], rhoa_d = S.rho[a];
     const double txx_d = txx.value() * SPH_C23_F, tyy_d = tyy.value() * SPH_C23_F, txy_d = txy.value();

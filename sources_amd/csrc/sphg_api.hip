@@ -1497,6 +1497,8 @@ int build_nlists(sphg_ctx* c)
     groups(S.il_same, c->P.nnps != 2 && (mx ? all : u.s), S.lg);
     groups(W.il_cross, u.x, W.lg);
     groups(S.il_cross, u.x, S.lg);
+    // (also in the plain steps of a learned run of a mixed context)
+    W.il_same.crowd = S.il_same.crowd = (mx || c->K.learned) && !mx_lists_crowded(c->P.skf);
     // the displacement trigger restarts (a past-the-skin bit stays for the check);
     // the rebuild has just permuted the state into cell order (no order lookups)
     RC(launch(c, "nlist", k_keep_bits, 1, TPB, c->d_nlflag, 2));
