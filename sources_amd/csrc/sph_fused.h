@@ -611,7 +611,7 @@ struct Masks {
 };
 
 // ------------------------------------------------------------------------
-// Neighbour lists with a skin (FP64 fused step).  At a rebuild the cell
+// Neighbour lists with a skin (fused step).  At a rebuild the cell
 // list is built on a grid of cell size >= R + skin (R the largest support
 // radius), the records are written in its order, and every particle keeps
 // (a) the key of its cell, (b) the candidates within R + skin (same phase and
@@ -639,18 +639,18 @@ constexpr int WIN_INTS = 8;
 constexpr int WIN_CAP = 846;             // records of a window in LDS: two workgroups' six chunks fill a CU's
 constexpr int WIN_STRIDE = WIN_CAP + 1;  // (and the stand-in record)
 // Lanes of a workgroup that take particles where its window is to fit the LDS (all
-// of them otherwise).  The window holds three rows' worth
-// of them: 633 records on average (848 at most) for 192 particles of a
-// lattice at h = 1.2 dx (whose cell rows hold two or three lattice rows); with
-// 240 particles one window in four does not fit, and its workgroup takes the
-// slow path at the occupancy the LDS leaves (1M slope, soil_ab 117 us against
-// 102, water_b 72 against 55).
+// of them otherwise).  The window holds three rows' worth of them: 633 records on
+// average (848 at most, and that workgroup reads by lane) for 192 particles of a
+// lattice at h = 1.2 dx (whose cell rows hold two or three lattice rows); with 240
+// particles one window in four does not fit, and its workgroup takes the slow path
+// at the occupancy the LDS leaves (1M slope, soil_ab 117 us against 102, water_b 72
+// against 55).
 constexpr int WIN_LANES = 192;
 
 struct NList {
     Masks same, cross;   // candidates within R + skin: same phase, other phase
     const int* cell;     // [n] key of the particle's cell at the rebuild (record order)
-    IdxList is, ix;      // the candidates as indices (FP64 stages): same phase, other phase
+    IdxList is, ix;      // the candidates as indices: same phase, other phase
     int lg;
 };
 

@@ -286,8 +286,8 @@ __device__ __forceinline__ CatMask cand_mask_f(const LaneRows& L, const Masks& M
 // (or where the window does not fit) it goes through its partner mask, reading
 // the records from global memory.
 // Stage 1 was bound by the gathers of the partners' records (1M slope, us per
-// launch: 140 -> 105); stage 2 is bound by its FP32 terms and their sums in
-// FP64, and pays for the candidates in the skin (150 -> 166).  us per step, masks
+// launch: 140 -> 112); stage 2 is bound by its FP32 terms and their sums in
+// FP64, and pays for the candidates in the skin (150 -> 168).  us per step, masks
 // -> windows: slope of 3k 56 -> 42, 33k 57 -> 46, 64k 61 -> 52, 1M 419 -> 400;
 // column of 33k 56 -> 43, 64k 60 -> 47 (below 1M 5 of these from the posted flag).
 // body(v, lim, other): record chunks v, the squared distance it has yet to be within
